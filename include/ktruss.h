@@ -107,7 +107,7 @@ int kt_solve_tsv(kt_context* ctx, const char* path, kt_result* res, double* pars
 int kt_parse_tsv_device(kt_context* ctx, const char* path, uint32_t* xs, uint32_t* ys, uint64_t cap,
                         uint64_t* lines, uint32_t* n, int* on_device);
 
-/* Survivors of the last solve: original ids, u < v, unordered.
+/* Survivors of the last solve: original ids, u < v, sorted by (u, v).
  * *count receives the truss size; at most cap pairs are written. */
 int kt_truss_edges(kt_context* ctx, uint32_t* pairs, uint64_t cap, uint64_t* count);
 
@@ -115,7 +115,7 @@ int kt_truss_edges(kt_context* ctx, uint32_t* pairs, uint64_t cap, uint64_t* cou
  * reference, which reports kmax and |T| only): a
  * full truss decomposition on the device, then (u, v, t) triples, u < v in
  * original ids, for every edge of trussness t >= 3 (every other edge has
- * trussness 2), unordered. *count receives how many; at most cap triples
+ * trussness 2), sorted by (u, v). *count receives how many; at most cap triples
  * are written. The decomposition runs once per input graph: a second call
  * (e.g. with a buffer sized by the first call's count) only copies. The last
  * solve's kmax-truss stays available to kt_truss_edges; kt_last_stats fails

@@ -312,11 +312,10 @@ class Context:
         sorted by (u, v)."""
         cnt = _U64()
         _check(self._lib.kt_truss_edges(self._h, None, 0, ctypes.byref(cnt)))
-        out = np.zeros((max(cnt.value, 1), 2), dtype=np.uint32)
-        _check(self._lib.kt_truss_edges(self._h, out.ctypes.data, cnt.value, ctypes.byref(cnt)))
-        out = out[: cnt.value]
-        order = np.lexsort((out[:, 1], out[:, 0]))
-        return out[order]
+        out = np.empty((cnt.value, 2), dtype=np.uint32)
+        if cnt.value:
+            _check(self._lib.kt_truss_edges(self._h, out.ctypes.data, cnt.value, ctypes.byref(cnt)))
+        return out
 
     def push_probe(self, mode: int) -> None:
         """Measurement of the vertex-peel push kernel: 1 stamps events at
@@ -341,10 +340,10 @@ class Context:
         returns the last solve's kmax-truss afterwards."""
         cnt = _U64()
         _check(self._lib.kt_trussness(self._h, None, 0, ctypes.byref(cnt)))
-        out = np.zeros((max(cnt.value, 1), 3), dtype=np.uint32)
-        _check(self._lib.kt_trussness(self._h, out.ctypes.data, cnt.value, ctypes.byref(cnt)))
-        out = out[: cnt.value]
-        return out[np.lexsort((out[:, 1], out[:, 0]))]
+        out = np.empty((cnt.value, 3), dtype=np.uint32)
+        if cnt.value:
+            _check(self._lib.kt_trussness(self._h, out.ctypes.data, cnt.value, ctypes.byref(cnt)))
+        return out
 
     def stats(self) -> KtStats:
         """Byte-model terms W(C+), W(C+ minus T+) of the last solve."""

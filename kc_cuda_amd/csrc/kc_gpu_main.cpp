@@ -8,7 +8,6 @@
 //              sorted by (u, v)
 //   -t <path>  per-edge trussness, "u\tv\tt" for every edge with t >= 3,
 //              sorted by (u, v); edges not listed have trussness 2
-#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -23,19 +22,13 @@ int usage() {
   return 1;
 }
 
-bool write_rows(const char* path, std::vector<uint32_t>& rows, int width) {
+// rows come sorted from the library
+bool write_rows(const char* path, const std::vector<uint32_t>& rows, int width) {
   const size_t count = rows.size() / width;
-  std::vector<size_t> order(count);
-  for (size_t i = 0; i < count; ++i) order[i] = i;
-  std::sort(order.begin(), order.end(), [&](size_t a, size_t b) {
-    const uint32_t* x = &rows[a * width];
-    const uint32_t* y = &rows[b * width];
-    return x[0] != y[0] ? x[0] < y[0] : x[1] < y[1];
-  });
   FILE* f = std::fopen(path, "w");
   if (!f) return false;
   bool ok = true;
-  for (size_t i : order) {
+  for (size_t i = 0; i < count; ++i) {
     const uint32_t* r = &rows[i * width];
     const int w = width == 2 ? std::fprintf(f, "%u\t%u\n", r[0], r[1]) : std::fprintf(f, "%u\t%u\t%u\n", r[0], r[1], r[2]);
     if (w < 0) {

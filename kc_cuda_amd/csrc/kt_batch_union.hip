@@ -129,21 +129,22 @@ __global__ __launch_bounds__(kBlock) void k_batch_results(const uint32_t* __rest
   }
 }
 
-// (u, v, t), u < v input ids, for every core edge of truss number t >= 3
-__global__ __launch_bounds__(kBlock) void k_truss_triples(const uint32_t* __restrict__ src0,
-                                                          const uint32_t* __restrict__ dst0,
-                                                          const uint32_t* __restrict__ inv,
-                                                          const uint32_t* __restrict__ del_thr, uint32_t mc0,
-                                                          uint32_t kall, uint32_t* out, uint32_t* count) {
-  for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < mc0; e += gridDim.x * blockDim.x) {
-    const uint32_t t = truss_of(del_thr, e, kall);
-    if (t < 3) continue;
-    const uint32_t a = inv[src0[e]], b = inv[dst0[e]];
-    const uint32_t at = atomicAdd(count, 1u);
-    out[3 * uint64_t(at)] = min(a, b);
-    out[3 * uint64_t(at) + 1] = max(a, b);
-    out[3 * uint64_t(at) + 2] = t;
-  }
+// every core edge of truss number t >= 3 as a sort key u << id_bits | v
+// (u < v input ids) with its t, in no order
+__global__ __launch_bounds__(kBlock) void k_truss_keys(const uint32_t* __restrict__ src0,
+                                                       const uint32_t* __restrict__ dst0,
+                                                       const uint32_t* __restrict__ inv,
+                                                       const uint32_t* __restrict__ del_thr, uint32_t mc0,
+                                                       uint32_t kall, uint32_t id_bits, uint64_t* keys, uint32_t* ts,
+                                                       uint32_t* count) {
+  tile_compact(
+      mc0, [&](uint64_t e) { return truss_of(del_thr, uint32_t(e), kall) >= 3; },
+      [&](uint32_t at, uint64_t e) {
+        const uint32_t a = inv[src0[e]], b = inv[dst0[e]];
+        keys[at] = uint64_t(min(a, b)) << id_bits | max(a, b);
+        ts[at] = truss_of(del_thr, uint32_t(e), kall);
+      },
+      count);
 }
 
 __global__ void k_fill_u8(uint8_t* p, uint64_t n, uint8_t v) {
@@ -178,10 +179,11 @@ void batch_results(const uint32_t* gk, const unsigned long long* gcnt, const uin
   if (count) k_batch_results<<<grid_for(count), kBlock, 0, s>>>(gk, gcnt, status, count, kmax, edges, status_out);
 }
 
-void truss_triples(const CoreView& cv, uint32_t kall, uint32_t* out, uint32_t* count, hipStream_t s) {
+void truss_keys(const CoreView& cv, uint32_t kall, uint32_t id_bits, uint64_t* keys, uint32_t* ts, uint32_t* count,
+                hipStream_t s) {
   if (cv.mc0)
-    k_truss_triples<<<grid_for(cv.mc0), kBlock, 0, s>>>(cv.src0, cv.adj_d0, cv.inv, cv.del_thr, cv.mc0, kall, out,
-                                                        count);
+    k_truss_keys<<<grid_tiles(cv.mc0), kBlock, 0, s>>>(cv.src0, cv.adj_d0, cv.inv, cv.del_thr, cv.mc0, kall, id_bits,
+                                                       keys, ts, count);
 }
 
 void fill_u8(uint8_t* p, uint64_t n, uint8_t v, hipStream_t s) {

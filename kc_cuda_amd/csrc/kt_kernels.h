@@ -222,7 +222,14 @@ void row_compact(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* o
                  uint32_t* adj2, uint32_t* src2, uint32_t* orig2, int32_t* sup2, hipStream_t s);
 void count_in_degrees(const uint32_t* adj, uint32_t m, uint32_t* din, hipStream_t s);
 void truss_pairs(const uint32_t* del_thr, uint32_t m0, int32_t floor, const uint32_t* src0,
-                 const uint32_t* dst0, const uint32_t* inv, uint32_t* out, uint32_t* count,
+                 const uint32_t* dst0, const uint32_t* inv, uint32_t id_bits, uint32_t cap, void* out,
+                 uint32_t* count, hipStream_t s);
+// rows (u, v) -- or (u, v, vals[i]) -- of keys u << id_bits | v: sorted ones,
+// and at most kRowSortCap in any order, whose rows come out sorted
+constexpr uint32_t kRowSortCap = 4096;
+void sort_unpack_rows(const uint64_t* keys, const uint32_t* vals, uint32_t n, uint32_t id_bits, uint32_t* out,
+                      hipStream_t s);
+void unpack_rows(const uint64_t* keys, const uint32_t* vals, uint32_t n, uint32_t id_bits, uint32_t* out,
                  hipStream_t s);
 
 }  // namespace kt

@@ -1757,25 +1757,85 @@ __global__ void k_count_din(const uint32_t* __restrict__ adj, uint32_t m, uint32
     atomicAdd(&din[adj[i]], 1u);
 }
 
-// Survivors of the level with threshold `floor` among the base edges.
-__global__ void k_truss_pairs(const uint32_t* __restrict__ del_thr, uint32_t m0, int32_t floor,
-                              const uint32_t* __restrict__ src0, const uint32_t* __restrict__ dst0,
-                              const uint32_t* __restrict__ inv, uint2* out, uint32_t* count) {
-  for (uint64_t base = uint64_t(blockIdx.x) * blockDim.x; base < m0;
-       base += uint64_t(gridDim.x) * blockDim.x) {
-    const uint64_t e = base + threadIdx.x;
-    bool p = false;
-    uint2 pr = make_uint2(0, 0);
-    if (e < m0) {
-      const uint32_t d = del_thr[e];
-      p = (d == kNone) || (int64_t(d) > int64_t(floor));
-      if (p) {
+// Survivors of the level with threshold `floor` among the base edges, in no
+// order: (u, v) pairs (id_bits 0), or sort keys u << id_bits | v. At most cap
+// are written; *count receives their number.
+__global__ __launch_bounds__(kBlock) void k_truss_pairs(const uint32_t* __restrict__ del_thr, uint32_t m0,
+                                                        int32_t floor, const uint32_t* __restrict__ src0,
+                                                        const uint32_t* __restrict__ dst0,
+                                                        const uint32_t* __restrict__ inv, uint32_t id_bits,
+                                                        uint32_t cap, void* out, uint32_t* count) {
+  tile_compact(
+      m0,
+      [&](uint64_t e) {
+        const uint32_t d = del_thr[e];
+        return d == kNone || int64_t(d) > int64_t(floor);
+      },
+      [&](uint32_t at, uint64_t e) {
+        if (at >= cap) return;
         const uint32_t a = inv[src0[e]], b = inv[dst0[e]];
-        pr = make_uint2(min(a, b), max(a, b));
-      }
-    }
-    wave_append<uint2>(p, pr, out, count);
+        const uint32_t u = min(a, b), v = max(a, b);
+        if (id_bits)
+          static_cast<uint64_t*>(out)[at] = uint64_t(u) << id_bits | v;
+        else
+          static_cast<uint2*>(out)[at] = make_uint2(u, v);
+      },
+      count);
+}
+
+// Sorted key u << id_bits | v back to row i: (u, v), or (u, v, *val).
+__device__ __forceinline__ void unpack_row(uint64_t key, const uint32_t* val, uint64_t i, uint32_t id_bits,
+                                           uint32_t* __restrict__ out) {
+  const uint32_t u = uint32_t(key >> id_bits), v = uint32_t(key & ((uint64_t(1) << id_bits) - 1));
+  if (val) {
+    out[3 * i] = u;
+    out[3 * i + 1] = v;
+    out[3 * i + 2] = *val;
+  } else {
+    reinterpret_cast<uint2*>(out)[i] = make_uint2(u, v);
   }
+}
+
+__global__ __launch_bounds__(kBlock) void k_unpack_rows(const uint64_t* __restrict__ keys,
+                                                        const uint32_t* __restrict__ vals, uint32_t n,
+                                                        uint32_t id_bits, uint32_t* __restrict__ out) {
+  for (uint64_t i = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; i < n; i += uint64_t(gridDim.x) * blockDim.x)
+    unpack_row(keys[i], vals ? &vals[i] : nullptr, i, id_bits, out);
+}
+
+// Up to kRowSortCap rows sorted and unpacked by one workgroup (a bitonic
+// network in LDS): a small edge set pays one launch instead of the radix
+// sort's several and the unpacking.
+constexpr uint32_t kRowSortBlock = 1024;
+__global__ __launch_bounds__(kRowSortBlock) void k_sort_unpack_rows(const uint64_t* __restrict__ keys,
+                                                                    const uint32_t* __restrict__ vals, uint32_t n,
+                                                                    uint32_t id_bits, uint32_t* __restrict__ out) {
+  __shared__ uint64_t s_key[kRowSortCap];
+  __shared__ uint32_t s_val[kRowSortCap];
+  uint32_t P = 2;
+  while (P < n) P <<= 1;
+  for (uint32_t i = threadIdx.x; i < P; i += kRowSortBlock) {
+    s_key[i] = i < n ? keys[i] : ~uint64_t(0);
+    s_val[i] = vals && i < n ? vals[i] : 0u;
+  }
+  __syncthreads();
+  for (uint32_t size = 2; size <= P; size <<= 1)
+    for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+      for (uint32_t t = threadIdx.x; t < P / 2; t += kRowSortBlock) {
+        const uint32_t lo = 2 * t - (t & (stride - 1)), hi = lo + stride;
+        const uint64_t a = s_key[lo], b = s_key[hi];
+        if ((a > b) == ((lo & size) == 0)) {
+          s_key[lo] = b;
+          s_key[hi] = a;
+          const uint32_t x = s_val[lo];
+          s_val[lo] = s_val[hi];
+          s_val[hi] = x;
+        }
+      }
+      __syncthreads();
+    }
+  for (uint32_t i = threadIdx.x; i < n; i += kRowSortBlock)
+    unpack_row(s_key[i], vals ? &s_val[i] : nullptr, i, id_bits, out);
 }
 
 // Byte-model terms of the last core: W(C+) = sum over oriented edges of
@@ -1869,10 +1929,19 @@ void count_in_degrees(const uint32_t* adj, uint32_t m, uint32_t* din, hipStream_
   if (m) k_count_din<<<grid_for(m), kBlock, 0, s>>>(adj, m, din);
 }
 void truss_pairs(const uint32_t* del_thr, uint32_t m0, int32_t floor, const uint32_t* src0,
-                 const uint32_t* dst0, const uint32_t* inv, uint32_t* out, uint32_t* count, hipStream_t s) {
+                 const uint32_t* dst0, const uint32_t* inv, uint32_t id_bits, uint32_t cap, void* out,
+                 uint32_t* count, hipStream_t s) {
   if (m0)
-    k_truss_pairs<<<grid_for(m0), kBlock, 0, s>>>(del_thr, m0, floor, src0, dst0, inv,
-                                                 reinterpret_cast<uint2*>(out), count);
+    k_truss_pairs<<<grid_tiles(m0), kBlock, 0, s>>>(del_thr, m0, floor, src0, dst0, inv, id_bits, cap, out, count);
+}
+void sort_unpack_rows(const uint64_t* keys, const uint32_t* vals, uint32_t n, uint32_t id_bits, uint32_t* out,
+                      hipStream_t s) {
+  if (n > kRowSortCap) fail("sort_unpack_rows: more rows than one workgroup holds");
+  if (n) k_sort_unpack_rows<<<1, kRowSortBlock, 0, s>>>(keys, vals, n, id_bits, out);
+}
+void unpack_rows(const uint64_t* keys, const uint32_t* vals, uint32_t n, uint32_t id_bits, uint32_t* out,
+                 hipStream_t s) {
+  if (n) k_unpack_rows<<<grid_for(n), kBlock, 0, s>>>(keys, vals, n, id_bits, out);
 }
 
 void fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s) {

@@ -89,6 +89,7 @@ uint64_t noalloc_solve_pairs(int device, const uint32_t* d_pairs, uint64_t m, ui
   uint64_t count = res->truss_edges;
   if (d_truss) count = s.truss_edges_to_device(d_truss, cap);
   KT_HIP(hipStreamSynchronize(s.stream()));
+  if (d_truss) s.check_truss_count();
   return count;
 }
 

@@ -141,13 +141,18 @@ class Solver {
   // Directed line list (x into row y) resident on the device.
   void solve_lines_device(const uint32_t* d_xs, const uint32_t* d_ys, uint64_t L, uint32_t n,
                           kt_result* res);
-  // Copies the survivors of the last solve (original ids, u < v) to host.
+  // Copies the survivors of the last solve (original ids, u < v, sorted by
+  // (u, v)) to host.
   uint64_t truss_edges(uint32_t* host_pairs, uint64_t cap);
-  // The same into device memory (queued on the solver's stream, not waited for).
+  // The same into device memory (queued on the solver's stream, not waited
+  // for); in arena mode in no order.
   uint64_t truss_edges_to_device(uint32_t* dev_pairs, uint64_t cap);
+  // After the stream has drained: fails when the number of edges written
+  // is not the last solve's |T|.
+  void check_truss_count();
   // Truss decomposition of the last input graph: (u, v, t) with u < v for
-  // every edge of trussness t >= 3 (the others have 2), unordered; returns
-  // the count, copies at most cap triples. Replaces the last solve's
+  // every edge of trussness t >= 3 (the others have 2), sorted by (u, v);
+  // returns the count, copies at most cap triples. Replaces the last solve's
   // survivors (truss_edges fails afterwards).
   uint64_t trussness(uint32_t* host_triples, uint64_t cap);
   // Byte-model terms of the last pass-2 core.
@@ -292,7 +297,9 @@ class Solver {
   void exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint32_t n_plus_1);
   uint32_t reduce_max_u32(const uint32_t* in, uint32_t n);
   void sort_pairs_u64(const uint64_t* k_in, uint64_t* k_out, const uint32_t* v_in, uint32_t* v_out,
-                      uint32_t count);
+                      uint32_t count, int end_bit = 64);
+  void sort_keys_u64(const uint64_t* k_in, uint64_t* k_out, uint32_t count, int end_bit);
+  uint32_t id_bits() const;
 
   void init_common();
   int device_;
@@ -366,7 +373,12 @@ class Solver {
   uint64_t truss_count_ = 0, triples_count_ = 0;
   DevBuf truss_out_;
   void new_input();            // a new graph: results of the previous one are gone
+  // word of pinned_ (past the control block's) that gets the number of
+  // kmax-truss edges found
+  static constexpr uint32_t kTrussCountWord = 63;
   void materialize_truss();
+  uint64_t truss_size() const;
+  void sort_rows_by_key(DevBuf* vals, uint32_t count, uint32_t bits, uint32_t* out);
 };
 
 }  // namespace kt

@@ -228,12 +228,20 @@ uint32_t Solver::reduce_max_u32(const uint32_t* in, uint32_t count) {
 }
 
 void Solver::sort_pairs_u64(const uint64_t* k_in, uint64_t* k_out, const uint32_t* v_in, uint32_t* v_out,
-                            uint32_t count) {
+                            uint32_t count, int end_bit) {
   if (!count) return;
   size_t tb = 0;
-  KT_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k_in, k_out, v_in, v_out, count, 0, 64, stream_));
+  KT_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k_in, k_out, v_in, v_out, count, 0, end_bit, stream_));
   temp_.ensure(tb);
-  KT_HIP(hipcub::DeviceRadixSort::SortPairs(temp_.p, tb, k_in, k_out, v_in, v_out, count, 0, 64, stream_));
+  KT_HIP(hipcub::DeviceRadixSort::SortPairs(temp_.p, tb, k_in, k_out, v_in, v_out, count, 0, end_bit, stream_));
+}
+
+void Solver::sort_keys_u64(const uint64_t* k_in, uint64_t* k_out, uint32_t count, int end_bit) {
+  if (!count) return;
+  size_t tb = 0;
+  KT_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, tb, k_in, k_out, count, 0, end_bit, stream_));
+  temp_.ensure(tb);
+  KT_HIP(hipcub::DeviceRadixSort::SortKeys(temp_.p, tb, k_in, k_out, count, 0, end_bit, stream_));
 }
 
 // ------------------------------------------------------------- (a) CSR ---

@@ -1022,8 +1022,20 @@ void Solver::last_stats(kt_stats* out) {
   out->w_peeled = h[1];
 }
 
+// Bits that hold any vertex id of the input.
+uint32_t Solver::id_bits() const {
+  uint32_t b = 1;
+  while (b < 32 && (uint64_t(1) << b) < n_) ++b;
+  return b;
+}
+
 // The kmax-truss of the last solve as (u, v) pairs in input ids, written
-// once into truss_out_ (from the core view's deletion thresholds).
+// once into truss_out_ (from the core view's deletion thresholds). Sorted
+// by (u, v) on the device -- a radix sort of the packed pairs takes 0.1 ms
+// for 180 k of them, where a caller's sort on the host takes 16 -- except in
+// arena mode, whose scratch is sized for the solve alone and whose caller is
+// given them in no order. Queued on the stream, not waited for: a caller
+// synchronises and then calls check_truss_count.
 void Solver::materialize_truss() {
   if (truss_ready_) return;
   if (!have_truss_) fail("no solve has completed on this context");
@@ -1031,13 +1043,50 @@ void Solver::materialize_truss() {
   const CoreView& cv = last_core_;
   truss_count_ = 0;
   if (cv.mc0 && last_truss_) {
-    truss_out_.ensure(sizeof(uint32_t) * 2 * size_t(cv.mc0));
+    const uint32_t cap = uint32_t(last_truss_), bits = arena_ ? 0 : id_bits();
+    truss_out_.ensure(sizeof(uint32_t) * 2 * size_t(cap));
+    if (bits) keys_.ensure(sizeof(uint64_t) * size_t(cap));
     zero_u32(&ctl_->nalive);
-    truss_pairs(cv.del_thr, cv.mc0, last_floor_, cv.src0, cv.adj_d0, cv.inv, truss_out_.as<uint32_t>(),
-                &ctl_->nalive, stream_);
-    truss_count_ = read_u32(&ctl_->nalive);
+    truss_pairs(cv.del_thr, cv.mc0, last_floor_, cv.src0, cv.adj_d0, cv.inv, bits, cap,
+                bits ? keys_.p : truss_out_.p, &ctl_->nalive, stream_);
+    KT_HIP(hipMemcpyAsync(pinned_ + kTrussCountWord, &ctl_->nalive, sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
+    truss_count_ = last_truss_;
+    if (bits) sort_rows_by_key(nullptr, cap, bits, truss_out_.as<uint32_t>());
   }
   truss_ready_ = true;
+}
+
+void Solver::check_truss_count() {
+  if (truss_count_ && pinned_[kTrussCountWord] != uint32_t(truss_count_)) {
+    truss_ready_ = false;
+    fail("kmax-truss bookkeeping mismatch");
+  }
+}
+
+// The count keys in keys_ (with a value each in *vals, or none) sorted and
+// unpacked into rows of out.
+void Solver::sort_rows_by_key(DevBuf* vals, uint32_t count, uint32_t bits, uint32_t* out) {
+  if (count <= kRowSortCap) {
+    sort_unpack_rows(keys_.as<uint64_t>(), vals ? vals->as<uint32_t>() : nullptr, count, bits, out, stream_);
+    return;
+  }
+  keys2_.ensure(sizeof(uint64_t) * size_t(count));
+  if (vals) {
+    vals2_.ensure(sizeof(uint32_t) * size_t(count));
+    sort_pairs_u64(keys_.as<uint64_t>(), keys2_.as<uint64_t>(), vals->as<uint32_t>(), vals2_.as<uint32_t>(), count,
+                   int(2 * bits));
+  } else {
+    sort_keys_u64(keys_.as<uint64_t>(), keys2_.as<uint64_t>(), count, int(2 * bits));
+  }
+  unpack_rows(keys2_.as<uint64_t>(), vals ? vals2_.as<uint32_t>() : nullptr, count, bits, out, stream_);
+}
+
+// How many edges materialize_truss has or will have.
+uint64_t Solver::truss_size() const {
+  if (truss_ready_) return truss_count_;
+  if (!have_truss_) fail("no solve has completed on this context");
+  if (!core_valid_) fail("the last solve's core view is gone");
+  return last_core_.mc0 ? last_truss_ : 0;
 }
 
 uint64_t Solver::trussness(uint32_t* host_triples, uint64_t cap) {
@@ -1047,7 +1096,11 @@ uint64_t Solver::trussness(uint32_t* host_triples, uint64_t cap) {
     // full decomposition of the last input's CSR (level 0 is never modified
     // after its build); the core view buffers are reused, so the last
     // solve's kmax-truss is saved first
-    if (have_truss_ && core_valid_) materialize_truss();
+    if (have_truss_ && core_valid_) {
+      materialize_truss();
+      KT_HIP(hipStreamSynchronize(stream_));
+      check_truss_count();
+    }
     core_valid_ = false;
     depth_ = 1;
     LevelGraph& g = level0();
@@ -1060,10 +1113,16 @@ uint64_t Solver::trussness(uint32_t* host_triples, uint64_t cap) {
     if (cv.mc0) {
       count_support(&cv, nullptr);
       const uint32_t kall = truss_search(&cv, 1, 0, 0).kmax;
-      out_pairs_.ensure(sizeof(uint32_t) * 3 * size_t(cv.mc0));
+      const size_t mm = cv.mc0;
+      const uint32_t bits = id_bits();
+      keys_.ensure(sizeof(uint64_t) * mm);
+      vals_.ensure(sizeof(uint32_t) * mm);
       zero_u32(&ctl_->nalive);
-      truss_triples(cv, kall, out_pairs_.as<uint32_t>(), &ctl_->nalive, stream_);
-      triples_count_ = read_u32(&ctl_->nalive);
+      truss_keys(cv, kall, bits, keys_.as<uint64_t>(), vals_.as<uint32_t>(), &ctl_->nalive, stream_);
+      const uint32_t count = read_u32(&ctl_->nalive);
+      out_pairs_.ensure(sizeof(uint32_t) * 3 * std::max<size_t>(count, 1));
+      sort_rows_by_key(&vals_, count, bits, out_pairs_.as<uint32_t>());
+      triples_count_ = count;
     }
     triples_ready_ = true;
   }
@@ -1085,11 +1144,12 @@ uint64_t Solver::truss_edges_to_device(uint32_t* dev_pairs, uint64_t cap) {
 
 uint64_t Solver::truss_edges(uint32_t* host_pairs, uint64_t cap) {
   KT_HIP(hipSetDevice(device_));
+  const uint64_t take = std::min<uint64_t>(truss_size(), cap);
+  if (!take || !host_pairs) return truss_size();
   materialize_truss();
-  const uint64_t take = std::min<uint64_t>(truss_count_, cap);
-  if (take && host_pairs)
-    KT_HIP(hipMemcpyAsync(host_pairs, truss_out_.p, sizeof(uint32_t) * 2 * take, hipMemcpyDeviceToHost, stream_));
+  KT_HIP(hipMemcpyAsync(host_pairs, truss_out_.p, sizeof(uint32_t) * 2 * take, hipMemcpyDeviceToHost, stream_));
   KT_HIP(hipStreamSynchronize(stream_));
+  check_truss_count();
   return truss_count_;
 }
 

@@ -84,3 +84,17 @@ def test_cli_edge_and_trussness_files(tmp_path):
     bad = subprocess.run([str(kc_gpu_binary()), "-f", str(path), "-x", "y"], capture_output=True, text=True,
                          timeout=60)
     assert bad.returncode == 1
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 65535, 65536, 65537, (1 << 20) + 1])
+def test_edge_sets_come_sorted_up_to_the_last_id(ctx, n):
+    """The device sorts by packed (u, v): ids at both ends of the range, with
+    n on either side of a power of two."""
+    ids = sorted({0, 1, 2, n // 2, n - 3, n - 2, n - 1} & set(range(n)))
+    rng = np.random.default_rng(n)
+    pairs = canon_pairs(np.array([(a, b) for i, a in enumerate(ids) for b in ids[i + 1:]], dtype=np.uint32))
+    want = pairs if len(ids) >= 3 else pairs[:0]
+    r = ctx.solve_pairs(pairs[rng.permutation(len(pairs))], n)
+    assert (r.kmax, r.truss_edges) == ((len(ids), len(pairs)) if len(ids) >= 3 else (0, 0))
+    np.testing.assert_array_equal(ctx.truss_edges(), want)
+    np.testing.assert_array_equal(ctx.trussness(), np.column_stack([want, np.full(len(want), len(ids), np.uint32)]))
