@@ -244,11 +244,12 @@ int kt_serve_counters_get(kt_server* srv, kt_serve_counters* out);
 /* Admission charge of a query of m edges on n vertices (bytes). */
 uint64_t kt_serve_footprint(uint64_t m, uint32_t n);
 
-/* Measurement hook for the vertex-peel push kernel (k_core_push), the
- * largest kernel of a solve. mode bit 1 (KT_PROBE_TIME): each launch stamps
+/* Measurement hook for the vertex peel: the sweeps that find a level's core
+ * numbers (k_core_est_step), or the peel's push kernel or cascade. mode bit 1 (KT_PROBE_TIME): each launch stamps
  * HIP events at its own start and end on the context's stream; bit 2
- * (KT_PROBE_COUNT): each launch counts the row slots it walks (rows up to
- * 8192 slots; longer ones go to the sliced kernel) and the vertices it takes,
+ * (KT_PROBE_COUNT): each launch counts the row slots it walks (a push: rows up
+ * to 8192 slots; longer ones go to the sliced kernel) and the vertices it
+ * takes -- of the sweeps over a level the first, which takes every row once --
  * with atomics that slow it, so time and count in separate solves. 0 turns
  * the probe off. kt_push_stats_get returns the sums since the last
  * kt_push_probe. */
@@ -263,8 +264,7 @@ typedef struct kt_push_stats {
 int kt_push_probe(kt_context* ctx, int mode);
 int kt_push_stats_get(kt_context* ctx, kt_push_stats* out);
 /* The same measurement for another kernel: KT_PROBE_VERTEX_PEEL is what
- * kt_push_probe measures (the vertex-peel cascade launch, or the push of
- * the round-based peel); KT_PROBE_DENSE_PEEL is the bit-matrix edge-peel
+ * kt_push_probe measures; KT_PROBE_DENSE_PEEL is the bit-matrix edge-peel
  * round (k_dense_peel_round), whose counters in kt_push_stats are slots =
  * the frontier edges' oriented out-degrees d+(u) + d+(v) summed, vertices =
  * the frontier edges walked. */

@@ -85,16 +85,38 @@ void core_alive_degrees(const uint64_t* off, const uint32_t* adj, const uint32_t
 // lvl[v] = (lvl[v] > k) ? kNone : (lvl[v] == kNone ? kNone : k) -- used to
 // re-open every vertex whose removal threshold exceeds k.
 void core_reopen_above(uint32_t* lvl, uint32_t n, uint32_t k, hipStream_t s);
-// Max core of a level of at most core_decompose_max_n() vertices in one
-// workgroup, from its current state (the alive vertices, their alive-
-// neighbour degrees, every alive degree >= k0 - 1): thresholds walked upward
-// from k0 without restores; afterwards the max core is alive with its
-// degrees, every other vertex v of the level removed here has lvl[v] = its
-// core number + 1, out[0] = the max core's k (0 if nothing was alive) and
-// out[1] its vertex count. q holds n entries.
-uint32_t core_decompose_max_n();
-void core_decompose(const uint64_t* off, const uint32_t* adj, uint32_t n, uint32_t k0, uint32_t* lvl, uint32_t* deg,
-                    uint32_t* q, uint32_t* out, hipStream_t s);
+// Core numbers of a level's alive vertices by local updates (kt_core.hip).
+// est has n entries, due / due_next n bytes each, flags room for the longest
+// batch of sweeps + 1; medium / heavy (n entries) and counts (2) are
+// written by init and read by the sweeps. floor >= 1: cores below it are not told apart (their vertices end
+// with est 0). steps queues `count` sweeps (lanes per row: 8, 16, 32 or 64;
+// stats, for measurement: the first one's row slots and vertices);
+// flags[count] == 0 afterwards: the estimates are the core numbers. max:
+// *top = the largest one. apply: lvl of the alive vertices below *top = their
+// core number + 1 (floor below floor).
+struct CoreEst {
+  const uint64_t* off;
+  const uint32_t* adj;
+  uint32_t n, floor;
+  uint32_t* est;
+  uint8_t *due, *due_next;
+  uint32_t *medium, *heavy, *counts;
+  uint32_t* flags;
+};
+void core_est_init(const CoreEst& a, const uint32_t* deg, const uint32_t* lvl, int lanes, hipStream_t s);
+void core_est_steps(CoreEst* a, int lanes, uint32_t count, hipStream_t s, unsigned long long* stats, hipEvent_t* ev);
+void core_est_max(const CoreEst& a, uint32_t* top, hipStream_t s);
+void core_est_apply(const CoreEst& a, const uint32_t* top, uint32_t* lvl, hipStream_t s);
+// The whole of it for a small level (core_small_fits) in one launch: lvl as
+// after apply, deg of the max core's vertices = their degree in it; out[0] =
+// the largest core number, out[1] = 0 when the sweeps did not converge.
+bool core_small_fits(uint32_t n, uint64_t slots);
+void core_small(const uint64_t* off, const uint32_t* adj, uint32_t n, uint32_t floor, uint32_t* lvl, uint32_t* deg,
+                int lanes, uint32_t* out, hipStream_t s, unsigned long long* stats, hipEvent_t* ev);
+// lvl[v] = k for every vertex of the alive bitmap (alive_words) with fewer
+// than k alive neighbours; *alive (starts at 0) += the others.
+void core_prune(const uint64_t* off, const uint32_t* adj, const uint32_t* bits, uint32_t n, uint32_t k, uint32_t* lvl,
+                uint32_t* alive, hipStream_t s);
 // Degree histogram (kDegBins bins: exact below kDegExact, then one per power
 // of two) and the degree filter of the max-core search (lvl = k for every
 // vertex of degree < k, kNone otherwise; *alive += vertices kept).

@@ -209,6 +209,7 @@ uint64_t Solver::filtered_core(uint32_t k) {
   depth_ = 1;
   LevelGraph& g0 = *levels_[0];
   const uint32_t n = g0.n;
+  g0.exact_from = g0.exact_to = 0;  // its stamps are overwritten
   degrees_from_offsets(g0.off, n, g0.deg, stream_);
   zero_u32(&ctl_->nalive);
   core_filter(g0.deg, n, k, g0.lvl, &ctl_->nalive, stream_);
@@ -224,23 +225,12 @@ uint64_t Solver::filtered_core(uint32_t k) {
   return kept - removed;
 }
 
-// Start of the max-core search from a high threshold: a sixteenth of a lower
-// bound of the degree h-index H (at least H vertices have degree >= H; the
-// max core is at most H), reached by filtered_core. On power-law graphs the
-// row slots of the vertices of degree >= d shrink very slowly with d, so a
-// low threshold costs the cut little more than a high one, and it leaves a
-// cut level that pass 2's (L-1)-core usually lies in (no second cut from
-// level 0). When its core is empty the threshold drops by 4x, and when the
-// filter would keep more than a quarter of the vertices the plain search
-// from 1 runs instead. On success *gp is the cut level with the kf-core
-// alive, *k_out = kf and *alive_out its vertex count. The degree histogram
-// stays for later filtered cuts.
-bool Solver::filtered_start(LevelGraph** gp, uint32_t* k_out, uint64_t* alive_out) {
-  LevelGraph& g0 = **gp;
-  const uint32_t n = g0.n;
-  if (n < 4 * kMinCut) return false;
+// Lower bound of the degree h-index H of level 0 (at least H vertices have
+// degree >= H), from a histogram of its degrees that stays for later
+// filtered cuts.
+uint32_t Solver::degree_hindex(const LevelGraph& g0) {
   dhist_.ensure(sizeof(uint32_t) * kDegBins);
-  degree_hist(g0.deg, n, dhist_.as<uint32_t>(), stream_);
+  degree_hist(g0.deg, g0.n, dhist_.as<uint32_t>(), stream_);
   // into pinned host memory (arena mode has none and copies to pageable memory)
   std::vector<uint32_t> paged(pinned_hist_ ? 0 : kDegBins);
   uint32_t* h = pinned_hist_ ? pinned_hist_ : paged.data();
@@ -254,7 +244,165 @@ bool Solver::filtered_start(LevelGraph** gp, uint32_t* k_out, uint64_t* alive_ou
     const uint64_t lo = uint32_t(b) < kDegExact ? uint64_t(b) : uint64_t(1) << (b - kDegExact + kDegExactLog2);
     hidx = std::max(hidx, std::min(deg_at_least_[b], lo));
   }
-  for (uint32_t kf = uint32_t(hidx / 16); kf >= 3; kf /= 4) {
+  return uint32_t(hidx);
+}
+
+// Core numbers of the alive vertices of g (kt_core.hip), from their alive
+// degrees; cores below floor are not told apart. On success *top is the
+// largest core number: its vertices stay alive with their degrees in it, and
+// every other vertex is stamped with its core number + 1 (floor below floor),
+// so every cut of g from floor to *top is exact; with *top == 0 (no core of
+// floor) every vertex is stamped. False (lvl and deg untouched) when the
+// sweeps have not converged after kCoreSweeps: each sweep moves a removal one
+// vertex along, so a core that unravels along a path of many vertices is left
+// to the peel.
+bool Solver::core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top) {
+  constexpr uint32_t kBatch = 16, kMaxBatch = 32, kCoreSweeps = 512;
+  const uint32_t n = g.n;
+  core_out_.ensure(sizeof(uint32_t) * (kMaxBatch + 4));  // top | flags | medium and heavy counts
+  uint32_t* out = core_out_.as<uint32_t>();
+  const int lanes = auto_lanes(double(g.slots) / std::max<uint32_t>(n, 1));
+  // measurement of the vertex peel
+  const bool probe = probe_kernel_ == kProbeVertexPeel;
+  auto events = [&](uint32_t count) { return probe && (probe_push_ & 1) ? probe_events(int(count)) : nullptr; };
+  unsigned long long* ps = probe && (probe_push_ & 2) ? probe_stats_.as<unsigned long long>() : nullptr;
+  if (trace_) trace_ms();
+  uint32_t sweeps = 0;
+  if (core_small_fits(n, g.slots)) {
+    core_small(g.off, g.adj, n, floor, g.lvl, g.deg, lanes, out, stream_, ps, events(1));
+    KT_HIP(hipMemcpyAsync(pinned_, out, sizeof(uint32_t) * 2, hipMemcpyDeviceToHost, stream_));
+    KT_HIP(hipStreamSynchronize(stream_));
+    if (!pinned_[1]) return false;
+    *top = pinned_[0];
+  } else {
+    // extraction scratch, free at this point
+    keys_.ensure(sizeof(uint64_t) * (size_t(n_) + 1));
+    keys2_.ensure(sizeof(uint64_t) * (size_t(n_) + 1));
+    const HeavyList hl = heavy();
+    CoreEst a{};
+    a.off = g.off;
+    a.adj = g.adj;
+    a.n = n;
+    a.floor = floor;
+    a.est = keys_.as<uint32_t>();
+    a.due = keys2_.as<uint8_t>();
+    a.due_next = a.due + n;
+    a.medium = hl.slices;
+    a.heavy = hl.items;
+    a.flags = out + 1;
+    a.counts = a.flags + kMaxBatch + 1;
+    core_est_init(a, g.deg, g.lvl, lanes, stream_);
+    for (uint32_t batch = kBatch;;) {
+      core_est_steps(&a, lanes, batch, stream_, sweeps ? nullptr : ps, events(batch));
+      core_est_max(a, out, stream_);
+      KT_HIP(hipMemcpyAsync(pinned_, out, sizeof(uint32_t) * (batch + 2), hipMemcpyDeviceToHost, stream_));
+      KT_HIP(hipStreamSynchronize(stream_));
+      sweeps += batch;
+      if (pinned_[1 + batch] == 0) break;
+      if (sweeps >= kCoreSweeps) return false;
+      batch = std::min(batch * 2, kMaxBatch);
+    }
+    *top = pinned_[0];
+    if (*top) {
+      core_est_apply(a, out, g.lvl, stream_);
+      core_alive_degrees(g.off, g.adj, g.lvl, n, g.deg, heavy(), stream_);
+    } else {
+      fill_u32(g.lvl, n, floor, stream_);
+    }
+  }
+  if (trace_)
+    std::fprintf(stderr, "[kt] core numbers level_n=%u slots=%llu from k=%u: max core %u, at most %u sweeps (%.2f ms)\n",
+                 n, (unsigned long long)g.slots, floor, *top, sweeps, trace_ms());
+  vertex_rounds_ = false;
+  if (*top) {
+    g.ok.push_back(*top);
+    g.exact_from = floor;
+    g.exact_to = *top;
+  }
+  return true;
+}
+
+// Stamps most of the vertices outside g's k-core removed at k: those of degree
+// < k, and those with fewer than k neighbours among the rest. Returns the
+// vertices left; their degrees are stale.
+uint32_t Solver::prune_level(LevelGraph& g, uint32_t k) {
+  const size_t words = (size_t(g.n) + 31) / 32;
+  new_id_.ensure(sizeof(uint32_t) * 2 * (words + 1));
+  uint32_t* bits = new_id_.as<uint32_t>();
+  zero_u32(&ctl_->nalive);
+  core_filter(g.deg, g.n, k, g.lvl, &ctl_->nalive, stream_);
+  alive_words(g.lvl, g.n, bits, bits + words + 1, stream_);
+  zero_u32(&ctl_->nalive);
+  core_prune(g.off, g.adj, bits, g.n, k, g.lvl, &ctl_->nalive, stream_);
+  const uint32_t left = read_u32(&ctl_->nalive);
+  if (trace_) std::fprintf(stderr, "[kt] prune level_n=%u k=%u: %u left\n", g.n, k, left);
+  return left;
+}
+
+// The max core from core numbers. The k-core lies in the subgraph induced by
+// the vertices of degree >= k, so with allow_cut the search starts on that
+// subgraph for k = a twelfth of the degree h-index (the max core is at most
+// the h-index): on power-law graphs the row slots of the vertices of degree
+// >= d shrink slowly with d, so a low threshold costs the cut little more
+// than a high one, and its level then holds pass 2's (L-1)-core (L - 1 was
+// 0.11 to 0.25 of the h-index on R-MAT and Chung-Lu graphs of 200 k to 500 M
+// edges). Most of what the filter keeps has fewer than k neighbours among the
+// kept: that and one pass over the rows of the rest is pruned, and what is
+// left is cut again when it is at most 3/4 (50M-vertex Chung-Lu: 129 k
+// vertices kept, 30 k left). When the core is empty the threshold drops by
+// 4x, and when the filter would keep more than a quarter of the vertices the
+// whole graph is taken if it has at most kCoreWholeSlots row slots. False:
+// not converged, or too large (the level 0 state is as it was, or fresh).
+bool Solver::max_core_numbers(bool allow_cut, bool fresh, uint32_t* k) {
+  LevelGraph& g0 = levels_.empty() || fresh ? level0() : *levels_[0];
+  if (fresh) degrees_from_offsets(g0.off, g0.n, g0.deg, stream_);
+  if (allow_cut && fresh && g0.n >= 4 * kMinCut) {
+    const uint32_t hidx = degree_hindex(g0);
+    for (uint32_t kf = hidx / 12; kf >= 3; kf /= 4) {
+      if (degree_at_least(kf) > g0.n / 4) break;
+      zero_u32(&ctl_->nalive);
+      core_filter(g0.deg, g0.n, kf, g0.lvl, &ctl_->nalive, stream_);
+      const uint32_t kept = read_u32(&ctl_->nalive);
+      depth_ = 1;
+      if (kept == 0) continue;
+      LevelGraph* s = &cut_level(g0, kf, kept, true);
+      if (s->slots >= kPruneMinSlots) {
+        const uint32_t left = prune_level(*s, kf);
+        if (left == 0) continue;
+        if (uint64_t(left) * 4 <= uint64_t(s->n) * 3) s = &cut_level(*s, kf, left, true);
+      }
+      if (!core_numbers(*s, kf, k)) return false;
+      if (*k) return true;
+    }
+  }
+  depth_ = 1;
+  if (fresh) fill_u32(g0.lvl, g0.n, kNone, stream_);
+  return g0.slots <= kCoreWholeSlots && core_numbers(g0, 1, k);
+}
+
+// The largest k with a non-empty k-core (0: no edges); leaves the max-core
+// alive on the deepest level. By core numbers, or (a large graph whose degrees
+// do not set a core apart, sweeps that did not converge, or a peel forced by
+// set_vertex_mode) by a galloping search.
+uint32_t Solver::max_core(bool allow_cut, bool fresh) {
+  depth_ = 1;
+  uint32_t top = 0;
+  if (n_ && vertex_mode_ == 0 && max_core_numbers(allow_cut, fresh, &top)) return top;
+  depth_ = 1;
+  return max_core_gallop(allow_cut, fresh);
+}
+
+// Start of the galloping search from a high threshold: a sixteenth of the
+// degree h-index's lower bound, reached by filtered_core, dropping by 4x while
+// its core is empty; the plain search from 1 runs when the filter would keep
+// more than a quarter of the vertices. On success *gp is the cut level with
+// the kf-core alive, *k_out = kf and *alive_out its vertex count.
+bool Solver::filtered_start(LevelGraph** gp, uint32_t* k_out, uint64_t* alive_out) {
+  LevelGraph& g0 = **gp;
+  const uint32_t n = g0.n;
+  if (n < 4 * kMinCut) return false;
+  const uint32_t hidx = degree_hindex(g0);
+  for (uint32_t kf = hidx / 16; kf >= 3; kf /= 4) {
     if (degree_at_least(kf) > n / 4) break;
     const uint64_t alive = filtered_core(kf);
     if (trace_)
@@ -274,10 +422,9 @@ bool Solver::filtered_start(LevelGraph** gp, uint32_t* k_out, uint64_t* alive_ou
   return false;
 }
 
-// Galloping search for the largest k with a non-empty k-core. Leaves the
-// max-core alive on the deepest level and returns its k (0: no edges).
-uint32_t Solver::max_core(bool allow_cut, bool fresh) {
-  depth_ = 1;
+// Galloping search for the largest k with a non-empty k-core; once a step
+// leaves few enough alive for a cut, the core numbers of the cut level end it.
+uint32_t Solver::max_core_gallop(bool allow_cut, bool fresh) {
   LevelGraph* g = levels_.empty() || fresh ? &level0() : levels_[0].get();
   deg_bak_.ensure(sizeof(uint32_t) * (size_t(n_) + 1));
   q0_.ensure(sizeof(uint32_t) * (size_t(n_) + 1));
@@ -301,18 +448,13 @@ uint32_t Solver::max_core(bool allow_cut, bool fresh) {
     g->exact_from = g->exact_to = 0;
     if (allow_cut && alive * 4 <= g->n && alive >= kMinCut) g = &cut_level(*g, 1, uint32_t(alive));
   }
-  bool grow = true;
-  uint32_t hi = ~0u;  // smallest threshold known to empty the level
+  bool grow = true, tried = false;
   while (step > 0) {
-    // A small level finishes in one workgroup that walks every threshold
-    // (each costs about a row length of latency), the gallop in cascades of
-    // the whole level (about log2 of the range): walk when few thresholds
-    // are left, or on a cut level (its threshold already near the max core)
-    // whose rows are short.
-    if (vertex_mode_ == 0 && g->n <= core_decompose_max_n() && g->slots <= kDecomposeMaxSlots &&
-        (uint64_t(hi) - k <= kDecomposeMaxRange ||
-         (depth_ > 1 && g->slots <= uint64_t(kDecomposeMaxRow) * g->n)))
-      return decompose_level(*g, k);
+    if (vertex_mode_ == 0 && depth_ > 1 && !tried && g->slots <= kCoreWholeSlots) {
+      uint32_t top = 0;
+      if (core_numbers(*g, k, &top) && top) return top;
+      tried = true;
+    }
     const uint32_t kk = k + step;
     KT_HIP(hipMemcpyAsync(deg_bak_.p, g->deg, sizeof(uint32_t) * g->n, hipMemcpyDeviceToDevice, stream_));
     const uint64_t removed = peel_vertices(*g, kk, alive);  // an overshoot is restored below
@@ -321,10 +463,9 @@ uint32_t Solver::max_core(bool allow_cut, bool fresh) {
       k = kk;
       g->ok.push_back(k);
       step = grow ? step * 2 : step / 2;
-      if (allow_cut && alive * 4 <= g->n && alive >= kMinCut) g = &cut_level(*g, k, uint32_t(alive));
+      if (allow_cut && alive * 4 <= g->n && alive >= kMinCut) g = &cut_level(*g, k, uint32_t(alive)), tried = false;
     } else {
       // overshoot: re-open what this step removed and restore degrees
-      hi = std::min(hi, kk);
       core_reopen_above(g->lvl, g->n, k, stream_);
       KT_HIP(hipMemcpyAsync(g->deg, deg_bak_.p, sizeof(uint32_t) * g->n, hipMemcpyDeviceToDevice, stream_));
       if (step == 1) break;
@@ -335,29 +476,6 @@ uint32_t Solver::max_core(bool allow_cut, bool fresh) {
   return k;
 }
 
-// The rest of the max-core search on a small level in one workgroup
-// (core_decompose): from the k-core alive on g, thresholds walk upward with
-// no restores. Leaves the max core alive on g with its degrees and every
-// vertex removed on the way stamped with its core number + 1, so every cut
-// of g from k up to the max core is exact; returns the max core's k.
-uint32_t Solver::decompose_level(LevelGraph& g, uint32_t k) {
-  dec_out_.ensure(sizeof(uint32_t) * 2);
-  q0_.ensure(sizeof(uint32_t) * (size_t(g.n) + 1));
-  if (trace_) trace_ms();
-  core_decompose(g.off, g.adj, g.n, k, g.lvl, g.deg, q0_.as<uint32_t>(), dec_out_.as<uint32_t>(), stream_);
-  KT_HIP(hipMemcpyAsync(pinned_, dec_out_.p, sizeof(uint32_t) * 2, hipMemcpyDeviceToHost, stream_));
-  KT_HIP(hipStreamSynchronize(stream_));
-  const uint32_t kmax = pinned_[0], alive = pinned_[1];
-  if (kmax < k || alive == 0 || alive > g.n) fail("vertex peel bookkeeping mismatch (core decomposition)");
-  if (trace_)
-    std::fprintf(stderr, "[kt] core decomposition level_n=%u slots=%llu from k=%u: max core %u, %u vertices (%.2f ms)\n",
-                 g.n, (unsigned long long)g.slots, k, kmax, alive, trace_ms());
-  g.ok.push_back(kmax);
-  g.exact_from = k;
-  g.exact_to = kmax;
-  return kmax;
-}
-
 // Leaves the k-core alive on the deepest level whose vertices all have core
 // number >= its entry threshold <= k: re-open everything that level removed
 // above its largest successful threshold kj <= k (k itself when the level's
@@ -365,7 +483,9 @@ uint32_t Solver::decompose_level(LevelGraph& g, uint32_t k) {
 void Solver::core_at(uint32_t k) {
   size_t d = depth_ - 1;
   while (d > 0 && levels_[d]->k_enter > k) --d;
-  if (d == 0 && k >= 3 && levels_[0]->n >= 4 * kMinCut && degree_at_least(k) <= levels_[0]->n / 4) {
+  auto exact_at = [&](const LevelGraph& g) { return g.exact_from && g.exact_from <= k && k <= g.exact_to; };
+  if (d == 0 && !exact_at(*levels_[0]) && k >= 3 && levels_[0]->n >= 4 * kMinCut &&
+      degree_at_least(k) <= levels_[0]->n / 4) {
     // no cut level holds the k-core, but few vertices have degree >= k:
     // filter and cut again rather than re-peel the whole graph
     const uint64_t alive = filtered_core(k);
@@ -378,7 +498,7 @@ void Solver::core_at(uint32_t k) {
   uint32_t kj = std::max<uint32_t>(g.k_enter, 1);
   for (uint32_t t : g.ok)
     if (t <= k) kj = std::max(kj, t);
-  const bool exact = g.exact_from && g.exact_from <= k && k <= g.exact_to;
+  const bool exact = exact_at(g);
   if (exact) kj = k;
   core_reopen_above(g.lvl, g.n, kj, stream_);
   core_alive_degrees(g.off, g.adj, g.lvl, g.n, g.deg, heavy(), stream_);

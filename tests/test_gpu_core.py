@@ -1,0 +1,62 @@
+"""The max-core search by core numbers: every branch of its sweeps (one
+workgroup; estimates in LDS or in memory; rows of a lane group, a wave, a
+workgroup in registers and longer) and the peel that takes over when they do
+not converge, against the oracle."""
+import numpy as np
+import pytest
+
+from conftest import canon_pairs
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _hubs(n, degrees, m, clique, seed):
+    """m random edges, a clique, and hubs joined to the first `degree` other vertices."""
+    rng = np.random.default_rng(seed)
+    e = [rng.integers(0, n, (m, 2))]
+    vs = rng.choice(n, clique, replace=False)
+    e.append(np.array([(a, b) for i, a in enumerate(vs) for b in vs[i + 1:]]).reshape(-1, 2))
+    for h, d in enumerate(degrees):
+        e.append(np.column_stack([np.full(d, h), (h + 1 + np.arange(d)) % n]))
+    e = np.concatenate(e)
+    return np.unique(canon_pairs(e[e[:, 0] != e[:, 1]].astype(np.uint32)), axis=0)
+
+
+def _lollipop(path, clique):
+    """A clique with a path hanging off it."""
+    e = [(a, b) for a in range(clique) for b in range(a + 1, clique)]
+    e += [(clique - 1 + i, clique + i) for i in range(path)]
+    return np.array(e, dtype=np.uint32)
+
+
+CASES = {
+    # one workgroup, up to its limits of 4,096 vertices and 8,192 row slots, and past them
+    "tiny": (40, [], 100, 6), "one_wg": (4096, [900], 3000, 9), "past_n": (4097, [900], 3000, 9),
+    "past_slots": (900, [], 4200, 9),
+    # LDS estimates: rows past a lane group, a wave (4,096) and the registers of a workgroup (16,384)
+    "lds_rows": (30_000, [300, 1200, 4096, 4097, 16_384, 16_385, 29_000], 60_000, 20),
+    "lds_dense": (3_000, [2_999, 2_500], 200_000, 60),
+    "lds_last_n": (65_536, [17_000], 40_000, 12),
+    # estimates in memory: one workgroup of 256 holds 4,096 row entries in registers
+    "memory": (65_537, [300, 1200, 4096, 4097, 20_000], 100_000, 14),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_max_core_of_every_row_length(ctx, name):
+    n, hubs, m, clique = CASES[name]
+    pairs = _hubs(n, hubs, m, clique, len(name))
+    ref = O.solve_pairs(pairs, n, want_edges=True)
+    r = ctx.solve_pairs(pairs, n)
+    assert (r.max_core, r.k_hat, r.kmax, r.truss_edges) == (ref.max_core, ref.k_hat, ref.kmax, ref.truss_edges)
+    np.testing.assert_array_equal(ctx.truss_edges(), canon_pairs(ref.truss))
+
+
+@pytest.mark.parametrize("path", [1, 511, 513, 1200, 5000])
+def test_cores_that_unravel_along_a_path(ctx, path):
+    """Each sweep moves the end of the path by one vertex; past the sweeps'
+    limit the peel takes over."""
+    pairs = _lollipop(path, 7)
+    r = ctx.solve_pairs(pairs, 7 + path)
+    assert (r.max_core, r.kmax, r.truss_edges) == (6, 7, 21)
