@@ -54,7 +54,7 @@ typedef struct kt_result {
   float ms_count;         /* (c) pass-2 support count */
   float ms_peel;          /* (d) pass-2 edge peeling */
   float ms_count_kernel;  /* device time of the pass-2 support kernel alone */
-  uint32_t compactions;   /* edge-set compactions, both passes (src/kc.cu:1059-1138) */
+  uint32_t compactions;   /* edge sets or live-edge lists rewritten, both passes (src/kc.cu:1059-1138) */
   uint32_t recounts;      /* dropped frontiers recounted exactly (src/kc.cu:1206-1233) */
 } kt_result;
 

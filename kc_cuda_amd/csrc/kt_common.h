@@ -142,4 +142,50 @@ struct PeelArgs {
   const uint32_t *pref0, *eidm;
 };
 
+// ------------------------------------- truss levels over triangle lists --
+
+constexpr uint32_t kListStart = 0;  // nothing done yet
+constexpr uint32_t kListWalk = 1;   // walk the frontier's triangles
+constexpr uint32_t kListLook = 2;   // collect the live edges below the threshold
+constexpr uint32_t kListEmpty = 3;  // the level empties: every live edge dies now
+constexpr uint32_t kListDone = 4;
+
+// What a step of the search does (kt_list.hip).
+struct ListState {
+  uint32_t phase;
+  uint32_t round;    // stamp of the frontier walked
+  uint32_t cur;      // queue that holds it
+  uint32_t rounds;   // frontiers walked
+  int32_t thr;       // threshold of the level being peeled or looked for
+  uint32_t closing;  // look: the level at thr - 1 is complete
+  uint32_t compact;  // look: list the live edges anew
+  uint32_t live;     // entries of the edge list looked at (dead ones among them)
+  uint32_t listed;   // it is live[buf] (else every edge)
+  uint32_t buf;
+  uint32_t err;      // live edges left, but none found
+  // levels and the search's end, as in Ctl and SearchRule
+  uint32_t levels, first, level_kmax;
+  int32_t level_floor;
+  uint32_t early_k, exact_early, relists;  // relists: live edges listed anew
+  unsigned long long alive, level_count, early_ans;
+};
+
+// What a step finds; one cache line each.
+struct ListCounters {
+  uint32_t frontier;  // edges appended to the next frontier
+  uint32_t live;      // live edges listed
+  uint32_t min;       // least support among the live edges
+  uint32_t pad[29];
+};
+
+struct ListArgs {
+  ListState* states;       // two, alternating
+  ListCounters* counters;  // three, rotating
+  const uint32_t* tri_off;  // lists: mc + 1 offsets, pairs of partner edges
+  const uint2* tri;
+  uint32_t *state, *del_thr;
+  int32_t* sup;
+  uint32_t *q[2], *live[2];
+};
+
 }  // namespace kt

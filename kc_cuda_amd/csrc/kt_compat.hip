@@ -163,7 +163,7 @@ void Solver::view_from_oriented_host(uint32_t nc, const uint32_t* h_off_d, const
   inv_orig_.ensure(sizeof(uint32_t) * (size_t(nc) + 1));
   orig0_.ensure(sizeof(uint32_t) * mm);
   del_thr_.ensure(sizeof(uint32_t) * mm);
-  sup_.ensure(sizeof(int32_t) * mm);
+  sup_.ensure(sizeof(int32_t) * (mm + 1));
   state_.ensure(sizeof(uint32_t) * mm);
   eq0_.ensure(sizeof(uint32_t) * mm);
   eq1_.ensure(sizeof(uint32_t) * mm);

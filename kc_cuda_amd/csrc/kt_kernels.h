@@ -243,6 +243,15 @@ void row_compact(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* o
                  const int32_t* sup, const uint32_t* state, uint32_t nc, const uint32_t* off2,
                  uint32_t* adj2, uint32_t* src2, uint32_t* orig2, int32_t* sup2, hipStream_t s);
 void count_in_degrees(const uint32_t* adj, uint32_t m, uint32_t* din, hipStream_t s);
+// Truss levels over triangle lists (kt_list.hip). sum_u32: *total (starts at
+// 0) += the sum. tri_fill: every triangle's entries, cursor starting as a copy
+// of the offsets (bitmap, lanes: as the support count's kernels). list_steps:
+// steps from, from + 1, ... after list_start.
+void sum_u32(const uint32_t* in, uint32_t n, uint64_t* total, hipStream_t s);
+void tri_fill(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* src, uint32_t nc, uint32_t mc,
+              uint32_t max_dout, bool bitmap, int lanes, uint32_t* cursor, uint32_t* tri, hipStream_t s);
+void list_start(const ListArgs& a, const ListState& first, hipStream_t s);
+void list_steps(const ListArgs& a, uint32_t mc, uint32_t from, uint32_t count, hipStream_t s);
 void truss_pairs(const uint32_t* del_thr, uint32_t m0, int32_t floor, const uint32_t* src0,
                  const uint32_t* dst0, const uint32_t* inv, uint32_t id_bits, uint32_t cap, void* out,
                  uint32_t* count, hipStream_t s);

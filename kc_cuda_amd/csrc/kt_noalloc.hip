@@ -58,6 +58,7 @@ void set_up(NoAllocDevice& d, int device) {
     d.arena.size = KT_NOALLOC_SCRATCH_BYTES;
     Solver* s = new Solver(device, &d.arena);
     s->set_eidm_budget(kNoAllocEidmBytes);
+    s->set_list_budget(kNoAllocListBytes);
     d.solver = s;
   }
 }

@@ -23,6 +23,9 @@ namespace kt {
 
 // Edge-id matrix cap of a serving slot's dense cores (bytes).
 constexpr uint64_t kServeEidmBytes = uint64_t(256) << 20;
+// Triangle lists of a sorted-row core, per core edge: a slot then holds at
+// most 120 B an edge where the footprint counts 160.
+constexpr uint64_t kServeListBytes = 48;
 // Bytes an idle slot may keep after freeing its buffers (control block).
 constexpr uint64_t kServeSlotFloor = uint64_t(1) << 20;
 // Continuous batching: while more queries wait than the idle slots can take,

@@ -122,6 +122,8 @@ class Solver {
   void release_buffers();
   // Largest edge-id matrix a dense core may allocate (bytes).
   void set_eidm_budget(uint64_t bytes) { eidm_budget_ = bytes; }
+  // Largest triangle lists of a sorted-row core, in bytes a core edge.
+  void set_list_budget(uint64_t bytes_per_edge) { tri_per_edge_ = bytes_per_edge; }
 
   // Input already resident on the device: m canonical pairs (interleaved).
   void solve_pairs_device(const uint32_t* d_pairs, uint64_t m, uint32_t n, kt_result* res);
@@ -295,6 +297,8 @@ class Solver {
   PeelArgs peel_args(const CoreView& cv);
   // frontier of the live edges below thr, stamped; the rounds' starting state
   // (reset: a new search with its early-exit rule)
+  bool list_triangles(const CoreView& cv);
+  TrussOutcome run_lists(const CoreView& cv, int32_t thr0, const SearchRule& search);
   void start_rounds(CoreView* cv, int32_t thr, uint32_t r, uint64_t alive, bool reset, const SearchRule& search);
   TrussOutcome run_levels(CoreView* cv, int32_t thr, uint64_t alive, uint32_t* r_io, const SearchRule& search,
                           bool allow_redensify);
@@ -324,12 +328,14 @@ class Solver {
   int64_t gallop_growth_ = 2;  // KT_GALLOP_GROWTH: factor of the pass-1 probe steps
 
   int core_mode_ = 0;
-  DevBuf bits0_, bits_, fbits_, pref0_, eidm_, heavy_, vflag_, vmap_, roff_, dhist_, vq_, core_out_;
+  DevBuf bits0_, bits_, fbits_, pref0_, eidm_, heavy_, vflag_, vmap_, roff_, dhist_, vq_, core_out_, list_ctl_, tri_off_, tri_, live_[2];
   int vertex_mode_ = 0;        // see set_vertex_mode
   bool vertex_rounds_ = false;  // the last vertex peel ran synchronous rounds (reported by last_stats)
   std::vector<uint64_t> deg_at_least_;  // input degree histogram, suffix sums per bin (empty: none)
   DevBuf bk_state_, bk_sup_, bk_bits_, bk_del_;  // threshold-probe backups
   uint64_t eidm_budget_ = uint64_t(4) << 30;  // bytes for the edge-id matrix
+  // triangle lists: in all, and a core edge (a context of its own is not bound there)
+  uint64_t tri_budget_ = uint64_t(16) << 30, tri_per_edge_ = ~uint64_t(0) >> 32;
   double dense_tri_cost_ = 10.0, sparse_drop_ratio_ = 3.0, default_drop_ratio_ = 3.0;
   double dense_drop_fixed_ = 32e6;  // about what a drop's host round trip and restart cost
   bool trace_ = false;  // KT_TRACE=1: per-round frontier sizes on stderr

@@ -124,6 +124,7 @@ void Solver::init_common() {
   if (const char* v = std::getenv("KT_WALK_WINDOW")) walk_window_ = std::max<int64_t>(1, std::atoll(v));
   if (const char* v = std::getenv("KT_GALLOP_GROWTH")) gallop_growth_ = std::max<int64_t>(2, std::atoll(v));
   if (const char* v = std::getenv("KT_EIDM_BUDGET_MB")) eidm_budget_ = uint64_t(std::atoll(v)) << 20;
+  if (const char* v = std::getenv("KT_LIST_BUDGET_MB")) tri_budget_ = uint64_t(std::atoll(v)) << 20;
   if (const char* v = std::getenv("KT_WALK_LEVELS")) walk_levels_ = std::max(1, std::atoi(v));
   if (const char* v = std::getenv("KT_BUILD_TILES")) build_tiles_ = uint32_t(std::max(1, std::atoi(v)));
   if (const char* v = std::getenv("KT_VERTEX_PEEL"))
@@ -138,7 +139,7 @@ void Solver::each_buffer(F f) const {
                          &adj_d_, &src_, &din_, &din_off_, &tkeys_, &tvals_, &tiota_, &in_src_, &off_u_,
                          &adj_u_, &eid_u_, &sup_, &state_, &eq0_, &eq1_, &out_pairs_, &truss_out_, &del_thr_, &orig0_,
                          &temp_, &hist_, &hoff_, &part_, &bits0_, &bits_, &fbits_, &pref0_, &eidm_, &heavy_,
-                         &vflag_, &vmap_, &roff_, &dhist_, &vq_, &core_out_, &bk_state_, &bk_sup_, &bk_bits_, &bk_del_, &text_,
+                         &vflag_, &vmap_, &roff_, &dhist_, &vq_, &core_out_, &list_ctl_, &tri_off_, &tri_, &live_[0], &live_[1], &bk_state_, &bk_sup_, &bk_bits_, &bk_del_, &text_,
                          &tile_cnt_, &tile_off_, &lx_, &ly_, &lkind_, &lx2_, &ly2_, &lkeep_, &lkeep_off_,
                          &lstat_, &probe_stats_};
   for (const DevBuf* b : all) f(*b);

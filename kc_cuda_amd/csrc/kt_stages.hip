@@ -569,7 +569,7 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   sort_oriented_rows(nc, mc, cv->max_dout);
   orig0_.ensure(sizeof(uint32_t) * mm);
   del_thr_.ensure(sizeof(uint32_t) * mm);
-  sup_.ensure(sizeof(int32_t) * mm);
+  sup_.ensure(sizeof(int32_t) * (mm + 1));
   state_.ensure(sizeof(uint32_t) * mm);
   eq0_.ensure(sizeof(uint32_t) * mm);
   eq1_.ensure(sizeof(uint32_t) * mm);
@@ -587,8 +587,10 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   cv->sup = sup_.as<int32_t>();
   cv->state = state_.as<uint32_t>();
   cv->work = -1;
-  build_undirected_view(cv);
-  if (core_mode_ == 2 ? cv->nc <= 65536 : (core_mode_ == 0 && dense_fits(cv->nc, cv->mc))) make_dense(cv);
+  if (core_mode_ == 2 ? cv->nc <= 65536 : (core_mode_ == 0 && dense_fits(cv->nc, cv->mc))) {
+    build_undirected_view(cv);
+    make_dense(cv);
+  }  // a sorted-row view gets its undirected rows only if its triangles are not listed
 }
 
 // Bit-matrix rows of the core (all edges, live edges) plus per-word prefix
@@ -813,8 +815,98 @@ TrussOutcome Solver::truss_search(CoreView* cv, int32_t thr0, uint64_t early_ans
   search.early_ans = early_ans;
   search.early_k = early_k;
   search.exact_early = exact_early ? 1u : 0u;
+  if (!cv->dense) {
+    if (list_triangles(*cv)) return run_lists(*cv, thr0, search);
+    if (!cv->off_u) build_undirected_view(cv);
+  }
   uint32_t r = 1;
   return run_levels(cv, thr0, cv->mc, &r, search, true);
+}
+
+// Triangle lists of a base view whose supports are counted: offsets in
+// tri_off_, the pairs of partner edges in tri_. False when they do not fit
+// the budget (tri_budget_ bytes, tri_per_edge_ a core edge, and of more than
+// 1 GiB half of the device memory that is free).
+bool Solver::list_triangles(const CoreView& cv) {
+  const uint32_t mc = cv.mc;
+  if (cv.work != -1) return false;
+  list_ctl_.ensure(sizeof(ListState) * 2 + sizeof(ListCounters) * 3 + sizeof(uint64_t));
+  uint64_t* total = reinterpret_cast<uint64_t*>(list_ctl_.as<uint8_t>() + sizeof(ListState) * 2 + sizeof(ListCounters) * 3);
+  fill_u64(total, 1, 0, stream_);
+  sum_u32(reinterpret_cast<const uint32_t*>(cv.sup), mc, total, stream_);
+  const uint64_t entries = read_u64(total), bytes = entries * sizeof(uint2);
+  if (entries >= (uint64_t(1) << 31) || bytes > tri_budget_ || bytes > tri_per_edge_ * mc) return false;
+  if (bytes > tri_.bytes && bytes > (uint64_t(1) << 30)) {
+    size_t free_bytes = 0, total_bytes = 0;
+    KT_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
+    if (bytes > (free_bytes + tri_.bytes) / 2) return false;
+  }
+  tri_off_.ensure(sizeof(uint32_t) * (size_t(mc) + 1));
+  live_[0].ensure(sizeof(uint32_t) * (size_t(mc) + 1));
+  live_[1].ensure(sizeof(uint32_t) * (size_t(mc) + 1));
+  tri_.ensure(std::max<uint64_t>(bytes, 1));
+  uint32_t* off = tri_off_.as<uint32_t>();
+  uint32_t* cursor = live_[0].as<uint32_t>();  // free until the search lists live edges
+  fill_u32(reinterpret_cast<uint32_t*>(cv.sup) + mc, 1, 0, stream_);
+  exclusive_scan_u32(reinterpret_cast<const uint32_t*>(cv.sup), off, mc + 1);
+  KT_HIP(hipMemcpyAsync(cursor, off, sizeof(uint32_t) * mc, hipMemcpyDeviceToDevice, stream_));
+  const double avg = cv.nc ? double(mc) / cv.nc : 0.0;
+  tri_fill(cv.off_d, cv.adj_d, cv.src, cv.nc, mc, cv.max_dout, support_bitmap_fits(cv.nc, cv.max_dout),
+           lanes_count_ ? lanes_count_ : auto_lanes(avg), cursor, tri_.as<uint32_t>(), stream_);
+  return true;
+}
+
+// The search over the lists; steps are queued in batches and the state read
+// once per batch.
+TrussOutcome Solver::run_lists(const CoreView& cv, int32_t thr0, const SearchRule& search) {
+  constexpr uint32_t kFirstBatch = 8, kMaxBatch = 64;
+  const uint32_t mc = cv.mc;
+  ListArgs a{};
+  a.states = list_ctl_.as<ListState>();
+  a.counters = reinterpret_cast<ListCounters*>(a.states + 2);
+  a.tri_off = tri_off_.as<uint32_t>();
+  a.tri = tri_.as<uint2>();
+  a.state = cv.state;
+  a.del_thr = cv.del_thr;
+  a.sup = cv.sup;
+  a.q[0] = eq0_.as<uint32_t>();
+  a.q[1] = eq1_.as<uint32_t>();
+  a.live[0] = live_[0].as<uint32_t>();
+  a.live[1] = live_[1].as<uint32_t>();
+  ListState h{};
+  h.thr = thr0;
+  h.live = mc;
+  h.alive = mc;
+  h.first = 1;
+  h.level_floor = -1;
+  h.early_k = search.early_k;
+  h.exact_early = search.exact_early;
+  h.early_ans = search.early_ans;
+  list_start(a, h, stream_);
+  uint64_t steps = 0;
+  for (uint32_t batch = kFirstBatch;; batch = std::min(batch * 2, kMaxBatch)) {
+    if (steps > 4 * uint64_t(mc) + 4 * kMaxBatch) fail("edge peel did not converge");
+    list_steps(a, mc, uint32_t(steps), batch, stream_);
+    steps += batch;
+    static_assert(sizeof(ListState) <= 252, "state exceeds the pinned readback buffer");
+    KT_HIP(hipMemcpyAsync(pinned_, a.states + (steps & 1), sizeof(ListState), hipMemcpyDeviceToHost, stream_));
+    KT_HIP(hipStreamSynchronize(stream_));
+    std::memcpy(&h, pinned_, sizeof(h));
+    if (trace_)
+      std::fprintf(stderr, "[kt] list steps=%llu phase=%u thr=%d alive=%llu live=%u levels=%u rounds=%u\n",
+                   (unsigned long long)steps, h.phase, h.thr, h.alive, h.live, h.levels, h.rounds);
+    if (h.err) fail("edge peel bookkeeping mismatch (live count)");
+    if (h.phase == kListDone || h.phase == kListEmpty) break;
+  }
+  TrussOutcome out;
+  out.kmax = h.level_kmax;
+  out.count = h.level_count;
+  out.alive = h.phase == kListEmpty ? 0 : h.alive;
+  out.floor_thr = h.level_floor;
+  out.levels = h.levels;
+  out.rounds = h.rounds;
+  out.compactions = h.relists;
+  return out;
 }
 
 // Runs levels from threshold thr with `alive` live edges on the device until

@@ -1,0 +1,62 @@
+"""Truss levels over triangle lists against the oracle, and against the rows
+that a core whose triangles do not fit the budget is peeled with."""
+import numpy as np
+import pytest
+
+from conftest import canon_pairs
+from graphs import closed_forms, random_graph
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _graphs():
+    from kc_cuda_amd import gen
+    out = [(name, np.asarray(p, np.uint32).reshape(-1, 2), n) for name, p, n, _, _ in closed_forms()]
+    for seed, (n, p, cl) in enumerate([(60, 0.4, (9,)), (300, 0.06, (12, 9)), (700, 0.05, ())]):
+        out.append((f"er{seed}", random_graph(n, p, seed, cliques=cl), n))
+    out.append(("rmat11", *gen.rmat(11, 8, 0.57, 0.19, 0.19, True, 9, 3)))
+    return out
+
+
+@pytest.fixture(scope="module", params=["lists", "rows"])
+def sparse_ctx(request):
+    """A context that keeps every core in sorted rows; "rows": no room for lists."""
+    from kc_cuda_amd import Context
+    mp = pytest.MonkeyPatch()
+    if request.param == "rows":
+        mp.setenv("KT_LIST_BUDGET_MB", "0")
+    c = Context(0)
+    mp.undo()
+    c.tune(core="sparse")
+    yield c
+    c.close()
+
+
+def test_sparse_cores_match_oracle(sparse_ctx):
+    for name, pairs, n in _graphs():
+        print(f"[gpu] {name} m={len(pairs)}", flush=True)
+        ref = O.solve_pairs(pairs, n, want_edges=True)
+        r = sparse_ctx.solve_pairs(pairs, n)
+        assert (r.k_hat, r.kmax, r.truss_edges) == (ref.k_hat, ref.kmax, ref.truss_edges), name
+        np.testing.assert_array_equal(sparse_ctx.truss_edges(), canon_pairs(ref.truss), err_msg=name)
+        t = O.trussness(pairs)
+        want = np.array(sorted((u, v, k) for (u, v), k in t.items() if k >= 3), dtype=np.uint32).reshape(-1, 3)
+        np.testing.assert_array_equal(sparse_ctx.trussness(), want, err_msg=name)
+
+
+@pytest.mark.parametrize("scale,lanes", [(14, 8), (14, 64), (15, 0)])
+def test_lists_equal_rows(ctx, sparse_ctx, scale, lanes):
+    """Frontiers from one edge to hundreds of thousands (several edges a wave,
+    several waves an edge), live lists rewritten on the way: every trussness."""
+    from kc_cuda_amd import gen
+    pairs, n = gen.rmat(scale, 16, 0.57, 0.19, 0.19, True, 20, 4)
+    sparse_ctx.tune(core="sparse", count_lanes=lanes)
+    try:
+        r = sparse_ctx.solve_pairs(pairs, n)
+        got = sparse_ctx.trussness()
+    finally:
+        sparse_ctx.tune(core="sparse")
+    ref = ctx.solve_pairs(pairs, n)
+    assert (r.kmax, r.truss_edges, r.k_hat) == (ref.kmax, ref.truss_edges, ref.k_hat)
+    np.testing.assert_array_equal(got, ctx.trussness())
