@@ -97,24 +97,11 @@ constexpr uint32_t kRoundMinSup = 5;   // level done: reduce the live supports
 constexpr uint32_t kRoundSweep = 6;    // next level: collect its frontier
 constexpr uint32_t kRoundDone = 7;     // search finished (early exit, no edges)
 
-// Measurement of a round kernel (all optional): ev holds a start and an end
-// event per launch, stamped at the kernel's own start and end; stats gains
-// [0] the oriented out-degrees d+(u) + d+(v) of the frontier edges walked
-// and [1] their count.
-struct LaunchProbe {
-  hipEvent_t* ev = nullptr;
-  unsigned long long* stats = nullptr;
-};
-
 // Host-set parameters of the device round decision (drop or walk a frontier).
 struct RoundRule {
-  uint32_t dense;     // bit-matrix core
-  uint32_t ws;        // words per bit-matrix row
   uint32_t mc;        // edges of the current edge set (compaction rule)
   uint32_t pad;
-  double tri_cost;    // dense: cost of one triangle visit in word ANDs
-  double drop_ratio;  // sparse: drop when frontier * ratio >= alive
-  double drop_fixed;  // dense: fixed cost of a drop (host round trip, restart) in word ANDs
+  double drop_ratio;  // drop when frontier * ratio >= alive
 };
 
 // How a truss search ends: early exit on a first level of early_ans edges at
@@ -128,64 +115,85 @@ struct SearchRule {
   uint32_t pad;
 };
 
-// Arrays of a core view that the edge-peel round kernels touch.
+// Arrays of a sorted-row core view that the edge-peel round kernels touch.
 struct PeelArgs {
   uint32_t *q0, *q1;
   const uint32_t *src, *dst, *orig;  // oriented edges and their base ids
   uint32_t *state, *del_thr;
   int32_t* sup;
-  uint32_t mc, nc, ws;
+  uint32_t mc;
   const uint32_t *off_u, *adj_u, *eid_u;  // undirected view (sorted rows)
-  const uint32_t* off_d;                  // oriented rows (out-degrees, for measurement)
-  uint64_t *bits, *fbits;                 // dense views: live / frontier bits
-  const uint64_t* bits0;
-  const uint32_t *pref0, *eidm;
 };
 
-// ------------------------------------- truss levels over triangle lists --
+// ------------------------------------------ truss levels, step by step --
 
-constexpr uint32_t kListStart = 0;  // nothing done yet
-constexpr uint32_t kListWalk = 1;   // walk the frontier's triangles
-constexpr uint32_t kListLook = 2;   // collect the live edges below the threshold
-constexpr uint32_t kListEmpty = 3;  // the level empties: every live edge dies now
-constexpr uint32_t kListDone = 4;
+constexpr uint32_t kStepStart = 0;    // nothing done yet
+constexpr uint32_t kStepResume = 1;   // the host left a dropped frontier as it was
+constexpr uint32_t kStepWalk = 2;     // walk the frontier's triangles
+constexpr uint32_t kStepLook = 3;     // collect the live edges below the threshold
+constexpr uint32_t kStepClear = 4;    // dense: a dropped frontier leaves the rows ...
+constexpr uint32_t kStepRecount = 5;  // ... and the supports of the rest are counted anew
+constexpr uint32_t kStepEmpty = 6;    // the level empties: every live edge dies now
+constexpr uint32_t kStepHost = 7;     // dense: a frontier is dropped, the host may shrink the matrix first
+constexpr uint32_t kStepDone = 8;
 
-// What a step of the search does (kt_list.hip).
-struct ListState {
+// What a step of the search does (kt_step.hip).
+struct StepState {
   uint32_t phase;
-  uint32_t round;    // stamp of the frontier walked
-  uint32_t cur;      // queue that holds it
-  uint32_t rounds;   // frontiers walked
-  int32_t thr;       // threshold of the level being peeled or looked for
-  uint32_t closing;  // look: the level at thr - 1 is complete
-  uint32_t compact;  // look: list the live edges anew
-  uint32_t live;     // entries of the edge list looked at (dead ones among them)
-  uint32_t listed;   // it is live[buf] (else every edge)
-  uint32_t buf;
-  uint32_t err;      // live edges left, but none found
+  uint32_t round;           // stamp of the frontier walked
+  uint32_t cur, cnt;        // queue that holds it, its edges
+  uint32_t pend, pend_cnt;  // dense: the frontier walked before it, still in the rows (0: none)
+  uint32_t rounds;          // frontiers so far
+  int32_t thr;              // threshold of the level being peeled or looked for
+  uint32_t closing;         // look: the level at thr - 1 is complete
+  uint32_t peek;            // look: collect nothing
+  uint32_t compact;         // look: list the live edges anew
+  uint32_t live;            // entries of the edge list looked at (dead ones among them)
+  uint32_t listed, buf;     // it is live[buf] (else every edge)
+  uint32_t err;             // live edges left, but none found
+  uint32_t recounts;        // dropped frontiers
+  uint32_t relists;         // live edges listed anew
   // levels and the search's end, as in Ctl and SearchRule
   uint32_t levels, first, level_kmax;
   int32_t level_floor;
-  uint32_t early_k, exact_early, relists;  // relists: live edges listed anew
+  uint32_t early_k, exact_early, max_levels;
   unsigned long long alive, level_count, early_ans;
+  unsigned long long host_at;  // live edges when the host last looked at shrinking the matrix
 };
 
-// What a step finds; one cache line each.
-struct ListCounters {
+// What a step finds.
+struct StepCounters {
   uint32_t frontier;  // edges appended to the next frontier
   uint32_t live;      // live edges listed
   uint32_t min;       // least support among the live edges
-  uint32_t pad[29];
+  uint32_t pad[29];   // 128 bytes
 };
 
-struct ListArgs {
-  ListState* states;       // two, alternating
-  ListCounters* counters;  // three, rotating
-  const uint32_t* tri_off;  // lists: mc + 1 offsets, pairs of partner edges
-  const uint2* tri;
+struct StepRule {
+  uint32_t dense, ws;
+  uint32_t relist;    // list live edges anew once half of the list is dead
+  uint32_t host;      // stop for the host before shrinkable recounts
+  double tri_cost;    // dense: cost of one triangle visit in word ANDs
+  double drop_fixed;  // dense: fixed cost of a recount in word ANDs
+};
+
+struct StepArgs {
+  StepState* states;       // two, alternating
+  StepCounters* counters;  // three, rotating
+  const uint32_t* orig;    // base edge of each edge (null: itself)
   uint32_t *state, *del_thr;
   int32_t* sup;
-  uint32_t *q[2], *live[2];
+  uint32_t *q[3], *live[2];
+  // sorted-row cores: lists of mc + 1 offsets, pairs of partner edges
+  const uint32_t* tri_off;
+  const uint2* tri;
+  // dense cores
+  const uint32_t *src, *dst, *off_d;
+  uint32_t nc, ws;
+  unsigned long long* bits;
+  const unsigned long long* bits0;
+  const uint32_t *pref0, *off_u, *adj_u, *eid_u, *eidm;
+  unsigned long long* stats;  // measurement (null: none)
 };
 
 }  // namespace kt

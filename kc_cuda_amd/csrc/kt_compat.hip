@@ -167,6 +167,7 @@ void Solver::view_from_oriented_host(uint32_t nc, const uint32_t* h_off_d, const
   state_.ensure(sizeof(uint32_t) * mm);
   eq0_.ensure(sizeof(uint32_t) * mm);
   eq1_.ensure(sizeof(uint32_t) * mm);
+  eq2_.ensure(sizeof(uint32_t) * mm);
   KT_HIP(hipMemcpyAsync(off_d_.p, h_off_d, sizeof(uint32_t) * (size_t(nc) + 1), hipMemcpyHostToDevice, stream_));
   if (mc) KT_HIP(hipMemcpyAsync(adj_d_.p, h_adj_d, sizeof(uint32_t) * mc, hipMemcpyHostToDevice, stream_));
   row_src(off_d_.as<uint32_t>(), nc, src_.as<uint32_t>(), stream_);

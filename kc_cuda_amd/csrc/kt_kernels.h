@@ -203,13 +203,15 @@ void w_stats(const uint32_t* off_d, const uint32_t* src, const uint32_t* dst, co
 
 // Dense cores: neighbourhoods as bit-matrix rows of ws = ceil(nc / 64) words.
 uint32_t dense_words(uint32_t nc);
+int dense_lanes(uint32_t ws);  // lanes per edge of the support count
 bool dense_fits(uint32_t nc, uint32_t mc);
 void dense_rows(const uint32_t* off_u, const uint32_t* adj_u, uint32_t nc, uint32_t ws,
                 uint64_t* bits0, uint64_t* bits, uint32_t* pref0, hipStream_t s);
 void dense_support(const uint32_t* off_d, const uint32_t* dst, uint32_t nc, uint32_t mc, const uint64_t* bits,
                    uint32_t ws, const uint32_t* state, int32_t* sup, hipStream_t s);
 
-// Device-driven edge-peel rounds and truss levels (kt_peel.hip). q0/q1 are
+// Device-driven edge-peel rounds and truss levels of a sorted-row core whose
+// triangles are not listed (kt_peel.hip). q0/q1 are
 // the two frontier queues; ctl->cur says which one holds the current
 // frontier, ctl->thr the level threshold, ctl->action what comes next.
 // Starts a frontier already collected into q0 (count in ctl->qcount[0]) at
@@ -219,9 +221,7 @@ void round_start(Ctl* ctl, uint32_t r, uint64_t alive, int32_t thr, const RoundR
                  const SearchRule& search, hipStream_t s);
 void round_stamp(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, hipStream_t s);
 // `count` rounds of (peel, advance, stamp)
-void peel_rounds(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, int lanes, int count, hipStream_t s,
-                 const LaunchProbe& probe = LaunchProbe{});
-void frontier_clear(const PeelArgs& a, const Ctl* ctl, hipStream_t s);
+void peel_rounds(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, int lanes, int count, hipStream_t s);
 void dense_eidm(const uint32_t* off_u, const uint32_t* adj_u, const uint32_t* eid_u, uint32_t nc,
                 uint32_t* eidm, hipStream_t s);
 // Vertex compaction of a core view: flag the endpoints of live edges (flag
@@ -243,15 +243,18 @@ void row_compact(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* o
                  const int32_t* sup, const uint32_t* state, uint32_t nc, const uint32_t* off2,
                  uint32_t* adj2, uint32_t* src2, uint32_t* orig2, int32_t* sup2, hipStream_t s);
 void count_in_degrees(const uint32_t* adj, uint32_t m, uint32_t* din, hipStream_t s);
-// Truss levels over triangle lists (kt_list.hip). sum_u32: *total (starts at
-// 0) += the sum. tri_fill: every triangle's entries, cursor starting as a copy
-// of the offsets (bitmap, lanes: as the support count's kernels). list_steps:
-// steps from, from + 1, ... after list_start.
+// Triangle lists (kt_list.hip). sum_u32: *total (starts at 0) += the sum.
+// tri_fill: every triangle's entries, cursor starting as a copy of the offsets
+// (bitmap, lanes: as the support count's kernels).
 void sum_u32(const uint32_t* in, uint32_t n, uint64_t* total, hipStream_t s);
 void tri_fill(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* src, uint32_t nc, uint32_t mc,
               uint32_t max_dout, bool bitmap, int lanes, uint32_t* cursor, uint32_t* tri, hipStream_t s);
-void list_start(const ListArgs& a, const ListState& first, hipStream_t s);
-void list_steps(const ListArgs& a, uint32_t mc, uint32_t from, uint32_t count, hipStream_t s);
+// Truss levels of a core with triangle lists or dense rows (kt_step.hip):
+// steps from, from + 1, ... after steps_start (mc: edges of the core; ev, for
+// measurement: a start and an end event per step).
+void steps_start(const StepArgs& a, const StepState& first, hipStream_t s);
+void steps_run(const StepArgs& a, const StepRule& rule, uint32_t mc, uint32_t from, uint32_t count, hipStream_t s,
+               hipEvent_t* ev = nullptr);
 void truss_pairs(const uint32_t* del_thr, uint32_t m0, int32_t floor, const uint32_t* src0,
                  const uint32_t* dst0, const uint32_t* inv, uint32_t id_bits, uint32_t cap, void* out,
                  uint32_t* count, hipStream_t s);

@@ -1748,7 +1748,7 @@ bool dense_fits(uint32_t nc, uint32_t mc) {
   // a bitmap row (ws words of 8 bytes) no larger than two average sorted rows
   return uint64_t(dense_words(nc)) * nc <= 2ull * mc;
 }
-static int dense_lanes(uint32_t ws) {  // tuning only: KT_DENSE_COUNT_WORDS words per lane
+int dense_lanes(uint32_t ws) {  // tuning only: KT_DENSE_COUNT_WORDS words per lane
   static const uint32_t per = [] {
     const char* v = std::getenv("KT_DENSE_COUNT_WORDS");
     return v ? uint32_t(std::max(1, std::atoi(v))) : 8u;

@@ -9,9 +9,9 @@ namespace kt {
 // Edge-id matrix cap of a dense core in the allocation-free solve.
 constexpr uint64_t kNoAllocEidmBytes = uint64_t(32) << 20;
 // Triangle lists of a sorted-row core, per core edge: with their offsets and
-// live-edge lists (12 B) no more than the undirected rows and their sort (40
+// live-edge lists and third queue (16 B) no more than the undirected rows and their sort (40
 // B) that a core without lists takes instead.
-constexpr uint64_t kNoAllocListBytes = 24;
+constexpr uint64_t kNoAllocListBytes = 20;
 
 // Upper bound of the scratch bytes a solve of m edges on n vertices carves
 // (the serving footprint with the allocation-free solve's matrix cap).

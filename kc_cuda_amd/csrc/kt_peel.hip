@@ -1,4 +1,5 @@
-// Device-driven edge-peel rounds (truss levels) on CDNA4.
+// Device-driven edge-peel rounds (truss levels) of sorted-row cores whose
+// triangles are not listed, on CDNA4.
 //
 // A level removes, round by round, every edge whose support is below the
 // threshold (reference: src/kc.cu:886-1056, __delete_edge / ktruss), and the
@@ -8,12 +9,11 @@
 //   peel     walk the triangles of the frontier, decrement the partners,
 //            append edges that cross below the threshold to the next queue;
 //            at a level change: collect the new level's frontier;
-//   next     clear the walked frontier from the live bit matrix (dense
-//            cores); every workgroup takes the same decision on the next
-//            frontier from the control block and stamps it (state, deletion
-//            threshold, frontier bits), or, when it is empty, reduces the
-//            live supports; the last workgroup switches queues, records a
-//            finished level and sets what the next round does.
+//   next     every workgroup takes the same decision on the next frontier
+//            from the control block and stamps it (state, deletion
+//            threshold), or, when it is empty, reduces the live supports; the
+//            last workgroup switches queues, records a finished level and
+//            sets what the next round does.
 // The host enqueues rounds in batches, reads the control block once per batch
 // and steps in only to drop a frontier, compact, or collect the answer; a
 // kernel whose action does not concern it does nothing. k_round_stamp stamps
@@ -32,9 +32,7 @@ namespace {
 // the edges, for a level's minimum support).
 constexpr int kStampGrid = 256;
 constexpr int kPeelGrid = 1024;
-constexpr uint32_t kPeelUnroll = 8;      // triangles per lane per step of the dense peel
 constexpr uint32_t kSparseStage = 4096;  // LDS words per workgroup for the sparse peel's staged rows
-constexpr int kClearGrid = 512;
 
 // What the next round does with a frontier of c edges when `alive` edges are
 // live and unstamped.
@@ -49,10 +47,7 @@ __device__ __forceinline__ uint32_t decide_round(uint32_t c, unsigned long long 
   if (c == alive || (thr > 0 && alive - c < (unsigned long long)(thr + 2) * (unsigned long long)(thr + 1) / 2))
     return kRoundEmpty;
   if (allow_compact && 2ull * alive <= rule.mc) return kRoundCompact;
-  const bool drop = rule.dense ? double(c) * (double(rule.ws) + rule.tri_cost * double(thr)) >=
-                                     double(alive) * double(rule.ws) + rule.drop_fixed
-                               : double(c) * rule.drop_ratio >= double(alive);
-  return drop ? kRoundDrop : kRoundPeel;
+  return double(c) * rule.drop_ratio >= double(alive) ? kRoundDrop : kRoundPeel;
 }
 
 __device__ __forceinline__ void set_action(Ctl* ctl, uint32_t a) {
@@ -138,23 +133,16 @@ __device__ __forceinline__ void level_end(Ctl* ctl, const uint32_t* __restrict__
       return;
     }
     ctl->thr = int32_t(ms) + 1;
-    ctl->action = (!rule.dense && 2ull * alive <= rule.mc) ? kRoundCompact : kRoundSweep;
+    ctl->action = 2ull * alive <= rule.mc ? kRoundCompact : kRoundSweep;
   }
 }
 
 // Stamp of a frontier edge: state = round, deletion threshold of its base
-// edge = thr, and (frontiers walked on dense cores) its frontier bits.
+// edge = thr.
 __device__ __forceinline__ void stamp_edge(uint32_t e, uint32_t r, uint32_t thr, uint32_t* state,
-                                           const uint32_t* __restrict__ orig, uint32_t* del_thr,
-                                           const uint32_t* __restrict__ src, const uint32_t* __restrict__ dst,
-                                           unsigned long long* fbits, uint32_t ws) {
+                                           const uint32_t* __restrict__ orig, uint32_t* del_thr) {
   state[e] = r;
   del_thr[orig[e]] = thr;
-  if (fbits) {
-    const uint32_t u = src[e], v = dst[e];
-    atomicOr(&fbits[uint64_t(u) * ws + (v >> 6)], 1ull << (v & 63));
-    atomicOr(&fbits[uint64_t(v) * ws + (u >> 6)], 1ull << (u & 63));
-  }
 }
 
 // An emptied level (kRoundEmpty): every live edge of the edge set, the
@@ -174,9 +162,7 @@ __device__ __forceinline__ void stamp_all_live(uint32_t mc, uint32_t r, uint32_t
 __global__ __launch_bounds__(kBlock) void k_round_stamp(uint32_t* q0, uint32_t* q1, Ctl* ctl, uint32_t* state,
                                                         const int32_t* __restrict__ sup,
                                                         const uint32_t* __restrict__ orig, uint32_t* del_thr,
-                                                        const uint32_t* __restrict__ src,
-                                                        const uint32_t* __restrict__ dst,
-                                                        unsigned long long* fbits, uint32_t ws, RoundRule rule) {
+                                                        RoundRule rule) {
   const uint32_t a = ctl->action;
   if (a == kRoundMinSup) {
     level_end(ctl, state, sup, rule, [] {});
@@ -186,12 +172,11 @@ __global__ __launch_bounds__(kBlock) void k_round_stamp(uint32_t* q0, uint32_t* 
   const uint32_t cur = ctl->cur, cnt = ctl->qcount[cur], r = ctl->round;
   const uint32_t thr = uint32_t(ctl->thr);
   const uint32_t* q = cur ? q1 : q0;
-  const bool fb = fbits && a == kRoundPeel;
   if (a == kRoundEmpty)
     stamp_all_live(rule.mc, r, thr, state, orig, del_thr);
   else
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += gridDim.x * blockDim.x)
-      stamp_edge(q[i], r, thr, state, orig, del_thr, src, dst, fb ? fbits : nullptr, ws);
+      stamp_edge(q[i], r, thr, state, orig, del_thr);
   if (last_block(&ctl->ticket) && threadIdx.x == 0) {
     ctl->alive = a == kRoundEmpty ? 0 : ctl->alive - cnt;
     ctl->rounds_done += 1;
@@ -212,21 +197,8 @@ __device__ __forceinline__ void sweep_frontier(uint32_t* q0, uint32_t* q1, Ctl* 
       [&](uint32_t at, uint64_t e) { q[at] = uint32_t(e); }, &ctl->qcount[cur]);
 }
 
-__device__ __forceinline__ void clear_edge_bits(uint32_t u, uint32_t v, unsigned long long* bits,
-                                                unsigned long long* fbits, uint32_t ws) {
-  const uint64_t a = uint64_t(u) * ws + (v >> 6), b = uint64_t(v) * ws + (u >> 6);
-  const unsigned long long ma = ~(1ull << (v & 63)), mb = ~(1ull << (u & 63));
-  atomicAnd(&bits[a], ma);
-  atomicAnd(&bits[b], mb);
-  if (fbits) {
-    atomicAnd(&fbits[a], ma);
-    atomicAnd(&fbits[b], mb);
-  }
-}
-
-// Close a round. After a walked round: clear its frontier from the bit
-// matrices; the next frontier is the peel's next queue. After a sweep: the
-// next frontier is the swept queue. Every workgroup reads the same frontier
+// Close a round. After a walked round the next frontier is the peel's next
+// queue, after a sweep the swept queue. Every workgroup reads the same frontier
 // size, live count and threshold, so all take the same decision on the next
 // round and stamp the frontier it walks, drops or empties the level with (a
 // compaction takes it unstamped); an empty frontier completes the level
@@ -235,9 +207,7 @@ __device__ __forceinline__ void clear_edge_bits(uint32_t u, uint32_t v, unsigned
 __global__ __launch_bounds__(kBlock) void k_round_next(uint32_t* q0, uint32_t* q1, Ctl* ctl, uint32_t* state,
                                                        const int32_t* __restrict__ sup,
                                                        const uint32_t* __restrict__ orig, uint32_t* del_thr,
-                                                       const uint32_t* __restrict__ src,
-                                                       const uint32_t* __restrict__ dst, unsigned long long* bits,
-                                                       unsigned long long* fbits, uint32_t ws, RoundRule rule) {
+                                                       RoundRule rule) {
   const uint32_t a = ctl->action;
   if (a == kRoundMinSup) {
     level_end(ctl, state, sup, rule, [] {});
@@ -248,14 +218,6 @@ __global__ __launch_bounds__(kBlock) void k_round_next(uint32_t* q0, uint32_t* q
   const uint32_t cur = ctl->cur, r = ctl->round;
   const int32_t thr = ctl->thr;
   const unsigned long long alive = ctl->alive;
-  if (walked && bits) {
-    const uint32_t cnt = ctl->qcount[cur];
-    const uint32_t* q = cur ? q1 : q0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += gridDim.x * blockDim.x) {
-      const uint32_t e = q[i];
-      clear_edge_bits(src[e], dst[e], bits, fbits, ws);
-    }
-  }
   const uint32_t nq = walked ? cur ^ 1u : cur;  // queue of the next frontier
   const uint32_t c = ctl->qcount[nq];
   auto switch_queue = [&] {
@@ -269,17 +231,16 @@ __global__ __launch_bounds__(kBlock) void k_round_next(uint32_t* q0, uint32_t* q
     level_end(ctl, state, sup, rule, switch_queue);
     return;
   }
-  const uint32_t d = decide_round(c, alive, thr, rule, walked && !rule.dense);
+  const uint32_t d = decide_round(c, alive, thr, rule, walked);
   const bool stamp = d == kRoundPeel || d == kRoundDrop || d == kRoundEmpty;
   if (stamp) {
     const uint32_t rs = walked ? r + 1 : r;
     const uint32_t* q = nq ? q1 : q0;
-    unsigned long long* fb = d == kRoundPeel ? fbits : nullptr;
     if (d == kRoundEmpty)
       stamp_all_live(rule.mc, rs, uint32_t(thr), state, orig, del_thr);
     else
       for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < c; i += gridDim.x * blockDim.x)
-        stamp_edge(q[i], rs, uint32_t(thr), state, orig, del_thr, src, dst, fb, ws);
+        stamp_edge(q[i], rs, uint32_t(thr), state, orig, del_thr);
   }
   if (last_block(&ctl->ticket) && threadIdx.x == 0) {
     switch_queue();
@@ -292,152 +253,8 @@ __global__ __launch_bounds__(kBlock) void k_round_next(uint32_t* q0, uint32_t* q
   }
 }
 
-// Clear the current frontier from the bit matrices (a dropped frontier).
-__global__ __launch_bounds__(kBlock) void k_frontier_clear(const uint32_t* q0, const uint32_t* q1, const Ctl* ctl,
-                                                           const uint32_t* __restrict__ src,
-                                                           const uint32_t* __restrict__ dst,
-                                                           unsigned long long* bits, unsigned long long* fbits,
-                                                           uint32_t ws) {
-  const uint32_t cur = ctl->cur, cnt = ctl->qcount[cur];
-  const uint32_t* q = cur ? q1 : q0;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += gridDim.x * blockDim.x) {
-    const uint32_t e = q[i];
-    clear_edge_bits(src[e], dst[e], bits, fbits, ws);
-  }
-}
-
 __device__ __forceinline__ bool dec_crosses(uint32_t x, int32_t thr, int32_t* sup) {
   return x != kNone && atomicSub(&sup[x], 1) == thr;
-}
-
-// Walked round on a bit-matrix core. One wave per (frontier edge, chunk of
-// its rows); a chunk is 64 words, or 32 or 16 when the frontier is too small
-// to give every wave of the grid an item (a short cascade round then spreads
-// each edge's triangles over more waves). The common neighbours w of
-// e = (u, v) in the chunk are
-// the set bits of live[u] & live[v]; their count is scanned across the wave
-// and the triangles are dealt out evenly, one per lane per step, whatever
-// words they sit in. Frontier bits say at word level whether (u, w) and
-// (v, w) are in the frontier, so a triangle costs only the edge-id lookups
-// of the partners it decrements. Round-synchronous rule: a triangle with one
-// frontier edge charges both partners; with two, the third edge is charged
-// once -- by the frontier edge whose non-shared endpoint is larger than the
-// apex (z < x for the third edge (x, z)); with three, nobody. The supports
-// after the round equal the reference's `2 - #frontier` decrements on
-// doubled counts (src/kc.cu:122-146).
-template <bool kEidm>
-__global__ __launch_bounds__(kBlock) void k_dense_peel_round(
-    uint32_t* q0, uint32_t* q1, Ctl* ctl, const uint32_t* __restrict__ src, const uint32_t* __restrict__ dst,
-    const unsigned long long* __restrict__ bits, const unsigned long long* __restrict__ fbits, uint32_t ws,
-    const uint32_t* __restrict__ eidm, uint32_t nc, const unsigned long long* __restrict__ bits0,
-    const uint32_t* __restrict__ pref0, const uint32_t* __restrict__ off_u, const uint32_t* __restrict__ eid_u,
-    const uint32_t* __restrict__ state, int32_t* sup, uint32_t mc, const uint32_t* __restrict__ off_d,
-    unsigned long long* stats) {
-  const uint32_t action = ctl->action;
-  if (action == kRoundSweep) {
-    sweep_frontier(q0, q1, ctl, state, sup, mc);
-    return;
-  }
-  if (action != kRoundPeel || !ctl->stamped) return;
-  const int32_t thr = ctl->thr;
-  const uint32_t cur = ctl->cur;
-  const uint32_t cnt = ctl->qcount[cur];
-  const uint32_t* q = cur ? q1 : q0;
-  uint32_t* qn = cur ? q0 : q1;
-  uint32_t* qn_count = &ctl->qcount[cur ^ 1u];
-  __shared__ unsigned long long s_t[kBlock], s_fa[kBlock], s_fb[kBlock];
-  __shared__ uint32_t s_inc[kBlock];
-  const int lane = lane64();
-  const uint32_t wbase = threadIdx.x & ~uint32_t(kWave - 1);
-  const uint64_t nw = uint64_t(gridDim.x) * (kBlock / kWave);
-  uint32_t cw = kWave;  // words per chunk
-  while (cw > 16 && uint64_t(cnt) * ((ws + cw - 1) / cw) < nw) cw >>= 1;
-  const uint32_t nch = (ws + cw - 1) / cw;
-  const uint64_t items = uint64_t(cnt) * nch;
-  auto eid_of = [&](uint32_t a, uint32_t w) -> uint32_t {
-    if (kEidm) return eidm[uint64_t(a) * nc + w];
-    const uint64_t ra = uint64_t(a) * ws;
-    const uint32_t i = w >> 6;
-    const unsigned long long below = bits0[ra + i] & ((1ull << (w & 63)) - 1ull);
-    return eid_u[off_u[a] + pref0[ra + i] + uint32_t(__popcll(below))];
-  };
-  for (uint64_t it = uint64_t(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave; it < items; it += nw) {
-    const uint32_t qi = uint32_t(it / nch), ch = uint32_t(it - uint64_t(qi) * nch);
-    const uint32_t e = q[qi];
-    const uint32_t u = src[e], v = dst[e];
-    if (stats && ch == 0 && lane == 0) {  // measurement: the edge's merge work, d+(u) + d+(v)
-      atomicAdd(&stats[0], (unsigned long long)(off_d[u + 1] - off_d[u] + off_d[v + 1] - off_d[v]));
-      atomicAdd(&stats[1], 1ull);
-    }
-    const uint64_t ru = uint64_t(u) * ws, rv = uint64_t(v) * ws;
-    const uint32_t i = ch * cw + uint32_t(lane);
-    unsigned long long t = 0, fa = 0, fb = 0;
-    if (uint32_t(lane) < cw && i < ws) {
-      t = bits[ru + i] & bits[rv + i];
-      fa = fbits[ru + i] & t;
-      fb = fbits[rv + i] & t;
-      t &= ~(fa & fb);  // both partners in the frontier: nobody is charged
-    }
-    uint32_t inc = uint32_t(__popcll(t));
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t y = __shfl_up(inc, o);
-      if (lane >= o) inc += y;
-    }
-    const uint32_t total = __shfl(inc, kWave - 1);
-    s_t[threadIdx.x] = t;
-    s_fa[threadIdx.x] = fa;
-    s_fb[threadIdx.x] = fb;
-    s_inc[threadIdx.x] = inc;
-    wave_sync();
-    // kPeelUnroll triangles per lane per step: their partner lookups, then
-    // all their decrements, are in flight together (the returning atomics
-    // are performed past the L2, so one round trip per triangle would leave
-    // the wave waiting)
-    for (uint32_t j0 = 0; j0 < total; j0 += kWave * kPeelUnroll) {
-      uint32_t xa[kPeelUnroll], xb[kPeelUnroll];  // partner edges (u, w) and (v, w) to decrement
-#pragma unroll
-      for (uint32_t k = 0; k < kPeelUnroll; ++k) {
-        xa[k] = kNone;
-        xb[k] = kNone;
-        const uint32_t j = j0 + k * kWave + uint32_t(lane);
-        if (j < total) {
-          uint32_t lo = 0, hi = kWave - 1;  // owner: first lane whose inclusive count exceeds j
-          while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (s_inc[wbase + mid] > j)
-              hi = mid;
-            else
-              lo = mid + 1;
-          }
-          const unsigned long long tw = s_t[wbase + lo];
-          const uint32_t b = select_bit(tw, j - (s_inc[wbase + lo] - uint32_t(__popcll(tw))));
-          const uint32_t w = ((ch * cw + lo) << 6) + b;
-          const bool ina = (s_fa[wbase + lo] >> b) & 1ull, inb = (s_fb[wbase + lo] >> b) & 1ull;
-          if (!ina && !inb) {
-            xa[k] = eid_of(u, w);
-            xb[k] = eid_of(v, w);
-          } else if (ina) {  // (u, w) in the frontier, third edge (v, w)
-            if (w < v) xb[k] = eid_of(v, w);
-          } else {  // (v, w) in the frontier, third edge (u, w)
-            if (w < u) xa[k] = eid_of(u, w);
-          }
-        }
-      }
-      int32_t oa[kPeelUnroll], ob[kPeelUnroll];  // supports before the decrements
-#pragma unroll
-      for (uint32_t k = 0; k < kPeelUnroll; ++k) {
-        oa[k] = xa[k] != kNone ? atomicSub(&sup[xa[k]], 1) : 0;
-        ob[k] = xb[k] != kNone ? atomicSub(&sup[xb[k]], 1) : 0;
-      }
-#pragma unroll
-      for (uint32_t k = 0; k < kPeelUnroll; ++k) {  // a partner that falls below thr now joins the next frontier
-        wave_append(xa[k] != kNone && oa[k] == thr, xa[k], qn, qn_count);
-        wave_append(xb[k] != kNone && ob[k] == thr, xb[k], qn, qn_count);
-      }
-    }
-    wave_sync();
-  }
 }
 
 // Walked round on a sorted-row core: G lanes per frontier edge stream the
@@ -591,19 +408,12 @@ static int work_grid(uint64_t items, uint64_t per_block, int cap) {
   return int(std::max<uint64_t>(1, std::min<uint64_t>(g, uint64_t(cap))));
 }
 
-static void launch_stamp(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, hipStream_t s) {
-  k_round_stamp<<<work_grid(a.mc, 4 * kBlock, kStampGrid), kBlock, 0, s>>>(
-      a.q0, a.q1, ctl, a.state, a.sup, a.orig, a.del_thr, a.src, a.dst,
-      reinterpret_cast<unsigned long long*>(a.fbits), a.ws, rule);
+void round_stamp(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, hipStream_t s) {
+  k_round_stamp<<<work_grid(a.mc, 4 * kBlock, kStampGrid), kBlock, 0, s>>>(a.q0, a.q1, ctl, a.state, a.sup, a.orig,
+                                                                           a.del_thr, rule);
 }
 
-void round_stamp(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, hipStream_t s) { launch_stamp(a, ctl, rule, s); }
-
-void peel_rounds(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, int lanes, int count, hipStream_t s,
-                 const LaunchProbe& probe) {
-  auto bits = reinterpret_cast<unsigned long long*>(a.bits);
-  auto fbits = reinterpret_cast<unsigned long long*>(a.fbits);
-  auto b0 = reinterpret_cast<const unsigned long long*>(a.bits0);
+void peel_rounds(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, int lanes, int count, hipStream_t s) {
   static const int next_cap = [] {  // tuning only
     const char* v = std::getenv("KT_NEXT_GRID");
     return v ? std::max(1, std::atoi(v)) : kStampGrid;
@@ -611,48 +421,18 @@ void peel_rounds(const PeelArgs& a, Ctl* ctl, const RoundRule& rule, int lanes, 
   const int peel_grid = work_grid(a.mc, kBlock, kPeelGrid);
   const int next_grid = work_grid(a.mc, 4 * kBlock, next_cap);
   for (int i = 0; i < count; ++i) {
-    if (rule.dense) {
-      // every argument as an lvalue for the event-stamped launch
-      uint32_t *q0 = a.q0, *q1 = a.q1;
-      Ctl* c = ctl;
-      const uint32_t *src = a.src, *dst = a.dst, *eidm = a.eidm, *pref0 = a.pref0, *off_u = a.off_u,
-                     *eid_u = a.eid_u, *state = a.state, *off_d = a.off_d;
-      unsigned long long *lb = bits, *fb = fbits;
-      const unsigned long long* b0c = b0;
-      uint32_t ws = a.ws, nc = a.nc, mc = a.mc;
-      int32_t* sup = a.sup;
-      unsigned long long* st = probe.stats;
-      void* args[] = {&q0, &q1, &c, &src, &dst, &lb, &fb, &ws, &eidm, &nc, &b0c, &pref0, &off_u, &eid_u,
-                      &state, &sup, &mc, &off_d, &st};
-      const void* fn = a.eidm ? reinterpret_cast<const void*>(&k_dense_peel_round<true>)
-                              : reinterpret_cast<const void*>(&k_dense_peel_round<false>);
-      if (probe.ev)
-        KT_HIP(hipExtLaunchKernel(fn, dim3(peel_grid), dim3(kBlock), args, 0, s, probe.ev[2 * i],
-                                  probe.ev[2 * i + 1], 0));
-      else
-        KT_HIP(hipLaunchKernel(fn, dim3(peel_grid), dim3(kBlock), args, 0, s));
-    } else {
 #define KT_SPARSE_ROUND(G)                                                                                 \
   k_sparse_peel_round<G><<<peel_grid, kBlock, 0, s>>>(a.q0, a.q1, ctl, a.off_u, a.adj_u, a.eid_u, a.src, a.dst, \
                                                       a.state, a.sup, a.mc)
-      switch (lanes) {
-        case 8: KT_SPARSE_ROUND(8); break;
-        case 16: KT_SPARSE_ROUND(16); break;
-        case 32: KT_SPARSE_ROUND(32); break;
-        default: KT_SPARSE_ROUND(64); break;
-      }
-#undef KT_SPARSE_ROUND
+    switch (lanes) {
+      case 8: KT_SPARSE_ROUND(8); break;
+      case 16: KT_SPARSE_ROUND(16); break;
+      case 32: KT_SPARSE_ROUND(32); break;
+      default: KT_SPARSE_ROUND(64); break;
     }
-    k_round_next<<<next_grid, kBlock, 0, s>>>(a.q0, a.q1, ctl, a.state, a.sup, a.orig, a.del_thr, a.src, a.dst,
-                                              rule.dense ? bits : nullptr, rule.dense ? fbits : nullptr, a.ws,
-                                              rule);
+#undef KT_SPARSE_ROUND
+    k_round_next<<<next_grid, kBlock, 0, s>>>(a.q0, a.q1, ctl, a.state, a.sup, a.orig, a.del_thr, rule);
   }
-}
-
-void frontier_clear(const PeelArgs& a, const Ctl* ctl, hipStream_t s) {
-  k_frontier_clear<<<work_grid(a.mc, kBlock, kClearGrid), kBlock, 0, s>>>(a.q0, a.q1, ctl, a.src, a.dst,
-                                                 reinterpret_cast<unsigned long long*>(a.bits),
-                                                 reinterpret_cast<unsigned long long*>(a.fbits), a.ws);
 }
 
 void dense_eidm(const uint32_t* off_u, const uint32_t* adj_u, const uint32_t* eid_u, uint32_t nc, uint32_t* eidm,

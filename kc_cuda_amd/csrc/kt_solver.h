@@ -76,12 +76,11 @@ struct CoreView {
   uint32_t mc0 = 0, max_dout0 = 0;
   uint32_t *off_d0 = nullptr, *adj_d0 = nullptr, *src0 = nullptr, *del_thr = nullptr;
   int work = -1;  // which work set holds the current edges (-1: base)
-  // dense cores: bit-matrix rows (ws words each) of all / live / frontier
-  // edges, per-word prefix popcounts of the static rows, and (when nc^2
+  // dense cores: bit-matrix rows (ws words each) of all / live edges, per-word prefix popcounts of the static rows, and (when nc^2
   // entries fit the budget) the edge id of every (u, w) pair
   bool dense = false;
   uint32_t ws = 0;
-  uint64_t *bits0 = nullptr, *bits = nullptr, *fbits = nullptr;
+  uint64_t *bits0 = nullptr, *bits = nullptr;
   uint32_t* pref0 = nullptr;
   uint32_t* eidm = nullptr;
 };
@@ -293,15 +292,15 @@ class Solver {
   uint32_t read_u32(const uint32_t* dptr);
   uint64_t read_u64(const uint64_t* dptr);
   Ctl read_ctl();
-  RoundRule round_rule(const CoreView& cv) const;
   PeelArgs peel_args(const CoreView& cv);
   // frontier of the live edges below thr, stamped; the rounds' starting state
   // (reset: a new search with its early-exit rule)
   bool list_triangles(const CoreView& cv);
-  TrussOutcome run_lists(const CoreView& cv, int32_t thr0, const SearchRule& search);
+  StepArgs step_args(const CoreView& cv);
+  TrussOutcome run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32_t* r_io, const SearchRule& search,
+                         bool allow_host);
   void start_rounds(CoreView* cv, int32_t thr, uint32_t r, uint64_t alive, bool reset, const SearchRule& search);
-  TrussOutcome run_levels(CoreView* cv, int32_t thr, uint64_t alive, uint32_t* r_io, const SearchRule& search,
-                          bool allow_redensify);
+  TrussOutcome run_levels(CoreView* cv, int32_t thr, const SearchRule& search);
   void zero_u32(uint32_t* dptr);
   void exclusive_scan_u32_to_u64(const uint32_t* in, uint64_t* out, uint32_t n_plus_1);
   void exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint32_t n_plus_1);
@@ -328,7 +327,7 @@ class Solver {
   int64_t gallop_growth_ = 2;  // KT_GALLOP_GROWTH: factor of the pass-1 probe steps
 
   int core_mode_ = 0;
-  DevBuf bits0_, bits_, fbits_, pref0_, eidm_, heavy_, vflag_, vmap_, roff_, dhist_, vq_, core_out_, list_ctl_, tri_off_, tri_, live_[2];
+  DevBuf bits0_, bits_, pref0_, eidm_, heavy_, vflag_, vmap_, roff_, dhist_, vq_, core_out_, step_ctl_, tri_off_, tri_, live_[2];
   int vertex_mode_ = 0;        // see set_vertex_mode
   bool vertex_rounds_ = false;  // the last vertex peel ran synchronous rounds (reported by last_stats)
   std::vector<uint64_t> deg_at_least_;  // input degree histogram, suffix sums per bin (empty: none)
@@ -337,7 +336,7 @@ class Solver {
   // triangle lists: in all, and a core edge (a context of its own is not bound there)
   uint64_t tri_budget_ = uint64_t(16) << 30, tri_per_edge_ = ~uint64_t(0) >> 32;
   double dense_tri_cost_ = 10.0, sparse_drop_ratio_ = 3.0, default_drop_ratio_ = 3.0;
-  double dense_drop_fixed_ = 32e6;  // about what a drop's host round trip and restart cost
+  double dense_drop_fixed_ = 12e6;  // about what the two steps of a recount take
   bool trace_ = false;  // KT_TRACE=1: per-round frontier sizes on stderr
   // trace only: milliseconds since the previous call, after the stream drains
   double trace_ms();
@@ -368,7 +367,7 @@ class Solver {
   DevBuf list_, new_id_, keys_, keys2_, vals_, vals2_, to_;
   // core
   DevBuf inv_, inv_orig_, dout_, off_d_, adj_d_, src_, din_, din_off_, tkeys_, tvals_, tiota_,
-      in_src_, off_u_, adj_u_, eid_u_, sup_, state_, eq0_, eq1_, out_pairs_, del_thr_, orig0_;
+      in_src_, off_u_, adj_u_, eid_u_, sup_, state_, eq0_, eq1_, eq2_, out_pairs_, del_thr_, orig0_;
   EdgeSet work_[2];
   DevBuf temp_;
   // device-side text ingest: bytes, per-tile line counts and offsets, lines
@@ -388,6 +387,7 @@ class Solver {
   // word of pinned_ (past the control block's) that gets the number of
   // kmax-truss edges found
   static constexpr uint32_t kTrussCountWord = 63;
+  static constexpr size_t kStepCtlBytes = 1024;  // states and counters of kt_step.hip
   void materialize_truss();
   uint64_t truss_size() const;
   void sort_rows_by_key(DevBuf* vals, uint32_t count, uint32_t bits, uint32_t* out);

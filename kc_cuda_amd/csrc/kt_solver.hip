@@ -137,9 +137,9 @@ void Solver::each_buffer(F f) const {
   const DevBuf* all[] = {&off_, &adj_, &deg_, &lvl_, &q0_, &q1_, &deg_bak_, &cursor_, &list_, &new_id_,
                          &keys_, &keys2_, &vals_, &vals2_, &to_, &inv_, &inv_orig_, &dout_, &off_d_,
                          &adj_d_, &src_, &din_, &din_off_, &tkeys_, &tvals_, &tiota_, &in_src_, &off_u_,
-                         &adj_u_, &eid_u_, &sup_, &state_, &eq0_, &eq1_, &out_pairs_, &truss_out_, &del_thr_, &orig0_,
-                         &temp_, &hist_, &hoff_, &part_, &bits0_, &bits_, &fbits_, &pref0_, &eidm_, &heavy_,
-                         &vflag_, &vmap_, &roff_, &dhist_, &vq_, &core_out_, &list_ctl_, &tri_off_, &tri_, &live_[0], &live_[1], &bk_state_, &bk_sup_, &bk_bits_, &bk_del_, &text_,
+                         &adj_u_, &eid_u_, &sup_, &state_, &eq0_, &eq1_, &eq2_, &out_pairs_, &truss_out_, &del_thr_, &orig0_,
+                         &temp_, &hist_, &hoff_, &part_, &bits0_, &bits_, &pref0_, &eidm_, &heavy_,
+                         &vflag_, &vmap_, &roff_, &dhist_, &vq_, &core_out_, &step_ctl_, &tri_off_, &tri_, &live_[0], &live_[1], &bk_state_, &bk_sup_, &bk_bits_, &bk_del_, &text_,
                          &tile_cnt_, &tile_off_, &lx_, &ly_, &lkind_, &lx2_, &ly2_, &lkeep_, &lkeep_off_,
                          &lstat_, &probe_stats_};
   for (const DevBuf* b : all) f(*b);

@@ -573,6 +573,7 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   state_.ensure(sizeof(uint32_t) * mm);
   eq0_.ensure(sizeof(uint32_t) * mm);
   eq1_.ensure(sizeof(uint32_t) * mm);
+  eq2_.ensure(sizeof(uint32_t) * mm);
   iota_u32(orig0_.as<uint32_t>(), mc, stream_);
   fill_u32(del_thr_.as<uint32_t>(), mc, kNone, stream_);
   fill_u32(state_.as<uint32_t>(), mc, kNone, stream_);
@@ -600,16 +601,13 @@ void Solver::make_dense(CoreView* cv) {
   const size_t words = size_t(cv->nc) * ws;
   bits0_.ensure(sizeof(uint64_t) * std::max<size_t>(words, 1));
   bits_.ensure(sizeof(uint64_t) * std::max<size_t>(words, 1));
-  fbits_.ensure(sizeof(uint64_t) * std::max<size_t>(words, 1));
   pref0_.ensure(sizeof(uint32_t) * std::max<size_t>(words, 1));
   cv->dense = true;
   cv->ws = ws;
   cv->bits0 = bits0_.as<uint64_t>();
   cv->bits = bits_.as<uint64_t>();
-  cv->fbits = fbits_.as<uint64_t>();
   cv->pref0 = pref0_.as<uint32_t>();
   dense_rows(cv->off_u, cv->adj_u, cv->nc, ws, cv->bits0, cv->bits, cv->pref0, stream_);
-  fill_u64(cv->fbits, words, 0, stream_);
   cv->eidm = nullptr;
   const uint64_t eb = sizeof(uint32_t) * uint64_t(cv->nc) * cv->nc;
   if (eb && eb <= eidm_budget_) {
@@ -741,29 +739,6 @@ bool Solver::try_redensify(CoreView* cv) {
 
 // ------------------------------------------------------------- (d) peel ---
 
-// The round rule decides on the device whether a frontier of c edges
-// (supports < thr) is cheaper to drop with an exact recount of the alive
-// edges than to walk triangle by triangle. Dense cores: a recount is
-// alive * ws word ANDs, a frontier walk c * (ws + tri_cost * thr) random
-// lookups and atomics, so a few percent of the alive edges already favour
-// the recount. Sorted-row cores pay a compaction and a rebuild first: the
-// reference's third (src/kc.cu:988) scaled by drop_ratio.
-// Truss levels on the core view, upward from threshold thr0 (an edge stays
-// while its support >= thr, i.e. in the (thr+2)-truss). Empty levels are
-// skipped by jumping to the minimum live support. With early_ans != 0, a
-// first level of exactly early_ans edges at kmax early_k ends the search
-// (src/kc.cu:1240-1241).
-RoundRule Solver::round_rule(const CoreView& cv) const {
-  RoundRule rule{};
-  rule.dense = cv.dense ? 1u : 0u;
-  rule.ws = cv.ws;
-  rule.mc = cv.mc;
-  rule.tri_cost = dense_tri_cost_;
-  rule.drop_fixed = dense_drop_fixed_;
-  rule.drop_ratio = sparse_drop_ratio_;
-  return rule;
-}
-
 PeelArgs Solver::peel_args(const CoreView& cv) {
   PeelArgs a{};
   a.q0 = eq0_.as<uint32_t>();
@@ -775,19 +750,9 @@ PeelArgs Solver::peel_args(const CoreView& cv) {
   a.del_thr = cv.del_thr;
   a.sup = cv.sup;
   a.mc = cv.mc;
-  a.nc = cv.nc;
-  a.ws = cv.ws;
   a.off_u = cv.off_u;
   a.adj_u = cv.adj_u;
   a.eid_u = cv.eid_u;
-  a.off_d = cv.off_d;
-  if (cv.dense) {
-    a.bits = cv.bits;
-    a.fbits = cv.fbits;
-    a.bits0 = cv.bits0;
-    a.pref0 = cv.pref0;
-    a.eidm = cv.eidm;
-  }
   return a;
 }
 
@@ -796,7 +761,7 @@ void Solver::start_rounds(CoreView* cv, int32_t thr, uint32_t r, uint64_t alive,
   const PeelArgs a = peel_args(*cv);
   zero_u32(&ctl_->qcount[0]);
   edge_frontier_init(cv->state, cv->sup, cv->mc, thr, a.q0, &ctl_->qcount[0], stream_);
-  const RoundRule rule = round_rule(*cv);
+  const RoundRule rule{cv->mc, 0, sparse_drop_ratio_};
   round_start(ctl_, r, alive, thr, rule, reset, search, stream_);
   round_stamp(a, ctl_, rule, stream_);
 }
@@ -815,12 +780,10 @@ TrussOutcome Solver::truss_search(CoreView* cv, int32_t thr0, uint64_t early_ans
   search.early_ans = early_ans;
   search.early_k = early_k;
   search.exact_early = exact_early ? 1u : 0u;
-  if (!cv->dense) {
-    if (list_triangles(*cv)) return run_lists(*cv, thr0, search);
-    if (!cv->off_u) build_undirected_view(cv);
-  }
   uint32_t r = 1;
-  return run_levels(cv, thr0, cv->mc, &r, search, true);
+  if (cv->dense || list_triangles(*cv)) return run_steps(cv, thr0, cv->mc, &r, search, true);
+  if (!cv->off_u) build_undirected_view(cv);
+  return run_levels(cv, thr0, search);
 }
 
 // Triangle lists of a base view whose supports are counted: offsets in
@@ -830,8 +793,8 @@ TrussOutcome Solver::truss_search(CoreView* cv, int32_t thr0, uint64_t early_ans
 bool Solver::list_triangles(const CoreView& cv) {
   const uint32_t mc = cv.mc;
   if (cv.work != -1) return false;
-  list_ctl_.ensure(sizeof(ListState) * 2 + sizeof(ListCounters) * 3 + sizeof(uint64_t));
-  uint64_t* total = reinterpret_cast<uint64_t*>(list_ctl_.as<uint8_t>() + sizeof(ListState) * 2 + sizeof(ListCounters) * 3);
+  step_ctl_.ensure(kStepCtlBytes + sizeof(uint64_t));
+  uint64_t* total = reinterpret_cast<uint64_t*>(step_ctl_.as<uint8_t>() + kStepCtlBytes);
   fill_u64(total, 1, 0, stream_);
   sum_u32(reinterpret_cast<const uint32_t*>(cv.sup), mc, total, stream_);
   const uint64_t entries = read_u64(total), bytes = entries * sizeof(uint2);
@@ -856,80 +819,135 @@ bool Solver::list_triangles(const CoreView& cv) {
   return true;
 }
 
-// The search over the lists; steps are queued in batches and the state read
-// once per batch.
-TrussOutcome Solver::run_lists(const CoreView& cv, int32_t thr0, const SearchRule& search) {
-  constexpr uint32_t kFirstBatch = 8, kMaxBatch = 64;
-  const uint32_t mc = cv.mc;
-  ListArgs a{};
-  a.states = list_ctl_.as<ListState>();
-  a.counters = reinterpret_cast<ListCounters*>(a.states + 2);
-  a.tri_off = tri_off_.as<uint32_t>();
-  a.tri = tri_.as<uint2>();
-  a.state = cv.state;
-  a.del_thr = cv.del_thr;
-  a.sup = cv.sup;
-  a.q[0] = eq0_.as<uint32_t>();
-  a.q[1] = eq1_.as<uint32_t>();
-  a.live[0] = live_[0].as<uint32_t>();
-  a.live[1] = live_[1].as<uint32_t>();
-  ListState h{};
-  h.thr = thr0;
-  h.live = mc;
-  h.alive = mc;
+// Levels from threshold thr with `alive` live edges over triangle lists or
+// dense rows (kt_step.hip), until the search rule ends them or the level
+// empties. Steps are queued in batches and the state is read once per batch;
+// with allow_host the search stops at dropped frontiers of a dense core that
+// may shrink its matrix (try_redensify). *r is the next round stamp on entry
+// and on exit.
+TrussOutcome Solver::run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32_t* r_io, const SearchRule& search,
+                               bool allow_host) {
+  constexpr uint32_t kFirstBatch = 8, kMaxBatch = 32;
+  static_assert(sizeof(StepState) * 2 + sizeof(StepCounters) * 3 <= kStepCtlBytes, "step control block too small");
+  static_assert(sizeof(StepState) <= 4 * kTrussCountWord, "state exceeds the pinned readback buffer");
+  step_ctl_.ensure(kStepCtlBytes + sizeof(uint64_t));
+  TrussOutcome out;
+  StepState h{};
+  h.round = *r_io - 1;
+  h.thr = thr;
+  h.live = cv->mc;
+  h.alive = h.host_at = alive;
   h.first = 1;
   h.level_floor = -1;
   h.early_k = search.early_k;
   h.exact_early = search.exact_early;
   h.early_ans = search.early_ans;
-  list_start(a, h, stream_);
-  uint64_t steps = 0;
-  for (uint32_t batch = kFirstBatch;; batch = std::min(batch * 2, kMaxBatch)) {
-    if (steps > 4 * uint64_t(mc) + 4 * kMaxBatch) fail("edge peel did not converge");
-    list_steps(a, mc, uint32_t(steps), batch, stream_);
-    steps += batch;
-    static_assert(sizeof(ListState) <= 252, "state exceeds the pinned readback buffer");
-    KT_HIP(hipMemcpyAsync(pinned_, a.states + (steps & 1), sizeof(ListState), hipMemcpyDeviceToHost, stream_));
-    KT_HIP(hipStreamSynchronize(stream_));
-    std::memcpy(&h, pinned_, sizeof(h));
-    if (trace_)
-      std::fprintf(stderr, "[kt] list steps=%llu phase=%u thr=%d alive=%llu live=%u levels=%u rounds=%u\n",
-                   (unsigned long long)steps, h.phase, h.thr, h.alive, h.live, h.levels, h.rounds);
-    if (h.err) fail("edge peel bookkeeping mismatch (live count)");
-    if (h.phase == kListDone || h.phase == kListEmpty) break;
+  h.max_levels = search.max_levels;
+  for (;;) {  // until the search ends; again after each stop for the host
+    const StepArgs a = step_args(*cv);
+    StepRule rule{};
+    rule.dense = cv->dense ? 1u : 0u;
+    rule.ws = cv->ws;
+    rule.relist = cv->dense ? 0u : 1u;
+    rule.host = cv->dense && allow_host ? 1u : 0u;
+    rule.tri_cost = dense_tri_cost_;
+    rule.drop_fixed = dense_drop_fixed_;
+    steps_start(a, h, stream_);
+    uint64_t steps = 0;
+    uint32_t batch = kFirstBatch;
+    do {
+      // a step removes an edge, completes a level or prepares one that does
+      if (steps > 4 * uint64_t(cv->mc) + 4 * kMaxBatch) fail("edge peel did not converge");
+      const bool probe = cv->dense && probe_kernel_ == kProbeDensePeel;  // measurement
+      steps_run(a, rule, cv->mc, uint32_t(steps), batch, stream_,
+                probe && (probe_push_ & 1) ? probe_events(int(batch)) : nullptr);
+      steps += batch;
+      KT_HIP(hipMemcpyAsync(pinned_, a.states + (steps & 1), sizeof(StepState), hipMemcpyDeviceToHost, stream_));
+      KT_HIP(hipStreamSynchronize(stream_));
+      std::memcpy(&h, pinned_, sizeof(h));
+      if (trace_)
+        std::fprintf(stderr, "[kt] edge-peel batch=%u phase=%u thr=%d alive=%llu mc=%u frontier=%u levels=%u rounds=%u recounts=%u\n",
+                     batch, h.phase, h.thr, h.alive, cv->mc, h.cnt, h.levels, h.rounds, h.recounts);
+      if (h.err) fail("edge peel bookkeeping mismatch (live count)");
+      if (steps >= 2 * batch) batch = std::min(batch * 2, kMaxBatch);
+    } while (h.phase != kStepDone && h.phase != kStepEmpty && h.phase != kStepHost);
+    if (h.phase != kStepHost) break;
+    h.host_at = h.alive;
+    if (try_redensify(cv)) {  // smaller matrix on the vertices left, exact recount
+      if (cv->mc != h.alive) fail("edge peel bookkeeping mismatch (redensify)");
+      ++out.compactions;
+      h.phase = kStepStart;
+      h.live = cv->mc;
+      h.round = h.cur = h.cnt = h.pend_cnt = 0;
+    } else {
+      h.phase = kStepResume;
+    }
   }
-  TrussOutcome out;
+  if (h.phase == kStepEmpty) h.alive = 0;
+  *r_io = h.round + 1;
   out.kmax = h.level_kmax;
   out.count = h.level_count;
-  out.alive = h.phase == kListEmpty ? 0 : h.alive;
+  out.alive = h.alive;
+  out.cut_short = h.alive > 0 && search.max_levels && h.levels >= search.max_levels;
   out.floor_thr = h.level_floor;
   out.levels = h.levels;
   out.rounds = h.rounds;
-  out.compactions = h.relists;
+  out.compactions += h.relists;
+  out.recounts = h.recounts;
   return out;
 }
 
-// Runs levels from threshold thr with `alive` live edges on the device until
-// the search rule ends it (or the level empties); handles dropped frontiers
-// and compactions. *r is the next round stamp on entry and on exit.
-TrussOutcome Solver::run_levels(CoreView* cv, int32_t thr, uint64_t alive, uint32_t* r_io, const SearchRule& search,
-                                bool allow_redensify) {
+StepArgs Solver::step_args(const CoreView& cv) {
+  StepArgs a{};
+  a.states = step_ctl_.as<StepState>();
+  a.counters = reinterpret_cast<StepCounters*>(a.states + 2);
+  a.orig = cv.work == -1 ? nullptr : cv.orig;
+  a.state = cv.state;
+  a.del_thr = cv.del_thr;
+  a.sup = cv.sup;
+  a.q[0] = eq0_.as<uint32_t>();
+  a.q[1] = eq1_.as<uint32_t>();
+  a.q[2] = eq2_.as<uint32_t>();
+  if (!cv.dense) {
+    a.live[0] = live_[0].as<uint32_t>();
+    a.live[1] = live_[1].as<uint32_t>();
+    a.tri_off = tri_off_.as<uint32_t>();
+    a.tri = tri_.as<uint2>();
+    return a;
+  }
+  a.src = cv.src;
+  a.dst = cv.adj_d;
+  a.off_d = cv.off_d;
+  a.nc = cv.nc;
+  a.ws = cv.ws;
+  a.bits = reinterpret_cast<unsigned long long*>(cv.bits);
+  a.bits0 = reinterpret_cast<const unsigned long long*>(cv.bits0);
+  a.pref0 = cv.pref0;
+  a.off_u = cv.off_u;
+  a.adj_u = cv.adj_u;
+  a.eid_u = cv.eid_u;
+  a.eidm = cv.eidm;
+  if (probe_kernel_ == kProbeDensePeel && (probe_push_ & 2)) a.stats = probe_stats_.as<unsigned long long>();
+  return a;
+}
+
+// Levels of a sorted-row core without triangle lists from threshold thr until
+// the search rule ends them or the level empties; handles dropped frontiers
+// (a recount costs a compaction and a rebuild first: the reference's third of
+// the live edges, src/kc.cu:988, scaled by drop_ratio) and compactions.
+TrussOutcome Solver::run_levels(CoreView* cv, int32_t thr, const SearchRule& search) {
   constexpr int kMaxBatch = 32;
   TrussOutcome out;
-  uint32_t r = *r_io;
+  uint32_t r = 1;
+  uint64_t alive = cv->mc;
   start_rounds(cv, thr, r, alive, true, search);
   int batch = 2;
   uint64_t queued = 0;  // rounds since the last restart; each removes an edge or changes level
   for (;;) {
     if (queued > 3 * uint64_t(cv->mc) + 4 * kMaxBatch) fail("edge peel did not converge");
     const double avg = cv->nc ? double(2ull * cv->mc) / cv->nc : 0.0;
-    LaunchProbe probe;
-    if (probe_kernel_ == kProbeDensePeel && cv->dense) {  // measurement of the dense peel round
-      if (probe_push_ & 1) probe.ev = probe_events(batch);
-      if (probe_push_ & 2) probe.stats = probe_stats_.as<unsigned long long>();
-    }
-    peel_rounds(peel_args(*cv), ctl_, round_rule(*cv), lanes_peel_ ? lanes_peel_ : auto_lanes(avg), batch, stream_,
-                probe);
+    const RoundRule rule{cv->mc, 0, sparse_drop_ratio_};
+    peel_rounds(peel_args(*cv), ctl_, rule, lanes_peel_ ? lanes_peel_ : auto_lanes(avg), batch, stream_);
     queued += batch;
     const Ctl h = read_ctl();
     if (trace_)
@@ -946,43 +964,25 @@ TrussOutcome Solver::run_levels(CoreView* cv, int32_t thr, uint64_t alive, uint3
       continue;
     }
     out.alive = h.alive;
-    r = h.round + 1;
-    if (h.action == kRoundDone || h.action == kRoundEmpty) {
-      out.cut_short = h.action == kRoundDone && h.alive > 0 && search.max_levels && h.levels >= search.max_levels;
-      break;
-    }
+    if (h.action == kRoundDone || h.action == kRoundEmpty) break;
     alive = h.alive;
     thr = h.thr;
     if (h.action == kRoundDrop) {  // drop the stamped frontier, recount the rest exactly
       ++out.recounts;
-      if (cv->dense) {
-        if (allow_redensify && try_redensify(cv)) {  // smaller matrix on the vertices left, exact recount
-          if (cv->mc != alive) fail("edge peel bookkeeping mismatch (redensify)");
-          ++out.compactions;
-          r = 1;
-        } else {
-          frontier_clear(peel_args(*cv), ctl_, stream_);
-          dense_support(cv->off_d, cv->adj_d, cv->nc, cv->mc, cv->bits, cv->ws, cv->state, cv->sup, stream_);
-        }
-      } else {
-        compact_core(cv, false);
-        ++out.compactions;
-        alive = cv->mc;
-        r = 1;
-      }
+      compact_core(cv, false);
+      alive = cv->mc;
     } else if (h.action == kRoundCompact) {  // half the edges are dead: compact, keep supports
       compact_core(cv, true);
-      ++out.compactions;
       if (cv->mc != alive) fail("edge peel bookkeeping mismatch (compaction)");
-      r = 1;
     } else {
       fail("edge peel: unexpected round action");
     }
+    ++out.compactions;
+    r = 1;
     start_rounds(cv, thr, r, alive, false, search);
     batch = 2;
     queued = 0;
   }
-  *r_io = r;
   return out;
 }
 
@@ -1007,7 +1007,7 @@ TrussOutcome Solver::truss_gallop(CoreView* cv, int64_t empty_from) {
   walk.max_levels = walk_levels_;
   uint32_t r = 1;
   if (trace_) trace_ms();
-  TrussOutcome lv = run_levels(cv, 1, cv->mc, &r, walk, true);
+  TrussOutcome lv = run_steps(cv, 1, cv->mc, &r, walk, true);
   if (trace_)
     std::fprintf(stderr, "[kt] gallop walk of %u levels: lo=%d alive=%llu rounds=%llu (%.2f ms)\n", lv.levels,
                  int(lv.kmax) - 2, (unsigned long long)lv.count, (unsigned long long)lv.rounds, trace_ms());
@@ -1052,7 +1052,7 @@ TrussOutcome Solver::truss_gallop(CoreView* cv, int64_t empty_from) {
       // view costs a full cascade and is then undone; the walk's only empty
       // level is the last one.
       SearchRule all{};
-      const TrussOutcome w = run_levels(cv, int32_t(lo + 1), alive, &r, all, true);
+      const TrussOutcome w = run_steps(cv, int32_t(lo + 1), alive, &r, all, true);
       out.rounds += w.rounds;
       out.levels += w.levels;
       out.compactions += w.compactions;
@@ -1072,7 +1072,7 @@ TrussOutcome Solver::truss_gallop(CoreView* cv, int64_t empty_from) {
     // probe has emptied the view
     const int64_t t = hi < 0 ? lo + step : !probed_empty ? std::min(lo + step, hi - 1) : lo + (hi - lo) / 2;
     save();
-    const TrussOutcome p = run_levels(cv, int32_t(t), alive, &r, single, false);
+    const TrussOutcome p = run_steps(cv, int32_t(t), alive, &r, single, false);
     out.rounds += p.rounds;
     out.levels += 1;
     out.compactions += p.compactions;

@@ -60,3 +60,43 @@ def test_lists_equal_rows(ctx, sparse_ctx, scale, lanes):
     ref = ctx.solve_pairs(pairs, n)
     assert (r.kmax, r.truss_edges, r.k_hat) == (ref.kmax, ref.truss_edges, ref.k_hat)
     np.testing.assert_array_equal(got, ctx.trussness())
+
+
+@pytest.fixture(scope="module", params=["eid_matrix", "prefix_counts"])
+def dense_ctx(request):
+    """A context that keeps every core in bit-matrix rows; "prefix_counts": no
+    room for the matrix of edge ids."""
+    from kc_cuda_amd import Context
+    mp = pytest.MonkeyPatch()
+    if request.param == "prefix_counts":
+        mp.setenv("KT_EIDM_BUDGET_MB", "0")
+    c = Context(0)
+    mp.undo()
+    c.tune(core="dense")
+    yield c
+    c.close()
+
+
+# row words: one, two, the support count's lane steps (128 and 256), the last
+@pytest.mark.parametrize("n", [64, 65, 2048, 8191, 16385, 65536])
+def test_dense_rows_equal_lists(dense_ctx, n):
+    """The whole decomposition over bit-matrix rows: walks, dropped frontiers
+    cleared edge by edge or by rebuilding the rows, recounts, the stops where
+    the host shrinks the matrix or leaves it."""
+    from kc_cuda_amd import Context
+    rng = np.random.default_rng(n)
+    m = min(n * (n - 1) // 4, 60_000)
+    e = rng.integers(0, n, (m, 2))
+    k = min(n, 300)  # a dense corner: sparse edges go first, in drops
+    c = rng.integers(0, k, (25 * k, 2))
+    e = np.concatenate([e, c, np.column_stack([np.arange(n), (np.arange(n) + 1) % n]),
+                        np.column_stack([np.arange(n), (np.arange(n) + 2) % n])])
+    pairs = np.unique(canon_pairs(e[e[:, 0] != e[:, 1]].astype(np.uint32)), axis=0)
+    r = dense_ctx.solve_pairs(pairs, n)
+    got = dense_ctx.trussness()
+    with Context(0) as other:
+        other.tune(core="sparse")
+        ref = other.solve_pairs(pairs, n)
+        want = other.trussness()
+    assert (r.kmax, r.truss_edges, r.k_hat) == (ref.kmax, ref.truss_edges, ref.k_hat)
+    np.testing.assert_array_equal(got, want)
