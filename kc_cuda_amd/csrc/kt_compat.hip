@@ -189,7 +189,7 @@ void Solver::view_from_oriented_host(uint32_t nc, const uint32_t* h_off_d, const
   cv->state = state_.as<uint32_t>();
   cv->work = -1;
   build_undirected_view(cv);
-  if (core_mode_ == 2 ? nc <= 65536 : (core_mode_ == 0 && dense_fits(nc, mc))) make_dense(cv);
+  if (wants_dense(nc, mc)) make_dense(cv);
 }
 
 void Solver::undirected_to_host(const CoreView& cv, uint32_t* adj_u, uint32_t* eid_u, uint32_t* lson,
@@ -269,7 +269,7 @@ int kc_count_deg_with_mask(const uint32_t* nbr, const uint32_t* nbr_u, uint32_t 
     std::vector<uint32_t> dm(N);
     s.level0_degrees_to_host(dm.data());
     kt::CoreView cv;
-    s.extract_core(s.level0(), &cv);
+    s.extract_core(s.level0(), &cv, false);
     const uint32_t nc = cv.nc;
     std::vector<uint32_t> inv(nc), dout(nc), pos(N, 0);
     s.core_ranks_to_host(cv, inv.data(), dout.data());

@@ -127,9 +127,11 @@ void degree_hist(const uint32_t* deg, uint32_t n, uint32_t* hist, hipStream_t s)
 void core_filter(const uint32_t* deg, uint32_t n, uint32_t k, uint32_t* lvl, uint32_t* alive, hipStream_t s);
 
 // (a1-a3) core subgraph extraction.
-// key = degree << 32 | ~original id (to_orig may be null: identity), val = local id
+// key = degree << 32 | ~original id (to_orig may be null: identity), val =
+// local id of every alive vertex; to = kNone for the others; found[0] (low
+// word) = how many, found[1] = the sum of their degrees
 void core_collect(const uint32_t* lvl, const uint32_t* deg, const uint32_t* to_orig, uint32_t n,
-                  uint64_t* keys, uint32_t* vals, uint32_t* count, hipStream_t s);
+                  uint64_t* keys, uint32_t* vals, uint32_t* to, uint64_t* found, hipStream_t s);
 void core_assign_rank(const uint64_t* sorted_keys, const uint32_t* sorted_vals, uint32_t nc,
                       uint32_t* to, uint32_t* inv, uint32_t* inv_orig, hipStream_t s);
 // (b') induced subgraph of the alive vertices
@@ -243,6 +245,19 @@ void row_compact(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* o
                  const int32_t* sup, const uint32_t* state, uint32_t nc, const uint32_t* off2,
                  uint32_t* adj2, uint32_t* src2, uint32_t* orig2, int32_t* sup2, hipStream_t s);
 void count_in_degrees(const uint32_t* adj, uint32_t m, uint32_t* din, hipStream_t s);
+// Dense core views through their bit-matrix rows (kt_dense.hip), in this
+// order: rows of the level's vertices inv[0..nc) in rank ids (to); the offsets
+// (*simple = 0 and no edge when the bits do not stand for `slots` row slots);
+// every array of the view (eidm nullable). max_row: *out = the longest row.
+void rank_rows(const uint64_t* off, const uint32_t* adj, const uint32_t* to, const uint32_t* inv, uint32_t nc,
+               uint32_t ws, uint64_t* bits0, uint64_t* bits, uint32_t* pref0, uint32_t* du, uint32_t* dout,
+               hipStream_t s);
+void rank_scan(const uint32_t* du, const uint32_t* dout, uint32_t nc, uint64_t slots, uint32_t* off_d,
+               uint32_t* off_u, uint32_t* ebase, uint32_t* simple, hipStream_t s);
+void rank_fill(const uint64_t* bits0, const uint32_t* pref0, const uint32_t* off_u, const uint32_t* ebase, uint32_t nc,
+               uint32_t ws, uint32_t* adj_u, uint32_t* eid_u, uint32_t* adj_d, uint32_t* src, uint32_t* orig,
+               uint32_t* state, uint32_t* del_thr, uint32_t* eidm, hipStream_t s);
+void max_row(const uint32_t* off, uint32_t rows, uint32_t* out, hipStream_t s);
 // Triangle lists (kt_list.hip). sum_u32: *total (starts at 0) += the sum.
 // tri_fill: every triangle's entries, cursor starting as a copy of the offsets
 // (bitmap, lanes: as the support count's kernels).

@@ -889,15 +889,26 @@ __global__ void k_core_reopen_above(uint32_t* lvl, uint32_t n, uint32_t k) {
 __global__ __launch_bounds__(kBlock) void k_core_collect(const uint32_t* __restrict__ lvl,
                                                          const uint32_t* __restrict__ deg,
                                                          const uint32_t* __restrict__ to_orig, uint32_t n,
-                                                         uint64_t* keys, uint32_t* vals, uint32_t* count) {
+                                                         uint64_t* keys, uint32_t* vals, uint32_t* to,
+                                                         unsigned long long* found) {
+  unsigned long long sum = 0;
   tile_compact(
-      n, [&](uint64_t v) { return lvl[v] == kNone; },
-      [&](uint32_t at, uint64_t v) {
-        const uint32_t id = to_orig ? to_orig[v] : uint32_t(v);
-        keys[at] = uint64_t(deg[v]) << 32 | uint64_t(0xFFFFFFFFu - id);
-        vals[at] = uint32_t(v);
+      n,
+      [&](uint64_t v) {
+        const bool alive = lvl[v] == kNone;
+        if (!alive) to[v] = kNone;
+        return alive;
       },
-      count);
+      [&](uint32_t at, uint64_t v) {
+        const uint32_t id = to_orig ? to_orig[v] : uint32_t(v), d = deg[v];
+        keys[at] = uint64_t(d) << 32 | uint64_t(0xFFFFFFFFu - id);
+        vals[at] = uint32_t(v);
+        sum += d;
+      },
+      reinterpret_cast<uint32_t*>(&found[0]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+  if (lane64() == 0 && sum) atomicAdd(&found[1], sum);
 }
 
 // sorted (key, local id) -> rank maps; inv_orig carries the input's ids
@@ -2007,8 +2018,11 @@ void core_reopen_above(uint32_t* lvl, uint32_t n, uint32_t k, hipStream_t s) {
 }
 
 void core_collect(const uint32_t* lvl, const uint32_t* deg, const uint32_t* to_orig, uint32_t n,
-                  uint64_t* keys, uint32_t* vals, uint32_t* count, hipStream_t s) {
-  if (n) k_core_collect<<<grid_tiles(n), kBlock, 0, s>>>(lvl, deg, to_orig, n, keys, vals, count);
+                  uint64_t* keys, uint32_t* vals, uint32_t* to, uint64_t* found, hipStream_t s) {
+  fill_u64(found, 2, 0, s);
+  if (n)
+    k_core_collect<<<grid_tiles(n), kBlock, 0, s>>>(lvl, deg, to_orig, n, keys, vals, to,
+                                                    reinterpret_cast<unsigned long long*>(found));
 }
 void core_assign_rank(const uint64_t* keys, const uint32_t* vals, uint32_t nc, uint32_t* to, uint32_t* inv,
                       uint32_t* inv_orig, hipStream_t s) {

@@ -242,7 +242,11 @@ class Solver {
   // bound), from the degree histogram of the current input; ~0 when none.
   uint64_t degree_at_least(uint32_t k) const;
   void core_at(uint32_t k);  // leaves the k-core alive on the deepest usable level
-  void extract_core(LevelGraph& g, CoreView* cv);
+  // symmetric: every row slot has its mirror (false: the rows come from the
+  // caller unchecked)
+  void extract_core(LevelGraph& g, CoreView* cv, bool symmetric = true);
+  bool extract_dense(LevelGraph& g, CoreView* cv, uint64_t slots);
+  bool wants_dense(uint32_t nc, uint32_t mc) const;
   void sort_oriented_rows(uint32_t nc, uint32_t mc, uint32_t max_row);
   void build_undirected_view(CoreView* cv);
   void count_support(CoreView* cv, float* ms);
@@ -318,7 +322,7 @@ class Solver {
   uint32_t* pinned_ = nullptr;
   uint32_t* pinned_hist_ = nullptr;  // kDegBins words of pinned memory (none in arena mode)
   uint32_t host_rb_[64] = {};  // readback buffer in arena mode
-  hipEvent_t ev_[10];
+  hipEvent_t ev_[11];
   int lanes_count_ = 0, lanes_peel_ = 0;
   bool force_edge_count_ = false;
   bool force_atomic_build_ = false;

@@ -532,7 +532,7 @@ void Solver::sort_oriented_rows(uint32_t nc, uint32_t mc, uint32_t max_row) {
   KT_HIP(hipMemcpyAsync(adj_d_.p, tkeys_.p, sizeof(uint32_t) * mc, hipMemcpyDeviceToDevice, stream_));
 }
 
-void Solver::extract_core(LevelGraph& g, CoreView* cv) {
+void Solver::extract_core(LevelGraph& g, CoreView* cv, bool symmetric) {
   core_valid_ = false;  // the core buffers are rewritten
   const uint32_t n = g.n;
   const size_t nn = size_t(n_) + 1;
@@ -541,19 +541,34 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   vals_.ensure(sizeof(uint32_t) * nn);
   vals2_.ensure(sizeof(uint32_t) * nn);
   to_.ensure(sizeof(uint32_t) * nn);
-  zero_u32(&ctl_->nalive);
-  core_collect(g.lvl, g.deg, g.to_orig, n, keys_.as<uint64_t>(), vals_.as<uint32_t>(), &ctl_->nalive, stream_);
-  const uint32_t nc = read_u32(&ctl_->nalive);
+  core_out_.ensure(64);
+  uint64_t* found = core_out_.as<uint64_t>();
+  core_collect(g.lvl, g.deg, g.to_orig, n, keys_.as<uint64_t>(), vals_.as<uint32_t>(), to_.as<uint32_t>(), found,
+               stream_);
+  KT_HIP(hipMemcpyAsync(pinned_, found, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_));
+  KT_HIP(hipStreamSynchronize(stream_));
+  uint64_t got[2];
+  std::memcpy(got, pinned_, sizeof(got));
+  const uint32_t nc = uint32_t(got[0]);
+  const uint64_t by_degree = got[1] / 2;  // the core's edges
   *cv = CoreView{};
   cv->nc = cv->nc0 = nc;
   inv_.ensure(sizeof(uint32_t) * (size_t(nc) + 1));
   inv_orig_.ensure(sizeof(uint32_t) * (size_t(nc) + 1));
   dout_.ensure(sizeof(uint32_t) * (size_t(nc) + 1));
   off_d_.ensure(sizeof(uint32_t) * (size_t(nc) + 1));
-  sort_pairs_u64(keys_.as<uint64_t>(), keys2_.as<uint64_t>(), vals_.as<uint32_t>(), vals2_.as<uint32_t>(), nc);
-  fill_u32(to_.as<uint32_t>(), n, kNone, stream_);
+  // a degree in the core is below nc
+  int deg_bits = 1;
+  while (deg_bits < 32 && (uint64_t(1) << deg_bits) < nc) ++deg_bits;
+  sort_pairs_u64(keys_.as<uint64_t>(), keys2_.as<uint64_t>(), vals_.as<uint32_t>(), vals2_.as<uint32_t>(), nc,
+                 32 + deg_bits);
   core_assign_rank(keys2_.as<uint64_t>(), vals2_.as<uint32_t>(), nc, to_.as<uint32_t>(), inv_.as<uint32_t>(),
                    inv_orig_.as<uint32_t>(), stream_);
+  // rows that repeat a neighbour or hold their own vertex do not survive as
+  // bits: their view is built from the rows themselves
+  if (symmetric && by_degree < 0x7FFFFFFFull && wants_dense(nc, uint32_t(by_degree)) &&
+      extract_dense(g, cv, got[1]))
+    return;
   fill_u32(dout_.as<uint32_t>(), uint64_t(nc) + 1, 0, stream_);
   orient_count(g.off, g.adj, to_.as<uint32_t>(), inv_.as<uint32_t>(), nc, dout_.as<uint32_t>(), stream_);
   exclusive_scan_u32(dout_.as<uint32_t>(), off_d_.as<uint32_t>(), nc + 1);
@@ -588,10 +603,75 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   cv->sup = sup_.as<int32_t>();
   cv->state = state_.as<uint32_t>();
   cv->work = -1;
-  if (core_mode_ == 2 ? cv->nc <= 65536 : (core_mode_ == 0 && dense_fits(cv->nc, cv->mc))) {
+  // a sorted-row view gets its undirected rows only if its triangles are not
+  // listed
+  if (wants_dense(nc, mc)) {
     build_undirected_view(cv);
     make_dense(cv);
-  }  // a sorted-row view gets its undirected rows only if its triangles are not listed
+  }
+}
+
+// Whether a core of this size gets bit-matrix rows.
+bool Solver::wants_dense(uint32_t nc, uint32_t mc) const {
+  return core_mode_ == 2 ? nc <= 65536 : (core_mode_ == 0 && dense_fits(nc, mc));
+}
+
+// The view of a dense core through its bit-matrix rows (kt_dense.hip): no
+// count, sort or transpose of its rows, and one wait, taken while the view is
+// filled. `slots` = the sum of the core's degrees. False: the rows do not
+// describe a simple graph, nothing is filled.
+bool Solver::extract_dense(LevelGraph& g, CoreView* cv, uint64_t slots) {
+  const uint32_t mc = uint32_t(slots / 2), nc = cv->nc, ws = dense_words(nc);
+  const size_t mm = std::max<uint32_t>(mc, 1), words = std::max<size_t>(size_t(nc) * ws, 1);
+  const size_t rows = sizeof(uint32_t) * (size_t(nc) + 1);
+  din_.ensure(rows);      // degrees
+  din_off_.ensure(rows);  // edge id bases
+  off_u_.ensure(rows);
+  bits0_.ensure(sizeof(uint64_t) * words);
+  bits_.ensure(sizeof(uint64_t) * words);
+  pref0_.ensure(sizeof(uint32_t) * words);
+  for (DevBuf* b : {&adj_d_, &src_, &orig0_, &del_thr_, &state_, &eq0_, &eq1_, &eq2_}) b->ensure(sizeof(uint32_t) * mm);
+  sup_.ensure(sizeof(int32_t) * (mm + 1));
+  adj_u_.ensure(sizeof(uint32_t) * 2 * mm);
+  eid_u_.ensure(sizeof(uint32_t) * 2 * mm);
+  const uint64_t eb = sizeof(uint32_t) * uint64_t(nc) * nc;
+  uint32_t* eidm = nullptr;
+  if (eb && eb <= eidm_budget_) {
+    eidm_.ensure(eb);
+    eidm = eidm_.as<uint32_t>();
+  }
+  rank_rows(g.off, g.adj, to_.as<uint32_t>(), inv_.as<uint32_t>(), nc, ws, bits0_.as<uint64_t>(),
+            bits_.as<uint64_t>(), pref0_.as<uint32_t>(), din_.as<uint32_t>(), dout_.as<uint32_t>(), stream_);
+  uint32_t* simple = core_out_.as<uint32_t>();
+  rank_scan(din_.as<uint32_t>(), dout_.as<uint32_t>(), nc, slots, off_d_.as<uint32_t>(), off_u_.as<uint32_t>(),
+            din_off_.as<uint32_t>(), simple, stream_);
+  KT_HIP(hipMemcpyAsync(pinned_, simple, sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
+  KT_HIP(hipEventRecord(ev_[10], stream_));
+  rank_fill(bits0_.as<uint64_t>(), pref0_.as<uint32_t>(), off_u_.as<uint32_t>(), din_off_.as<uint32_t>(), nc, ws,
+            adj_u_.as<uint32_t>(), eid_u_.as<uint32_t>(), adj_d_.as<uint32_t>(), src_.as<uint32_t>(),
+            orig0_.as<uint32_t>(), state_.as<uint32_t>(), del_thr_.as<uint32_t>(), eidm, stream_);
+  KT_HIP(hipEventSynchronize(ev_[10]));
+  if (!pinned_[0]) return false;
+  cv->mc = cv->mc0 = mc;
+  cv->inv = inv_orig_.as<uint32_t>();
+  cv->off_d = cv->off_d0 = off_d_.as<uint32_t>();
+  cv->adj_d = cv->adj_d0 = adj_d_.as<uint32_t>();
+  cv->src = cv->src0 = src_.as<uint32_t>();
+  cv->orig = orig0_.as<uint32_t>();
+  cv->del_thr = del_thr_.as<uint32_t>();
+  cv->sup = sup_.as<int32_t>();
+  cv->state = state_.as<uint32_t>();
+  cv->off_u = off_u_.as<uint32_t>();
+  cv->adj_u = adj_u_.as<uint32_t>();
+  cv->eid_u = eid_u_.as<uint32_t>();
+  cv->work = -1;
+  cv->dense = true;
+  cv->ws = ws;
+  cv->bits0 = bits0_.as<uint64_t>();
+  cv->bits = bits_.as<uint64_t>();
+  cv->pref0 = pref0_.as<uint32_t>();
+  cv->eidm = eidm;
+  return true;
 }
 
 // Bit-matrix rows of the core (all edges, live edges) plus per-word prefix
@@ -657,7 +737,8 @@ void Solver::build_undirected_view(CoreView* cv) {
 // ------------------------------------------------------------ (c) count ---
 
 void Solver::count_support(CoreView* cv, float* ms) {
-  fill_u32(reinterpret_cast<uint32_t*>(cv->sup), cv->mc, 0, stream_);
+  // (the dense count writes every support)
+  if (!cv->dense) fill_u32(reinterpret_cast<uint32_t*>(cv->sup), cv->mc, 0, stream_);
   const double avg = cv->nc ? double(cv->mc) / cv->nc : 0.0;
   const int lanes = lanes_count_ ? lanes_count_ : auto_lanes(avg);
   KT_HIP(hipEventRecord(ev_[8], stream_));
@@ -1221,6 +1302,10 @@ void Solver::last_stats(kt_stats* out) {
   out->truss_edges = last_truss_;
   if (cv.mc0 == 0) return;
   out->max_out_degree = cv.max_dout0;
+  if (cv.dense && !cv.max_dout0) {  // a dense view does not need it
+    max_row(cv.off_d0, cv.nc0, &ctl_->pad[0], stream_);
+    out->max_out_degree = read_u32(&ctl_->pad[0]);
+  }
   DevBuf tmp;
   tmp.ensure(16);
   fill_u64(tmp.as<uint64_t>(), 2, 0, stream_);

@@ -100,3 +100,19 @@ def test_dense_rows_equal_lists(dense_ctx, n):
         want = other.trussness()
     assert (r.kmax, r.truss_edges, r.k_hat) == (ref.kmax, ref.truss_edges, ref.k_hat)
     np.testing.assert_array_equal(got, want)
+
+
+# a row: one word, whole runs of words and one more, more slots than one pass
+# over a row takes
+@pytest.mark.parametrize("n", [3, 64, 1024, 1025, 2050])
+def test_dense_views_of_cliques(dense_ctx, n):
+    """A clique hung with triangles: the level's rows hold vertices outside
+    the core, ranks run against ids."""
+    u, v = np.triu_indices(n, 1)
+    t = np.arange(n)
+    pairs = np.concatenate([np.column_stack([u, v]), np.column_stack([t, n + t])]).astype(np.uint32)
+    pairs = canon_pairs((2 * n - 1 - pairs).astype(np.uint32))
+    r = dense_ctx.solve_pairs(pairs, 2 * n)
+    assert (r.kmax, r.truss_edges, r.max_core) == (n, n * (n - 1) // 2, n - 1)
+    got = dense_ctx.truss_edges()
+    assert (got >= n).all() and len(np.unique(got[:, 0].astype(np.uint64) * (2 * n) + got[:, 1])) == len(got)
