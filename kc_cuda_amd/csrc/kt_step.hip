@@ -24,7 +24,13 @@
 namespace kt {
 namespace {
 
+// Workgroups a step gets: the most, and the core's edges for each. A core of
+// 200 edges is walked 64 edges at a time: by one workgroup in 36 us, by one
+// per 32 edges in 9 (256 and 32 edges each, whole solves: 40 vertices 0.61 ->
+// 0.51 ms, 200k edges 3.25 -> 3.02 ms with the two round trips less; the same
+// from 16 to 64 edges each, and for cores that fill the grid).
 constexpr int kStepGrid = 1024;
+constexpr uint32_t kGridEdges = 32;
 constexpr uint32_t kListUnroll = 4;   // list entries a lane has in flight
 constexpr uint32_t kDenseUnroll = 8;  // triangles a lane has in flight (dense walk)
 // a dropped frontier of at least 1/32 of the core's edges has the rows rebuilt
@@ -156,7 +162,7 @@ __device__ __forceinline__ void stamp_dead(const StepArgs& a, uint32_t e, uint32
 // leaves 160 k took 585 us, 35 without its appends).
 constexpr uint32_t kOutCap = 1024;
 struct Out {
-  uint32_t e[kOutCap];
+  uint32_t item[kOutCap];
   uint32_t n, base;
 };
 
@@ -165,10 +171,16 @@ __device__ __forceinline__ void out_begin(Out& o) {
   __syncthreads();
 }
 
+// A queue's entry for edge e = (u, v): of a sorted-row core the edge, of a
+// dense one its ends (16 bits each), which name its rows without a detour
+// through the edge's arrays; its id comes from the edge-id matrix while the
+// rows are read.
+__device__ __forceinline__ uint32_t ends(uint32_t u, uint32_t v) { return u << 16 | v; }
+
 // Edges that fall below thr join the next frontier. Every lane of the wave
 // must reach this; what no longer fits in LDS goes to the queue directly.
-__device__ __forceinline__ void append_dead(const StepArgs& a, Out& o, bool p, uint32_t e, uint32_t round, int32_t thr,
-                                            uint32_t* qn, uint32_t* qn_count) {
+__device__ __forceinline__ void append_dead(const StepArgs& a, Out& o, bool p, uint32_t e, uint32_t item,
+                                            uint32_t round, int32_t thr, uint32_t* qn, uint32_t* qn_count) {
   const unsigned long long mask = __ballot(p);
   if (!mask) return;
   const int lane = lane64(), leader = __ffsll(mask) - 1;
@@ -177,9 +189,9 @@ __device__ __forceinline__ void append_dead(const StepArgs& a, Out& o, bool p, u
   at = __shfl(at, leader) + uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
   if (p) {
     stamp_dead(a, e, round, uint32_t(thr));
-    if (at < kOutCap) o.e[at] = e;
+    if (at < kOutCap) o.item[at] = item;
   }
-  wave_append(p && at >= kOutCap, e, qn, qn_count);
+  wave_append(p && at >= kOutCap, item, qn, qn_count);
 }
 
 // Every thread of the workgroup, after its last append.
@@ -188,7 +200,7 @@ __device__ __forceinline__ void out_end(Out& o, uint32_t* qn, uint32_t* qn_count
   const uint32_t n = min(o.n, kOutCap);
   if (threadIdx.x == 0 && n) o.base = atomicAdd(qn_count, n);
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < n; i += kBlock) qn[o.base + i] = o.e[i];
+  for (uint32_t i = threadIdx.x; i < n; i += kBlock) qn[o.base + i] = o.item[i];
 }
 
 // Whom a triangle of frontier edge e with partner edges xa, xb charges
@@ -283,8 +295,8 @@ __device__ __forceinline__ void walk_lists(const StepArgs& a, const StepState& s
       }
 #pragma unroll
       for (uint32_t k = 0; k < kListUnroll; ++k) {
-        append_dead(a, out, da[k] && oa[k] == thr, xa[k], r + 1, thr, qn, qn_count);
-        append_dead(a, out, db[k] && ob[k] == thr, xb[k], r + 1, thr, qn, qn_count);
+        append_dead(a, out, da[k] && oa[k] == thr, xa[k], xa[k], r + 1, thr, qn, qn_count);
+        append_dead(a, out, db[k] && ob[k] == thr, xb[k], xb[k], r + 1, thr, qn, qn_count);
       }
     }
     wave_sync();
@@ -294,7 +306,7 @@ __device__ __forceinline__ void walk_lists(const StepArgs& a, const StepState& s
 
 __device__ __forceinline__ void clear_bits(const StepArgs& a, const uint32_t* q, uint32_t cnt) {
   for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < cnt; i += gridDim.x * kBlock) {
-    const uint32_t e = q[i], u = a.src[e], v = a.dst[e];
+    const uint32_t x = q[i], u = x >> 16, v = x & 0xFFFFu;
     atomicAnd(&a.bits[uint64_t(u) * a.ws + (v >> 6)], ~(1ull << (v & 63)));
     atomicAnd(&a.bits[uint64_t(v) * a.ws + (u >> 6)], ~(1ull << (u & 63)));
   }
@@ -352,8 +364,8 @@ __device__ __forceinline__ void walk_dense(const StepArgs& a, const StepState& s
   };
   for (uint64_t it = uint64_t(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave; it < items; it += nw) {
     const uint32_t qi = uint32_t(it / nch), ch = uint32_t(it - uint64_t(qi) * nch);
-    const uint32_t e = q[qi];
-    const uint32_t u = a.src[e], v = a.dst[e];
+    const uint32_t x = q[qi], u = x >> 16, v = x & 0xFFFFu;
+    const uint32_t e = eid_of(u, v);
     if (a.stats && ch == 0 && lane == 0) {  // measurement: the edge's merge work, d+(u) + d+(v)
       atomicAdd(&a.stats[0], (unsigned long long)(a.off_d[u + 1] - a.off_d[u] + a.off_d[v + 1] - a.off_d[v]));
       atomicAdd(&a.stats[1], 1ull);
@@ -372,10 +384,11 @@ __device__ __forceinline__ void walk_dense(const StepArgs& a, const StepState& s
     s_inc[threadIdx.x] = inc;
     wave_sync();
     for (uint32_t j0 = 0; j0 < total; j0 += kWave * kDenseUnroll) {
-      uint32_t xa[kDenseUnroll], xb[kDenseUnroll], ma[kDenseUnroll], mb[kDenseUnroll];
+      uint32_t w[kDenseUnroll], xa[kDenseUnroll], xb[kDenseUnroll], ma[kDenseUnroll], mb[kDenseUnroll];
 #pragma unroll
       for (uint32_t k = 0; k < kDenseUnroll; ++k) {
         xa[k] = xb[k] = kNone;
+        w[k] = 0;
         const uint32_t j = j0 + k * kWave + uint32_t(lane);
         if (j < total) {
           uint32_t lo = 0, hi = kWave - 1;  // owner: first lane whose inclusive count exceeds j
@@ -388,9 +401,9 @@ __device__ __forceinline__ void walk_dense(const StepArgs& a, const StepState& s
           }
           const unsigned long long tw = s_t[wbase + lo];
           const uint32_t b = select_bit(tw, j - (s_inc[wbase + lo] - uint32_t(__popcll(tw))));
-          const uint32_t w = ((ch * cw + lo) << 6) + b;
-          xa[k] = eid_of(u, w);
-          xb[k] = eid_of(v, w);
+          w[k] = ((ch * cw + lo) << 6) + b;
+          xa[k] = eid_of(u, w[k]);
+          xb[k] = eid_of(v, w[k]);
         }
       }
 #pragma unroll
@@ -408,8 +421,8 @@ __device__ __forceinline__ void walk_dense(const StepArgs& a, const StepState& s
       }
 #pragma unroll
       for (uint32_t k = 0; k < kDenseUnroll; ++k) {
-        append_dead(a, out, da[k] && oa[k] == thr, xa[k], r + 1, thr, qn, qn_count);
-        append_dead(a, out, db[k] && ob[k] == thr, xb[k], r + 1, thr, qn, qn_count);
+        append_dead(a, out, da[k] && oa[k] == thr, xa[k], ends(u, w[k]), r + 1, thr, qn, qn_count);
+        append_dead(a, out, db[k] && ob[k] == thr, xb[k], ends(v, w[k]), r + 1, thr, qn, qn_count);
       }
     }
     wave_sync();
@@ -433,6 +446,7 @@ __device__ __forceinline__ void put_min(uint32_t best, StepCounters* mine) {
 // The live edges below the threshold become the next frontier (none on a
 // peek), the least support among all live edges is found, and where half of
 // the edge list is dead the rest is listed anew.
+template <bool kDense>
 __device__ __forceinline__ void look(const StepArgs& a, const StepState& s, uint32_t* qn, StepCounters* mine) {
   __shared__ uint32_t s_base[2];
   const uint32_t* list = s.listed ? a.live[s.buf] : nullptr;
@@ -498,7 +512,7 @@ __device__ __forceinline__ void look(const StepArgs& a, const StepState& s, uint
     for (uint32_t k = 0; k < kItems; ++k) {
       if ((front >> k) & 1u) {
         stamp_dead(a, e[k], r, uint32_t(thr));
-        qn[at++] = e[k];
+        qn[at++] = kDense ? ends(a.src[e[k]], a.dst[e[k]]) : e[k];
       }
       if (s.compact && ((keep >> k) & 1u)) next[kept++] = e[k];
     }
@@ -541,7 +555,8 @@ __device__ __forceinline__ void recount(const StepArgs& a, const StepState& s, u
         a.sup[e] = int32_t(c);
         best = min(best, c);
       }
-      append_dead(a, out, mine_edge && int32_t(c) < thr, e, r, thr, qn, &mine->frontier);
+      append_dead(a, out, mine_edge && int32_t(c) < thr, e, ends(u, mine_edge ? a.dst[e] : 0u), r, thr, qn,
+                  &mine->frontier);
     }
   }
   out_end(out, qn, &mine->frontier);
@@ -549,17 +564,20 @@ __device__ __forceinline__ void recount(const StepArgs& a, const StepState& s, u
 }
 
 // Step `it`. Bound on the short rounds that a search is mostly made of: a
-// chain of seven dependent memory round trips (state and counters, queue,
-// edge or list bounds, rows or entries, partner ids and stamps, decrements).
+// chain of dependent memory round trips of about 0.7 us each, past the L2
+// (state and counters, queue, rows or list bounds, partner ids or entries,
+// stamps, decrements, append), 7 to 9 us in all. One workgroup that walks
+// short rounds in a loop, without launches, takes as long for each.
 template <bool kDense, bool kEidm, int G>
 __global__ __launch_bounds__(kBlock) void k_step(StepArgs a, StepRule rule, uint32_t it) {
-  const uint32_t phase = a.states[it & 1u].phase;
-  if (phase == kStepDone || phase == kStepHost) {  // nothing to do: a short way out for every other workgroup
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.states[(it + 1) & 1u] = a.states[it & 1u];
+  // (loaded together: one round trip)
+  const StepState was = a.states[it & 1u];
+  const StepCounters got = a.counters[(it + 2) % 3];
+  if (was.phase == kStepDone || was.phase == kStepHost) {  // nothing to do
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.states[(it + 1) & 1u] = was;
     return;
   }
-  const StepState was = a.states[it & 1u];
-  const StepState s = next_step(was, a.counters[(it + 2) % 3], rule);
+  const StepState s = next_step(was, got, rule);
   StepCounters* mine = &a.counters[it % 3];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     a.states[(it + 1) & 1u] = s;
@@ -579,7 +597,7 @@ __global__ __launch_bounds__(kBlock) void k_step(StepArgs a, StepRule rule, uint
     else
       walk_lists(a, s, qn, &mine->frontier);
   } else if (s.phase == kStepLook) {
-    look(a, s, qn, mine);
+    look<kDense>(a, s, qn, mine);
   } else if (kDense && s.phase == kStepClear) {
     if (rebuild)
       rebuild_rows(a);
@@ -627,7 +645,7 @@ void steps_start(const StepArgs& a, const StepState& first, hipStream_t s) {
 void steps_run(const StepArgs& a, const StepRule& rule, uint32_t mc, uint32_t from, uint32_t count, hipStream_t s,
                hipEvent_t* ev) {
   if (rule.dense && a.ws > kDenseMaxWords) fail("dense core: rows longer than the LDS stage");
-  const int grid = int(std::max<uint64_t>(1, std::min<uint64_t>((uint64_t(mc) + kBlock - 1) / kBlock, kStepGrid)));
+  const int grid = int(std::max<uint64_t>(1, std::min<uint64_t>((uint64_t(mc) + kGridEdges - 1) / kGridEdges, kStepGrid)));
   const void* fn = !rule.dense ? reinterpret_cast<const void*>(&k_step<false, false, 8>)
                    : a.eidm    ? dense_step<true>(a.ws)
                                : dense_step<false>(a.ws);
