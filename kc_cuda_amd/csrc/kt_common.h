@@ -152,6 +152,7 @@ struct StepState {
   uint32_t listed, buf;     // it is live[buf] (else every edge)
   uint32_t err;             // live edges left, but none found
   uint32_t recounts;        // dropped frontiers
+  uint32_t pairs;           // recount by all pairs of rows (else by live edge)
   uint32_t relists;         // live edges listed anew
   // levels and the search's end, as in Ctl and SearchRule
   uint32_t levels, first, level_kmax;
@@ -175,6 +176,7 @@ struct StepRule {
   uint32_t host;      // stop for the host before shrinkable recounts
   double tri_cost;    // dense: cost of one triangle visit in word ANDs
   double drop_fixed;  // dense: fixed cost of a recount in word ANDs
+  double pair_cost;   // dense: cost of a recount by all pairs of rows
 };
 
 struct StepArgs {

@@ -18,6 +18,7 @@
 
 #include "kt_device.h"
 #include "kt_kernels.h"
+#include "kt_tile.h"
 
 namespace kt {
 namespace {
@@ -178,6 +179,33 @@ __global__ __launch_bounds__(kBlock) void k_rank_fill(const unsigned long long* 
   }
 }
 
+// Every edge's support through the matrix cores (kt_tile.h): 2 x 2 waves of 64
+// x 64 pairs per workgroup. Bound on the rows' reads: a block of pairs reads
+// 256 rows, so blocks go to the dies (workgroups in turn) in squares of side x
+// side, which share their rows in a die's L2.
+constexpr uint32_t kTileRows = 128;
+template <bool kEidm>
+__global__ __launch_bounds__(kBlock) void k_dense_count(const unsigned long long* __restrict__ bits,
+                                                        EidOf<kEidm> eid_of, uint32_t nb, uint32_t side,
+                                                        int32_t* sup) {
+  constexpr uint32_t kDies = 8;
+  const uint32_t ns = (nb + side - 1) / side, cells = side * side;
+  const uint32_t q = blockIdx.x / kDies, sq = q / cells * kDies + blockIdx.x % kDies, in = q % cells;
+  uint32_t si, sj;
+  if (sq >= tile_items(ns) || !tile_of(sq, ns, &si, &sj)) return;
+  const uint32_t bi = si * side + in / side, bj = sj * side + in % side;
+  if (bi > bj || bj >= nb) return;
+  const uint32_t wave = threadIdx.x / kWave;
+  const uint32_t u0 = bi * kTileRows + wave / 2 * 64, v0 = bj * kTileRows + wave % 2 * 64;
+  if (u0 > v0 || v0 >= eid_of.nc) return;
+  Acc4 acc[4][4];
+  count_tile<4, 4>(bits, eid_of.nc, eid_of.ws, u0, v0, acc);
+  tile_edges<4, 4>(bits, eid_of.nc, eid_of.ws, u0, v0, acc, eid_of,
+                   [&](bool live, uint32_t e, uint32_t, uint32_t, uint32_t c) {
+                     if (live) sup[e] = int32_t(c);
+                   });
+}
+
 // *out = the longest of the rows (starts at 0)
 __global__ __launch_bounds__(kBlock) void k_max_row(const uint32_t* __restrict__ off, uint32_t rows, uint32_t* out) {
   uint32_t m = 0;
@@ -213,6 +241,29 @@ void rank_fill(const uint64_t* bits0, const uint32_t* pref0, const uint32_t* off
     k_rank_fill<<<std::min(grid_for(waves * kWave), 8192), kBlock, 0, s>>>(
         reinterpret_cast<const unsigned long long*>(bits0), pref0, off_u, ebase, nc, ws, adj_u, eid_u, adj_d, src,
         orig, state, del_thr, eidm);
+}
+// Measured (vertices, edges; by edge -> by pairs): 1,268, 483 k: 20 -> 23 us;
+// 1,535, 912 k: 37 -> 23; 2,867, 878 k: 39 -> 34; 3,150, 3.05 M: 136 -> 39;
+// 4,048, 945 k: 59 -> 61; 5,701, 2.35 M: 170 -> 112; 9,109, 6.25 M: 645 -> 331;
+// 14,697, 15.8 M: 2,530 -> 1,020. By edge about 10^6 word ANDs a us, by pairs
+// 12 * 10^6 plus some 15 us.
+double dense_pair_cost(uint32_t nc, uint32_t ws) { return double(nc) * nc / 24.0 * ws; }
+bool dense_by_pairs(uint32_t nc, uint32_t mc, uint32_t ws) {
+  return double(mc) * ws > 15e6 + dense_pair_cost(nc, ws);
+}
+void dense_count(const uint64_t* bits, const uint32_t* pref0, const uint32_t* off_u, const uint32_t* eid_u,
+                 const uint32_t* eidm, uint32_t nc, uint32_t ws, int32_t* sup, hipStream_t s) {
+  if (!nc) return;
+  auto b = reinterpret_cast<const unsigned long long*>(bits);
+  const uint32_t nb = (nc + kTileRows - 1) / kTileRows;
+  // squares once the rows outgrow a die's L2 (4 MB)
+  const uint32_t side = uint64_t(nc) * ws * 8 > (4u << 20) ? 8u : 1u;
+  const uint32_t squares = (tile_items((nb + side - 1) / side) + 7) / 8 * 8;
+  const uint32_t grid = squares * side * side;
+  if (eidm)
+    k_dense_count<true><<<grid, kBlock, 0, s>>>(b, EidOf<true>{eidm, b, pref0, off_u, eid_u, nc, ws}, nb, side, sup);
+  else
+    k_dense_count<false><<<grid, kBlock, 0, s>>>(b, EidOf<false>{eidm, b, pref0, off_u, eid_u, nc, ws}, nb, side, sup);
 }
 void max_row(const uint32_t* off, uint32_t rows, uint32_t* out, hipStream_t s) {
   fill_u32(out, 1, 0, s);

@@ -258,6 +258,14 @@ void rank_fill(const uint64_t* bits0, const uint32_t* pref0, const uint32_t* off
                uint32_t ws, uint32_t* adj_u, uint32_t* eid_u, uint32_t* adj_d, uint32_t* src, uint32_t* orig,
                uint32_t* state, uint32_t* del_thr, uint32_t* eidm, hipStream_t s);
 void max_row(const uint32_t* off, uint32_t rows, uint32_t* out, hipStream_t s);
+// A count by all pairs of rows in word ANDs of one by edge, and whether it is
+// the faster one for a fresh view.
+double dense_pair_cost(uint32_t nc, uint32_t ws);
+bool dense_by_pairs(uint32_t nc, uint32_t mc, uint32_t ws);
+// sup of every edge of a dense core whose rows hold all of its edges: by all
+// pairs of rows (dense_support: by edge)
+void dense_count(const uint64_t* bits, const uint32_t* pref0, const uint32_t* off_u, const uint32_t* eid_u,
+                 const uint32_t* eidm, uint32_t nc, uint32_t ws, int32_t* sup, hipStream_t s);
 // Triangle lists (kt_list.hip). sum_u32: *total (starts at 0) += the sum.
 // tri_fill: every triangle's entries, cursor starting as a copy of the offsets
 // (bitmap, lanes: as the support count's kernels).

@@ -339,8 +339,8 @@ class Solver {
   uint64_t eidm_budget_ = uint64_t(4) << 30;  // bytes for the edge-id matrix
   // triangle lists: in all, and a core edge (a context of its own is not bound there)
   uint64_t tri_budget_ = uint64_t(16) << 30, tri_per_edge_ = ~uint64_t(0) >> 32;
-  double dense_tri_cost_ = 10.0, sparse_drop_ratio_ = 3.0, default_drop_ratio_ = 3.0;
-  double dense_drop_fixed_ = 12e6;  // about what the two steps of a recount take
+  double dense_tri_cost_ = 14.0, sparse_drop_ratio_ = 3.0, default_drop_ratio_ = 3.0;
+  double dense_drop_fixed_ = 8e6;  // about what the two steps of a recount take
   bool trace_ = false;  // KT_TRACE=1: per-round frontier sizes on stderr
   // trace only: milliseconds since the previous call, after the stream drains
   double trace_ms();

@@ -745,7 +745,10 @@ void Solver::count_support(CoreView* cv, float* ms) {
   uint32_t kind = 1;
   if (cv->dense) {
     kind = 2;
-    dense_support(cv->off_d, cv->adj_d, cv->nc, cv->mc, cv->bits, cv->ws, nullptr, cv->sup, stream_);
+    if (dense_by_pairs(cv->nc, cv->mc, cv->ws))
+      dense_count(cv->bits, cv->pref0, cv->off_u, cv->eid_u, cv->eidm, cv->nc, cv->ws, cv->sup, stream_);
+    else
+      dense_support(cv->off_d, cv->adj_d, cv->nc, cv->mc, cv->bits, cv->ws, nullptr, cv->sup, stream_);
   } else if (!force_edge_count_ && support_bitmap_fits(cv->nc, cv->max_dout)) {
     kind = 0;
     support_bitmap(cv->off_d, cv->adj_d, cv->nc, cv->max_dout, lanes, cv->sup, ctl_, stream_);
@@ -933,6 +936,7 @@ TrussOutcome Solver::run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32
     rule.host = cv->dense && allow_host ? 1u : 0u;
     rule.tri_cost = dense_tri_cost_;
     rule.drop_fixed = dense_drop_fixed_;
+    rule.pair_cost = cv->dense ? dense_pair_cost(cv->nc, cv->ws) : 0.0;
     steps_start(a, h, stream_);
     uint64_t steps = 0;
     uint32_t batch = kFirstBatch;

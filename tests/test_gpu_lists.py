@@ -116,3 +116,23 @@ def test_dense_views_of_cliques(dense_ctx, n):
     assert (r.kmax, r.truss_edges, r.max_core) == (n, n * (n - 1) // 2, n - 1)
     got = dense_ctx.truss_edges()
     assert (got >= n).all() and len(np.unique(got[:, 0].astype(np.uint64) * (2 * n) + got[:, 1])) == len(got)
+
+
+# rows one bit past a word, one short of it, whole chunks of eight words, and
+# squares of row blocks
+@pytest.mark.parametrize("n,p", [(1601, 0.6), (1727, 0.6), (2048, 0.4), (6000, 0.1)])
+def test_counts_by_pairs_equal_rows(dense_ctx, n, p):
+    """Cores whose supports are counted by all pairs of rows on the matrix
+    cores, at first and after every dropped frontier: every trussness."""
+    from kc_cuda_amd import Context
+    rng = np.random.default_rng(n)
+    pairs = np.argwhere(np.triu(rng.random((n, n), dtype=np.float32) < p, 1)).astype(np.uint32)
+    r = dense_ctx.solve_pairs(pairs, n)
+    got = dense_ctx.trussness()
+    assert r.recounts > 0
+    with Context(0) as other:
+        other.tune(core="sparse")
+        ref = other.solve_pairs(pairs, n)
+        want = other.trussness()
+    assert (r.kmax, r.truss_edges, r.k_hat) == (ref.kmax, ref.truss_edges, ref.k_hat)
+    np.testing.assert_array_equal(got, want)
