@@ -327,7 +327,8 @@ __global__ __launch_bounds__(kBucketBlock) void k_bucket_rows(const uint2* __res
 // for some i. With hpos / tpos (lines), each run of equal rows r < n also
 // records hpos[r] = its first index and tpos[r] = its last index + 1 (valid
 // when the keys are sorted; rows without lines keep what the caller
-// filled); a row >= n sets *err.
+// filled); a row >= n sets *err. Stride 2: the keys are the first ids of
+// pairs, and either id >= n sets *err.
 template <int Stride>
 __global__ __launch_bounds__(kBlock) void k_sorted_runs(const uint32_t* __restrict__ keys, uint64_t items,
                                                         uint32_t n, uint64_t* hpos, uint64_t* tpos,
@@ -336,6 +337,7 @@ __global__ __launch_bounds__(kBlock) void k_sorted_runs(const uint32_t* __restri
   const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
   for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < items; i += stride) {
     const uint32_t k = keys[i * Stride];
+    if (Stride == 2) big |= max(k, keys[i * 2 + 1]) >= n;
     const bool has_next = i + 1 < items;
     const uint32_t nx = has_next ? keys[(i + 1) * Stride] : 0u;
     bad |= has_next && nx < k;
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(kBlock) void k_sorted_runs(const uint32_t* __restri
     }
   }
   if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(unsorted, 1u);
-  if (hpos && __syncthreads_or(big) && threadIdx.x == 0) atomicOr(err, 1u);
+  if ((hpos || Stride == 2) && __syncthreads_or(big) && threadIdx.x == 0) atomicOr(err, 1u);
 }
 
 // deg[r] = tpos[r] - hpos[r] for r < n, deg[n] = 0.

@@ -256,16 +256,23 @@ bool Solver::build_partitioned(int mode, const uint32_t* a, const uint32_t* b, u
   // pairs sorted by their first id: the first entries of a bucket's rows lie
   // in order in the input, so only the second entries are bucketed
   bool fwd_sorted = false;
-  if (mode == 0 && sorted_build_ && items > 1) {
+  zero_u32(&ctl_->err);
+  const bool checked = mode == 0 && sorted_build_ && items > 1;
+  if (checked) {
     zero_u32(&ctl_->pad[0]);
     csr_sorted_check(0, a, items, n, nullptr, nullptr, &ctl_->pad[0], &ctl_->err, stream_);
-    fwd_sorted = read_u32(&ctl_->pad[0]) == 0;
+    const Ctl h = read_ctl();
+    if (h.err) fail("edge list holds a vertex id >= n");
+    fwd_sorted = h.pad[0] == 0;
   }
   const int pmode = fwd_sorted ? 2 : mode;
   const uint64_t entries = mode == 0 && !fwd_sorted ? 2 * items : items;  // bucketed entries
-  // at most build_tiles_ tiles of at least 65536 items
+  // at most build_tiles_ tiles, of at least 1024 items and 16 per bucket, whose
+  // counters a tile clears and writes (16 k pairs, one bucket: 25 + 85 us for
+  // counting and scattering by one tile of 65536, 6 + 8 by 16 tiles)
   const uint64_t tiles = std::max<uint32_t>(1, build_tiles_);
-  const uint64_t tile = std::max<uint64_t>(65536, (items + tiles - 1) / tiles);
+  const uint64_t least = std::min<uint64_t>(65536, std::max<uint64_t>(1024, 16 * uint64_t(B)));
+  const uint64_t tile = std::max<uint64_t>(least, (items + tiles - 1) / tiles);
   const uint32_t T = uint32_t(std::max<uint64_t>(1, (items + tile - 1) / tile));
   const uint64_t bt = uint64_t(B) * T;
   hist_.ensure(sizeof(uint32_t) * (2 * bt + 1));   // tile-major counts, then bucket-major
@@ -277,9 +284,8 @@ bool Solver::build_partitioned(int mode, const uint32_t* a, const uint32_t* b, u
   uint64_t* hoff_t = hoff_b + bt + 1;
   uint64_t* f0 = fwd_sorted ? cursor_.as<uint64_t>() : nullptr;  // B + 1 <= n + 1 words
   fill_u32(hist_b + bt, 1, 0, stream_);
-  zero_u32(&ctl_->err);
   csr_part_hist(pmode, a, b, items, tile, n, S, B, T, hist_t, &ctl_->err, stream_);
-  if (read_u32(&ctl_->err)) fail("edge list holds a vertex id >= n");
+  if (!checked && read_u32(&ctl_->err)) fail("edge list holds a vertex id >= n");
   transpose_u32(hist_t, T, B, hist_b, stream_);
   exclusive_scan_u32_to_u64(hist_b, hoff_b, uint32_t(bt + 1));
   transpose_u64(hoff_b, B, T, hoff_t, stream_);
@@ -327,6 +333,7 @@ void Solver::build_from_pairs(const uint32_t* d_pairs, uint64_t m, uint32_t n) {
   if (2 * m >= (uint64_t(1) << 40)) fail("edge list too large");
   n_ = n;
   m_ = m;
+  slots_ = 2 * m;
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   cursor_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
@@ -346,6 +353,7 @@ void Solver::build_from_lines(const uint32_t* d_xs, const uint32_t* d_ys, uint64
   new_input();
   n_ = n;
   m_ = L / 2;
+  slots_ = L;
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   cursor_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
@@ -366,6 +374,7 @@ void Solver::load_csr_host(uint32_t n, const uint64_t* off, const uint32_t* adj)
   new_input();
   n_ = n;
   m_ = off[n] / 2;
+  slots_ = off[n];
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   adj_.ensure(sizeof(uint32_t) * std::max<uint64_t>(off[n], 1));
@@ -388,7 +397,7 @@ LevelGraph& Solver::level0() {
   LevelGraph& g = *levels_[0];
   lvl_.ensure(sizeof(uint32_t) * (size_t(n_) + 1));
   g.n = n_;
-  g.slots = read_u64(off() + n_);
+  g.slots = slots_;
   g.off = off();
   g.adj = adj();
   g.deg = deg();
