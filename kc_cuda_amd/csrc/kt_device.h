@@ -36,9 +36,36 @@ __device__ __forceinline__ void wave_append(bool pred, T item, T* q, uint32_t* c
   if (pred) q[base + uint32_t(__popcll(mask & ((1ull << lane) - 1ull)))] = item;
 }
 
-// Block-wide exclusive scan of one value per thread (blockDim == kBlock).
+// Runs of equal keys in consecutive lanes (sorted inputs put a row's entries
+// next to each other): the first lane of each run adds the whole run with
+// one LDS atomic instead of one per lane, which would serialise on one
+// address. Inactive lanes end runs. head: first lane of this lane's run;
+// len: the run's length (meaningful at the head).
+struct LaneRun {
+  int head;
+  uint32_t len;
+  bool is_head;
+};
+__device__ __forceinline__ LaneRun lane_run(uint32_t key, bool active) {
+  const int lane = lane64();
+  const uint32_t prev = __shfl_up(key, 1);
+  const bool prev_active = __shfl_up(int(active), 1) != 0;
+  const bool head = active && (lane == 0 || !prev_active || prev != key);
+  const unsigned long long heads = __ballot(head);
+  const unsigned long long ends = heads | ~__ballot(active);  // a run stops at the next head or inactive lane
+  const unsigned long long le = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+  LaneRun r;
+  r.is_head = head;
+  r.head = 63 - __clzll((long long)(heads & le));  // valid for active lanes (lane 0 of a run is a head)
+  const unsigned long long after = ends & ~le;
+  r.len = uint32_t((after ? __ffsll((unsigned long long)after) - 1 : 64) - lane);
+  return r;
+}
+
+// Block-wide exclusive scan of one value per thread (blockDim == kThreads).
+template <int kThreads = kBlock>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* total) {
-  __shared__ uint32_t s_w[kBlock / kWave];
+  __shared__ uint32_t s_w[kThreads / kWave];
   const int lane = lane64(), wid = int(threadIdx.x) / kWave;
   uint32_t inc = v;
 #pragma unroll
@@ -50,7 +77,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* t
   __syncthreads();
   uint32_t before = 0, tot = 0;
 #pragma unroll
-  for (int k = 0; k < kBlock / kWave; ++k) {
+  for (int k = 0; k < kThreads / kWave; ++k) {
     const uint32_t w = s_w[k];
     if (k < wid) before += w;
     tot += w;

@@ -121,32 +121,6 @@ struct EntrySrc {
   }
 };
 
-// Runs of equal keys in consecutive lanes (sorted inputs put a row's entries
-// next to each other): the first lane of each run adds the whole run with
-// one LDS atomic instead of one per lane, which would serialise on one
-// address. Inactive lanes end runs. head: first lane of this lane's run;
-// len: the run's length (meaningful at the head).
-struct LaneRun {
-  int head;
-  uint32_t len;
-  bool is_head;
-};
-__device__ __forceinline__ LaneRun lane_run(uint32_t key, bool active) {
-  const int lane = lane64();
-  const uint32_t prev = __shfl_up(key, 1);
-  const bool prev_active = __shfl_up(int(active), 1) != 0;
-  const bool head = active && (lane == 0 || !prev_active || prev != key);
-  const unsigned long long heads = __ballot(head);
-  const unsigned long long ends = heads | ~__ballot(active);  // a run stops at the next head or inactive lane
-  const unsigned long long le = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-  LaneRun r;
-  r.is_head = head;
-  r.head = 63 - __clzll((long long)(heads & le));  // valid for active lanes (lane 0 of a run is a head)
-  const unsigned long long after = ends & ~le;
-  r.len = uint32_t((after ? __ffsll((unsigned long long)after) - 1 : 64) - lane);
-  return r;
-}
-
 // kBwd (pairs only): count and scatter only each pair's second entry (row v,
 // column u); the first entries of row-sorted pairs are placed in order by
 // k_bucket_rows_sorted instead.

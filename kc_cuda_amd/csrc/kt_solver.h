@@ -101,6 +101,8 @@ struct EdgeSet {
   DevBuf off, adj, src, orig, sup;
 };
 
+struct SplitPlan;  // kt_kernels.h
+
 class Solver {
  public:
   explicit Solver(int device);
@@ -291,6 +293,7 @@ class Solver {
   void build_from_pairs(const uint32_t* d_pairs, uint64_t m, uint32_t n);
   void build_from_lines(const uint32_t* d_xs, const uint32_t* d_ys, uint64_t L, uint32_t n);
   bool build_partitioned(int mode, const uint32_t* a, const uint32_t* b, uint64_t items, uint32_t n);
+  void build_split(const SplitPlan& p, const uint32_t* pairs, uint64_t items, uint32_t n);
   bool build_sorted_lines(const uint32_t* xs, const uint32_t* ys, uint64_t L, uint32_t n);
   void solve_csr(kt_result* res);
   uint32_t read_u32(const uint32_t* dptr);
@@ -348,6 +351,7 @@ class Solver {
   bool gallop_ = true;
   uint32_t count_kind_ = 0, count_words_ = 0;  // the last timed support count
   uint32_t walk_levels_ = 16;
+  uint64_t split_build_min_ = uint64_t(1) << 22;  // fewest pairs of the build by two splits (see split_plan)
   uint32_t build_tiles_ = 4096;  // most tiles of the partitioned CSR build
   int probe_push_ = 0;               // measurement of a kernel (mode bits)
   int probe_kernel_ = kProbeVertexPeel;
@@ -364,7 +368,7 @@ class Solver {
   uint32_t n_ = 0;
   uint64_t m_ = 0, slots_ = 0;  // edges and row slots of the input
   // full graph
-  DevBuf off_, adj_, deg_, lvl_, q0_, q1_, deg_bak_, cursor_, hist_, hoff_, part_;
+  DevBuf off_, adj_, deg_, lvl_, q0_, q1_, deg_bak_, cursor_, hist_, hoff_, part_, split_;
   std::vector<std::unique_ptr<LevelGraph>> levels_;
   size_t depth_ = 0;  // levels in use
   // scratch for level cuts and extraction

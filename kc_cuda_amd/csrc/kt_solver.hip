@@ -126,6 +126,7 @@ void Solver::init_common() {
   if (const char* v = std::getenv("KT_EIDM_BUDGET_MB")) eidm_budget_ = uint64_t(std::atoll(v)) << 20;
   if (const char* v = std::getenv("KT_LIST_BUDGET_MB")) tri_budget_ = uint64_t(std::atoll(v)) << 20;
   if (const char* v = std::getenv("KT_WALK_LEVELS")) walk_levels_ = std::max(1, std::atoi(v));
+  if (const char* v = std::getenv("KT_SPLIT_BUILD_MIN")) split_build_min_ = uint64_t(std::atoll(v));
   if (const char* v = std::getenv("KT_BUILD_TILES")) build_tiles_ = uint32_t(std::max(1, std::atoi(v)));
   if (const char* v = std::getenv("KT_VERTEX_PEEL"))
     vertex_mode_ = std::strcmp(v, "rounds") == 0 ? 1 : std::strcmp(v, "cascade") == 0 ? 2 : 0;
@@ -138,7 +139,7 @@ void Solver::each_buffer(F f) const {
                          &keys_, &keys2_, &vals_, &vals2_, &to_, &inv_, &inv_orig_, &dout_, &off_d_,
                          &adj_d_, &src_, &din_, &din_off_, &tkeys_, &tvals_, &tiota_, &in_src_, &off_u_,
                          &adj_u_, &eid_u_, &sup_, &state_, &eq0_, &eq1_, &eq2_, &out_pairs_, &truss_out_, &del_thr_, &orig0_,
-                         &temp_, &hist_, &hoff_, &part_, &bits0_, &bits_, &pref0_, &eidm_, &heavy_,
+                         &temp_, &hist_, &hoff_, &part_, &split_, &bits0_, &bits_, &pref0_, &eidm_, &heavy_,
                          &vflag_, &vmap_, &roff_, &dhist_, &vq_, &core_out_, &step_ctl_, &tri_off_, &tri_, &live_[0], &live_[1], &bk_state_, &bk_sup_, &bk_bits_, &bk_del_, &text_,
                          &tile_cnt_, &tile_off_, &lx_, &ly_, &lkind_, &lx2_, &ly2_, &lkeep_, &lkeep_off_,
                          &lstat_, &probe_stats_};
@@ -265,6 +266,11 @@ bool Solver::build_partitioned(int mode, const uint32_t* a, const uint32_t* b, u
     if (h.err) fail("edge list holds a vertex id >= n");
     fwd_sorted = h.pad[0] == 0;
   }
+  SplitPlan plan;
+  if (fwd_sorted && items >= split_build_min_ && split_plan(n, items, &plan)) {
+    build_split(plan, a, items, n);
+    return true;
+  }
   const int pmode = fwd_sorted ? 2 : mode;
   const uint64_t entries = mode == 0 && !fwd_sorted ? 2 * items : items;  // bucketed entries
   // at most build_tiles_ tiles, of at least 1024 items and 16 per bucket, whose
@@ -298,6 +304,40 @@ bool Solver::build_partitioned(int mode, const uint32_t* a, const uint32_t* b, u
   else
     KT_HIP(hipMemcpyAsync(off() + n, hoff_b + bt, sizeof(uint64_t), hipMemcpyDeviceToDevice, stream_));
   return true;
+}
+
+// Pairs sorted by their first id, valid ids: the second entries go to their
+// groups of rows in two splits (kt_build.hip), by way of adj.
+void Solver::build_split(const SplitPlan& p, const uint32_t* pairs, uint64_t items, uint32_t n) {
+  const uint32_t lows = 1u << p.low_bits, highs = 1u << p.high_bits;
+  const uint64_t bt = std::max(uint64_t(lows) * p.tiles1, uint64_t(highs) * p.tiles2);
+  hist_.ensure(sizeof(uint32_t) * (2 * bt + 1));
+  hoff_.ensure(sizeof(uint64_t) * (2 * bt + 1));
+  part_.ensure(sizeof(uint32_t) * 2 * items);
+  split_.ensure((sizeof(uint64_t) + sizeof(uint32_t)) * (size_t(lows) + 1));
+  uint64_t* start = split_.as<uint64_t>();
+  uint32_t* tiles = reinterpret_cast<uint32_t*>(start + lows + 1);
+  uint64_t* f0 = cursor_.as<uint64_t>();  // groups + 1 <= n + 1 words
+  for (const bool first : {true, false}) {
+    const uint32_t T = first ? p.tiles1 : p.tiles2, digits = first ? lows : highs;
+    const uint64_t cells = uint64_t(digits) * T;
+    uint32_t* hist_t = hist_.as<uint32_t>();
+    uint32_t* hist_b = hist_t + cells;
+    uint64_t* off_b = hoff_.as<uint64_t>();
+    uint64_t* off_t = off_b + cells + 1;
+    const uint32_t* from = first ? pairs : adj();
+    uint32_t* to = first ? adj() : part_.as<uint32_t>();
+    fill_u32(hist_b + cells, 1, 0, stream_);
+    split_hist(first, p, from, items, start, tiles, hist_t, stream_);
+    transpose_u32(hist_t, T, digits, hist_b, stream_);
+    exclusive_scan_u32_to_u64(hist_b, off_b, uint32_t(cells + 1));
+    transpose_u64(off_b, digits, T, off_t, stream_);
+    split(first, p, from, items, start, tiles, off_t, to, stream_);
+    if (first) split_tiles(p, off_b, start, tiles, stream_);
+  }
+  csr_fwd_start(pairs, items, p.shift, p.groups, f0, stream_);
+  group_rows(p, part_.as<uint32_t>(), hoff_.as<uint64_t>(), tiles, pairs, f0, n, off(), deg(), adj(), stream_);
+  fill_u64(off() + n, 1, 2 * items, stream_);
 }
 
 // Lines sorted by row (the reference's edge-list order): each row is a run
