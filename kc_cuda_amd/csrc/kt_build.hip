@@ -1,6 +1,7 @@
-// CSR build of large sorted pair lists by two staged splits, on CDNA4.
+// CSR build of large pair lists by two staged splits, on CDNA4.
 //
-// The second entries (row v, column u) of pairs sorted by u are in no order.
+// The second entries (row v, column u) of pairs sorted by u are in no order,
+// nor are any of pairs that are not sorted.
 // k_part_scatter writes each one straight to its bucket: with thousands of
 // buckets per workgroup and thousands of workgroups, the lines being filled
 // outgrow the L2 many times over, every 8-byte store becomes a memory
@@ -27,12 +28,15 @@ constexpr uint32_t kRowsPer = 16;
 constexpr uint32_t kRowsStage = kRowsBlock * kRowsPer;  // slots of a group put in order in LDS: 32 KB
 constexpr uint32_t kMaxGroupRows = kRowsBlock;
 
-// The entries of tile t. First split: a run of the pairs, entry (v, u). Second:
-// of the first one's output, cut at its bucket bounds (so that a tile holds
-// one low digit and the order within it does not matter): start[d] the first
-// entry of bucket d, tiles[d] its first tile.
-template <bool kFirst>
+// The entries of tile t. First split: a run of the pairs' second entries (v, u)
+// or of both of each pair's. Second: a run of the first one's output, cut at
+// its bucket bounds (so that a tile holds one low digit and the order within
+// it does not matter): start[d] the first entry of bucket d, tiles[d] its
+// first tile.
+constexpr int kSecondOnes = 0, kBothOnes = 1, kSplitOnce = 2;
+template <int kFrom>
 struct SplitSrc {
+  static constexpr bool kFirst = kFrom != kSplitOnce;
   const uint2* entries;
   uint64_t items, tile;
   uint32_t buckets;  // of the first split
@@ -60,14 +64,15 @@ struct SplitSrc {
     *hi = min(start[d0 + 1], *lo + tile);
   }
   __device__ __forceinline__ uint2 get(uint64_t i) const {
-    const uint2 p = entries[i];
-    return kFirst ? make_uint2(p.y, p.x) : p;
+    const uint2 p = entries[kFrom == kBothOnes ? i >> 1 : i];
+    const bool turn = kFrom == kSecondOnes || (kFrom == kBothOnes && (i & 1u));
+    return turn ? make_uint2(p.y, p.x) : p;
   }
 };
 
 // hist[t * digits + d] = tile t's entries of digit d
-template <bool kFirst>
-__global__ __launch_bounds__(kSplitBlock) void k_split_hist(SplitSrc<kFirst> src, uint32_t shift, uint32_t digits,
+template <int kFrom>
+__global__ __launch_bounds__(kSplitBlock) void k_split_hist(SplitSrc<kFrom> src, uint32_t shift, uint32_t digits,
                                                             uint32_t* hist) {
   __shared__ uint32_t s_cnt[kMaxDigits];
   uint64_t lo, hi;
@@ -101,8 +106,8 @@ __device__ __forceinline__ uint32_t digit_scan(uint32_t v) {
 
 // Tile t's entries to their digits' places, off_t[t * digits + d] on. 8192
 // entries at a time are put in digit order in LDS and written in runs.
-template <bool kFirst>
-__global__ __launch_bounds__(kSplitBlock) void k_split(SplitSrc<kFirst> src, uint32_t shift, uint32_t digits,
+template <int kFrom>
+__global__ __launch_bounds__(kSplitBlock) void k_split(SplitSrc<kFrom> src, uint32_t shift, uint32_t digits,
                                                        const uint64_t* __restrict__ off_t, uint2* __restrict__ out) {
   __shared__ uint2 s_stage[kSplitStage];
   __shared__ uint32_t s_cnt[kMaxDigits], s_at[kMaxDigits];
@@ -171,7 +176,7 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_tiles(const uint64_t* __r
 // A group of 2^S rows per workgroup: its second entries are part[beg .. end),
 // its first ones fwd[f0[g] .. f0[g + 1]). Ranks within the rows come from one
 // LDS counter a row while the entries are read, the columns are put in order
-// in LDS and leave as one run. A group with more slots than the stage holds
+// in LDS and leave as one run (fwd null: part holds all entries). A group with more slots than the stage holds
 // (hubs) is counted and placed from memory as k_bucket_rows does.
 __global__ __launch_bounds__(kRowsBlock) void k_group_rows(const uint2* __restrict__ part,
                                                            const uint64_t* __restrict__ off_b,
@@ -184,7 +189,7 @@ __global__ __launch_bounds__(kRowsBlock) void k_group_rows(const uint2* __restri
   const uint32_t g = blockIdx.x, tid = threadIdx.x;
   const uint32_t low = g & ((1u << low_bits) - 1u), high = g >> low_bits;
   const uint64_t beg = off_b[uint64_t(high) * T + tiles[low]], end = off_b[uint64_t(high) * T + tiles[low + 1]];
-  const uint64_t fb = f0[g], fe = f0[g + 1], base = beg + fb;
+  const uint64_t fb = fwd ? f0[g] : 0, fe = fwd ? f0[g + 1] : 0, base = beg + fb;
   const uint32_t r0 = g << S, nrows = min(1u << S, n - r0);
   const int lane = lane64();
   const uint64_t slots = (end - beg) + (fe - fb);
@@ -263,12 +268,15 @@ __global__ __launch_bounds__(kRowsBlock) void k_group_rows(const uint2* __restri
 // 2^21 pairs 0.121 -> 0.154, 2^22 0.187 -> 0.184, 2^23 0.319 -> 0.244, 2^24
 // 0.77 -> 0.40, 2^25 1.55 -> 0.72 (80 slots a row: the same); 505 M pairs 19.0
 // -> 10.8 (two counts 1.4, splits 3.2 and 2.5, rows 3.5; 2.7 to 3.5 TB/s). It
-// is taken from 2^22 pairs on.
+// is taken from 2^22 pairs on, shuffled ones too: 2^21 0.158 -> 0.186, 2^22
+// 0.288 -> 0.255, 2^23 0.525 -> 0.385, 2^25 2.67 -> 1.43.
 // Groups of as many rows as average 6,144 slots or fewer (the stage takes
 // 8,192), split by at most nine bits twice.
-bool split_plan(uint32_t n, uint64_t items, SplitPlan* p) {
+bool split_plan(uint32_t n, uint64_t pairs, bool sorted, SplitPlan* p) {
+  p->sorted = sorted;
+  p->entries = sorted ? pairs : 2 * pairs;
   uint32_t s = 9;  // kMaxGroupRows
-  while (s > 0 && double(2 * items) / n * double(1u << s) > 6144.0) --s;
+  while (s > 0 && double(2 * pairs) / n * double(1u << s) > 6144.0) --s;
   const uint64_t groups = (uint64_t(n) + (1u << s) - 1) >> s;
   uint32_t bits = 2;
   while (bits < 32 && (uint64_t(1) << bits) < groups) ++bits;
@@ -278,34 +286,43 @@ bool split_plan(uint32_t n, uint64_t items, SplitPlan* p) {
   p->low_bits = bits / 2;
   p->high_bits = bits - bits / 2;
   // tiles of whole stages, about 4096 of them
-  const uint64_t stages = (items + 4096ull * kSplitStage - 1) / (4096ull * kSplitStage);
+  const uint64_t stages = (p->entries + 4096ull * kSplitStage - 1) / (4096ull * kSplitStage);
   p->tile = kSplitStage * std::max<uint64_t>(2, stages);
-  p->tiles1 = uint32_t((items + p->tile - 1) / p->tile);
+  p->tiles1 = uint32_t((p->entries + p->tile - 1) / p->tile);
   p->tiles2 = p->tiles1 + (1u << p->low_bits);
   return true;
 }
-void split_hist(bool first, const SplitPlan& p, const uint32_t* entries, uint64_t items, const uint64_t* start,
-                const uint32_t* tiles, uint32_t* hist, hipStream_t s) {
-  auto e = reinterpret_cast<const uint2*>(entries);
-  const uint32_t lows = 1u << p.low_bits, highs = 1u << p.high_bits;
-  if (first)
-    k_split_hist<true><<<p.tiles1, kSplitBlock, 0, s>>>(SplitSrc<true>{e, items, p.tile, lows, start, tiles}, p.shift,
-                                                        lows, hist);
-  else
-    k_split_hist<false><<<p.tiles2, kSplitBlock, 0, s>>>(SplitSrc<false>{e, items, p.tile, lows, start, tiles},
-                                                         p.shift + p.low_bits, highs, hist);
+template <int kFrom>
+static SplitSrc<kFrom> split_src(const SplitPlan& p, const uint32_t* from, const uint64_t* start,
+                                 const uint32_t* tiles) {
+  return SplitSrc<kFrom>{reinterpret_cast<const uint2*>(from), p.entries, p.tile, 1u << p.low_bits, start, tiles};
 }
-void split(bool first, const SplitPlan& p, const uint32_t* entries, uint64_t items, const uint64_t* start,
-           const uint32_t* tiles, const uint64_t* off_t, uint32_t* out, hipStream_t s) {
-  auto e = reinterpret_cast<const uint2*>(entries);
-  auto o = reinterpret_cast<uint2*>(out);
+void split_hist(bool first, const SplitPlan& p, const uint32_t* from, const uint64_t* start, const uint32_t* tiles,
+                uint32_t* hist, hipStream_t s) {
   const uint32_t lows = 1u << p.low_bits, highs = 1u << p.high_bits;
-  if (first)
-    k_split<true><<<p.tiles1, kSplitBlock, 0, s>>>(SplitSrc<true>{e, items, p.tile, lows, start, tiles}, p.shift, lows,
-                                                   off_t, o);
+  if (!first)
+    k_split_hist<kSplitOnce><<<p.tiles2, kSplitBlock, 0, s>>>(split_src<kSplitOnce>(p, from, start, tiles),
+                                                              p.shift + p.low_bits, highs, hist);
+  else if (p.sorted)
+    k_split_hist<kSecondOnes><<<p.tiles1, kSplitBlock, 0, s>>>(split_src<kSecondOnes>(p, from, start, tiles), p.shift,
+                                                               lows, hist);
   else
-    k_split<false><<<p.tiles2, kSplitBlock, 0, s>>>(SplitSrc<false>{e, items, p.tile, lows, start, tiles},
-                                                    p.shift + p.low_bits, highs, off_t, o);
+    k_split_hist<kBothOnes><<<p.tiles1, kSplitBlock, 0, s>>>(split_src<kBothOnes>(p, from, start, tiles), p.shift,
+                                                             lows, hist);
+}
+void split(bool first, const SplitPlan& p, const uint32_t* from, const uint64_t* start, const uint32_t* tiles,
+           const uint64_t* off_t, uint32_t* to, hipStream_t s) {
+  auto o = reinterpret_cast<uint2*>(to);
+  const uint32_t lows = 1u << p.low_bits, highs = 1u << p.high_bits;
+  if (!first)
+    k_split<kSplitOnce><<<p.tiles2, kSplitBlock, 0, s>>>(split_src<kSplitOnce>(p, from, start, tiles),
+                                                         p.shift + p.low_bits, highs, off_t, o);
+  else if (p.sorted)
+    k_split<kSecondOnes><<<p.tiles1, kSplitBlock, 0, s>>>(split_src<kSecondOnes>(p, from, start, tiles), p.shift,
+                                                          lows, off_t, o);
+  else
+    k_split<kBothOnes><<<p.tiles1, kSplitBlock, 0, s>>>(split_src<kBothOnes>(p, from, start, tiles), p.shift, lows,
+                                                        off_t, o);
 }
 void split_tiles(const SplitPlan& p, const uint64_t* off_b, uint64_t* start, uint32_t* tiles, hipStream_t s) {
   k_split_tiles<<<1, kSplitBlock, 0, s>>>(off_b, p.tiles1, 1u << p.low_bits, p.tile, start, tiles);

@@ -245,20 +245,22 @@ void row_compact(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* o
                  const int32_t* sup, const uint32_t* state, uint32_t nc, const uint32_t* off2,
                  uint32_t* adj2, uint32_t* src2, uint32_t* orig2, int32_t* sup2, hipStream_t s);
 void count_in_degrees(const uint32_t* adj, uint32_t m, uint32_t* din, hipStream_t s);
-// CSR build of large sorted pair lists by two splits (kt_build.hip): groups of
-// 2^shift rows, split by the low and the high bits of their number in tiles of
-// `tile` entries, tiles1 of the first split and at most tiles2 of the second.
+// CSR build of large pair lists by two splits (kt_build.hip): groups of 2^shift
+// rows, split by the low and the high bits of their number in tiles of `tile`
+// entries, tiles1 of the first split and at most tiles2 of the second.
+// sorted: by the first ids; the second entries are split.
 struct SplitPlan {
+  bool sorted;
   uint32_t shift, groups, low_bits, high_bits, tiles1, tiles2;
-  uint64_t tile;
+  uint64_t entries, tile;
 };
-bool split_plan(uint32_t n, uint64_t items, SplitPlan* p);
-// first: of the pairs' second entries, else of its output (start, tiles: from
-// split_tiles); hist and off_t tile-major, off_b bucket-major
-void split_hist(bool first, const SplitPlan& p, const uint32_t* entries, uint64_t items, const uint64_t* start,
-                const uint32_t* tiles, uint32_t* hist, hipStream_t s);
-void split(bool first, const SplitPlan& p, const uint32_t* entries, uint64_t items, const uint64_t* start,
-           const uint32_t* tiles, const uint64_t* off_t, uint32_t* out, hipStream_t s);
+bool split_plan(uint32_t n, uint64_t pairs, bool sorted, SplitPlan* p);
+// first: from the pairs, else from its output (start, tiles: of split_tiles);
+// hist and off_t tile-major, off_b bucket-major
+void split_hist(bool first, const SplitPlan& p, const uint32_t* from, const uint64_t* start, const uint32_t* tiles,
+                uint32_t* hist, hipStream_t s);
+void split(bool first, const SplitPlan& p, const uint32_t* from, const uint64_t* start, const uint32_t* tiles,
+           const uint64_t* off_t, uint32_t* to, hipStream_t s);
 void split_tiles(const SplitPlan& p, const uint64_t* off_b, uint64_t* start, uint32_t* tiles, hipStream_t s);
 void group_rows(const SplitPlan& p, const uint32_t* part, const uint64_t* off_b, const uint32_t* tiles,
                 const uint32_t* fwd, const uint64_t* f0, uint32_t n, uint64_t* off, uint32_t* deg, uint32_t* adj,

@@ -368,7 +368,7 @@ class Solver {
   uint32_t n_ = 0;
   uint64_t m_ = 0, slots_ = 0;  // edges and row slots of the input
   // full graph
-  DevBuf off_, adj_, deg_, lvl_, q0_, q1_, deg_bak_, cursor_, hist_, hoff_, part_, split_;
+  DevBuf off_, adj_, deg_, lvl_, q0_, q1_, deg_bak_, cursor_, hist_, hoff_, part_, part2_, split_;
   std::vector<std::unique_ptr<LevelGraph>> levels_;
   size_t depth_ = 0;  // levels in use
   // scratch for level cuts and extraction

@@ -139,7 +139,7 @@ void Solver::each_buffer(F f) const {
                          &keys_, &keys2_, &vals_, &vals2_, &to_, &inv_, &inv_orig_, &dout_, &off_d_,
                          &adj_d_, &src_, &din_, &din_off_, &tkeys_, &tvals_, &tiota_, &in_src_, &off_u_,
                          &adj_u_, &eid_u_, &sup_, &state_, &eq0_, &eq1_, &eq2_, &out_pairs_, &truss_out_, &del_thr_, &orig0_,
-                         &temp_, &hist_, &hoff_, &part_, &split_, &bits0_, &bits_, &pref0_, &eidm_, &heavy_,
+                         &temp_, &hist_, &hoff_, &part_, &part2_, &split_, &bits0_, &bits_, &pref0_, &eidm_, &heavy_,
                          &vflag_, &vmap_, &roff_, &dhist_, &vq_, &core_out_, &step_ctl_, &tri_off_, &tri_, &live_[0], &live_[1], &bk_state_, &bk_sup_, &bk_bits_, &bk_del_, &text_,
                          &tile_cnt_, &tile_off_, &lx_, &ly_, &lkind_, &lx2_, &ly2_, &lkeep_, &lkeep_off_,
                          &lstat_, &probe_stats_};
@@ -267,7 +267,7 @@ bool Solver::build_partitioned(int mode, const uint32_t* a, const uint32_t* b, u
     fwd_sorted = h.pad[0] == 0;
   }
   SplitPlan plan;
-  if (fwd_sorted && items >= split_build_min_ && split_plan(n, items, &plan)) {
+  if (checked && items >= split_build_min_ && split_plan(n, items, fwd_sorted, &plan)) {
     build_split(plan, a, items, n);
     return true;
   }
@@ -306,14 +306,17 @@ bool Solver::build_partitioned(int mode, const uint32_t* a, const uint32_t* b, u
   return true;
 }
 
-// Pairs sorted by their first id, valid ids: the second entries go to their
-// groups of rows in two splits (kt_build.hip), by way of adj.
+// Pairs of valid ids: their entries go to their groups of rows in two splits
+// (kt_build.hip). The first one's output has room in adj if the pairs are
+// sorted (only half of the entries are split).
 void Solver::build_split(const SplitPlan& p, const uint32_t* pairs, uint64_t items, uint32_t n) {
   const uint32_t lows = 1u << p.low_bits, highs = 1u << p.high_bits;
   const uint64_t bt = std::max(uint64_t(lows) * p.tiles1, uint64_t(highs) * p.tiles2);
   hist_.ensure(sizeof(uint32_t) * (2 * bt + 1));
   hoff_.ensure(sizeof(uint64_t) * (2 * bt + 1));
-  part_.ensure(sizeof(uint32_t) * 2 * items);
+  part_.ensure(sizeof(uint32_t) * 2 * p.entries);
+  if (!p.sorted) part2_.ensure(sizeof(uint32_t) * 2 * p.entries);
+  uint32_t* once = p.sorted ? adj() : part2_.as<uint32_t>();
   split_.ensure((sizeof(uint64_t) + sizeof(uint32_t)) * (size_t(lows) + 1));
   uint64_t* start = split_.as<uint64_t>();
   uint32_t* tiles = reinterpret_cast<uint32_t*>(start + lows + 1);
@@ -325,18 +328,18 @@ void Solver::build_split(const SplitPlan& p, const uint32_t* pairs, uint64_t ite
     uint32_t* hist_b = hist_t + cells;
     uint64_t* off_b = hoff_.as<uint64_t>();
     uint64_t* off_t = off_b + cells + 1;
-    const uint32_t* from = first ? pairs : adj();
-    uint32_t* to = first ? adj() : part_.as<uint32_t>();
+    const uint32_t* from = first ? pairs : once;
+    uint32_t* to = first ? once : part_.as<uint32_t>();
     fill_u32(hist_b + cells, 1, 0, stream_);
-    split_hist(first, p, from, items, start, tiles, hist_t, stream_);
+    split_hist(first, p, from, start, tiles, hist_t, stream_);
     transpose_u32(hist_t, T, digits, hist_b, stream_);
     exclusive_scan_u32_to_u64(hist_b, off_b, uint32_t(cells + 1));
     transpose_u64(off_b, digits, T, off_t, stream_);
-    split(first, p, from, items, start, tiles, off_t, to, stream_);
+    split(first, p, from, start, tiles, off_t, to, stream_);
     if (first) split_tiles(p, off_b, start, tiles, stream_);
   }
-  csr_fwd_start(pairs, items, p.shift, p.groups, f0, stream_);
-  group_rows(p, part_.as<uint32_t>(), hoff_.as<uint64_t>(), tiles, pairs, f0, n, off(), deg(), adj(), stream_);
+  if (p.sorted) csr_fwd_start(pairs, items, p.shift, p.groups, f0, stream_);
+  group_rows(p, part_.as<uint32_t>(), hoff_.as<uint64_t>(), tiles, p.sorted ? pairs : nullptr, f0, n, off(), deg(), adj(), stream_);
   fill_u64(off() + n, 1, 2 * items, stream_);
 }
 

@@ -56,3 +56,19 @@ def test_split_build_matches_sorted_rows(split_ctx, kind, n, m):
     np.testing.assert_array_equal(off.astype(np.int64), want)
     rows = np.repeat(np.arange(n, dtype=np.int64), np.diff(want))
     np.testing.assert_array_equal(np.sort(rows * n + adj), key)
+
+
+@pytest.mark.parametrize("kind,n,m", [
+    ("dense", 1025, TILE // 2 - 1), ("dense", 1536, TILE // 2), ("sparse", 40000, TILE + 5), ("hub", 30000, 0)])
+def test_split_build_of_shuffled_pairs(split_ctx, kind, n, m):
+    """Both entries of every pair are split."""
+    pairs = _pairs(kind, n, m)
+    pairs = np.ascontiguousarray(pairs[np.random.default_rng(1).permutation(len(pairs))])
+    split_ctx.solve_pairs(pairs, n)
+    off, adj = split_ctx.last_csr(n, 2 * len(pairs))
+    p = pairs.astype(np.int64)
+    key = np.sort(np.concatenate([p[:, 0] * n + p[:, 1], p[:, 1] * n + p[:, 0]]))
+    want = np.concatenate([[0], np.cumsum(np.bincount(key // n, minlength=n))])
+    np.testing.assert_array_equal(off.astype(np.int64), want)
+    rows = np.repeat(np.arange(n, dtype=np.int64), np.diff(want))
+    np.testing.assert_array_equal(np.sort(rows * n + adj), key)
