@@ -15,11 +15,24 @@
 namespace kt {
 namespace {
 
-__device__ __forceinline__ void put_triangle(uint32_t a, uint32_t b, uint32_t c, uint32_t* cursor, uint2* tri) {
-  const uint32_t pa = atomicAdd(&cursor[a], 1u), pb = atomicAdd(&cursor[b], 1u), pc = atomicAdd(&cursor[c], 1u);
-  tri[pa] = make_uint2(b, c);
-  tri[pb] = make_uint2(a, c);
-  tri[pc] = make_uint2(a, b);
+// A group of G lanes found triangles of one edge e, at most one a lane (hit),
+// with partner edges x and y. They share one atomic of e's cursor: one each
+// would queue up on its address (a union of 40 M edges: 27 ms, shared 13).
+template <int G>
+__device__ __forceinline__ void put_triangles(bool hit, uint32_t e, uint32_t x, uint32_t y, uint32_t* cursor,
+                                              uint2* tri) {
+  const int lane = lane64();
+  const unsigned long long group = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << (lane / G * G);
+  const unsigned long long hits = __ballot(hit) & group;
+  if (!hit) return;
+  const uint32_t ax = atomicAdd(&cursor[x], 1u), ay = atomicAdd(&cursor[y], 1u);
+  const int first = __ffsll(hits) - 1;
+  uint32_t at = 0;
+  if (lane == first) at = atomicAdd(&cursor[e], uint32_t(__popcll(hits)));
+  at = __shfl(at, first) + uint32_t(__popcll(hits & ((1ull << lane) - 1ull)));
+  tri[at] = make_uint2(x, y);
+  tri[ax] = make_uint2(e, y);
+  tri[ay] = make_uint2(e, x);
 }
 
 // One workgroup per vertex u: out(u) in LDS as a bitmap and a list, the
@@ -52,11 +65,13 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill_bitmap(const uint32_t* __re
       for (uint32_t j0 = vb; j0 < ve; j0 += G) {
         if (adj_d[j0] > wmax) break;  // rows are sorted: nothing further can hit
         const uint32_t j = j0 + lane;
+        uint32_t w = 0;
+        bool hit = false;
         if (j < ve) {
-          const uint32_t w = adj_d[j];
-          if (w >= list[0] && w <= wmax && ((bits[w >> 5] >> (w & 31)) & 1u))
-            put_triangle(beg + i, beg + lower_bound_u32(list, i + 1, du, w), j, cursor, tri);
+          w = adj_d[j];
+          hit = w >= list[0] && w <= wmax && ((bits[w >> 5] >> (w & 31)) & 1u);
         }
+        put_triangles<G>(hit, beg + i, hit ? beg + lower_bound_u32(list, i + 1, du, w) : 0u, j, cursor, tri);
       }
     }
     __syncthreads();
@@ -79,10 +94,16 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill_edges(const uint32_t* __res
       uint32_t t = ab; ab = bb; bb = t;
       t = ae; ae = be; be = t;
     }
-    for (uint32_t i = ab + lane; i < ae; i += G) {
-      const uint32_t x = adj_d[i];
-      const uint32_t p = lower_bound_u32(adj_d, bb, be, x);
-      if (p < be && adj_d[p] == x) put_triangle(e, i, p, cursor, tri);
+    for (uint32_t i0 = ab; i0 < ae; i0 += G) {  // group-uniform
+      const uint32_t i = i0 + lane;
+      uint32_t p = 0;
+      bool hit = false;
+      if (i < ae) {
+        const uint32_t x = adj_d[i];
+        p = lower_bound_u32(adj_d, bb, be, x);
+        hit = p < be && adj_d[p] == x;
+      }
+      put_triangles<G>(hit, e, i, p, cursor, tri);
     }
   }
 }
