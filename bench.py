@@ -16,9 +16,9 @@ rmat22` is RMAT scale 22, edge factor 16, (.57,.19,.19,.05), seed 1.
 
 Prints one JSON line on stdout (everything else goes to stderr):
   value        edges/s = m / wall time per solve
-  roofline     of the vertex-peel kernels (k_core_push, k_core_cascade) and
-               the bit-matrix edge-peel round (k_dense_peel_round), the one with more device
-               time per solve: its algorithmic bytes per launch (KERNEL_MODELS,
+  roofline     of the vertex peel's kernel (k_core_est_step, the core-number
+               sweeps) and the truss-level step of bit-matrix cores (k_step),
+               the one with more device time per solve: its algorithmic bytes per launch (KERNEL_MODELS,
                the path's per-unit byte figures times the units the launches
                process) over its average launch duration, measured with HIP
                events stamped at each launch's start and end on the solver's
@@ -32,8 +32,9 @@ Prints one JSON line on stdout (everything else goes to stderr):
                solve over the same time when profiles/ holds them
   config.count_kernel
                the pass-2 support count: for a bit-matrix core, the bytes its
-               rows are read with (one source row per workgroup plus one
-               destination row per oriented edge, 8 B words, plus 4 B per
+               rows are read with (256 rows per block of pairs on the matrix
+               cores; by edge, one source row per workgroup plus one
+               destination row per oriented edge; 8 B words, plus 4 B per
                support written) over its event-timed duration
   config.batch, config.serve
                the 4096-graph batched solve (graphs/s against sequential plain
@@ -175,10 +176,10 @@ def _traffic(kernel: str, workload: str) -> dict | None:
 
 KERNEL_MODELS = {
     # kernel probe -> (kernel name, bytes from the counters, per-unit figure)
-    # levels of up to 2^24 row slots are peeled by k_core_cascade, larger ones by k_core_push rounds
-    "vertex_peel": ("k_core_push+k_core_cascade", lambda slots, items: 4 * slots + 12 * items,
+    # (the row slots and vertices of the first sweep of each search alone: the model's one pass)
+    "vertex_peel": ("k_core_est_step", lambda slots, items: 4 * slots + 12 * items,
                     "4 B per row slot walked + 12 B per vertex taken (the vertex-peel term 8m + 12n + 8)"),
-    "dense_peel": ("k_dense_peel_round", lambda slots, items: 4 * slots,
+    "dense_peel": ("k_step", lambda slots, items: 4 * slots,
                    "4 B x (d+(u) + d+(v)) per frontier edge walked (the peel term 4 W(C+ minus T+))"),
 }
 
@@ -251,8 +252,14 @@ def plain_line(args) -> dict:
     count_s = stages["ms_count_kernel"] / 1e3
     if st.count_kernel == 2:
         words = st.core_words
-        cbytes = (st.n_core + st.m_core) * words * 8 + 4 * st.m_core
-        cmodel = "(n_C + m_C) * ws * 8 B row words + 4 B per support (read from L2/MALL, not HBM)"
+        if st.m_core * words > 15e6 + st.n_core ** 2 / 24 * words:  # by all pairs of rows
+            kernel = "k_dense_count"
+            blocks = -(-st.n_core // 128)
+            cbytes = blocks * (blocks + 1) // 2 * 256 * words * 8 + 4 * st.m_core
+            cmodel = "256 rows of ws * 8 B per 128 x 128 pairs + 4 B per support (read from L2/MALL, not HBM)"
+        else:
+            cbytes = (st.n_core + st.m_core) * words * 8 + 4 * st.m_core
+            cmodel = "(n_C + m_C) * ws * 8 B row words + 4 B per support (read from L2/MALL, not HBM)"
     else:
         cbytes = 4 * st.w_core + 4 * st.m_core + 4 * (st.n_core + 1)
         cmodel = "4 W(C+) + 4 m_C + 4 (n_C + 1) (sorted-row merges)"
@@ -349,7 +356,7 @@ def batch_summary(args) -> dict:
     return {"workload": "batch4096", "graphs": count, "edges": total, "steps": steps, "warmup": warmup,
             "generator": "n log-uniform [64, 65536], ER or R-MAT(.57,.19,.19,.05) 50/50, avg degree U[8,32], "
                          "clique U[4,40], seed 3",
-            "engine": "the batch in 4 contiguous parts of about equal edges, each one truss decomposition "
+            "engine": "the batch in 2 contiguous parts of about equal edges, each one truss decomposition "
                       "of its union on its own stream, run concurrently; inputs in HBM",
             "ms_per_batch": wall * 1e3, "graphs_per_s": count / wall, "edges_per_s": total / wall,
             "sequential_plain_graphs_per_s": seq_gps,

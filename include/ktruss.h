@@ -70,7 +70,7 @@ typedef struct kt_stats {
   uint64_t truss_edges;
   uint32_t count_kernel;  /* pass-2 support count: 0 LDS bitmap, 1 per edge, 2 bit matrix */
   uint32_t core_words;    /* bit-matrix row words (count_kernel 2) */
-  uint32_t vertex_rounds; /* the last vertex peel: 0 one cascade launch, 1 synchronous rounds */
+  uint32_t vertex_rounds; /* the last vertex peel: 0 core numbers or one cascade launch, 1 synchronous rounds */
   uint32_t pad;
 } kt_stats;
 
@@ -140,10 +140,10 @@ int kt_parse_tsv(const char* path, uint32_t* xs, uint32_t* ys, uint64_t cap, uin
  * walked, then thresholds are probed), KT_FORCE_PROBES threshold probes right
  * after the first level, KT_FORCE_VERTEX_ROUNDS / KT_FORCE_VERTEX_CASCADE
  * the vertex peel by synchronous rounds / by one cascade launch per
- * threshold at every level (default: the cascade on levels of up to 2^24
- * row slots, rounds above, and the max-core search finished in one
- * workgroup on levels of up to 16,000 vertices, which either flag turns
- * off). Every variant computes the same result. The
+ * threshold at every level, and the max core by a galloping search over
+ * thresholds (default: the max core from core numbers found in sweeps over
+ * the level; where a peel remains, the cascade on levels of up to 2^24 row
+ * slots, rounds above). Every variant computes the same result. The
  * sparse-peel drop ratio returns to its default (KT_SPARSE_DROP_RATIO or
  * 3). */
 #define KT_FORCE_EDGE_COUNT 1
@@ -164,7 +164,7 @@ int kt_set_tuning(kt_context* ctx, int count_lanes, int peel_lanes, int flags);
  * (vertex counts) are host arrays. Per graph: d_kmax, d_count (edges in its
  * kmax-truss) and d_status (0 ok, 1 invalid input); d_keep (nullable) gets 1
  * for every pair in its graph's kmax-truss. The valid graphs are solved
- * together as disjoint unions: the batch is cut into up to four contiguous
+ * together as disjoint unions: the batch is cut into up to two contiguous
  * parts of about equal edges (KT_BATCH_PARTS sets the count), and each
  * part's union is decomposed on its own solver and stream (the context's
  * for the first), all at once; every graph's answer is read off its part's
@@ -245,9 +245,9 @@ int kt_serve_counters_get(kt_server* srv, kt_serve_counters* out);
 uint64_t kt_serve_footprint(uint64_t m, uint32_t n);
 
 /* Measurement hook for the vertex peel: the sweeps that find a level's core
- * numbers (k_core_est_step), or the peel's push kernel or cascade. mode bit 1 (KT_PROBE_TIME): each launch stamps
- * HIP events at its own start and end on the context's stream; bit 2
- * (KT_PROBE_COUNT): each launch counts the row slots it walks (a push: rows up
+ * numbers (k_core_est_step), or the peel's push kernel or cascade. mode bit 1
+ * (KT_PROBE_TIME): each launch stamps HIP events at its own start and end on
+ * the context's stream; bit 2 (KT_PROBE_COUNT): each launch counts the row slots it walks (a push: rows up
  * to 8192 slots; longer ones go to the sliced kernel) and the vertices it
  * takes -- of the sweeps over a level the first, which takes every row once --
  * with atomics that slow it, so time and count in separate solves. 0 turns
@@ -264,10 +264,11 @@ typedef struct kt_push_stats {
 int kt_push_probe(kt_context* ctx, int mode);
 int kt_push_stats_get(kt_context* ctx, kt_push_stats* out);
 /* The same measurement for another kernel: KT_PROBE_VERTEX_PEEL is what
- * kt_push_probe measures; KT_PROBE_DENSE_PEEL is the bit-matrix edge-peel
- * round (k_dense_peel_round), whose counters in kt_push_stats are slots =
- * the frontier edges' oriented out-degrees d+(u) + d+(v) summed, vertices =
- * the frontier edges walked. */
+ * kt_push_probe measures; KT_PROBE_DENSE_PEEL is the truss-level step of
+ * bit-matrix cores (k_step: looks, recounts and steps after the search's end
+ * are launches too), whose counters in kt_push_stats are slots = the frontier
+ * edges' oriented out-degrees d+(u) + d+(v) summed, vertices = the frontier
+ * edges walked. */
 #define KT_PROBE_VERTEX_PEEL 0
 #define KT_PROBE_DENSE_PEEL 1
 int kt_kernel_probe(kt_context* ctx, int kernel, int mode);

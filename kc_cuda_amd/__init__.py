@@ -257,8 +257,9 @@ class Context:
         pass1 on bit-matrix cores: "auto" (walk 16 levels, then probe
         thresholds), "walk" (every level) or "probe" (probe after level 1);
         vertex: the vertex peel as one "cascade" launch per threshold, as
-        synchronous "rounds", or "auto" (the cascade on levels of up to
-        2^24 row slots); unsorted_build: the bucketed CSR build even for
+        synchronous "rounds", or "auto" (the max core from core numbers;
+        where a peel remains, the cascade on levels of up to 2^24 row
+        slots); unsorted_build: the bucketed CSR build even for
         inputs sorted by row."""
         flags = (1 if force_edge_count else 0) | (2 if force_atomic_build else 0)
         flags |= {"auto": 0, "sparse": 4, "dense": 8}[core]
@@ -318,13 +319,14 @@ class Context:
         return out
 
     def push_probe(self, mode: int) -> None:
-        """Measurement of the vertex-peel push kernel: 1 stamps events at
-        each launch's start and end, 2 counts its slots and vertices, 0 off."""
+        """Measurement of the vertex peel's kernel (the core-number sweeps): 1
+        stamps events at each launch's start and end, 2 counts its slots and
+        vertices, 0 off."""
         _check(self._lib.kt_push_probe(self._h, int(mode)))
 
     def kernel_probe(self, kernel: str, mode: int) -> None:
         """Measurement of "vertex_peel" (as push_probe) or "dense_peel" (the
-        bit-matrix edge-peel round; push_stats then gives slots = the
+        truss-level step of bit-matrix cores; push_stats then gives slots = the
         frontier edges' d+(u) + d+(v) summed, vertices = frontier edges)."""
         _check(self._lib.kt_kernel_probe(self._h, {"vertex_peel": 0, "dense_peel": 1}[kernel], int(mode)))
 

@@ -1,19 +1,20 @@
 // Stage logic of the device-resident two-pass k-max-truss solve (host side).
 //
 // Flow (reference: src/kc_gpu.cpp:129-208, 336-341; src/kc.cu:770-884, 1140-1309):
-//   (b) vertex peel with a galloping threshold -> max-core C0. When a step
-//       leaves few vertices alive, the rest of the peel continues on their
-//       induced subgraph (a new level with dense ids), so high thresholds
-//       never rescan the rows of vertices already gone.
+//   (b) core numbers of the subgraph induced by the vertices of high degree
+//       (a new level with dense ids) -> max-core C0; or, where degrees do not
+//       set a core apart, a vertex peel with a galloping threshold, which
+//       continues on the induced subgraph once few vertices are alive.
 //   pass 1: rank + orient C0, exact supports, truss levels -> k̂ <= kmax.
 //   pass 2: the (L-1)-core C, L = max(k̂, 3) (it holds the kmax-truss),
 //       recovered from the deepest level that contains it; rank + orient,
 //       exact supports, truss levels upward from L with the reference's early
 //       exit (first level equal to pass 1's truss, src/kc.cu:1240-1241).
-//   Peeling drops a frontier holding a third of the live edges and recounts
-//   the rest (src/kc.cu:988, 1206-1233), and compacts once half the edges
-//   are dead, carrying supports (src/kc.cu:1174-1178).
-// Only scalar counters cross to the host.
+//   Levels advance on the device, one launch per step (kt_step.hip); dropping
+//   a frontier for a recount of the rest (src/kc.cu:988, 1206-1233) is a
+//   decision of cost there, and so is listing the live edges anew once half
+//   are dead (src/kc.cu:1174-1178).
+// Only scalar counters and the search's state cross to the host.
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
