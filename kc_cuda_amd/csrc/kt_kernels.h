@@ -197,8 +197,6 @@ void support_edges(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t*
 //     < r: deleted earlier.
 void edge_frontier_init(const uint32_t* state, const int32_t* sup, uint32_t mc, int32_t thr,
                         uint32_t* q, uint32_t* qcount, hipStream_t s);
-void edge_min_support(const uint32_t* state, const int32_t* sup, uint32_t mc, uint32_t* out,
-                      hipStream_t s);
 
 void w_stats(const uint32_t* off_d, const uint32_t* src, const uint32_t* dst, const uint32_t* del_thr,
              uint32_t mc, int32_t floor, uint64_t* out2, hipStream_t s);

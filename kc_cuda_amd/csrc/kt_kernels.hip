@@ -1439,23 +1439,6 @@ __global__ __launch_bounds__(kBlock) void k_edge_frontier(const uint32_t* __rest
       [&](uint32_t at, uint64_t e) { q[at] = uint32_t(e); }, qcount);
 }
 
-__global__ __launch_bounds__(kBlock) void k_min_support(const uint32_t* __restrict__ state,
-                                                        const int32_t* __restrict__ sup, uint32_t mc,
-                                                        uint32_t* out) {
-  __shared__ uint32_t s_min[kBlock / kWave];
-  uint32_t best = kNone;
-  for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < mc; e += gridDim.x * blockDim.x)
-    if (state[e] == kNone) best = min(best, uint32_t(sup[e]));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) best = min(best, uint32_t(__shfl_xor(best, o)));
-  if (lane64() == 0) s_min[threadIdx.x / kWave] = best;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < kBlock / kWave; ++k) best = min(best, s_min[k]);
-    if (best != kNone) atomicMin(out, best);
-  }
-}
-
 // Row index of every slot of a CSR with uint32 offsets.
 __global__ __launch_bounds__(kBlock) void k_row_src(const uint32_t* __restrict__ off, uint32_t rows,
                                                     uint32_t* src) {
@@ -2120,9 +2103,6 @@ void support_edges(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t*
 void edge_frontier_init(const uint32_t* state, const int32_t* sup, uint32_t mc, int32_t thr, uint32_t* q,
                         uint32_t* qcount, hipStream_t s) {
   if (mc) k_edge_frontier<<<grid_tiles(mc), kBlock, 0, s>>>(state, sup, mc, thr, q, qcount);
-}
-void edge_min_support(const uint32_t* state, const int32_t* sup, uint32_t mc, uint32_t* out, hipStream_t s) {
-  if (mc) k_min_support<<<std::min(grid_for(mc), 2048), kBlock, 0, s>>>(state, sup, mc, out);
 }
 
 }  // namespace kt
