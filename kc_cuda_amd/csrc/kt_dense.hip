@@ -81,7 +81,7 @@ __global__ __launch_bounds__(kBlock) void k_rank_rows(const uint64_t* __restrict
 // workgroup, and ebase[r] = off_d[r] less r's neighbours of a lower rank: the
 // neighbour at place k of row r has the edge id ebase[r] + k. *simple
 // = 1 when the bits stand for all of the rows' `slots` slots and
-// every edge has both of its bits; else the view is left without edges.
+// as many lie above the diagonal as below; else the view is left without edges.
 constexpr uint32_t kScanBlock = 1024;
 __global__ __launch_bounds__(kScanBlock) void k_rank_scan(const uint32_t* __restrict__ du,
                                                           const uint32_t* __restrict__ dout, uint32_t nc,
@@ -134,7 +134,9 @@ __global__ __launch_bounds__(kScanBlock) void k_rank_scan(const uint32_t* __rest
 }
 
 // The rows' entries: undirected (neighbour, edge id), oriented (neighbour,
-// source), the edge-id matrix (null: none) and fresh peel state. One wave per
+// source), the edge-id matrix (null: none) and fresh peel state; *simple = 0
+// when a bit below the diagonal has no mirror (as many lie above, so then all
+// have one). One wave per
 // row and run of words, a word's 64 bits on the wave's lanes, so every array
 // is written in order.
 constexpr uint32_t kFillWords = 16;
@@ -144,7 +146,7 @@ __global__ __launch_bounds__(kBlock) void k_rank_fill(const unsigned long long* 
                                                       const uint32_t* __restrict__ ebase, uint32_t nc, uint32_t ws,
                                                       uint32_t* adj_u, uint32_t* eid_u, uint32_t* adj_d,
                                                       uint32_t* src, uint32_t* orig, uint32_t* state,
-                                                      uint32_t* del_thr, uint32_t* eidm) {
+                                                      uint32_t* del_thr, uint32_t* eidm, uint32_t* simple) {
   const uint32_t lane = uint32_t(lane64());
   const unsigned long long below = (1ull << lane) - 1ull;
   const uint32_t runs = (ws + kFillWords - 1) / kFillWords;
@@ -170,6 +172,10 @@ __global__ __launch_bounds__(kBlock) void k_rank_fill(const unsigned long long* 
         del_thr[e] = kNone;
       } else {  // the edge of w's row
         const uint64_t q = uint64_t(w) * ws + (r >> 6);
+        if (!((bits0[q] >> (r & 63)) & 1ull)) {  // rows from lines need not mirror each other
+          *simple = 0;
+          continue;
+        }
         e = ebase[w] + pref0[q] + uint32_t(__popcll(bits0[q] & rbelow));
       }
       adj_u[ub + k] = w;
@@ -235,12 +241,12 @@ void rank_scan(const uint32_t* du, const uint32_t* dout, uint32_t nc, uint64_t s
 }
 void rank_fill(const uint64_t* bits0, const uint32_t* pref0, const uint32_t* off_u, const uint32_t* ebase, uint32_t nc,
                uint32_t ws, uint32_t* adj_u, uint32_t* eid_u, uint32_t* adj_d, uint32_t* src, uint32_t* orig,
-               uint32_t* state, uint32_t* del_thr, uint32_t* eidm, hipStream_t s) {
+               uint32_t* state, uint32_t* del_thr, uint32_t* eidm, uint32_t* simple, hipStream_t s) {
   const uint64_t waves = uint64_t(nc) * ((ws + kFillWords - 1) / kFillWords);
   if (nc)
     k_rank_fill<<<std::min(grid_for(waves * kWave), 8192), kBlock, 0, s>>>(
         reinterpret_cast<const unsigned long long*>(bits0), pref0, off_u, ebase, nc, ws, adj_u, eid_u, adj_d, src,
-        orig, state, del_thr, eidm);
+        orig, state, del_thr, eidm, simple);
 }
 // Measured (vertices, edges; by edge -> by pairs): 1,268, 483 k: 20 -> 23 us;
 // 1,535, 912 k: 37 -> 23; 2,867, 878 k: 39 -> 34; 3,150, 3.05 M: 136 -> 39;

@@ -266,7 +266,8 @@ void group_rows(const SplitPlan& p, const uint32_t* part, const uint64_t* off_b,
 // Dense core views through their bit-matrix rows (kt_dense.hip), in this
 // order: rows of the level's vertices inv[0..nc) in rank ids (to); the offsets
 // (*simple = 0 and no edge when the bits do not stand for `slots` row slots);
-// every array of the view (eidm nullable). max_row: *out = the longest row.
+// every array of the view (eidm nullable; *simple = 0 when rows do not mirror
+// each other). max_row: *out = the longest row.
 void rank_rows(const uint64_t* off, const uint32_t* adj, const uint32_t* to, const uint32_t* inv, uint32_t nc,
                uint32_t ws, uint64_t* bits0, uint64_t* bits, uint32_t* pref0, uint32_t* du, uint32_t* dout,
                hipStream_t s);
@@ -274,7 +275,7 @@ void rank_scan(const uint32_t* du, const uint32_t* dout, uint32_t nc, uint64_t s
                uint32_t* off_u, uint32_t* ebase, uint32_t* simple, hipStream_t s);
 void rank_fill(const uint64_t* bits0, const uint32_t* pref0, const uint32_t* off_u, const uint32_t* ebase, uint32_t nc,
                uint32_t ws, uint32_t* adj_u, uint32_t* eid_u, uint32_t* adj_d, uint32_t* src, uint32_t* orig,
-               uint32_t* state, uint32_t* del_thr, uint32_t* eidm, hipStream_t s);
+               uint32_t* state, uint32_t* del_thr, uint32_t* eidm, uint32_t* simple, hipStream_t s);
 void max_row(const uint32_t* off, uint32_t rows, uint32_t* out, hipStream_t s);
 // A count by all pairs of rows in word ANDs of one by edge, and whether it is
 // the faster one for a fresh view.

@@ -366,6 +366,7 @@ class Solver {
   }
 
   uint32_t n_ = 0;
+  bool mirrored_ = false;  // every row slot has its mirror (an input of pairs)
   uint64_t m_ = 0, slots_ = 0;  // edges and row slots of the input
   // full graph
   DevBuf off_, adj_, deg_, lvl_, q0_, q1_, deg_bak_, cursor_, hist_, hoff_, part_, part2_, split_;

@@ -377,6 +377,7 @@ void Solver::build_from_pairs(const uint32_t* d_pairs, uint64_t m, uint32_t n) {
   n_ = n;
   m_ = m;
   slots_ = 2 * m;
+  mirrored_ = true;
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   cursor_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
@@ -397,6 +398,7 @@ void Solver::build_from_lines(const uint32_t* d_xs, const uint32_t* d_ys, uint64
   n_ = n;
   m_ = L / 2;
   slots_ = L;
+  mirrored_ = false;
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   cursor_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
@@ -418,6 +420,7 @@ void Solver::load_csr_host(uint32_t n, const uint64_t* off, const uint32_t* adj)
   n_ = n;
   m_ = off[n] / 2;
   slots_ = off[n];
+  mirrored_ = false;
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   adj_.ensure(sizeof(uint32_t) * std::max<uint64_t>(off[n], 1));

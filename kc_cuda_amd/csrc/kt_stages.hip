@@ -618,8 +618,8 @@ bool Solver::wants_dense(uint32_t nc, uint32_t mc) const {
 }
 
 // The view of a dense core through its bit-matrix rows (kt_dense.hip): no
-// count, sort or transpose of its rows, and one wait, taken while the view is
-// filled. `slots` = the sum of the core's degrees. False: the rows do not
+// count, sort or transpose of its rows, and one wait, taken while the view of
+// an input of pairs is filled. `slots` = the sum of the core's degrees. False: the rows do not
 // describe a simple graph, nothing is filled.
 bool Solver::extract_dense(LevelGraph& g, CoreView* cv, uint64_t slots) {
   const uint32_t mc = uint32_t(slots / 2), nc = cv->nc, ws = dense_words(nc);
@@ -646,11 +646,15 @@ bool Solver::extract_dense(LevelGraph& g, CoreView* cv, uint64_t slots) {
   uint32_t* simple = core_out_.as<uint32_t>();
   rank_scan(din_.as<uint32_t>(), dout_.as<uint32_t>(), nc, slots, off_d_.as<uint32_t>(), off_u_.as<uint32_t>(),
             din_off_.as<uint32_t>(), simple, stream_);
-  KT_HIP(hipMemcpyAsync(pinned_, simple, sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
-  KT_HIP(hipEventRecord(ev_[10], stream_));
+  auto ask = [&] {
+    KT_HIP(hipMemcpyAsync(pinned_, simple, sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
+    KT_HIP(hipEventRecord(ev_[10], stream_));
+  };
+  if (mirrored_) ask();  // rows from pairs: nothing is found out while the view is filled
   rank_fill(bits0_.as<uint64_t>(), pref0_.as<uint32_t>(), off_u_.as<uint32_t>(), din_off_.as<uint32_t>(), nc, ws,
             adj_u_.as<uint32_t>(), eid_u_.as<uint32_t>(), adj_d_.as<uint32_t>(), src_.as<uint32_t>(),
-            orig0_.as<uint32_t>(), state_.as<uint32_t>(), del_thr_.as<uint32_t>(), eidm, stream_);
+            orig0_.as<uint32_t>(), state_.as<uint32_t>(), del_thr_.as<uint32_t>(), eidm, simple, stream_);
+  if (!mirrored_) ask();
   KT_HIP(hipEventSynchronize(ev_[10]));
   if (!pinned_[0]) return false;
   cv->mc = cv->mc0 = mc;

@@ -136,3 +136,27 @@ def test_counts_by_pairs_equal_rows(dense_ctx, n, p):
         want = other.trussness()
     assert (r.kmax, r.truss_edges, r.k_hat) == (ref.kmax, ref.truss_edges, ref.k_hat)
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_one_sided_lines_equal_rows(dense_ctx, seed):
+    """Lines that list some edges in one direction only, as many each way (two
+    copies of a graph, the other half of the lines left out in each), solve as
+    on a core of sorted rows."""
+    from kc_cuda_amd import Context
+    n = 130
+    e = np.asarray(random_graph(n, 0.4, seed, cliques=(12,)), np.uint32).reshape(-1, 2)
+    cut = np.random.default_rng(seed).random(len(e)) < 0.1
+    both = np.concatenate([e, e[:, ::-1]])
+    a = np.concatenate([both[:len(e)], both[len(e):][~cut]])
+    b = np.concatenate([both[:len(e)][~cut], both[len(e):]]) + n
+    lines = np.concatenate([a, b]).astype(np.uint32)
+    lines = lines[np.lexsort((lines[:, 0], lines[:, 1]))]
+    xs, ys = np.ascontiguousarray(lines[:, 0]), np.ascontiguousarray(lines[:, 1])
+    r = dense_ctx.solve_lines(xs, ys, 2 * n)
+    with Context(0) as other:
+        other.tune(core="sparse")
+        ref = other.solve_lines(xs, ys, 2 * n)
+        want = other.truss_edges()
+    assert (r.kmax, r.truss_edges, r.k_hat) == (ref.kmax, ref.truss_edges, ref.k_hat)
+    np.testing.assert_array_equal(dense_ctx.truss_edges(), want)
