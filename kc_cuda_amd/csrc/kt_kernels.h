@@ -285,10 +285,12 @@ bool dense_by_pairs(uint32_t nc, uint32_t mc, uint32_t ws);
 // pairs of rows (dense_support: by edge)
 void dense_count(const uint64_t* bits, const uint32_t* pref0, const uint32_t* off_u, const uint32_t* eid_u,
                  const uint32_t* eidm, uint32_t nc, uint32_t ws, int32_t* sup, hipStream_t s);
-// Triangle lists (kt_list.hip). sum_u32: *total (starts at 0) += the sum.
+// Triangle lists (kt_list.hip). list_size: found[0] = the sum of the supports,
+// found[1] = 1 when a row is not strictly ascending above its own vertex.
 // tri_fill: every triangle's entries, cursor starting as a copy of the offsets
-// (bitmap, lanes: as the support count's kernels).
-void sum_u32(const uint32_t* in, uint32_t n, uint64_t* total, hipStream_t s);
+// (bitmap: the enumeration that counted the supports; lanes: as the count's).
+void list_size(const int32_t* sup, const uint32_t* src, const uint32_t* adj, uint32_t mc, uint64_t* found,
+               hipStream_t s);
 void tri_fill(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* src, uint32_t nc, uint32_t mc,
               uint32_t max_dout, bool bitmap, int lanes, uint32_t* cursor, uint32_t* tri, hipStream_t s);
 // Truss levels of a core with triangle lists or dense rows (kt_step.hip):

@@ -108,21 +108,37 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill_edges(const uint32_t* __res
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_sum_u32(const uint32_t* __restrict__ in, uint32_t n,
-                                                    unsigned long long* total) {
+// found[0] += the sum of the supports, found[1] = 1 when a row is not strictly
+// ascending above its own vertex. The count and the fill need not agree on
+// such rows (a repeated neighbour is found once by a search, and by each of
+// its copies where they are streamed), so entries would miss their lists.
+__global__ __launch_bounds__(kBlock) void k_list_size(const uint32_t* __restrict__ sup,
+                                                      const uint32_t* __restrict__ src,
+                                                      const uint32_t* __restrict__ adj, uint32_t mc,
+                                                      unsigned long long* found) {
   unsigned long long c = 0;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) c += in[i];
+  bool odd = false;
+  for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < mc; i += gridDim.x * blockDim.x) {
+    const uint32_t u = src[i], v = adj[i];
+    c += sup[i];
+    odd |= v <= u || (i + 1 < mc && src[i + 1] == u && adj[i + 1] <= v);
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if (lane64() == 0 && c) atomicAdd(total, c);
+  if (lane64() == 0 && c) atomicAdd(&found[0], c);
+  if (__ballot(odd) && lane64() == 0) found[1] = 1;
 }
 
 }  // namespace
 
 // --------------------------------------------------------------- wrappers ---
 
-void sum_u32(const uint32_t* in, uint32_t n, uint64_t* total, hipStream_t s) {
-  if (n) k_sum_u32<<<std::min(grid_for(n), 1024), kBlock, 0, s>>>(in, n, reinterpret_cast<unsigned long long*>(total));
+void list_size(const int32_t* sup, const uint32_t* src, const uint32_t* adj, uint32_t mc, uint64_t* found,
+               hipStream_t s) {
+  fill_u64(found, 2, 0, s);
+  if (mc)
+    k_list_size<<<std::min(grid_for(mc), 1024), kBlock, 0, s>>>(reinterpret_cast<const uint32_t*>(sup), src, adj, mc,
+                                                                reinterpret_cast<unsigned long long*>(found));
 }
 
 void tri_fill(const uint32_t* off_d, const uint32_t* adj_d, const uint32_t* src, uint32_t nc, uint32_t mc,

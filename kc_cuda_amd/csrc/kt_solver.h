@@ -303,6 +303,7 @@ class Solver {
   // frontier of the live edges below thr, stamped; the rounds' starting state
   // (reset: a new search with its early-exit rule)
   bool list_triangles(const CoreView& cv);
+  bool counts_by_bitmap(const CoreView& cv) const;
   StepArgs step_args(const CoreView& cv);
   TrussOutcome run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32_t* r_io, const SearchRule& search,
                          bool allow_host);

@@ -741,6 +741,11 @@ void Solver::build_undirected_view(CoreView* cv) {
 
 // ------------------------------------------------------------ (c) count ---
 
+// Which enumeration counts a sorted-row core's triangles (and lists them).
+bool Solver::counts_by_bitmap(const CoreView& cv) const {
+  return !force_edge_count_ && support_bitmap_fits(cv.nc, cv.max_dout);
+}
+
 void Solver::count_support(CoreView* cv, float* ms) {
   // (the dense count writes every support)
   if (!cv->dense) fill_u32(reinterpret_cast<uint32_t*>(cv->sup), cv->mc, 0, stream_);
@@ -754,7 +759,7 @@ void Solver::count_support(CoreView* cv, float* ms) {
       dense_count(cv->bits, cv->pref0, cv->off_u, cv->eid_u, cv->eidm, cv->nc, cv->ws, cv->sup, stream_);
     else
       dense_support(cv->off_d, cv->adj_d, cv->nc, cv->mc, cv->bits, cv->ws, nullptr, cv->sup, stream_);
-  } else if (!force_edge_count_ && support_bitmap_fits(cv->nc, cv->max_dout)) {
+  } else if (counts_by_bitmap(*cv)) {
     kind = 0;
     support_bitmap(cv->off_d, cv->adj_d, cv->nc, cv->max_dout, lanes, cv->sup, ctl_, stream_);
   } else
@@ -878,16 +883,21 @@ TrussOutcome Solver::truss_search(CoreView* cv, int32_t thr0, uint64_t early_ans
 // Triangle lists of a base view whose supports are counted: offsets in
 // tri_off_, the pairs of partner edges in tri_. False when they do not fit
 // the budget (tri_budget_ bytes, tri_per_edge_ a core edge, and of more than
-// 1 GiB half of the device memory that is free).
+// 1 GiB half of the device memory that is free), or when rows repeat a
+// neighbour (or, given by a caller, are not in order): the lists are laid out
+// by the counted supports, which the fill then need not find again.
 bool Solver::list_triangles(const CoreView& cv) {
   const uint32_t mc = cv.mc;
   if (cv.work != -1) return false;
-  step_ctl_.ensure(kStepCtlBytes + sizeof(uint64_t));
-  uint64_t* total = reinterpret_cast<uint64_t*>(step_ctl_.as<uint8_t>() + kStepCtlBytes);
-  fill_u64(total, 1, 0, stream_);
-  sum_u32(reinterpret_cast<const uint32_t*>(cv.sup), mc, total, stream_);
-  const uint64_t entries = read_u64(total), bytes = entries * sizeof(uint2);
-  if (entries >= (uint64_t(1) << 31) || bytes > tri_budget_ || bytes > tri_per_edge_ * mc) return false;
+  step_ctl_.ensure(kStepCtlBytes);
+  uint64_t* found = step_ctl_.as<uint64_t>();  // free until the steps start
+  list_size(cv.sup, cv.src, cv.adj_d, mc, found, stream_);
+  KT_HIP(hipMemcpyAsync(pinned_, found, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_));
+  KT_HIP(hipStreamSynchronize(stream_));
+  uint64_t got[2];
+  std::memcpy(got, pinned_, sizeof(got));
+  const uint64_t entries = got[0], bytes = entries * sizeof(uint2);
+  if (got[1] || entries >= (uint64_t(1) << 31) || bytes > tri_budget_ || bytes > tri_per_edge_ * mc) return false;
   if (bytes > tri_.bytes && bytes > (uint64_t(1) << 30)) {
     size_t free_bytes = 0, total_bytes = 0;
     KT_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
@@ -903,7 +913,7 @@ bool Solver::list_triangles(const CoreView& cv) {
   exclusive_scan_u32(reinterpret_cast<const uint32_t*>(cv.sup), off, mc + 1);
   KT_HIP(hipMemcpyAsync(cursor, off, sizeof(uint32_t) * mc, hipMemcpyDeviceToDevice, stream_));
   const double avg = cv.nc ? double(mc) / cv.nc : 0.0;
-  tri_fill(cv.off_d, cv.adj_d, cv.src, cv.nc, mc, cv.max_dout, support_bitmap_fits(cv.nc, cv.max_dout),
+  tri_fill(cv.off_d, cv.adj_d, cv.src, cv.nc, mc, cv.max_dout, counts_by_bitmap(cv),
            lanes_count_ ? lanes_count_ : auto_lanes(avg), cursor, tri_.as<uint32_t>(), stream_);
   return true;
 }
@@ -919,7 +929,7 @@ TrussOutcome Solver::run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32
   constexpr uint32_t kFirstBatch = 8, kMaxBatch = 32;
   static_assert(sizeof(StepState) * 2 + sizeof(StepCounters) * 3 <= kStepCtlBytes, "step control block too small");
   static_assert(sizeof(StepState) <= 4 * kTrussCountWord, "state exceeds the pinned readback buffer");
-  step_ctl_.ensure(kStepCtlBytes + sizeof(uint64_t));
+  step_ctl_.ensure(kStepCtlBytes);
   TrussOutcome out;
   StepState h{};
   h.round = *r_io - 1;

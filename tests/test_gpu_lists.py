@@ -160,3 +160,25 @@ def test_one_sided_lines_equal_rows(dense_ctx, seed):
         want = other.truss_edges()
     assert (r.kmax, r.truss_edges, r.k_hat) == (ref.kmax, ref.truss_edges, ref.k_hat)
     np.testing.assert_array_equal(dense_ctx.truss_edges(), want)
+
+
+@pytest.mark.parametrize("by_edge", [False, True])
+def test_rows_that_repeat_a_neighbour_are_not_listed(by_edge):
+    """Pairs given more than once: the two support counts find different
+    triangles on such rows, so they are peeled by rows, whatever the budget."""
+    from kc_cuda_amd import Context
+    rng = np.random.default_rng(7)
+    once = np.argwhere(np.triu(rng.random((80, 80)) < 0.4, 1))
+    pairs = np.concatenate([once, once[rng.random(len(once)) < 0.3]]).astype(np.uint32)
+    mp = pytest.MonkeyPatch()
+    mp.setenv("KT_LIST_BUDGET_MB", "0")
+    with Context(0) as rows:
+        mp.undo()
+        rows.tune(core="sparse", force_edge_count=by_edge)
+        want = rows.solve_pairs(pairs, 80)
+        want_t = rows.trussness()
+    with Context(0) as lists:
+        lists.tune(core="sparse", force_edge_count=by_edge)
+        got = lists.solve_pairs(pairs, 80)
+        assert (got.kmax, got.truss_edges, got.k_hat) == (want.kmax, want.truss_edges, want.k_hat)
+        np.testing.assert_array_equal(lists.trussness(), want_t)
