@@ -123,8 +123,12 @@ uint64_t Solver::peel_vertices_rounds(LevelGraph& g, uint32_t k, uint64_t stop_a
   }
 }
 
-// Induced subgraph of the alive vertices of `p` as the next level.
+// Induced subgraph of the alive vertices of `p` as the next level. Rows that
+// need not mirror each other are always counted anew: what a peel leaves as a
+// vertex's degree (its slots less those of the removed vertices that name it)
+// is then not the number of alive vertices in its row, which sizes the cut's.
 LevelGraph& Solver::cut_level(LevelGraph& p, uint32_t k_enter, uint32_t alive, bool recount) {
+  recount |= !mirrored_;
   if (levels_.size() <= depth_) levels_.emplace_back(new LevelGraph);
   LevelGraph& s = *levels_[depth_];
   // alive bitmap | word popcounts | their exclusive scan, then the ranked list

@@ -60,3 +60,26 @@ def test_cores_that_unravel_along_a_path(ctx, path):
     pairs = _lollipop(path, 7)
     r = ctx.solve_pairs(pairs, 7 + path)
     assert (r.max_core, r.kmax, r.truss_edges) == (6, 7, 21)
+
+
+@pytest.mark.parametrize("down", [False, True])
+@pytest.mark.parametrize("vertex", ["cascade", "rounds"])
+def test_lines_in_one_direction_only(ctx, vertex, down):
+    """Rows that do not mirror each other, searched by peels with a cut at 275
+    of 2,000 vertices: the same answer twice, and the
+    right one for the next graph. The peels' degrees do not size such rows."""
+    from kc_cuda_amd import Context
+    rng = np.random.default_rng(6)
+    e = np.argwhere(np.triu(rng.random((2000, 2000), dtype=np.float32) < 0.012, 1))
+    x, y = (e[:, 1], e[:, 0]) if down else (e[:, 0], e[:, 1])
+    order = np.lexsort((x, y))
+    xs, ys = x[order].astype(np.uint32), y[order].astype(np.uint32)
+    pairs = e.astype(np.uint32)
+    ref = O.solve_pairs(pairs, 2000)
+    with Context(0) as c:
+        c.tune(vertex=vertex)
+        one = c.solve_lines(xs, ys, 2000)
+        two = c.solve_lines(xs, ys, 2000)
+        assert (one.max_core, one.k_hat, one.kmax, one.truss_edges) == (two.max_core, two.k_hat, two.kmax, two.truss_edges)
+        r = c.solve_pairs(pairs, 2000)
+        assert (r.max_core, r.kmax, r.truss_edges) == (ref.max_core, ref.kmax, ref.truss_edges)
