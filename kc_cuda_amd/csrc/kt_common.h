@@ -77,6 +77,7 @@ struct Ctl {
   uint32_t vq_chunks;
   uint32_t vq_err;
   uint32_t vq_removed;   // vertices queued so far (a lower bound while waves run)
+  uint64_t mirror;       // CSR build: 0 when every slot has its mirror
 };
 
 // ctl->vq_err values

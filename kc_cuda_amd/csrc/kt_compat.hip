@@ -269,7 +269,7 @@ int kc_count_deg_with_mask(const uint32_t* nbr, const uint32_t* nbr_u, uint32_t 
     std::vector<uint32_t> dm(N);
     s.level0_degrees_to_host(dm.data());
     kt::CoreView cv;
-    s.extract_core(s.level0(), &cv, false);
+    s.extract_core(s.level0(), &cv);
     const uint32_t nc = cv.nc;
     std::vector<uint32_t> inv(nc), dout(nc), pos(N, 0);
     s.core_ranks_to_host(cv, inv.data(), dout.data());

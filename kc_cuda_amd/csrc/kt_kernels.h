@@ -53,6 +53,9 @@ void csr_sorted_check(int mode, const uint32_t* keys, uint64_t items, uint32_t n
                       uint32_t* unsorted, uint32_t* err, hipStream_t s);
 void csr_deg_from_runs(const uint64_t* hpos, const uint64_t* tpos, uint32_t n, uint32_t* deg, hipStream_t s);
 void csr_copy_cols(const uint32_t* xs, uint64_t L, uint32_t n, uint32_t* adj, uint32_t* err, hipStream_t s);
+// *sum = 0 when every line or row slot (x in row y) has its mirror (y in row x)
+void mirror_lines(const uint32_t* xs, const uint32_t* ys, uint64_t L, uint64_t* sum, hipStream_t s);
+void mirror_rows(const uint64_t* off, const uint32_t* adj, uint32_t n, uint64_t* sum, hipStream_t s);
 void csr_fwd_start(const uint32_t* pairs, uint64_t items, uint32_t S, uint32_t B, uint64_t* f0, hipStream_t s);
 
 // (b) vertex peeling (k-core). lvl[v] == kNone: alive; otherwise the

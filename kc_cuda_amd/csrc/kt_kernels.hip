@@ -348,6 +348,41 @@ __global__ __launch_bounds__(kBlock) void k_copy_cols(const uint32_t* __restrict
   if (__syncthreads_or(big) && threadIdx.x == 0) atomicOr(err, 1u);
 }
 
+// Whether every slot (row y, column x) has its mirror: the sum of hash(x, y) -
+// hash(y, x) over the slots is 0 when it has, and but for one chance in 2^64
+// nothing else. One pass over what the build reads anyway (10M lines: 20 us).
+__device__ __forceinline__ unsigned long long slot_hash(uint32_t x, uint32_t y) {
+  unsigned long long z = (uint64_t(x) << 32 | y) * 0x9E3779B97F4A7C15ull;
+  z = (z ^ (z >> 32)) * 0xD6E8FEB86659FD93ull;
+  return z ^ (z >> 32);
+}
+__device__ __forceinline__ void add_mirror_sum(unsigned long long c, unsigned long long* sum) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+  if (lane64() == 0 && c) atomicAdd(sum, c);
+}
+__global__ __launch_bounds__(kBlock) void k_mirror_lines(const uint32_t* __restrict__ xs,
+                                                         const uint32_t* __restrict__ ys, uint64_t L,
+                                                         unsigned long long* sum) {
+  unsigned long long c = 0;
+  const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
+  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < L; i += stride) {
+    const uint32_t x = xs[i], y = ys[i];
+    c += slot_hash(x, y) - slot_hash(y, x);
+  }
+  add_mirror_sum(c, sum);
+}
+__global__ __launch_bounds__(kBlock) void k_mirror_rows(const uint64_t* __restrict__ off,
+                                                        const uint32_t* __restrict__ adj, uint32_t n,
+                                                        unsigned long long* sum) {
+  unsigned long long c = 0;
+  const uint32_t waves = gridDim.x * (kBlock / kWave);
+  for (uint32_t y = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; y < n; y += waves)
+    for (uint64_t j = off[y] + uint32_t(lane64()); j < off[y + 1]; j += kWave)
+      c += slot_hash(adj[j], y) - slot_hash(y, adj[j]);
+  add_mirror_sum(c, sum);
+}
+
 // f0[b] = index of the first pair whose first id is >= b << S (pairs sorted
 // by their first id), for b < B; f0[B] = items.
 __global__ void k_fwd_start(const uint2* __restrict__ pairs, uint64_t items, uint32_t S, uint32_t B,
@@ -1886,6 +1921,18 @@ void csr_deg_from_runs(const uint64_t* hpos, const uint64_t* tpos, uint32_t n, u
 }
 void csr_copy_cols(const uint32_t* xs, uint64_t L, uint32_t n, uint32_t* adj, uint32_t* err, hipStream_t s) {
   if (L) k_copy_cols<<<grid_for(L, 4 * kBlock), kBlock, 0, s>>>(xs, L, n, adj, err);
+}
+void mirror_lines(const uint32_t* xs, const uint32_t* ys, uint64_t L, uint64_t* sum, hipStream_t s) {
+  fill_u64(sum, 1, 0, s);
+  if (L)
+    k_mirror_lines<<<std::min(grid_for(L, 4 * kBlock), 2048), kBlock, 0, s>>>(
+        xs, ys, L, reinterpret_cast<unsigned long long*>(sum));
+}
+void mirror_rows(const uint64_t* off, const uint32_t* adj, uint32_t n, uint64_t* sum, hipStream_t s) {
+  fill_u64(sum, 1, 0, s);
+  if (n)
+    k_mirror_rows<<<std::min(grid_for(uint64_t(n) * kWave), 2048), kBlock, 0, s>>>(
+        off, adj, n, reinterpret_cast<unsigned long long*>(sum));
 }
 void csr_fwd_start(const uint32_t* pairs, uint64_t items, uint32_t S, uint32_t B, uint64_t* f0, hipStream_t s) {
   k_fwd_start<<<grid_for(uint64_t(B) + 1), kBlock, 0, s>>>(reinterpret_cast<const uint2*>(pairs), items, S, B, f0);

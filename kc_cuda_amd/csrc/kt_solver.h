@@ -244,9 +244,7 @@ class Solver {
   // bound), from the degree histogram of the current input; ~0 when none.
   uint64_t degree_at_least(uint32_t k) const;
   void core_at(uint32_t k);  // leaves the k-core alive on the deepest usable level
-  // symmetric: every row slot has its mirror (false: the rows come from the
-  // caller unchecked)
-  void extract_core(LevelGraph& g, CoreView* cv, bool symmetric = true);
+  void extract_core(LevelGraph& g, CoreView* cv);
   bool extract_dense(LevelGraph& g, CoreView* cv, uint64_t slots);
   bool wants_dense(uint32_t nc, uint32_t mc) const;
   void sort_oriented_rows(uint32_t nc, uint32_t mc, uint32_t max_row);
@@ -367,7 +365,8 @@ class Solver {
   }
 
   uint32_t n_ = 0;
-  bool mirrored_ = false;  // every row slot has its mirror (an input of pairs)
+  bool paired_ = false;    // an input of pairs: every row slot has its mirror
+  bool mirrored_ = false;  // so it has, as far as a sum of hashes tells (no access relies on it)
   uint64_t m_ = 0, slots_ = 0;  // edges and row slots of the input
   // full graph
   DevBuf off_, adj_, deg_, lvl_, q0_, q1_, deg_bak_, cursor_, hist_, hoff_, part_, part2_, split_;

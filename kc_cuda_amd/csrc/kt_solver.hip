@@ -354,8 +354,9 @@ bool Solver::build_sorted_lines(const uint32_t* xs, const uint32_t* ys, uint64_t
   zero_u32(&ctl_->pad[0]);
   zero_u32(&ctl_->err);
   csr_sorted_check(1, ys, L, n, hpos, tpos, &ctl_->pad[0], &ctl_->err, stream_);
-  if (read_u32(&ctl_->pad[0]) != 0) return false;
-  if (read_u32(&ctl_->err)) fail("edge list holds a vertex id >= n");
+  const Ctl h = read_ctl();
+  if (h.pad[0] != 0) return false;
+  if (h.err) fail("edge list holds a vertex id >= n");
   csr_deg_from_runs(hpos, tpos, n, deg(), stream_);
   exclusive_scan_u32_to_u64(deg(), off(), n + 1);
   csr_copy_cols(xs, L, n, adj(), &ctl_->err, stream_);
@@ -377,7 +378,7 @@ void Solver::build_from_pairs(const uint32_t* d_pairs, uint64_t m, uint32_t n) {
   n_ = n;
   m_ = m;
   slots_ = 2 * m;
-  mirrored_ = true;
+  paired_ = mirrored_ = true;
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   cursor_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
@@ -398,11 +399,13 @@ void Solver::build_from_lines(const uint32_t* d_xs, const uint32_t* d_ys, uint64
   n_ = n;
   m_ = L / 2;
   slots_ = L;
-  mirrored_ = false;
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   cursor_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   adj_.ensure(sizeof(uint32_t) * std::max<uint64_t>(L, 1));
+  paired_ = false;
+  mirror_lines(d_xs, d_ys, L, &ctl_->mirror, stream_);
+  mirrored_ = read_u64(&ctl_->mirror) == 0;
   if (!force_atomic_build_ && sorted_build_ && build_sorted_lines(d_xs, d_ys, L, n)) return;
   if (!force_atomic_build_ && build_partitioned(1, d_xs, d_ys, L, n)) return;
   fill_u32(deg(), uint64_t(n) + 1, 0, stream_);
@@ -420,14 +423,15 @@ void Solver::load_csr_host(uint32_t n, const uint64_t* off, const uint32_t* adj)
   n_ = n;
   m_ = off[n] / 2;
   slots_ = off[n];
-  mirrored_ = false;
   deg_.ensure(sizeof(uint32_t) * (size_t(n) + 1));
   off_.ensure(sizeof(uint64_t) * (size_t(n) + 1));
   adj_.ensure(sizeof(uint32_t) * std::max<uint64_t>(off[n], 1));
   KT_HIP(hipMemcpyAsync(off_.p, off, sizeof(uint64_t) * (size_t(n) + 1), hipMemcpyHostToDevice, stream_));
   if (off[n])
     KT_HIP(hipMemcpyAsync(adj_.p, adj, sizeof(uint32_t) * off[n], hipMemcpyHostToDevice, stream_));
-  KT_HIP(hipStreamSynchronize(stream_));
+  paired_ = false;
+  mirror_rows(off_.as<uint64_t>(), adj_.as<uint32_t>(), n, &ctl_->mirror, stream_);
+  mirrored_ = read_u64(&ctl_->mirror) == 0;
 }
 
 void Solver::csr_to_host(uint64_t* off, uint32_t* adj) {

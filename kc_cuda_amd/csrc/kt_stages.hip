@@ -128,7 +128,7 @@ uint64_t Solver::peel_vertices_rounds(LevelGraph& g, uint32_t k, uint64_t stop_a
 // vertex's degree (its slots less those of the removed vertices that name it)
 // is then not the number of alive vertices in its row, which sizes the cut's.
 LevelGraph& Solver::cut_level(LevelGraph& p, uint32_t k_enter, uint32_t alive, bool recount) {
-  recount |= !mirrored_;
+  recount |= !paired_;
   if (levels_.size() <= depth_) levels_.emplace_back(new LevelGraph);
   LevelGraph& s = *levels_[depth_];
   // alive bitmap | word popcounts | their exclusive scan, then the ranked list
@@ -387,12 +387,14 @@ bool Solver::max_core_numbers(bool allow_cut, bool fresh, uint32_t* k) {
 
 // The largest k with a non-empty k-core (0: no edges); leaves the max-core
 // alive on the deepest level. By core numbers, or (a large graph whose degrees
-// do not set a core apart, sweeps that did not converge, or a peel forced by
-// set_vertex_mode) by a galloping search.
+// do not set a core apart, sweeps that did not converge, rows that do not
+// mirror each other -- a fall marks the vertices of its own row as due, not
+// those whose rows name it --, or a peel forced by set_vertex_mode) by a
+// galloping search.
 uint32_t Solver::max_core(bool allow_cut, bool fresh) {
   depth_ = 1;
   uint32_t top = 0;
-  if (n_ && vertex_mode_ == 0 && max_core_numbers(allow_cut, fresh, &top)) return top;
+  if (n_ && vertex_mode_ == 0 && mirrored_ && max_core_numbers(allow_cut, fresh, &top)) return top;
   depth_ = 1;
   return max_core_gallop(allow_cut, fresh);
 }
@@ -455,7 +457,7 @@ uint32_t Solver::max_core_gallop(bool allow_cut, bool fresh) {
   }
   bool grow = true, tried = false;
   while (step > 0) {
-    if (vertex_mode_ == 0 && depth_ > 1 && !tried && g->slots <= kCoreWholeSlots) {
+    if (vertex_mode_ == 0 && mirrored_ && depth_ > 1 && !tried && g->slots <= kCoreWholeSlots) {
       uint32_t top = 0;
       if (core_numbers(*g, k, &top) && top) return top;
       tried = true;
@@ -537,7 +539,7 @@ void Solver::sort_oriented_rows(uint32_t nc, uint32_t mc, uint32_t max_row) {
   KT_HIP(hipMemcpyAsync(adj_d_.p, tkeys_.p, sizeof(uint32_t) * mc, hipMemcpyDeviceToDevice, stream_));
 }
 
-void Solver::extract_core(LevelGraph& g, CoreView* cv, bool symmetric) {
+void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   core_valid_ = false;  // the core buffers are rewritten
   const uint32_t n = g.n;
   const size_t nn = size_t(n_) + 1;
@@ -570,8 +572,9 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv, bool symmetric) {
   core_assign_rank(keys2_.as<uint64_t>(), vals2_.as<uint32_t>(), nc, to_.as<uint32_t>(), inv_.as<uint32_t>(),
                    inv_orig_.as<uint32_t>(), stream_);
   // rows that repeat a neighbour or hold their own vertex do not survive as
-  // bits: their view is built from the rows themselves
-  if (symmetric && by_degree < 0x7FFFFFFFull && wants_dense(nc, uint32_t(by_degree)) &&
+  // bits, and edge ids are looked up in the mirror: else the view is built from
+  // the rows themselves
+  if (mirrored_ && by_degree < 0x7FFFFFFFull && wants_dense(nc, uint32_t(by_degree)) &&
       extract_dense(g, cv, got[1]))
     return;
   fill_u32(dout_.as<uint32_t>(), uint64_t(nc) + 1, 0, stream_);
@@ -654,11 +657,11 @@ bool Solver::extract_dense(LevelGraph& g, CoreView* cv, uint64_t slots) {
     KT_HIP(hipMemcpyAsync(pinned_, simple, sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
     KT_HIP(hipEventRecord(ev_[10], stream_));
   };
-  if (mirrored_) ask();  // rows from pairs: nothing is found out while the view is filled
+  if (paired_) ask();  // rows from pairs: nothing is found out while the view is filled
   rank_fill(bits0_.as<uint64_t>(), pref0_.as<uint32_t>(), off_u_.as<uint32_t>(), din_off_.as<uint32_t>(), nc, ws,
             adj_u_.as<uint32_t>(), eid_u_.as<uint32_t>(), adj_d_.as<uint32_t>(), src_.as<uint32_t>(),
             orig0_.as<uint32_t>(), state_.as<uint32_t>(), del_thr_.as<uint32_t>(), eidm, simple, stream_);
-  if (!mirrored_) ask();
+  if (!paired_) ask();
   KT_HIP(hipEventSynchronize(ev_[10]));
   if (!pinned_[0]) return false;
   cv->mc = cv->mc0 = mc;

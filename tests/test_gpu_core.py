@@ -63,11 +63,12 @@ def test_cores_that_unravel_along_a_path(ctx, path):
 
 
 @pytest.mark.parametrize("down", [False, True])
-@pytest.mark.parametrize("vertex", ["cascade", "rounds"])
+@pytest.mark.parametrize("vertex", ["cascade", "rounds", "auto"])
 def test_lines_in_one_direction_only(ctx, vertex, down):
     """Rows that do not mirror each other, searched by peels with a cut at 275
-    of 2,000 vertices: the same answer twice, and the
-    right one for the next graph. The peels' degrees do not size such rows."""
+    of 2,000 vertices: the same answer twice, and the right one for the next
+    graph. The peels' degrees do not size such rows, and sweeps of core numbers,
+    which mark a vertex's own row, do not find their fixpoint."""
     from kc_cuda_amd import Context
     rng = np.random.default_rng(6)
     e = np.argwhere(np.triu(rng.random((2000, 2000), dtype=np.float32) < 0.012, 1))
