@@ -189,7 +189,10 @@ void Solver::view_from_oriented_host(uint32_t nc, const uint32_t* h_off_d, const
   cv->state = state_.as<uint32_t>();
   cv->work = -1;
   build_undirected_view(cv);
-  if (wants_dense(nc, mc)) make_dense(cv);
+  if (wants_dense(nc, mc)) {
+    find_repeats(cv);
+    make_dense(cv);
+  }
 }
 
 void Solver::undirected_to_host(const CoreView& cv, uint32_t* adj_u, uint32_t* eid_u, uint32_t* lson,

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill_edges(const uint32_t* __res
   }
 }
 
-// found[0] += the sum of the supports, found[1] = 1 when a row is not strictly
+// found[0] += the sum of the supports (null: none), found[1] = 1 when a row is not strictly
 // ascending above its own vertex. The count and the fill need not agree on
 // such rows (a repeated neighbour is found once by a search, and by each of
 // its copies where they are streamed), so entries would miss their lists.
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(kBlock) void k_list_size(const uint32_t* __restrict
   bool odd = false;
   for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < mc; i += gridDim.x * blockDim.x) {
     const uint32_t u = src[i], v = adj[i];
-    c += sup[i];
+    if (sup) c += sup[i];
     odd |= v <= u || (i + 1 < mc && src[i + 1] == u && adj[i + 1] <= v);
   }
 #pragma unroll

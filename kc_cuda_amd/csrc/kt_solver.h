@@ -79,6 +79,7 @@ struct CoreView {
   // dense cores: bit-matrix rows (ws words each) of all / live edges, per-word prefix popcounts of the static rows, and (when nc^2
   // entries fit the budget) the edge id of every (u, w) pair
   bool dense = false;
+  bool repeats = false;  // a row names a neighbour twice
   uint32_t ws = 0;
   uint64_t *bits0 = nullptr, *bits = nullptr;
   uint32_t* pref0 = nullptr;
@@ -359,6 +360,7 @@ class Solver {
   size_t probe_used_ = 0;
   DevBuf probe_stats_;
   void make_dense(CoreView* cv);
+  void find_repeats(CoreView* cv);
   HeavyList heavy() {
     heavy_.ensure(sizeof(uint32_t) * 2 * (size_t(n_) + 2));
     return HeavyList{heavy_.as<uint32_t>(), &ctl_->pad[1], heavy_.as<uint32_t>() + size_t(n_) + 2};

@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
@@ -615,8 +616,19 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   // listed
   if (wants_dense(nc, mc)) {
     build_undirected_view(cv);
+    find_repeats(cv);
     make_dense(cv);
   }
+}
+
+// Whether a row names a neighbour twice (or, given by a caller, is out of
+// order): bit-matrix rows then hold one bit for several edges, and what finds
+// edges by their bits (the counts by all pairs of rows) misses some.
+void Solver::find_repeats(CoreView* cv) {
+  step_ctl_.ensure(kStepCtlBytes);
+  uint64_t* found = step_ctl_.as<uint64_t>();
+  list_size(nullptr, cv->src, cv->adj_d, cv->mc, found, stream_);
+  cv->repeats = read_u64(found + 1) != 0;
 }
 
 // Whether a core of this size gets bit-matrix rows.
@@ -762,7 +774,7 @@ void Solver::count_support(CoreView* cv, float* ms) {
   uint32_t kind = 1;
   if (cv->dense) {
     kind = 2;
-    if (dense_by_pairs(cv->nc, cv->mc, cv->ws))
+    if (!cv->repeats && dense_by_pairs(cv->nc, cv->mc, cv->ws))
       dense_count(cv->bits, cv->pref0, cv->off_u, cv->eid_u, cv->eidm, cv->nc, cv->ws, cv->sup, stream_);
     else
       dense_support(cv->off_d, cv->adj_d, cv->nc, cv->mc, cv->bits, cv->ws, nullptr, cv->sup, stream_);
@@ -958,7 +970,7 @@ TrussOutcome Solver::run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32
     rule.host = cv->dense && allow_host ? 1u : 0u;
     rule.tri_cost = dense_tri_cost_;
     rule.drop_fixed = dense_drop_fixed_;
-    rule.pair_cost = cv->dense ? dense_pair_cost(cv->nc, cv->ws) : 0.0;
+    rule.pair_cost = !cv->dense ? 0.0 : cv->repeats ? HUGE_VAL : dense_pair_cost(cv->nc, cv->ws);
     steps_start(a, h, stream_);
     uint64_t steps = 0;
     uint32_t batch = kFirstBatch;

@@ -182,3 +182,29 @@ def test_rows_that_repeat_a_neighbour_are_not_listed(by_edge):
         got = lists.solve_pairs(pairs, 80)
         assert (got.kmax, got.truss_edges, got.k_hat) == (want.kmax, want.truss_edges, want.k_hat)
         np.testing.assert_array_equal(lists.trussness(), want_t)
+
+
+def test_repeated_pairs_on_dense_cores(dense_ctx):
+    """Every copy of an edge has its support counted, at first and after
+    dropped frontiers, whatever the last solve left behind."""
+    n = 1300  # counted by all pairs of rows, were no pair repeated
+    u, v = np.triu_indices(n, 1)
+    once = np.column_stack([u, v]).astype(np.uint32)
+    twice = np.repeat(once, 2, axis=0)
+    for _ in range(2):
+        r = dense_ctx.solve_pairs(twice, n)
+        assert (r.kmax, r.truss_edges) == (n, len(twice))
+        np.testing.assert_array_equal(dense_ctx.truss_edges(), twice)
+        rng = np.random.default_rng(3)  # other supports in the same buffers
+        dense_ctx.solve_pairs(once[rng.random(len(once)) < 0.6], n)
+    # sparse edges on a repeated clique: they go first, in drops
+    tail = np.argwhere(np.triu(np.random.default_rng(4).random((3000, 3000), dtype=np.float32) < 0.05, 1)) + n // 2
+    pairs = np.concatenate([twice, tail[tail[:, 1] >= n].astype(np.uint32)])
+    got = []
+    for other in (once, tail.astype(np.uint32)):
+        dense_ctx.solve_pairs(other, n // 2 + 3000)
+        r = dense_ctx.solve_pairs(pairs, n // 2 + 3000)
+        got.append((r.kmax, r.truss_edges, dense_ctx.truss_edges()))
+    assert got[0][:2] == got[1][:2] == (n, len(twice))
+    np.testing.assert_array_equal(got[0][2], twice)
+    np.testing.assert_array_equal(got[1][2], twice)
