@@ -132,7 +132,8 @@ void core_filter(const uint32_t* deg, uint32_t n, uint32_t k, uint32_t* lvl, uin
 // (a1-a3) core subgraph extraction.
 // key = degree << 32 | ~original id (to_orig may be null: identity), val =
 // local id of every alive vertex; to = kNone for the others; found[0] (low
-// word) = how many, found[1] = the sum of their degrees
+// word) = how many, found[1] = the sum of their degrees, found[2] (low word) =
+// the highest
 void core_collect(const uint32_t* lvl, const uint32_t* deg, const uint32_t* to_orig, uint32_t n,
                   uint64_t* keys, uint32_t* vals, uint32_t* to, uint64_t* found, hipStream_t s);
 void core_assign_rank(const uint64_t* sorted_keys, const uint32_t* sorted_vals, uint32_t nc,

@@ -903,6 +903,7 @@ __global__ __launch_bounds__(kBlock) void k_core_collect(const uint32_t* __restr
                                                          uint64_t* keys, uint32_t* vals, uint32_t* to,
                                                          unsigned long long* found) {
   unsigned long long sum = 0;
+  uint32_t top = 0;
   tile_compact(
       n,
       [&](uint64_t v) {
@@ -915,11 +916,19 @@ __global__ __launch_bounds__(kBlock) void k_core_collect(const uint32_t* __restr
         keys[at] = uint64_t(d) << 32 | uint64_t(0xFFFFFFFFu - id);
         vals[at] = uint32_t(v);
         sum += d;
+        top = max(top, d);
       },
       reinterpret_cast<uint32_t*>(&found[0]));
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-  if (lane64() == 0 && sum) atomicAdd(&found[1], sum);
+  for (int o = 32; o > 0; o >>= 1) {
+    sum += __shfl_xor(sum, o);
+    top = max(top, uint32_t(__shfl_xor(top, o)));
+  }
+  if (lane64() == 0 && sum) {
+    atomicAdd(&found[1], sum);
+    uint32_t* highest = reinterpret_cast<uint32_t*>(&found[2]);
+    if (ld_agent(highest) < top) atomicMax(highest, top);
+  }
 }
 
 // sorted (key, local id) -> rank maps; inv_orig carries the input's ids
@@ -2025,7 +2034,7 @@ void core_reopen_above(uint32_t* lvl, uint32_t n, uint32_t k, hipStream_t s) {
 
 void core_collect(const uint32_t* lvl, const uint32_t* deg, const uint32_t* to_orig, uint32_t n,
                   uint64_t* keys, uint32_t* vals, uint32_t* to, uint64_t* found, hipStream_t s) {
-  fill_u64(found, 2, 0, s);
+  fill_u64(found, 3, 0, s);
   if (n)
     k_core_collect<<<grid_tiles(n), kBlock, 0, s>>>(lvl, deg, to_orig, n, keys, vals, to,
                                                     reinterpret_cast<unsigned long long*>(found));

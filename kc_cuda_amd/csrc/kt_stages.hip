@@ -553,9 +553,9 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   uint64_t* found = core_out_.as<uint64_t>();
   core_collect(g.lvl, g.deg, g.to_orig, n, keys_.as<uint64_t>(), vals_.as<uint32_t>(), to_.as<uint32_t>(), found,
                stream_);
-  KT_HIP(hipMemcpyAsync(pinned_, found, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_));
+  uint64_t got[3];
+  KT_HIP(hipMemcpyAsync(pinned_, found, sizeof(got), hipMemcpyDeviceToHost, stream_));
   KT_HIP(hipStreamSynchronize(stream_));
-  uint64_t got[2];
   std::memcpy(got, pinned_, sizeof(got));
   const uint32_t nc = uint32_t(got[0]);
   const uint64_t by_degree = got[1] / 2;  // the core's edges
@@ -565,9 +565,9 @@ void Solver::extract_core(LevelGraph& g, CoreView* cv) {
   inv_orig_.ensure(sizeof(uint32_t) * (size_t(nc) + 1));
   dout_.ensure(sizeof(uint32_t) * (size_t(nc) + 1));
   off_d_.ensure(sizeof(uint32_t) * (size_t(nc) + 1));
-  // a degree in the core is below nc
+  // bits of the highest degree (below nc unless rows repeat a neighbour)
   int deg_bits = 1;
-  while (deg_bits < 32 && (uint64_t(1) << deg_bits) < nc) ++deg_bits;
+  while (deg_bits < 32 && (got[2] >> deg_bits) != 0) ++deg_bits;
   sort_pairs_u64(keys_.as<uint64_t>(), keys2_.as<uint64_t>(), vals_.as<uint32_t>(), vals2_.as<uint32_t>(), nc,
                  32 + deg_bits);
   core_assign_rank(keys2_.as<uint64_t>(), vals2_.as<uint32_t>(), nc, to_.as<uint32_t>(), inv_.as<uint32_t>(),

@@ -183,3 +183,27 @@ def test_long_rows_clique_k8250(ctx):
     assert (tcd == 2 * (n - 2)).all()
     print(f"[gpu] K{n}: compat two-pass driver", flush=True)
     assert C.solve(n, nbr_u, nbr, deg) == (n, m)
+
+
+@pytest.mark.parametrize("copies", [2, 7, 300])
+def test_ranks_of_rows_that_repeat_neighbours(copies):
+    """Degrees of the core's vertex count and above: ranks by degree ascending,
+    id descending."""
+    from kc_cuda_amd import compat as C
+    from oracle import oracle as O
+    n = 24
+    rng = np.random.default_rng(copies)
+    once = np.argwhere(np.triu(np.ones((n, n)), 1))
+    pairs = np.concatenate([np.repeat(e[None], rng.integers(1, copies + 1), 0) for e in once])
+    both = np.concatenate([pairs, pairs[:, ::-1]])
+    both = both[np.lexsort((both[:, 0], both[:, 1]))].astype(np.uint32)
+    off, adj, _ = O.csr_from_lines(both[:, 0], both[:, 1], n)
+    kept = np.zeros(n, dtype=np.uint32)
+    nc, oto, inv, degc = O.rank(off, adj, n, kept)
+    assert degc.max() >= n
+    dwm, to = np.zeros(n, dtype=np.uint32), np.zeros(n, dtype=np.uint32)
+    li, new_n, cdeg, _ = C.count_deg_with_mask(adj, off.astype(np.uint32), n, kept, dwm, to)
+    assert new_n == nc == n
+    np.testing.assert_array_equal(li[:, 0], inv)
+    np.testing.assert_array_equal(cdeg, degc[inv])
+    np.testing.assert_array_equal(to, oto)
