@@ -169,7 +169,8 @@ __device__ __forceinline__ uint32_t row_estimate(const uint32_t (&x)[R], uint32_
 //
 // Bound: the gather of the neighbours' estimates. kLds: each workgroup copies
 // the level's estimates into LDS as 16-bit words (a level of at most 65,536
-// vertices, whose estimates are below that) and gathers there -- a wave's 64
+// vertices; larger ones, of rows that repeat a neighbour, count as 65,535, and a
+// level that ends with such a core is swept again from memory) and gathers there -- a wave's 64
 // random words cost a few LDS cycles where the vector cache takes one line a
 // cycle -- and sees its own updates at once. Rows of up to 16 * G entries are
 // taken by G lanes, rows of up to 4096 by a wave, that keep the estimates in
@@ -506,6 +507,8 @@ __global__ __launch_bounds__(kBlock) void k_core_est_apply(const uint32_t* __res
 constexpr uint32_t kCoreLdsN = 65536;
 constexpr int kCoreLdsGrid = 256;
 
+bool core_est_fits_lds(uint32_t n) { return n <= kCoreLdsN; }
+
 void core_est_init(const CoreEst& a, const uint32_t* deg, const uint32_t* lvl, int lanes, hipStream_t s) {
   fill_u32(a.counts, 2, 0, s);
   k_core_est_init<<<std::min(grid_for(a.n), 4096), kBlock, 0, s>>>(a.off, deg, lvl, a.n, a.floor,
@@ -527,7 +530,7 @@ void core_est_steps(CoreEst* a, int lanes, uint32_t count, hipStream_t s, unsign
                     hipEvent_t* ev) {
   fill_u32(a->flags, 1, 1, s);
   fill_u32(a->flags + 1, count, 0, s);
-  const bool lds = a->n <= kCoreLdsN;
+  const bool lds = a->lds;
   const void* fn = lds ? core_est_kernel<true>(lanes) : core_est_kernel<false>(lanes);
   const int block = lds ? int(kCoreLdsBlock) : kBlock;
   const int grid = std::min(grid_for(uint64_t(a->n) * uint64_t(lanes), block), lds ? kCoreLdsGrid : 4096);

@@ -94,7 +94,8 @@ void core_reopen_above(uint32_t* lvl, uint32_t n, uint32_t k, hipStream_t s);
 // written by init and read by the sweeps. floor >= 1: cores below it are not told apart (their vertices end
 // with est 0). steps queues `count` sweeps (lanes per row: 8, 16, 32 or 64;
 // stats, for measurement: the first one's row slots and vertices);
-// flags[count] == 0 afterwards: the estimates are the core numbers. max:
+// flags[count] == 0 afterwards: the estimates are the core numbers (lds: those
+// below 65,535 are, if the largest is). max:
 // *top = the largest one. apply: lvl of the alive vertices below *top = their
 // core number + 1 (floor below floor).
 struct CoreEst {
@@ -105,7 +106,9 @@ struct CoreEst {
   uint8_t *due, *due_next;
   uint32_t *medium, *heavy, *counts;
   uint32_t* flags;
+  bool lds;  // gather from LDS (core_est_fits_lds)
 };
+bool core_est_fits_lds(uint32_t n);
 void core_est_init(const CoreEst& a, const uint32_t* deg, const uint32_t* lvl, int lanes, hipStream_t s);
 void core_est_steps(CoreEst* a, int lanes, uint32_t count, hipStream_t s, unsigned long long* stats, hipEvent_t* ev);
 void core_est_max(const CoreEst& a, uint32_t* top, hipStream_t s);

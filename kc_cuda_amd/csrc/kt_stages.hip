@@ -297,6 +297,7 @@ bool Solver::core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top) {
     a.heavy = hl.items;
     a.flags = out + 1;
     a.counts = a.flags + kMaxBatch + 1;
+    a.lds = core_est_fits_lds(n);
     core_est_init(a, g.deg, g.lvl, lanes, stream_);
     for (uint32_t batch = kBatch;;) {
       core_est_steps(&a, lanes, batch, stream_, sweeps ? nullptr : ps, events(batch));
@@ -304,7 +305,12 @@ bool Solver::core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top) {
       KT_HIP(hipMemcpyAsync(pinned_, out, sizeof(uint32_t) * (batch + 2), hipMemcpyDeviceToHost, stream_));
       KT_HIP(hipStreamSynchronize(stream_));
       sweeps += batch;
-      if (pinned_[1 + batch] == 0) break;
+      if (pinned_[1 + batch] == 0) {
+        if (!a.lds || pinned_[0] < 65535) break;
+        a.lds = false;  // a core past 16 bits, of repeated pairs
+        core_est_init(a, g.deg, g.lvl, lanes, stream_);
+        continue;
+      }
       if (sweeps >= kCoreSweeps) return false;
       batch = std::min(batch * 2, kMaxBatch);
     }

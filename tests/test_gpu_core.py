@@ -84,3 +84,10 @@ def test_lines_in_one_direction_only(ctx, vertex, down):
         assert (one.max_core, one.k_hat, one.kmax, one.truss_edges) == (two.max_core, two.k_hat, two.kmax, two.truss_edges)
         r = c.solve_pairs(pairs, 2000)
         assert (r.max_core, r.kmax, r.truss_edges) == (ref.max_core, ref.kmax, ref.truss_edges)
+
+
+@pytest.mark.parametrize("copies", [4000, 65534, 65535, 65536, 70000])
+def test_cores_of_repeated_pairs_beyond_16_bits(ctx, copies):
+    """Two vertices joined many times: a core as large as the count of copies."""
+    r = ctx.solve_pairs(np.tile(np.array([[3, 9]], np.uint32), (copies, 1)), 12)
+    assert (r.max_core, r.kmax, r.truss_edges) == (copies, 0, 0)
