@@ -36,10 +36,21 @@ struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
   bool carved = false;  // p lies in an arena
+  bool busy = false;    // what it holds is needed
+  DevBuf* spare = nullptr;  // freed, unless busy, when this one cannot be allocated
   void ensure(size_t b);
   void release();
   template <typename T>
   T* as() const { return static_cast<T*>(p); }
+};
+
+// A buffer that must not be freed for another's sake meanwhile.
+struct BusyScope {
+  explicit BusyScope(DevBuf& buf) : b(buf) { b.busy = true; }
+  ~BusyScope() { b.busy = false; }
+  BusyScope(const BusyScope&) = delete;
+  BusyScope& operator=(const BusyScope&) = delete;
+  DevBuf& b;
 };
 
 // One graph of the vertex-peel nest. Level 0 is the input CSR; each deeper
@@ -340,7 +351,9 @@ class Solver {
   std::vector<uint64_t> deg_at_least_;  // input degree histogram, suffix sums per bin (empty: none)
   DevBuf bk_state_, bk_sup_, bk_bits_, bk_del_;  // threshold-probe backups
   uint64_t eidm_budget_ = uint64_t(4) << 30;  // bytes for the edge-id matrix
-  // triangle lists: in all, and a core edge (a context of its own is not bound there)
+  // triangle lists: in all, and a core edge (a context of its own is not bound there).
+  // The room they took, kept for the next core, is the first to go when another
+  // buffer finds none (DevBuf::spare).
   uint64_t tri_budget_ = uint64_t(16) << 30, tri_per_edge_ = ~uint64_t(0) >> 32;
   double dense_tri_cost_ = 14.0, sparse_drop_ratio_ = 3.0, default_drop_ratio_ = 3.0;
   double dense_drop_fixed_ = 8e6;  // about what the two steps of a recount take

@@ -46,7 +46,17 @@ void DevBuf::ensure(size_t b) {
   release();
   size_t want = std::max<size_t>(b, 256);
   want = (want + 4095) & ~size_t(4095);
-  KT_HIP(hipMalloc(&p, want));
+  hipError_t e = hipMalloc(&p, want);
+  if (e == hipErrorOutOfMemory && spare && spare != this && !spare->busy && spare->p) {
+    (void)hipGetLastError();
+    spare->release();
+    e = hipMalloc(&p, want);
+  }
+  if (e != hipSuccess) {
+    p = nullptr;
+    (void)hipGetLastError();  // the caller may go on without
+    throw Error{e, "hipMalloc of " + std::to_string(want) + " bytes -> " + hipGetErrorString(e)};
+  }
   bytes = want;
 }
 
@@ -113,6 +123,7 @@ void Solver::clear_control() { fill_u32(reinterpret_cast<uint32_t*>(ctl_), sizeo
 
 void Solver::init_common() {
   static_assert(sizeof(host_rb_) >= 256, "readback buffer smaller than the pinned one");
+  each_buffer([&](const DevBuf& b) { const_cast<DevBuf&>(b).spare = &tri_; });
   for (auto& e : ev_) KT_HIP(hipEventCreate(&e));
   for (auto& e : stage_ev_) KT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   KT_HIP(hipStreamSynchronize(stream_));

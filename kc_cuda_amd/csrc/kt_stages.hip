@@ -21,6 +21,7 @@
 #include <climits>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "kt_batch_union.h"
@@ -130,7 +131,11 @@ uint64_t Solver::peel_vertices_rounds(LevelGraph& g, uint32_t k, uint64_t stop_a
 // is then not the number of alive vertices in its row, which sizes the cut's.
 LevelGraph& Solver::cut_level(LevelGraph& p, uint32_t k_enter, uint32_t alive, bool recount) {
   recount |= !paired_;
-  if (levels_.size() <= depth_) levels_.emplace_back(new LevelGraph);
+  if (levels_.size() <= depth_) {
+    levels_.emplace_back(new LevelGraph);
+    LevelGraph& l = *levels_[depth_];
+    for (DevBuf* b : {&l.b_off, &l.b_adj, &l.b_deg, &l.b_lvl, &l.b_orig}) b->spare = &tri_;
+  }
   LevelGraph& s = *levels_[depth_];
   // alive bitmap | word popcounts | their exclusive scan, then the ranked list
   const size_t words = (size_t(p.n) + 31) / 32;
@@ -900,7 +905,11 @@ TrussOutcome Solver::truss_search(CoreView* cv, int32_t thr0, uint64_t early_ans
   search.early_k = early_k;
   search.exact_early = exact_early ? 1u : 0u;
   uint32_t r = 1;
-  if (cv->dense || list_triangles(*cv)) return run_steps(cv, thr0, cv->mc, &r, search, true);
+  if (cv->dense) return run_steps(cv, thr0, cv->mc, &r, search, true);
+  {
+    BusyScope lists(tri_);
+    if (list_triangles(*cv)) return run_steps(cv, thr0, cv->mc, &r, search, true);
+  }
   if (!cv->off_u) build_undirected_view(cv);
   return run_levels(cv, thr0, search);
 }
@@ -908,7 +917,7 @@ TrussOutcome Solver::truss_search(CoreView* cv, int32_t thr0, uint64_t early_ans
 // Triangle lists of a base view whose supports are counted: offsets in
 // tri_off_, the pairs of partner edges in tri_. False when they do not fit
 // the budget (tri_budget_ bytes, tri_per_edge_ a core edge, and of more than
-// 1 GiB half of the device memory that is free), or when rows repeat a
+// 1 GiB half of the device memory that is free) or cannot be allocated, or when rows repeat a
 // neighbour (or, given by a caller, are not in order): the lists are laid out
 // by the counted supports, which the fill then need not find again.
 bool Solver::list_triangles(const CoreView& cv) {
@@ -923,15 +932,28 @@ bool Solver::list_triangles(const CoreView& cv) {
   std::memcpy(got, pinned_, sizeof(got));
   const uint64_t entries = got[0], bytes = entries * sizeof(uint2);
   if (got[1] || entries >= (uint64_t(1) << 31) || bytes > tri_budget_ || bytes > tri_per_edge_ * mc) return false;
-  if (bytes > tri_.bytes && bytes > (uint64_t(1) << 30)) {
-    size_t free_bytes = 0, total_bytes = 0;
-    KT_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
-    if (bytes > (free_bytes + tri_.bytes) / 2) return false;
+  const size_t per_edge = sizeof(uint32_t) * (size_t(mc) + 1);
+  if (arena_) {
+    for (DevBuf* b : {&tri_off_, &live_[0], &live_[1]}) b->ensure(per_edge);
+    tri_.ensure(std::max<uint64_t>(bytes, 1));
+  } else if (bytes > tri_.bytes || per_edge > live_[1].bytes) {
+    // one solver at a time sees what is free and takes its part of it
+    static std::mutex taking;
+    std::lock_guard<std::mutex> lk(taking);
+    if (bytes > tri_.bytes && bytes > (uint64_t(1) << 30)) {
+      size_t free_bytes = 0, total_bytes = 0;
+      KT_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
+      if (bytes > (free_bytes + tri_.bytes) / 2) return false;
+    }
+    try {
+      for (DevBuf* b : {&tri_off_, &live_[0], &live_[1]}) b->ensure(per_edge);
+      tri_.ensure(std::max<uint64_t>(bytes, 1));
+    } catch (const Error& e) {
+      if (e.code != hipErrorOutOfMemory) throw;
+      for (DevBuf* b : {&tri_, &tri_off_, &live_[0], &live_[1]}) b->release();
+      return false;
+    }
   }
-  tri_off_.ensure(sizeof(uint32_t) * (size_t(mc) + 1));
-  live_[0].ensure(sizeof(uint32_t) * (size_t(mc) + 1));
-  live_[1].ensure(sizeof(uint32_t) * (size_t(mc) + 1));
-  tri_.ensure(std::max<uint64_t>(bytes, 1));
   uint32_t* off = tri_off_.as<uint32_t>();
   uint32_t* cursor = live_[0].as<uint32_t>();  // free until the search lists live edges
   fill_u32(reinterpret_cast<uint32_t*>(cv.sup) + mc, 1, 0, stream_);
