@@ -16,9 +16,9 @@ double ms_between(std::chrono::steady_clock::time_point a, std::chrono::steady_c
 // Per input edge: the pairs' device copy, the CSR and its build and sort
 // buffers, the vertex-peel nest's subgraphs, and for every core edge its
 // oriented and undirected slots with edge ids, support, state, deletion
-// level, queues, backups and both compaction sets (160 B in all; measured at
-// most 96 B on serving and batch mixes and RMAT scale 22, shuffled pairs from
-// 2^22 on take 16 B more while they are split); per vertex
+// level, queues, triangle lists, backups and both compaction sets (160 B in all;
+// measured at most 96 B on serving and batch mixes and RMAT scale 22, pairs in
+// no order 8 B more, and 24 from 2^22 on if the core has no lists); per vertex
 // offsets, degrees, levels and maps (64 B); a dense core's bit rows (at most
 // 72 B per edge, since a row is no longer than two sorted rows) and its
 // edge-id matrix (at most kServeEidmBytes); 16 MiB of fixed buffers.

@@ -23,8 +23,12 @@ namespace kt {
 
 // Edge-id matrix cap of a serving slot's dense cores (bytes).
 constexpr uint64_t kServeEidmBytes = uint64_t(256) << 20;
-// Triangle lists of a sorted-row core, per core edge: a slot then holds at
-// most 120 B an edge where the footprint counts 160.
+// Triangle lists of a sorted-row core, per core edge. A slot then holds at most
+// 120 B an edge for pairs sorted by their first id -- staged pairs 8, rows 8,
+// the build's entries 8, oriented core, state and queues 36, lists 48, their
+// offsets and live edges 12 -- and 128 for shuffled ones (entries 16; what their
+// build stages besides, 16, lies where the lists go), before the cut levels'
+// rows, where the footprint counts 160.
 constexpr uint64_t kServeListBytes = 48;
 // Bytes an idle slot may keep after freeing its buffers (control block).
 constexpr uint64_t kServeSlotFloor = uint64_t(1) << 20;

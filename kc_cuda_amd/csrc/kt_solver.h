@@ -352,8 +352,9 @@ class Solver {
   DevBuf bk_state_, bk_sup_, bk_bits_, bk_del_;  // threshold-probe backups
   uint64_t eidm_budget_ = uint64_t(4) << 30;  // bytes for the edge-id matrix
   // triangle lists: in all, and a core edge (a context of its own is not bound there).
-  // The room they took, kept for the next core, is the first to go when another
-  // buffer finds none (DevBuf::spare).
+  // The room they took, kept for the next core (and the build of shuffled pairs,
+  // which stages 16 B an edge there), is the first to go when another buffer
+  // finds none (DevBuf::spare).
   uint64_t tri_budget_ = uint64_t(16) << 30, tri_per_edge_ = ~uint64_t(0) >> 32;
   double dense_tri_cost_ = 14.0, sparse_drop_ratio_ = 3.0, default_drop_ratio_ = 3.0;
   double dense_drop_fixed_ = 8e6;  // about what the two steps of a recount take
@@ -384,7 +385,7 @@ class Solver {
   bool mirrored_ = false;  // so it has, as far as a sum of hashes tells (no access relies on it)
   uint64_t m_ = 0, slots_ = 0;  // edges and row slots of the input
   // full graph
-  DevBuf off_, adj_, deg_, lvl_, q0_, q1_, deg_bak_, cursor_, hist_, hoff_, part_, part2_, split_;
+  DevBuf off_, adj_, deg_, lvl_, q0_, q1_, deg_bak_, cursor_, hist_, hoff_, part_, split_;
   std::vector<std::unique_ptr<LevelGraph>> levels_;
   size_t depth_ = 0;  // levels in use
   // scratch for level cuts and extraction

@@ -150,7 +150,7 @@ void Solver::each_buffer(F f) const {
                          &keys_, &keys2_, &vals_, &vals2_, &to_, &inv_, &inv_orig_, &dout_, &off_d_,
                          &adj_d_, &src_, &din_, &din_off_, &tkeys_, &tvals_, &tiota_, &in_src_, &off_u_,
                          &adj_u_, &eid_u_, &sup_, &state_, &eq0_, &eq1_, &eq2_, &out_pairs_, &truss_out_, &del_thr_, &orig0_,
-                         &temp_, &hist_, &hoff_, &part_, &part2_, &split_, &bits0_, &bits_, &pref0_, &eidm_, &heavy_,
+                         &temp_, &hist_, &hoff_, &part_, &split_, &bits0_, &bits_, &pref0_, &eidm_, &heavy_,
                          &vflag_, &vmap_, &roff_, &dhist_, &vq_, &core_out_, &step_ctl_, &tri_off_, &tri_, &live_[0], &live_[1], &bk_state_, &bk_sup_, &bk_bits_, &bk_del_, &text_,
                          &tile_cnt_, &tile_off_, &lx_, &ly_, &lkind_, &lx2_, &ly2_, &lkeep_, &lkeep_off_,
                          &lstat_, &probe_stats_};
@@ -319,15 +319,17 @@ bool Solver::build_partitioned(int mode, const uint32_t* a, const uint32_t* b, u
 
 // Pairs of valid ids: their entries go to their groups of rows in two splits
 // (kt_build.hip). The first one's output has room in adj if the pairs are
-// sorted (only half of the entries are split).
+// sorted (only half of the entries are split), else where a later core's
+// triangle lists go.
 void Solver::build_split(const SplitPlan& p, const uint32_t* pairs, uint64_t items, uint32_t n) {
   const uint32_t lows = 1u << p.low_bits, highs = 1u << p.high_bits;
   const uint64_t bt = std::max(uint64_t(lows) * p.tiles1, uint64_t(highs) * p.tiles2);
   hist_.ensure(sizeof(uint32_t) * (2 * bt + 1));
   hoff_.ensure(sizeof(uint64_t) * (2 * bt + 1));
   part_.ensure(sizeof(uint32_t) * 2 * p.entries);
-  if (!p.sorted) part2_.ensure(sizeof(uint32_t) * 2 * p.entries);
-  uint32_t* once = p.sorted ? adj() : part2_.as<uint32_t>();
+  BusyScope staged(tri_);
+  if (!p.sorted) tri_.ensure(sizeof(uint32_t) * 2 * p.entries);
+  uint32_t* once = p.sorted ? adj() : tri_.as<uint32_t>();
   split_.ensure((sizeof(uint64_t) + sizeof(uint32_t)) * (size_t(lows) + 1));
   uint64_t* start = split_.as<uint64_t>();
   uint32_t* tiles = reinterpret_cast<uint32_t*>(start + lows + 1);

@@ -132,3 +132,22 @@ def test_serve_device_resident_inputs(ctx):
     for i, (r, (k, e)) in enumerate(zip(res, ref)):
         assert r.status == 0, r.error
         assert (r.kmax, r.truss_edges) == (k, e), f"query {i}"
+
+
+def test_shuffled_pairs_hold_no_second_staging_buffer():
+    """From 2^22 pairs on: the build of shuffled pairs stages where the core's
+    triangle lists go, so a slot holds 8 B an edge more than for sorted ones."""
+    from kc_cuda_amd import Server
+    n = 1_100_000  # every vertex joined to the next four on a ring
+    i = np.arange(n)
+    pairs = np.concatenate([np.column_stack([i, (i + d) % n]) for d in range(1, 5)]).astype(np.uint32)
+    pairs = canon_pairs(pairs)
+    assert len(pairs) >= 1 << 22
+    held = []
+    for p in (pairs, pairs[np.random.default_rng(2).permutation(len(pairs))]):
+        with Server(0, 1, 32 << 30) as srv:
+            r = srv.wait(srv.submit(np.ascontiguousarray(p), n))
+        assert (r.status, r.kmax, r.truss_edges) == (0, 5, len(pairs))
+        assert r.slot_bytes <= r.charged
+        held.append(r.slot_bytes)
+    assert held[1] - held[0] <= 9 * len(pairs)
