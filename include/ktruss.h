@@ -177,16 +177,18 @@ int kt_batch_solve(kt_context* ctx, const uint32_t* d_pairs, const uint64_t* h_o
  * kt_batch_solve on every sample_every-th graph of the batch (1: all) under
  * candidate settings, one at a time: sparse-peel lanes, support-count lanes,
  * support-count kernel, drop ratio (a candidate is kept when it is 3%
- * faster than the best so far). Every trial must give every graph the same
+ * faster than the best so far; peel lanes and drop ratio only if a part's
+ * triangles did not fit the list budget, since only the peel by rows reads
+ * them). Every trial must give every graph the same
  * answer (else an error is returned). The fastest settings stay on the
  * context for later solves (kt_set_tuning resets them) and the whole batch is
  * then solved into d_kmax / d_count / d_status as kt_batch_solve does. */
 typedef struct kt_batch_tuning {
   int32_t count_lanes;  /* support count: sub-wavefront lanes per row (0 automatic) */
-  int32_t peel_lanes;   /* sparse peel rounds: the same */
+  int32_t peel_lanes;   /* sparse peel rounds (cores without triangle lists): the same */
   int32_t edge_count;   /* 1: per-edge support kernel (as KT_FORCE_EDGE_COUNT) */
   uint32_t trials;      /* batch solves timed */
-  double drop_ratio;    /* sparse peel: recount when frontier * ratio >= live edges */
+  double drop_ratio;    /* the same rounds: recount when frontier * ratio >= live edges */
   double ms_default;    /* sampled batch time with the context's settings on entry */
   double ms_best;       /* with the chosen settings */
 } kt_batch_tuning;

@@ -385,9 +385,10 @@ class Context:
     def batch_autotune(self, dpairs: DeviceArray, offsets: np.ndarray, ns: np.ndarray,
                        sample_every: int = 1) -> tuple["BatchResult", dict]:
         """Times the batched solve of every sample_every-th graph under
-        candidate settings (peel lanes, count lanes, count kernel, drop
-        ratio), keeps the fastest on this context and returns the whole
-        batch's results with the chosen settings and timings."""
+        candidate settings (count lanes, count kernel; peel lanes and drop
+        ratio where triangles were not listed), keeps the fastest on this
+        context and returns the whole batch's results with the chosen
+        settings and timings."""
         out = _BatchBuffers(self, offsets, ns, False)
         t = KtBatchTuning()
         try:

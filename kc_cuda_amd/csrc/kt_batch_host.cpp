@@ -128,9 +128,13 @@ BatchTuning BatchRunner::autotune(const uint32_t* d_pairs, const uint64_t* h_off
     trial(best);  // buffers grow to the batch
     double best_ms = trial(best);
     out.ms_default = best_ms;
-    auto consider = [&](const Solver::Tuning& cand) {
+    // peel lanes and the drop ratio are read where a core is peeled by its rows
+    // alone: with every part's triangles listed, a faster trial is noise
+    bool rows = false;
+    for (size_t p = 0; p < parts_.size(); ++p) rows |= (parts_[p].own ? parts_[p].own.get() : solver_)->peeled_by_rows();
+    auto consider = [&](const Solver::Tuning& cand, bool read = true) {
       const double ms = trial(cand);
-      if (ms < 0.97 * best_ms) best_ms = ms, best = cand;
+      if (read && ms < 0.97 * best_ms) best_ms = ms, best = cand;
     };
     const int widths[] = {8, 16, 32, 64};
     const Solver::Tuning base1 = best;
@@ -138,7 +142,7 @@ BatchTuning BatchRunner::autotune(const uint32_t* d_pairs, const uint64_t* h_off
       if (l != base1.peel_lanes) {
         Solver::Tuning c = base1;
         c.peel_lanes = l;
-        consider(c);
+        consider(c, rows);
       }
     const Solver::Tuning base2 = best;
     for (int l : widths)
@@ -154,7 +158,7 @@ BatchTuning BatchRunner::autotune(const uint32_t* d_pairs, const uint64_t* h_off
     for (double f : {0.5, 2.0, 4.0}) {
       Solver::Tuning c = base4;
       c.drop_ratio = base4.drop_ratio * f;
-      consider(c);
+      consider(c, rows);
     }
     solver_->set_tuning(best);
     out.best = best;

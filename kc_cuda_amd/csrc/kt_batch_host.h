@@ -31,7 +31,7 @@ class BatchRunner {
   // Autotuner: times the batched solve of every `every`-th graph under
   // candidate solver settings, one setting at a time (peel lanes, count
   // lanes, count kernel, drop ratio; a candidate is kept when it is 3%
-  // faster), checks that every trial gives every graph the same answer,
+  // faster and the union's cores are peeled by what it sets), checks that every trial gives every graph the same answer,
   // leaves the fastest settings on the solver and solves the whole batch
   // into the outputs.
   BatchTuning autotune(const uint32_t* d_pairs, const uint64_t* h_off, const uint32_t* h_ns, uint32_t count,

@@ -194,6 +194,9 @@ class Solver {
     bool edge_count = false;              // per-edge support kernel
     double drop_ratio = 3.0;              // sparse peel: recount when frontier * ratio >= live edges
   };
+  // the last truss search walked rows (and so read peel_lanes and drop_ratio),
+  // not triangle lists or bit-matrix rows
+  bool peeled_by_rows() const { return peeled_by_rows_; }
   Tuning tuning() const { return Tuning{lanes_count_, lanes_peel_, force_edge_count_, sparse_drop_ratio_}; }
   void set_tuning(const Tuning& t) {
     lanes_count_ = t.count_lanes;
@@ -363,6 +366,7 @@ class Solver {
   double trace_ms();
   std::chrono::steady_clock::time_point trace_t0_{};
   bool gallop_ = true;
+  bool peeled_by_rows_ = false;
   uint32_t count_kind_ = 0, count_words_ = 0;  // the last timed support count
   uint32_t walk_levels_ = 16;
   uint64_t split_build_min_ = uint64_t(1) << 22;  // fewest pairs of the build by two splits (see split_plan)

@@ -905,12 +905,14 @@ TrussOutcome Solver::truss_search(CoreView* cv, int32_t thr0, uint64_t early_ans
   search.early_k = early_k;
   search.exact_early = exact_early ? 1u : 0u;
   uint32_t r = 1;
+  peeled_by_rows_ = false;
   if (cv->dense) return run_steps(cv, thr0, cv->mc, &r, search, true);
   {
     BusyScope lists(tri_);
     if (list_triangles(*cv)) return run_steps(cv, thr0, cv->mc, &r, search, true);
   }
   if (!cv->off_u) build_undirected_view(cv);
+  peeled_by_rows_ = true;
   return run_levels(cv, thr0, search);
 }
 

@@ -215,3 +215,26 @@ def test_batch_parts_agree(parts):
             np.testing.assert_array_equal(canon_pairs(kept), canon_pairs(ref.truss), err_msg=f"graph {g}")
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("lists", [True, False])
+def test_autotuner_keeps_what_its_route_reads(lists):
+    """Peel lanes and the drop ratio steer the peel by rows alone: with
+    triangle lists a trial's time says nothing about them."""
+    from kc_cuda_amd import Context, gen
+    pairs, offs, ns = gen.batch(12, 32, 600, 6.0, 20.0, 4, 12, 9)
+    mp = pytest.MonkeyPatch()
+    if not lists:
+        mp.setenv("KT_LIST_BUDGET_MB", "0")
+    with Context(0) as c:
+        c.tune(core="sparse")
+        d = c.to_device(np.ascontiguousarray(pairs))
+        ref = c.batch_solve(d, offs, ns)
+        for _ in range(4):
+            c.tune(core="sparse")
+            r, t = c.batch_autotune(d, offs, ns, sample_every=1)
+            np.testing.assert_array_equal(r.edges, ref.edges)
+            if lists:
+                assert (t["peel_lanes"], t["drop_ratio"]) == (0, 3.0)
+        d.free()
+    mp.undo()
