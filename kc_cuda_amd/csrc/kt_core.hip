@@ -22,7 +22,6 @@ constexpr uint32_t kCoreLdsBlock = 1024;  // workgroup of the kernels that keep 
 // Levels of one workgroup (34 KB of LDS); 8,192 row slots are 4 k edges.
 constexpr uint32_t kCoreSmallN = 4096;
 constexpr uint32_t kCoreSmallSlots = 1u << 13;
-constexpr uint32_t kCoreSmallSweeps = 512;
 constexpr uint32_t kLightRegs = 16;   // row entries a lane keeps: a light row has at most 16 * G
 constexpr uint32_t kMediumRegs = 64;  // a medium row, taken by one wave, at most 4096
 constexpr uint32_t kHeavyRegs = 16;   // and a heavy row, taken by a workgroup of NT threads, 16 * NT
@@ -341,14 +340,14 @@ __global__ __launch_bounds__(kLds ? kCoreLdsBlock : kBlock) void k_core_est_step
 // sweeps over every vertex until one changes nothing, then the results (lvl
 // as k_core_est_apply writes it, deg of the max core's vertices = their degree
 // in it). out[0] = the largest core number, out[1] = 1 when the sweeps
-// converged within `cap` (else nothing but out is written). A sweep from LDS
-// takes less than launching one.
+// converged within `cap`; else est and due (every vertex of an estimate) are
+// written for k_core_finish. A sweep from LDS takes less than launching one.
 template <int G>
 __global__ __launch_bounds__(kCoreLdsBlock) void k_core_small(const uint64_t* __restrict__ off,
                                                               const uint32_t* __restrict__ adj, uint32_t n,
                                                               uint32_t floor, uint32_t cap, uint32_t* lvl,
-                                                              uint32_t* deg, uint32_t* out,
-                                                              unsigned long long* stats) {
+                                                              uint32_t* deg, uint32_t* est, uint8_t* due,
+                                                              uint32_t* out, unsigned long long* stats) {
   __shared__ uint16_t s_adj[kCoreSmallSlots];
   __shared__ uint16_t s_off[kCoreSmallN + 1];  // at most kCoreSmallSlots
   __shared__ uint16_t s_e[kCoreSmallN];
@@ -403,6 +402,10 @@ __global__ __launch_bounds__(kCoreLdsBlock) void k_core_small(const uint64_t* __
     __syncthreads();
     if (!s_changed) break;
     if (sweep >= cap) {
+      for (uint32_t v = tid; v < n; v += kCoreLdsBlock) {
+        est[v] = s_e[v];
+        due[v] = s_e[v] != 0;
+      }
       if (tid == 0) out[0] = out[1] = 0;
       return;
     }
@@ -430,6 +433,247 @@ __global__ __launch_bounds__(kCoreLdsBlock) void k_core_small(const uint64_t* __
     out[0] = top;
     out[1] = 1;
   }
+}
+
+// What is left of a level of at most 65,536 vertices whose sweeps make slow
+// progress (a core that unravels along paths: each sweep moves the ends by one
+// vertex), by one workgroup, estimates and due marks in LDS: a sweep takes a
+// list of due vertices, so it costs what they cost and two barriers, not a
+// launch; where they are few, one wave runs sweeps on end with no barrier.
+//
+// From sweep `all` on only vertices of the largest estimate T are taken. Once
+// none of them is due, each has T neighbours among them: they are the max core
+// (no core is larger than the estimates), and the other estimates are left as
+// the upper bounds they are.
+//
+// out[0] = the largest estimate; out[1] = 1: every estimate is a core number,
+// 2: the largest is, 0: not done after `cap` sweeps.
+// Bound on a sweep's chain of dependent accesses (row bounds, entries, some ten
+// to LDS): 3 us where one vertex is due, as a path's 10 k vertices take 15 ms.
+constexpr uint32_t kOneQueue = 4096;  // listed vertices of one sweep (the others wait for a later one)
+template <int G>
+__global__ __launch_bounds__(kCoreLdsBlock) void k_core_finish(const uint64_t* __restrict__ off,
+                                                               const uint32_t* __restrict__ adj, uint32_t n,
+                                                               uint32_t floor, uint32_t all, uint32_t cap,
+                                                               uint32_t* est, const uint8_t* __restrict__ due,
+                                                               uint32_t* out) {
+  extern __shared__ __align__(16) uint32_t s_due[];  // marks: listed, or waiting
+  __shared__ uint16_t s_q[2][kOneQueue];
+  __shared__ uint32_t s_n[2];  // listed (past kOneQueue: waiting)
+  __shared__ uint32_t s_top, s_cnt, s_sweep;
+  constexpr uint32_t kSolo = 4 * (kWave / G);  // due vertices that one wave takes alone
+  const uint32_t words = (n + 31) / 32;
+  uint16_t* s_e = reinterpret_cast<uint16_t*>(s_due + words);
+  const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+  const uint32_t glane = tid % G, shift = lane / G * G;
+  const unsigned long long gmask = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << shift;
+  if (tid == 0) s_n[0] = 0;
+  __syncthreads();
+  for (uint32_t v0 = wid * kWave; v0 < n; v0 += kCoreLdsBlock) {  // at most kOneQueue are due
+    const uint32_t v = v0 + lane;
+    if (v < n) s_e[v] = uint16_t(min(est[v], 65535u));
+    const unsigned long long mask = __ballot(v < n && due[v] != 0);
+    uint32_t at = 0;
+    if (lane == 0 && mask) at = atomicAdd(&s_n[0], uint32_t(__popcll(mask)));
+    at = __shfl(at, 0) + uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
+    if (((mask >> lane) & 1ull) && at < kOneQueue) s_q[0][at] = uint16_t(v);
+    if (lane % 32 == 0 && v < n) s_due[v >> 5] = uint32_t(mask >> lane);
+  }
+  __syncthreads();
+
+  // the largest estimate and (counted) how many vertices have it
+  auto find_top = [&](bool counted) {
+    if (tid == 0) s_top = s_cnt = 0;
+    __syncthreads();
+    uint32_t m = 0;
+    for (uint32_t v = tid; v < n; v += kCoreLdsBlock) m = max(m, uint32_t(s_e[v]));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = max(m, uint32_t(__shfl_xor(m, o)));
+    if (lane == 0) atomicMax(&s_top, m);
+    __syncthreads();
+    m = s_top;
+    if (!counted) return m;
+    uint32_t c = 0;
+    for (uint32_t v = tid; v < n; v += kCoreLdsBlock) c += s_e[v] == m;
+    c = wave_sum(c);
+    if (lane == 0 && c) atomicAdd(&s_cnt, c);
+    __syncthreads();
+    return m;
+  };
+  // list `cur` from the marks, of vertices of estimate `only` (0: any); true
+  // when there are marks besides
+  constexpr uint32_t kWords = 2;  // due words a thread owns
+  auto list_due = [&](uint32_t cur, uint32_t only) {
+    uint32_t take[kWords], mine = 0;
+    bool other = false;
+#pragma unroll
+    for (uint32_t h = 0; h < kWords; ++h) {
+      const uint32_t w = h * kCoreLdsBlock + tid;
+      uint32_t x = w < words ? s_due[w] : 0u;
+      if (only)
+        for (uint32_t y = x; y; y &= y - 1)
+          if (s_e[w * 32 + __ffs(int(y)) - 1] != only) {
+            x &= ~(y & (0u - y));
+            other = true;
+          }
+      take[h] = x;
+      mine += uint32_t(__popc(x));
+    }
+    uint32_t total;
+    uint32_t at = block_exclusive_scan<kCoreLdsBlock>(mine, &total);
+#pragma unroll
+    for (uint32_t h = 0; h < kWords; ++h)
+      for (uint32_t y = take[h]; y && at < kOneQueue; y &= y - 1, ++at)
+        s_q[cur][at] = uint16_t((h * kCoreLdsBlock + tid) * 32 + __ffs(int(y)) - 1);
+    if (tid == 0) s_n[cur] = total;
+    return __syncthreads_or(other) != 0 || total > kOneQueue;
+  };
+
+  uint32_t top = 0;  // not 0: only vertices of this estimate
+  // a list's marks go before its sweep reads
+  auto unmark = [&](uint32_t cur, uint32_t count, uint32_t first, uint32_t step) {
+    for (uint32_t i = first; i < count; i += step) {
+      const uint32_t v = s_q[cur][i];
+      atomicAnd(&s_due[v >> 5], ~(1u << (v & 31)));
+    }
+  };
+  // a wave's entries of the list, first on and every step; a fall marks and
+  // lists vertices for the next sweep
+  auto sweep_list = [&](uint32_t cur, uint32_t count, uint32_t first, uint32_t step) {
+    auto mark = [&](uint32_t w, bool listed) {
+      const uint32_t bit = 1u << (w & 31);
+      if (!(atomicOr(&s_due[w >> 5], bit) & bit) && listed) {
+        const uint32_t at = atomicAdd(&s_n[cur ^ 1u], 1u);
+        if (at < kOneQueue) s_q[cur ^ 1u][at] = uint16_t(w);
+      }
+    };
+    for (uint32_t i0 = first; i0 < count; i0 += step) {  // wave-uniform
+      const uint32_t i = i0 + lane / G;
+      const uint32_t v = i < count ? s_q[cur][i] : 0u, e = i < count ? s_e[v] : 0u;
+      uint64_t b = 0;
+      uint32_t len = 0;
+      if (e) {
+        b = off[v];
+        len = uint32_t(off[v + 1] - b);
+      }
+      auto settle = [&](uint32_t h) {
+        s_e[v] = uint16_t(h);
+        if (h) mark(v, !top);
+        if (top && e == top) atomicSub(&s_cnt, 1u);
+      };
+      auto supported = [&](uint32_t w, uint32_t x, uint32_t h) {
+        if (x > h && x <= e) mark(w, !top || x == top);
+      };
+      if (!__ballot(len > G)) {  // a lane an entry
+        const uint32_t w = glane < len ? adj[b + glane] : kNone;
+        const uint32_t x[1] = {w != kNone ? s_e[w] : 0u};
+        uint32_t h = row_estimate(x, e, 1, gmask);
+        if (h < e) {
+          if (h < floor) h = 0;
+          if (glane == 0) settle(h);
+          if (w != kNone) supported(w, x[0], h);
+        }
+      } else if (!__ballot(len > kLightRegs * G)) {
+        uint32_t w[kLightRegs], x[kLightRegs];
+#pragma unroll
+        for (uint32_t r = 0; r < kLightRegs; ++r) {
+          const uint32_t j = r * G + glane;
+          w[r] = j < len ? adj[b + j] : kNone;
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < kLightRegs; ++r) x[r] = w[r] != kNone ? s_e[w[r]] : 0u;
+        uint32_t h = row_estimate(x, e, kLightRegs, gmask);
+        if (h < e) {
+          if (h < floor) h = 0;
+          if (glane == 0) settle(h);
+#pragma unroll
+          for (uint32_t r = 0; r < kLightRegs; ++r)
+            if (w[r] != kNone) supported(w[r], x[r], h);
+        }
+      } else {  // a long row in the wave: read anew for every count
+        auto count_row = [&](uint32_t t) {  // entries of the row of at least t >= 1, per group
+          uint32_t c = 0;
+          for (uint32_t j = glane; __ballot(j < len); j += G)
+            c += uint32_t(__popcll(__ballot(j < len && s_e[adj[b + j]] >= t) & gmask));
+          return c;
+        };
+        const uint32_t ce = count_row(max(e, 1u));
+        uint32_t lo = ce >= e ? e : ce, hi = ce >= e ? e + 1 : e;  // as row_estimate
+        while (__ballot(hi - lo > 1)) {
+          const uint32_t mid = lo + (hi - lo) / 2;
+          const bool ok = count_row(max(mid, 1u)) >= mid;
+          if (hi - lo > 1) (ok ? lo : hi) = mid;
+        }
+        if (lo < e) {
+          const uint32_t h = lo < floor ? 0u : lo;
+          if (glane == 0) settle(h);
+          for (uint32_t j = glane; j < len; j += G) {
+            const uint32_t w = adj[b + j];
+            supported(w, s_e[w], h);
+          }
+        }
+      }
+    }
+  };
+
+  uint32_t cur = 0, done = 0, sweep = 0;
+  bool left = s_n[0] > kOneQueue;  // there are marks that are not listed
+  while (sweep < cap) {            // (a barrier follows the last writes of s_n and s_cnt)
+    if (top ? s_cnt == 0 : sweep >= all && s_n[cur]) {
+      __syncthreads();
+      top = find_top(true);
+      if (top == 0) {
+        done = 1;
+        break;
+      }
+      left = list_due(cur, top);
+    } else if (s_n[cur] > kOneQueue) {
+      left = list_due(cur, top);
+    }
+    uint32_t count = s_n[cur];
+    if (count == 0) {
+      if (top || left) left = list_due(cur, top);
+      if (s_n[cur]) continue;
+      done = top && left ? 2u : 1u;
+      break;
+    }
+    count = min(count, kOneQueue);
+    if (count <= kSolo) {
+      if (wid == 0) {
+        for (;;) {
+          if (lane == 0) s_n[cur ^ 1u] = 0;
+          unmark(cur, count, lane, kWave);
+          wave_sync();
+          sweep_list(cur, count, 0, kWave / G);
+          wave_sync();
+          cur ^= 1u;
+          ++sweep;
+          count = s_n[cur];
+          if (count == 0 || count > kSolo || sweep >= cap || (top ? s_cnt == 0 : sweep >= all)) break;
+        }
+        if (lane == 0) s_sweep = sweep * 2 + cur;
+      }
+      __syncthreads();
+      sweep = s_sweep / 2;
+      cur = s_sweep & 1u;
+      __syncthreads();
+      continue;
+    }
+    if (tid == 0) s_n[cur ^ 1u] = 0;
+    unmark(cur, count, tid, kCoreLdsBlock);
+    __syncthreads();
+    sweep_list(cur, count, wid * (kWave / G), kCoreLdsBlock / G);
+    __syncthreads();
+    cur ^= 1u;
+    ++sweep;
+  }
+  __syncthreads();
+  top = find_top(false);
+  if (tid == 0) {
+    out[0] = top;
+    out[1] = done;
+  }
+  for (uint32_t v = tid; v < n; v += kCoreLdsBlock) est[v] = s_e[v];
 }
 
 // Alive vertices (the bitmap) with fewer than k alive neighbours are stamped
@@ -475,15 +719,20 @@ __global__ __launch_bounds__(kCoreLdsBlock) void k_core_prune(const uint64_t* __
   if (lane == 0 && kept) atomicAdd(alive, kept);
 }
 
-// out[0] = the largest estimate (out[0] starts at 0).
-__global__ __launch_bounds__(kBlock) void k_core_est_max(const uint32_t* __restrict__ est, uint32_t n,
+// out[0] = the largest estimate, out[1] = the vertices due (both start at 0).
+__global__ __launch_bounds__(kBlock) void k_core_est_max(const uint32_t* __restrict__ est,
+                                                         const uint8_t* __restrict__ due, uint32_t n,
                                                          uint32_t* out) {
-  uint32_t m = 0;
-  for (uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < n; v += uint64_t(gridDim.x) * blockDim.x)
+  uint32_t m = 0, c = 0;
+  for (uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < n; v += uint64_t(gridDim.x) * blockDim.x) {
     m = max(m, est[v]);
+    c += due[v] != 0;
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = max(m, uint32_t(__shfl_xor(m, o)));
+  c = wave_sum(c);
   if (lane64() == 0 && m) atomicMax(&out[0], m);
+  if (lane64() == 0 && c) atomicAdd(&out[1], c);
 }
 
 // Of the vertices alive before, those of the largest core number (*top) stay
@@ -496,6 +745,18 @@ __global__ __launch_bounds__(kBlock) void k_core_est_apply(const uint32_t* __res
     const uint32_t e = est[v];
     if (e < t && lvl[v] == kNone) lvl[v] = e ? e + 1 : floor;
   }
+}
+
+__global__ __launch_bounds__(kBlock) void k_core_est_prune(const uint32_t* __restrict__ est, uint32_t n, uint32_t k,
+                                                           uint32_t* __restrict__ lvl, uint32_t* removed) {
+  uint32_t c = 0;
+  for (uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < n; v += uint64_t(gridDim.x) * blockDim.x)
+    if (est[v] < k && lvl[v] == kNone) {
+      lvl[v] = k;
+      ++c;
+    }
+  c = wave_sum(c);
+  if (lane64() == 0 && c) atomicAdd(removed, c);
 }
 
 }  // namespace
@@ -547,19 +808,42 @@ void core_est_steps(CoreEst* a, int lanes, uint32_t count, hipStream_t s, unsign
   }
 }
 
+constexpr uint32_t kSmallSweeps = 16;     // most small levels take fewer; past them the work is in few vertices
+constexpr uint32_t kFinishAll = 64;       // sweeps over all due vertices
+constexpr uint32_t kFinishCap = 1u << 16;
+
 bool core_small_fits(uint32_t n, uint64_t slots) { return n <= kCoreSmallN && slots <= kCoreSmallSlots; }
-void core_small(const uint64_t* off, const uint32_t* adj, uint32_t n, uint32_t floor, uint32_t* lvl, uint32_t* deg,
-                int lanes, uint32_t* out, hipStream_t s, unsigned long long* stats, hipEvent_t* ev) {
+void core_small(const CoreEst& a, uint32_t* lvl, uint32_t* deg, int lanes, uint32_t* out, hipStream_t s,
+                unsigned long long* stats, hipEvent_t* ev) {
   const void* fn = lanes == 64   ? reinterpret_cast<const void*>(&k_core_small<64>)
                    : lanes == 32 ? reinterpret_cast<const void*>(&k_core_small<32>)
                    : lanes == 16 ? reinterpret_cast<const void*>(&k_core_small<16>)
                                  : reinterpret_cast<const void*>(&k_core_small<8>);
-  uint32_t cap = kCoreSmallSweeps;
-  void* args[] = {&off, &adj, &n, &floor, &cap, &lvl, &deg, &out, &stats};
+  CoreEst e = a;
+  uint32_t cap = kSmallSweeps;
+  void* args[] = {&e.off, &e.adj, &e.n, &e.floor, &cap, &lvl, &deg, &e.est, &e.due, &out, &stats};
   if (ev)
     KT_HIP(hipExtLaunchKernel(fn, dim3(1), dim3(kCoreLdsBlock), args, 0, s, ev[0], ev[1], 0));
   else
     KT_HIP(hipLaunchKernel(fn, dim3(1), dim3(kCoreLdsBlock), args, 0, s));
+}
+
+// Up to two rounds of its groups of lanes (256 vertices of short rows): a sweep
+// then takes about as long as launching one, 6 us, or half of that
+bool core_finish_fits(uint32_t n, uint32_t due, int lanes) {
+  return n <= kCoreLdsN && due <= 2 * kCoreLdsBlock / uint32_t(lanes);
+}
+void core_finish(const CoreEst& e, int lanes, uint32_t* out, hipStream_t s) {
+  const size_t bytes = sizeof(uint32_t) * ((e.n + 31) / 32) + sizeof(uint16_t) * size_t(e.n);
+  auto launch = [&](auto kernel) {
+    kernel<<<1, kCoreLdsBlock, bytes, s>>>(e.off, e.adj, e.n, e.floor, kFinishAll, kFinishCap, e.est, e.due, out);
+  };
+  switch (lanes) {
+    case 8: launch(k_core_finish<8>); break;
+    case 16: launch(k_core_finish<16>); break;
+    case 32: launch(k_core_finish<32>); break;
+    default: launch(k_core_finish<64>); break;
+  }
 }
 
 void core_prune(const uint64_t* off, const uint32_t* adj, const uint32_t* bits, uint32_t n, uint32_t k, uint32_t* lvl,
@@ -573,11 +857,14 @@ void core_prune(const uint64_t* off, const uint32_t* adj, const uint32_t* bits, 
     k_core_prune<false><<<grid, kCoreLdsBlock, 0, s>>>(off, adj, bits, n, k, lvl, alive);
 }
 
-void core_est_max(const CoreEst& a, uint32_t* top, hipStream_t s) {
-  fill_u32(top, 1, 0, s);
-  k_core_est_max<<<std::min(grid_for(a.n), 1024), kBlock, 0, s>>>(a.est, a.n, top);
+void core_est_max(const CoreEst& a, uint32_t* out, hipStream_t s) {
+  fill_u32(out, 2, 0, s);
+  k_core_est_max<<<std::min(grid_for(a.n), 1024), kBlock, 0, s>>>(a.est, a.due, a.n, out);
 }
 
+void core_est_prune(const uint32_t* est, uint32_t n, uint32_t k, uint32_t* lvl, uint32_t* removed, hipStream_t s) {
+  if (n) k_core_est_prune<<<std::min(grid_for(n), 1024), kBlock, 0, s>>>(est, n, k, lvl, removed);
+}
 void core_est_apply(const CoreEst& a, const uint32_t* top, uint32_t* lvl, hipStream_t s) {
   k_core_est_apply<<<std::min(grid_for(a.n), 4096), kBlock, 0, s>>>(a.est, a.n, a.floor, top, lvl);
 }

@@ -95,9 +95,9 @@ void core_reopen_above(uint32_t* lvl, uint32_t n, uint32_t k, hipStream_t s);
 // with est 0). steps queues `count` sweeps (lanes per row: 8, 16, 32 or 64;
 // stats, for measurement: the first one's row slots and vertices);
 // flags[count] == 0 afterwards: the estimates are the core numbers (lds: those
-// below 65,535 are, if the largest is). max:
-// *top = the largest one. apply: lvl of the alive vertices below *top = their
-// core number + 1 (floor below floor).
+// below 65,535 are, if the largest is). max: out[0] = the largest one, out[1] =
+// the vertices due. apply: lvl of the alive vertices below *top = their
+// estimate + 1 (floor below floor).
 struct CoreEst {
   const uint64_t* off;
   const uint32_t* adj;
@@ -111,14 +111,24 @@ struct CoreEst {
 bool core_est_fits_lds(uint32_t n);
 void core_est_init(const CoreEst& a, const uint32_t* deg, const uint32_t* lvl, int lanes, hipStream_t s);
 void core_est_steps(CoreEst* a, int lanes, uint32_t count, hipStream_t s, unsigned long long* stats, hipEvent_t* ev);
-void core_est_max(const CoreEst& a, uint32_t* top, hipStream_t s);
+void core_est_max(const CoreEst& a, uint32_t* out, hipStream_t s);
+// alive vertices of an estimate below k are stamped removed at k; *removed (starts
+// at 0) += how many
+void core_est_prune(const uint32_t* est, uint32_t n, uint32_t k, uint32_t* lvl, uint32_t* removed, hipStream_t s);
 void core_est_apply(const CoreEst& a, const uint32_t* top, uint32_t* lvl, hipStream_t s);
 // The whole of it for a small level (core_small_fits) in one launch: lvl as
 // after apply, deg of the max core's vertices = their degree in it; out[0] =
-// the largest core number, out[1] = 0 when the sweeps did not converge.
+// the largest core number, out[1] = 1; 0 (lvl and deg untouched) when it is not
+// done and left to finish.
 bool core_small_fits(uint32_t n, uint64_t slots);
-void core_small(const uint64_t* off, const uint32_t* adj, uint32_t n, uint32_t floor, uint32_t* lvl, uint32_t* deg,
-                int lanes, uint32_t* out, hipStream_t s, unsigned long long* stats, hipEvent_t* ev);
+void core_small(const CoreEst& a, uint32_t* lvl, uint32_t* deg, int lanes, uint32_t* out, hipStream_t s,
+                unsigned long long* stats, hipEvent_t* ev);
+// The rest of a level after small, or after steps (lds) that left few vertices
+// due (core_finish_fits) of a level without long rows, by one workgroup: out[0] = the largest estimate,
+// out[1] = 1 when all estimates are core numbers, 2 when only the largest is, 0
+// when none may be.
+bool core_finish_fits(uint32_t n, uint32_t due, int lanes);
+void core_finish(const CoreEst& a, int lanes, uint32_t* out, hipStream_t s);
 // lvl[v] = k for every vertex of the alive bitmap (alive_words) with fewer
 // than k alive neighbours; *alive (starts at 0) += the others.
 void core_prune(const uint64_t* off, const uint32_t* adj, const uint32_t* bits, uint32_t n, uint32_t k, uint32_t* lvl,

@@ -919,15 +919,27 @@ __global__ __launch_bounds__(kBlock) void k_core_collect(const uint32_t* __restr
         top = max(top, d);
       },
       reinterpret_cast<uint32_t*>(&found[0]));
+  __shared__ unsigned long long s_sum[kBlock / kWave];
+  __shared__ uint32_t s_top[kBlock / kWave];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     sum += __shfl_xor(sum, o);
     top = max(top, uint32_t(__shfl_xor(top, o)));
   }
-  if (lane64() == 0 && sum) {
-    atomicAdd(&found[1], sum);
-    uint32_t* highest = reinterpret_cast<uint32_t*>(&found[2]);
-    if (ld_agent(highest) < top) atomicMax(highest, top);
+  if (lane64() == 0) {
+    s_sum[threadIdx.x / kWave] = sum;
+    s_top[threadIdx.x / kWave] = top;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < kBlock / kWave; ++k) {
+      sum += s_sum[k];
+      top = max(top, s_top[k]);
+    }
+    if (sum) {
+      atomicAdd(&found[1], sum);
+      atomicMax(reinterpret_cast<uint32_t*>(&found[2]), top);
+    }
   }
 }
 

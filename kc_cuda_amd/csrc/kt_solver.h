@@ -67,8 +67,10 @@ struct LevelGraph {
   uint32_t k_enter = 0;          // every vertex here has core number >= k_enter
   std::vector<uint32_t> ok;      // thresholds whose peel left vertices alive
   // after a core decomposition: lvl is exact for thresholds in
-  // [exact_from, exact_to] (the t-core = alive or lvl > t); 0, 0 otherwise
+  // [exact_from, exact_to] (the t-core = alive or lvl > t; loose: that holds
+  // it); 0, 0 otherwise
   uint32_t exact_from = 0, exact_to = 0;
+  bool loose = false;
   DevBuf b_off, b_adj, b_deg, b_lvl, b_orig;
 };
 
@@ -230,8 +232,8 @@ class Solver {
   // fresh: start from full degrees with every vertex alive; otherwise from
   // the state already on level 0. allow_cut: continue on induced subgraphs.
   uint32_t max_core(bool allow_cut = true, bool fresh = true);
-  uint32_t max_core_gallop(bool allow_cut, bool fresh);
-  bool max_core_numbers(bool allow_cut, bool fresh, uint32_t* k);
+  uint32_t max_core_gallop(bool allow_cut, bool fresh, uint32_t hi);
+  bool max_core_numbers(bool allow_cut, bool fresh, uint32_t* k, uint32_t* hi);
   // Whole graphs (and cut levels of the gallop) up to this many row slots get
   // core numbers, larger ones the peel: a sweep gathers every row slot at
   // random, a peel round streams and walks only what it removes. Random graphs
@@ -242,7 +244,7 @@ class Solver {
   // levels of fewer row slots are not worth a prune and a second cut
   static constexpr uint64_t kPruneMinSlots = uint64_t(1) << 22;
   uint32_t prune_level(LevelGraph& g, uint32_t k);
-  bool core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top);
+  bool core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top, uint32_t* hi);
   uint32_t degree_hindex(const LevelGraph& g0);
   bool filtered_start(LevelGraph** gp, uint32_t* k_out, uint64_t* alive_out);
   LevelGraph& level0();
@@ -366,6 +368,7 @@ class Solver {
   double trace_ms();
   std::chrono::steady_clock::time_point trace_t0_{};
   bool gallop_ = true;
+  bool est_whole_ = false;  // keys_ holds upper bounds of the whole graph's core numbers
   bool peeled_by_rows_ = false;
   uint32_t count_kind_ = 0, count_words_ = 0;  // the last timed support count
   uint32_t walk_levels_ = 16;

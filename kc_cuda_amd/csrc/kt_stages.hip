@@ -263,14 +263,22 @@ uint32_t Solver::degree_hindex(const LevelGraph& g0) {
 // largest core number: its vertices stay alive with their degrees in it, and
 // every other vertex is stamped with its core number + 1 (floor below floor),
 // so every cut of g from floor to *top is exact; with *top == 0 (no core of
-// floor) every vertex is stamped. False (lvl and deg untouched) when the
-// sweeps have not converged after kCoreSweeps: each sweep moves a removal one
-// vertex along, so a core that unravels along a path of many vertices is left
-// to the peel.
-bool Solver::core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top) {
-  constexpr uint32_t kBatch = 16, kMaxBatch = 32, kCoreSweeps = 512;
+// floor) every vertex is stamped.
+// Each sweep moves a removal one vertex along. Where a core unravels along
+// paths of many vertices, so that few are due, one workgroup takes over, which
+// needs no launch a sweep and stops once the max core stands: other stamps are
+// then upper bounds (g.loose), which a cut still has to peel. False (lvl and
+// deg untouched, *hi = a threshold with an empty core, 0: none known) when a
+// level too large for that, or with long rows, has not converged after
+// kCoreSweeps; its estimates then bound and prune the peel.
+// Whole solves in ms, by a galloping peel alone, by sweeps given up after 512,
+// and so: a path of 3 k vertices 5.0, 12.4, 5.1; of 10 k 15.5, 26.7, 15.4; a
+// clique with a tail of 3 k 0.94, 5.7, 0.69; grids of 200^2 7.1, 2.9, 2.7; of
+// 600^2 79.5, 90.4, 16.7; of 1,000^2 185, 202, 65; triangulated 365, 363, 119.
+bool Solver::core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top, uint32_t* hi) {
+  constexpr uint32_t kBatch = 16, kMaxBatch = 32, kCoreSweeps = 512, kOutWords = kMaxBatch + 5;
   const uint32_t n = g.n;
-  core_out_.ensure(sizeof(uint32_t) * (kMaxBatch + 4));  // top | flags | medium and heavy counts
+  core_out_.ensure(sizeof(uint32_t) * kOutWords);  // top, due | flags | medium and heavy rows
   uint32_t* out = core_out_.as<uint32_t>();
   const int lanes = auto_lanes(double(g.slots) / std::max<uint32_t>(n, 1));
   // measurement of the vertex peel
@@ -278,63 +286,79 @@ bool Solver::core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top) {
   auto events = [&](uint32_t count) { return probe && (probe_push_ & 1) ? probe_events(int(count)) : nullptr; };
   unsigned long long* ps = probe && (probe_push_ & 2) ? probe_stats_.as<unsigned long long>() : nullptr;
   if (trace_) trace_ms();
+  // extraction scratch, free at this point
+  keys_.ensure(sizeof(uint64_t) * (size_t(n_) + 1));
+  keys2_.ensure(sizeof(uint64_t) * (size_t(n_) + 1));
+  const HeavyList hl = heavy();
+  CoreEst a{};
+  a.off = g.off;
+  a.adj = g.adj;
+  a.n = n;
+  a.floor = floor;
+  a.est = keys_.as<uint32_t>();
+  a.due = keys2_.as<uint8_t>();
+  a.due_next = a.due + n;
+  a.medium = hl.slices;
+  a.heavy = hl.items;
+  a.flags = out + 2;
+  a.counts = a.flags + kMaxBatch + 1;
+  a.lds = core_est_fits_lds(n);
   uint32_t sweeps = 0;
-  if (core_small_fits(n, g.slots)) {
-    core_small(g.off, g.adj, n, floor, g.lvl, g.deg, lanes, out, stream_, ps, events(1));
-    KT_HIP(hipMemcpyAsync(pinned_, out, sizeof(uint32_t) * 2, hipMemcpyDeviceToHost, stream_));
+  bool loose = false, small = core_small_fits(n, g.slots);
+  auto read = [&](uint32_t words) {  // the largest estimate, and what else out holds
+    KT_HIP(hipMemcpyAsync(pinned_, out, sizeof(uint32_t) * words, hipMemcpyDeviceToHost, stream_));
     KT_HIP(hipStreamSynchronize(stream_));
-    if (!pinned_[1]) return false;
     *top = pinned_[0];
+    *hi = a.lds && *top >= 65535 ? 0 : *top + 1;  // (0: cut off)
+  };
+  auto finish = [&] {
+    core_finish(a, lanes, out, stream_);
+    read(2);
+    loose = pinned_[1] == 2;
+    return pinned_[1] != 0 && *top < 65535;
+  };
+  if (small) {
+    core_small(a, g.lvl, g.deg, lanes, out, stream_, ps, events(1));
+    read(2);
+    small = pinned_[1] == 1;
+    if (!small && !finish()) return false;
   } else {
-    // extraction scratch, free at this point
-    keys_.ensure(sizeof(uint64_t) * (size_t(n_) + 1));
-    keys2_.ensure(sizeof(uint64_t) * (size_t(n_) + 1));
-    const HeavyList hl = heavy();
-    CoreEst a{};
-    a.off = g.off;
-    a.adj = g.adj;
-    a.n = n;
-    a.floor = floor;
-    a.est = keys_.as<uint32_t>();
-    a.due = keys2_.as<uint8_t>();
-    a.due_next = a.due + n;
-    a.medium = hl.slices;
-    a.heavy = hl.items;
-    a.flags = out + 1;
-    a.counts = a.flags + kMaxBatch + 1;
-    a.lds = core_est_fits_lds(n);
     core_est_init(a, g.deg, g.lvl, lanes, stream_);
     for (uint32_t batch = kBatch;;) {
       core_est_steps(&a, lanes, batch, stream_, sweeps ? nullptr : ps, events(batch));
       core_est_max(a, out, stream_);
-      KT_HIP(hipMemcpyAsync(pinned_, out, sizeof(uint32_t) * (batch + 2), hipMemcpyDeviceToHost, stream_));
-      KT_HIP(hipStreamSynchronize(stream_));
+      read(kOutWords);
       sweeps += batch;
-      if (pinned_[1 + batch] == 0) {
-        if (!a.lds || pinned_[0] < 65535) break;
+      if (pinned_[2 + batch] == 0) {
+        if (!a.lds || *top < 65535) break;
         a.lds = false;  // a core past 16 bits, of repeated pairs
         core_est_init(a, g.deg, g.lvl, lanes, stream_);
         continue;
       }
+      const bool long_rows = pinned_[kOutWords - 2] || pinned_[kOutWords - 1];
+      if (a.lds && !long_rows && core_finish_fits(n, pinned_[1], lanes)) {
+        if (!finish()) return false;
+        break;
+      }
       if (sweeps >= kCoreSweeps) return false;
       batch = std::min(batch * 2, kMaxBatch);
     }
-    *top = pinned_[0];
-    if (*top) {
-      core_est_apply(a, out, g.lvl, stream_);
-      core_alive_degrees(g.off, g.adj, g.lvl, n, g.deg, heavy(), stream_);
-    } else {
-      fill_u32(g.lvl, n, floor, stream_);
-    }
+  }
+  if (!*top) {
+    fill_u32(g.lvl, n, floor, stream_);
+  } else if (!small) {
+    core_est_apply(a, out, g.lvl, stream_);
+    core_alive_degrees(g.off, g.adj, g.lvl, n, g.deg, heavy(), stream_);
   }
   if (trace_)
-    std::fprintf(stderr, "[kt] core numbers level_n=%u slots=%llu from k=%u: max core %u, at most %u sweeps (%.2f ms)\n",
-                 n, (unsigned long long)g.slots, floor, *top, sweeps, trace_ms());
+    std::fprintf(stderr, "[kt] core numbers level_n=%u slots=%llu from k=%u: max core %u, at most %u sweeps%s (%.2f ms)\n",
+                 n, (unsigned long long)g.slots, floor, *top, sweeps, loose ? ", others bounds" : "", trace_ms());
   vertex_rounds_ = false;
   if (*top) {
     g.ok.push_back(*top);
     g.exact_from = floor;
     g.exact_to = *top;
+    g.loose = loose;
   }
   return true;
 }
@@ -369,8 +393,9 @@ uint32_t Solver::prune_level(LevelGraph& g, uint32_t k) {
 // vertices kept, 30 k left). When the core is empty the threshold drops by
 // 4x, and when the filter would keep more than a quarter of the vertices the
 // whole graph is taken if it has at most kCoreWholeSlots row slots. False:
-// not converged, or too large (the level 0 state is as it was, or fresh).
-bool Solver::max_core_numbers(bool allow_cut, bool fresh, uint32_t* k) {
+// not converged, or too large (the level 0 state is as it was, or fresh); *hi
+// is then the lowest threshold known to have an empty core, if any is.
+bool Solver::max_core_numbers(bool allow_cut, bool fresh, uint32_t* k, uint32_t* hi) {
   LevelGraph& g0 = levels_.empty() || fresh ? level0() : *levels_[0];
   if (fresh) degrees_from_offsets(g0.off, g0.n, g0.deg, stream_);
   if (allow_cut && fresh && g0.n >= 4 * kMinCut) {
@@ -388,13 +413,18 @@ bool Solver::max_core_numbers(bool allow_cut, bool fresh, uint32_t* k) {
         if (left == 0) continue;
         if (uint64_t(left) * 4 <= uint64_t(s->n) * 3) s = &cut_level(*s, kf, left, true);
       }
-      if (!core_numbers(*s, kf, k)) return false;
+      if (!core_numbers(*s, kf, k, hi)) {
+        if (*hi) *hi = std::max(*hi, kf);
+        return false;
+      }
       if (*k) return true;
     }
   }
   depth_ = 1;
   if (fresh) fill_u32(g0.lvl, g0.n, kNone, stream_);
-  return g0.slots <= kCoreWholeSlots && core_numbers(g0, 1, k);
+  *hi = 0;
+  est_whole_ = true;
+  return g0.slots <= kCoreWholeSlots && core_numbers(g0, 1, k, hi);
 }
 
 // The largest k with a non-empty k-core (0: no edges); leaves the max-core
@@ -405,10 +435,11 @@ bool Solver::max_core_numbers(bool allow_cut, bool fresh, uint32_t* k) {
 // galloping search.
 uint32_t Solver::max_core(bool allow_cut, bool fresh) {
   depth_ = 1;
-  uint32_t top = 0;
-  if (n_ && vertex_mode_ == 0 && mirrored_ && max_core_numbers(allow_cut, fresh, &top)) return top;
+  uint32_t top = 0, hi = 0;
+  est_whole_ = false;
+  if (n_ && vertex_mode_ == 0 && mirrored_ && max_core_numbers(allow_cut, fresh, &top, &hi)) return top;
   depth_ = 1;
-  return max_core_gallop(allow_cut, fresh);
+  return max_core_gallop(allow_cut, fresh, hi);
 }
 
 // Start of the galloping search from a high threshold: a sixteenth of the
@@ -443,7 +474,10 @@ bool Solver::filtered_start(LevelGraph** gp, uint32_t* k_out, uint64_t* alive_ou
 
 // Galloping search for the largest k with a non-empty k-core; once a step
 // leaves few enough alive for a cut, the core numbers of the cut level end it.
-uint32_t Solver::max_core_gallop(bool allow_cut, bool fresh) {
+// hi: a threshold known to have an empty core (0: none known), found by sweeps
+// that did not converge: cut levels are then not swept again, and while the
+// whole graph is peeled its estimates take the first part of every cascade.
+uint32_t Solver::max_core_gallop(bool allow_cut, bool fresh, uint32_t hi) {
   LevelGraph* g = levels_.empty() || fresh ? &level0() : levels_[0].get();
   deg_bak_.ensure(sizeof(uint32_t) * (size_t(n_) + 1));
   q0_.ensure(sizeof(uint32_t) * (size_t(n_) + 1));
@@ -467,24 +501,45 @@ uint32_t Solver::max_core_gallop(bool allow_cut, bool fresh) {
     g->exact_from = g->exact_to = 0;
     if (allow_cut && alive * 4 <= g->n && alive >= kMinCut) g = &cut_level(*g, 1, uint32_t(alive));
   }
-  bool grow = true, tried = false;
-  while (step > 0) {
+  bool grow = true, slow = hi != 0, tried = slow;
+  // what the sweeps over the whole graph left (a filter's cut has reused it)
+  const uint32_t* est = hi && depth_ == 1 && est_whole_ ? keys_.as<uint32_t>() : nullptr;
+  while (step > 0 && (!hi || k + 1 < hi)) {
     if (vertex_mode_ == 0 && mirrored_ && depth_ > 1 && !tried && g->slots <= kCoreWholeSlots) {
-      uint32_t top = 0;
-      if (core_numbers(*g, k, &top) && top) return top;
+      uint32_t top = 0, bound = 0;
+      if (core_numbers(*g, k, &top, &bound)) {
+        if (top) return top;
+      } else if (bound) {
+        slow = true;
+        hi = std::max(hi ? std::min(hi, bound) : bound, k + 1);
+      }
       tried = true;
+      continue;
     }
     const uint32_t kk = k + step;
+    if (hi && kk >= hi) {  // known to be empty
+      step /= 2;
+      grow = false;
+      continue;
+    }
     KT_HIP(hipMemcpyAsync(deg_bak_.p, g->deg, sizeof(uint32_t) * g->n, hipMemcpyDeviceToDevice, stream_));
-    const uint64_t removed = peel_vertices(*g, kk, alive);  // an overshoot is restored below
+    uint64_t removed = 0;
+    if (est && depth_ == 1) {  // no vertex of a lower estimate is in the kk-core
+      zero_u32(&ctl_->nalive);
+      core_est_prune(est, g->n, kk, g->lvl, &ctl_->nalive, stream_);
+      core_alive_degrees(g->off, g->adj, g->lvl, g->n, g->deg, heavy(), stream_);
+      removed = read_u32(&ctl_->nalive);
+    }
+    if (removed < alive) removed += peel_vertices(*g, kk, alive - removed);  // an overshoot is restored below
     if (removed < alive) {
       alive -= removed;
       k = kk;
       g->ok.push_back(k);
       step = grow ? step * 2 : step / 2;
-      if (allow_cut && alive * 4 <= g->n && alive >= kMinCut) g = &cut_level(*g, k, uint32_t(alive)), tried = false;
+      if (allow_cut && alive * 4 <= g->n && alive >= kMinCut) g = &cut_level(*g, k, uint32_t(alive)), tried = slow;
     } else {
       // overshoot: re-open what this step removed and restore degrees
+      hi = kk;
       core_reopen_above(g->lvl, g->n, k, stream_);
       KT_HIP(hipMemcpyAsync(g->deg, deg_bak_.p, sizeof(uint32_t) * g->n, hipMemcpyDeviceToDevice, stream_));
       if (step == 1) break;
@@ -521,7 +576,7 @@ void Solver::core_at(uint32_t k) {
   if (exact) kj = k;
   core_reopen_above(g.lvl, g.n, kj, stream_);
   core_alive_degrees(g.off, g.adj, g.lvl, g.n, g.deg, heavy(), stream_);
-  if (k > kj) peel_vertices(g, k);
+  if (k > kj || (exact && g.loose)) peel_vertices(g, k);
   // stamps at or below k are untouched; above k they are gone
   if (exact)
     g.exact_to = k;

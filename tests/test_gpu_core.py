@@ -91,3 +91,64 @@ def test_cores_of_repeated_pairs_beyond_16_bits(ctx, copies):
     """Two vertices joined many times: a core as large as the count of copies."""
     r = ctx.solve_pairs(np.tile(np.array([[3, 9]], np.uint32), (copies, 1)), 12)
     assert (r.max_core, r.kmax, r.truss_edges) == (copies, 0, 0)
+
+
+def _grid(side, diagonals):
+    i = np.arange(side * side).reshape(side, side)
+    e = [np.column_stack([i[:, :-1].ravel(), i[:, 1:].ravel()]), np.column_stack([i[:-1].ravel(), i[1:].ravel()])]
+    if diagonals:
+        e.append(np.column_stack([i[:-1, :-1].ravel(), i[1:, 1:].ravel()]))
+    return canon_pairs(np.concatenate(e).astype(np.uint32)), side * side
+
+
+def _ladder_into_expander(columns, n):
+    """A ladder, broken at one end, that leads into a random graph: every
+    vertex has three neighbours, so the 3-core unravels along the ladder and
+    then all over the graph at once."""
+    rng = np.random.default_rng(n)
+    ring = np.arange(n)
+    match = rng.permutation(n).reshape(-1, 2)  # a ring and a matching
+    e = np.concatenate([np.column_stack([ring, (ring + 1) % n])[:-1], match])  # the ring is cut between n - 1 and 0
+    u, v = n + np.arange(columns), n + columns + np.arange(columns)
+    e = np.concatenate([e, np.column_stack([u[:-1], u[1:]]), np.column_stack([v[:-1], v[1:]]), np.column_stack([u, v]),
+                        [[0, u[-1]], [n - 1, v[-1]]]])
+    return np.unique(canon_pairs(e.astype(np.uint32)), axis=0), n + 2 * columns
+
+
+LONG = {
+    # one workgroup from the start, from the first sweeps on, from later ones on; peel with bounds
+    "grid_20": lambda: _grid(20, False), "mesh_40": lambda: _grid(40, True), "grid_70": lambda: _grid(70, False),
+    "mesh_150": lambda: _grid(150, True), "grid_256": lambda: _grid(256, False), "grid_257": lambda: _grid(257, False),
+    "grid_640": lambda: _grid(640, False), "mesh_560": lambda: _grid(560, True),
+    "path_4096": lambda: (_lollipop(4089, 7), 4096), "path_65536": lambda: (_lollipop(65_529, 7), 65_536),
+    # more vertices due at once than one workgroup lists
+    "expander": lambda: _ladder_into_expander(300, 60_000),
+}
+
+
+@pytest.mark.parametrize("name", LONG)
+def test_cores_that_unravel_over_many_sweeps(ctx, name):
+    pairs, n = LONG[name]()
+    print(f"[gpu] {name} m={len(pairs)}", flush=True)
+    ref = O.solve_pairs(pairs, n, want_edges=True)
+    r = ctx.solve_pairs(pairs, n)
+    assert (r.max_core, r.k_hat, r.kmax, r.truss_edges) == (ref.max_core, ref.k_hat, ref.kmax, ref.truss_edges)
+    np.testing.assert_array_equal(ctx.truss_edges(), canon_pairs(ref.truss))
+
+
+@pytest.mark.parametrize("path", [300, 5000, 70_000])
+def test_second_core_from_bounds(ctx, path):
+    """A max core without triangles, known before the path that hangs off it has
+    unravelled: the 2-core of the second pass is peeled from upper bounds."""
+    k = 10
+    side = np.array([(a, k + b) for a in range(k) for b in range(k)])
+    walk = 2 * k - 1 + np.arange(path + 1)
+    end = int(walk[-1])
+    e = np.concatenate([side, np.column_stack([walk[:-1], walk[1:]]), [[end, end + 1], [end, end + 2], [end + 1, end + 2]],
+                        [[end + 2, end + 3]]])  # a triangle, and a spike on it
+    e = np.concatenate([e, np.column_stack([np.full(path, end + 3), end + 4 + np.arange(path)])[:1],
+                        np.column_stack([end + 4 + np.arange(path - 1), end + 5 + np.arange(path - 1)])])
+    n = end + 4 + path
+    r = ctx.solve_pairs(canon_pairs(e.astype(np.uint32)), n)
+    assert (r.max_core, r.kmax, r.truss_edges) == (k, 3, 3)
+    np.testing.assert_array_equal(ctx.truss_edges(), [[end, end + 1], [end, end + 2], [end + 1, end + 2]])
