@@ -370,6 +370,7 @@ class Solver {
   bool gallop_ = true;
   bool est_whole_ = false;  // keys_ holds upper bounds of the whole graph's core numbers
   bool peeled_by_rows_ = false;
+  uint64_t listed_ = 0;  // entries of the last core's triangle lists
   uint32_t count_kind_ = 0, count_words_ = 0;  // the last timed support count
   uint32_t walk_levels_ = 16;
   uint64_t split_build_min_ = uint64_t(1) << 22;  // fewest pairs of the build by two splits (see split_plan)

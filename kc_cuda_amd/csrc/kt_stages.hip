@@ -989,6 +989,8 @@ bool Solver::list_triangles(const CoreView& cv) {
   std::memcpy(got, pinned_, sizeof(got));
   const uint64_t entries = got[0], bytes = entries * sizeof(uint2);
   if (got[1] || entries >= (uint64_t(1) << 31) || bytes > tri_budget_ || bytes > tri_per_edge_ * mc) return false;
+  listed_ = entries;
+  if (entries == 0) return true;  // no walk will look for any
   const size_t per_edge = sizeof(uint32_t) * (size_t(mc) + 1);
   if (arena_) {
     for (DevBuf* b : {&tri_off_, &live_[0], &live_[1]}) b->ensure(per_edge);
@@ -1030,7 +1032,10 @@ bool Solver::list_triangles(const CoreView& cv) {
 // and on exit.
 TrussOutcome Solver::run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32_t* r_io, const SearchRule& search,
                                bool allow_host) {
-  constexpr uint32_t kFirstBatch = 8, kMaxBatch = 32;
+  constexpr uint32_t kMaxBatch = 32;
+  // without triangles a look and the level's end are all there is (a grid of 40
+  // x 40: 0.83 ms with empty lists and eight steps, 0.69 without)
+  const uint32_t first_batch = !cv->dense && listed_ == 0 ? 2 : 8;
   static_assert(sizeof(StepState) * 2 + sizeof(StepCounters) * 3 <= kStepCtlBytes, "step control block too small");
   static_assert(sizeof(StepState) <= 4 * kTrussCountWord, "state exceeds the pinned readback buffer");
   step_ctl_.ensure(kStepCtlBytes);
@@ -1058,7 +1063,7 @@ TrussOutcome Solver::run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32
     rule.pair_cost = !cv->dense ? 0.0 : cv->repeats ? HUGE_VAL : dense_pair_cost(cv->nc, cv->ws);
     steps_start(a, h, stream_);
     uint64_t steps = 0;
-    uint32_t batch = kFirstBatch;
+    uint32_t batch = first_batch;
     do {
       // a step removes an edge, completes a level or prepares one that does
       if (steps > 4 * uint64_t(cv->mc) + 4 * kMaxBatch) fail("edge peel did not converge");

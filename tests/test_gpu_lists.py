@@ -208,3 +208,17 @@ def test_repeated_pairs_on_dense_cores(dense_ctx):
     assert got[0][:2] == got[1][:2] == (n, len(twice))
     np.testing.assert_array_equal(got[0][2], twice)
     np.testing.assert_array_equal(got[1][2], twice)
+
+
+@pytest.mark.parametrize("side", [3, 40, 90])
+def test_cores_without_triangles(sparse_ctx, side):
+    """Nothing is listed; the levels end in their first look."""
+    i = np.arange(side * side).reshape(side, side)
+    pairs = canon_pairs(np.concatenate([np.column_stack([i[:, :-1].ravel(), i[:, 1:].ravel()]),
+                                        np.column_stack([i[:-1].ravel(), i[1:].ravel()])]).astype(np.uint32))
+    for _ in range(2):
+        r = sparse_ctx.solve_pairs(pairs, side * side)
+        assert (r.max_core, r.kmax, r.truss_edges) == (2, 0, 0)
+        assert len(sparse_ctx.truss_edges()) == 0 and len(sparse_ctx.trussness()) == 0
+        k5 = np.array([(a, b) for a in range(5) for b in range(a + 1, 5)], dtype=np.uint32)
+        assert sparse_ctx.solve_pairs(k5, 5).kmax == 5
