@@ -357,15 +357,23 @@ __device__ __forceinline__ unsigned long long slot_hash(uint32_t x, uint32_t y) 
   return z ^ (z >> 32);
 }
 __device__ __forceinline__ void add_mirror_sum(unsigned long long c, unsigned long long* sum) {
+  __shared__ unsigned long long s_c[kBlock / kWave];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if (lane64() == 0 && c) atomicAdd(sum, c);
+  if (lane64() == 0) s_c[threadIdx.x / kWave] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < kBlock / kWave; ++k) c += s_c[k];
+    atomicAdd(sum, c);
+  }
 }
+constexpr int kMirrorGrid = 512;  // workgroups, each with one atomic on the sum
 __global__ __launch_bounds__(kBlock) void k_mirror_lines(const uint32_t* __restrict__ xs,
                                                          const uint32_t* __restrict__ ys, uint64_t L,
                                                          unsigned long long* sum) {
   unsigned long long c = 0;
   const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
+#pragma unroll 4
   for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < L; i += stride) {
     const uint32_t x = xs[i], y = ys[i];
     c += slot_hash(x, y) - slot_hash(y, x);
@@ -1946,13 +1954,13 @@ void csr_copy_cols(const uint32_t* xs, uint64_t L, uint32_t n, uint32_t* adj, ui
 void mirror_lines(const uint32_t* xs, const uint32_t* ys, uint64_t L, uint64_t* sum, hipStream_t s) {
   fill_u64(sum, 1, 0, s);
   if (L)
-    k_mirror_lines<<<std::min(grid_for(L, 4 * kBlock), 2048), kBlock, 0, s>>>(
+    k_mirror_lines<<<std::min(grid_for(L, 4 * kBlock), kMirrorGrid), kBlock, 0, s>>>(
         xs, ys, L, reinterpret_cast<unsigned long long*>(sum));
 }
 void mirror_rows(const uint64_t* off, const uint32_t* adj, uint32_t n, uint64_t* sum, hipStream_t s) {
   fill_u64(sum, 1, 0, s);
   if (n)
-    k_mirror_rows<<<std::min(grid_for(uint64_t(n) * kWave), 2048), kBlock, 0, s>>>(
+    k_mirror_rows<<<std::min(grid_for(uint64_t(n) * kWave), kMirrorGrid), kBlock, 0, s>>>(
         off, adj, n, reinterpret_cast<unsigned long long*>(sum));
 }
 void csr_fwd_start(const uint32_t* pairs, uint64_t items, uint32_t S, uint32_t B, uint64_t* f0, hipStream_t s) {
