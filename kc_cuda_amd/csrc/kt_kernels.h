@@ -303,7 +303,8 @@ bool dense_by_pairs(uint32_t nc, uint32_t mc, uint32_t ws);
 void dense_count(const uint64_t* bits, const uint32_t* pref0, const uint32_t* off_u, const uint32_t* eid_u,
                  const uint32_t* eidm, uint32_t nc, uint32_t ws, int32_t* sup, hipStream_t s);
 // Triangle lists (kt_list.hip). list_size: found[0] = the sum of the supports
-// (null: 0), found[1] = 1 when a row is not strictly ascending above its own vertex.
+// (null: 0), found[1] = 1 when a row is not strictly ascending above its own
+// vertex, found[2], found[3] = the highest support and ~ of the lowest (low words).
 // tri_fill: every triangle's entries, cursor starting as a copy of the offsets
 // (bitmap: the enumeration that counted the supports; lanes: as the count's).
 void list_size(const int32_t* sup, const uint32_t* src, const uint32_t* adj, uint32_t mc, uint64_t* found,

@@ -108,25 +108,51 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill_edges(const uint32_t* __res
   }
 }
 
-// found[0] += the sum of the supports (null: none), found[1] = 1 when a row is not strictly
-// ascending above its own vertex. The count and the fill need not agree on
-// such rows (a repeated neighbour is found once by a search, and by each of
-// its copies where they are streamed), so entries would miss their lists.
+// found[0] += the sum of the supports (null: none), found[1] = 1 when a row is
+// not strictly ascending above its own vertex, found[2], found[3] = the highest
+// support and ~ of the lowest. The count and the fill need not agree on such
+// rows (a repeated neighbour is found once by a search, and by each of its
+// copies where they are streamed), so entries would miss their lists.
 __global__ __launch_bounds__(kBlock) void k_list_size(const uint32_t* __restrict__ sup,
                                                       const uint32_t* __restrict__ src,
                                                       const uint32_t* __restrict__ adj, uint32_t mc,
                                                       unsigned long long* found) {
+  __shared__ unsigned long long s_sum[kBlock / kWave];
+  __shared__ uint2 s_ends[kBlock / kWave];
   unsigned long long c = 0;
+  uint32_t high = 0, low = 0;  // low: ~ the lowest
   bool odd = false;
   for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < mc; i += gridDim.x * blockDim.x) {
     const uint32_t u = src[i], v = adj[i];
-    if (sup) c += sup[i];
+    if (sup) {
+      const uint32_t x = sup[i];
+      c += x;
+      high = max(high, x);
+      low = max(low, ~x);
+    }
     odd |= v <= u || (i + 1 < mc && src[i + 1] == u && adj[i + 1] <= v);
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if (lane64() == 0 && c) atomicAdd(&found[0], c);
-  if (__ballot(odd) && lane64() == 0) found[1] = 1;
+  for (int o = 32; o > 0; o >>= 1) {
+    c += __shfl_xor(c, o);
+    high = max(high, uint32_t(__shfl_xor(high, o)));
+    low = max(low, uint32_t(__shfl_xor(low, o)));
+  }
+  if (lane64() == 0) {
+    s_sum[threadIdx.x / kWave] = c;
+    s_ends[threadIdx.x / kWave] = make_uint2(high, low);
+  }
+  if (__syncthreads_or(odd) && threadIdx.x == 0) found[1] = 1;
+  if (threadIdx.x == 0 && sup) {
+    for (int k = 1; k < kBlock / kWave; ++k) {
+      c += s_sum[k];
+      high = max(high, s_ends[k].x);
+      low = max(low, s_ends[k].y);
+    }
+    atomicAdd(&found[0], c);
+    atomicMax(reinterpret_cast<uint32_t*>(&found[2]), high);
+    atomicMax(reinterpret_cast<uint32_t*>(&found[3]), low);
+  }
 }
 
 }  // namespace
@@ -135,7 +161,7 @@ __global__ __launch_bounds__(kBlock) void k_list_size(const uint32_t* __restrict
 
 void list_size(const int32_t* sup, const uint32_t* src, const uint32_t* adj, uint32_t mc, uint64_t* found,
                hipStream_t s) {
-  fill_u64(found, 2, 0, s);
+  fill_u64(found, 4, 0, s);
   if (mc)
     k_list_size<<<std::min(grid_for(mc), 1024), kBlock, 0, s>>>(reinterpret_cast<const uint32_t*>(sup), src, adj, mc,
                                                                 reinterpret_cast<unsigned long long*>(found));

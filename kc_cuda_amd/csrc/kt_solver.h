@@ -317,7 +317,7 @@ class Solver {
   PeelArgs peel_args(const CoreView& cv);
   // frontier of the live edges below thr, stamped; the rounds' starting state
   // (reset: a new search with its early-exit rule)
-  bool list_triangles(const CoreView& cv);
+  bool list_triangles(const CoreView& cv, int32_t thr, const SearchRule& search);
   bool counts_by_bitmap(const CoreView& cv) const;
   StepArgs step_args(const CoreView& cv);
   TrussOutcome run_steps(CoreView* cv, int32_t thr, uint64_t alive, uint32_t* r_io, const SearchRule& search,
@@ -370,7 +370,7 @@ class Solver {
   bool gallop_ = true;
   bool est_whole_ = false;  // keys_ holds upper bounds of the whole graph's core numbers
   bool peeled_by_rows_ = false;
-  uint64_t listed_ = 0;  // entries of the last core's triangle lists
+  bool walks_ = true;  // the search over triangle lists has frontiers to walk
   uint32_t count_kind_ = 0, count_words_ = 0;  // the last timed support count
   uint32_t walk_levels_ = 16;
   uint64_t split_build_min_ = uint64_t(1) << 22;  // fewest pairs of the build by two splits (see split_plan)

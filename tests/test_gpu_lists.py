@@ -222,3 +222,26 @@ def test_cores_without_triangles(sparse_ctx, side):
         assert len(sparse_ctx.truss_edges()) == 0 and len(sparse_ctx.trussness()) == 0
         k5 = np.array([(a, b) for a in range(5) for b in range(a + 1, 5)], dtype=np.uint32)
         assert sparse_ctx.solve_pairs(k5, 5).kmax == 5
+
+
+@pytest.mark.parametrize("kind,size", [("cliques", 5), ("cliques", 40), ("wheel", 4), ("wheel", 5), ("wheel", 900),
+                                       ("wheel_and_tail", 30)])
+def test_searches_that_walk_no_frontier(sparse_ctx, kind, size):
+    """Equal supports, or a first level that ends the search: nothing is
+    listed; and next to them searches that do walk."""
+    if kind == "cliques":
+        u, v = np.triu_indices(size, 1)
+        pairs, n = np.concatenate([np.column_stack([u, v]) + i * size for i in range(20)]), 20 * size
+    else:
+        rim = np.arange(1, size + 1)
+        pairs, n = np.concatenate([np.column_stack([np.zeros(size, int), rim]), np.column_stack([rim, rim % size + 1])]), size + 1
+        if kind == "wheel_and_tail":  # a square: supports below the first level
+            pairs, n = np.concatenate([pairs, [[0, n], [n, n + 1], [n + 1, 1]]]), n + 2
+    pairs = np.unique(canon_pairs(pairs.astype(np.uint32)), axis=0)
+    ref = O.solve_pairs(pairs, n, want_edges=True)
+    r = sparse_ctx.solve_pairs(pairs, n)
+    assert (r.k_hat, r.kmax, r.truss_edges) == (ref.k_hat, ref.kmax, ref.truss_edges)
+    np.testing.assert_array_equal(sparse_ctx.truss_edges(), canon_pairs(ref.truss))
+    t = O.trussness(pairs)
+    want = np.array(sorted((u, v, k) for (u, v), k in t.items() if k >= 3), dtype=np.uint32).reshape(-1, 3)
+    np.testing.assert_array_equal(sparse_ctx.trussness(), want)
