@@ -24,7 +24,7 @@ constexpr uint32_t kCoreSmallN = 4096;
 constexpr uint32_t kCoreSmallSlots = 1u << 13;
 constexpr uint32_t kLightRegs = 16;   // row entries a lane keeps: a light row has at most 16 * G
 constexpr uint32_t kMediumRegs = 64;  // a medium row, taken by one wave, at most 4096
-constexpr uint32_t kHeavyRegs = 16;   // and a heavy row, taken by a workgroup of NT threads, 16 * NT
+constexpr uint32_t kHeavyRegs = 16;   // and a heavy row, taken by a workgroup of kCoreLdsBlock, 16,384 (kLds)
 constexpr uint32_t kHistBins = 1024;  // heavy rows: bins per refinement of the new estimate
 
 // est[v] = deg[v], or 0 (no core of at least `floor` >= 1 holds v) when that
@@ -222,7 +222,11 @@ __global__ __launch_bounds__(kLds ? kCoreLdsBlock : kBlock) void k_core_est_step
     const uint64_t len = off[v + 1] - b;
     if (stats && tid == 0) counted(len);
     uint32_t h;
-    if (len <= uint64_t(kHeavyRegs) * NT) {  // read once, kept in registers
+    // a workgroup of kCoreLdsBlock holds rows of up to 16,384 entries in
+    // registers; one of kBlock would hold 4,096, which are no heavy rows yet
+    bool held = false;
+    if constexpr (kLds) held = len <= uint64_t(kHeavyRegs) * NT;
+    if (kLds && held) {  // read once
       uint32_t x[kHeavyRegs];
 #pragma unroll
       for (uint32_t r = 0; r < kHeavyRegs; ++r) {

@@ -152,3 +152,28 @@ def test_second_core_from_bounds(ctx, path):
     r = ctx.solve_pairs(canon_pairs(e.astype(np.uint32)), n)
     assert (r.max_core, r.kmax, r.truss_edges) == (k, 3, 3)
     np.testing.assert_array_equal(ctx.truss_edges(), [[end, end + 1], [end, end + 2], [end + 1, end + 2]])
+
+
+@pytest.mark.parametrize("kept,m", [(300_000, 2_200_000), (540_000, 2_300_000)])
+def test_pruned_and_cut_again(ctx, kept, m):
+    """A filtered cut of 2^22 row slots and more, pruned with the bitmap of its
+    vertices in LDS (up to 524,288 of them) or in memory, and, where enough of
+    its vertices hang by fewer than k neighbours, cut a second time."""
+    rng = np.random.default_rng(kept)
+    n = 4 * kept + 4096
+    hubs = 48  # a clique: the h-index is at least 48, the filter's k 4 or so
+    core = kept // 2  # joined at random among themselves; the others have a star's centre and two more
+    e = [rng.integers(hubs, core, (m, 2))]
+    leaf = np.arange(core, kept)
+    e.append(np.column_stack([leaf, rng.integers(hubs, core, len(leaf))]))
+    e += [np.column_stack([leaf, kept + (leaf * 3 + d) % (n - kept)]) for d in range(5)]
+    u, v = np.triu_indices(hubs, 1)
+    e.append(np.column_stack([u, v]))
+    e.append(np.column_stack([np.arange(hubs), hubs + np.arange(hubs)]))
+    e = np.concatenate(e)
+    pairs = np.unique(canon_pairs(e[e[:, 0] != e[:, 1]].astype(np.uint32)), axis=0)
+    print(f"[gpu] {len(pairs)} edges", flush=True)
+    ref = O.solve_pairs(pairs, n, want_edges=True)
+    r = ctx.solve_pairs(pairs, n)
+    assert (r.max_core, r.k_hat, r.kmax, r.truss_edges) == (ref.max_core, ref.k_hat, ref.kmax, ref.truss_edges)
+    np.testing.assert_array_equal(ctx.truss_edges(), canon_pairs(ref.truss))
