@@ -252,7 +252,7 @@ def plain_line(args) -> dict:
     count_s = stages["ms_count_kernel"] / 1e3
     if st.count_kernel == 2:
         words = st.core_words
-        if st.m_core * words > 15e6 + st.n_core ** 2 / 24 * words:  # by all pairs of rows
+        if st.count_by_pairs:
             kernel = "k_dense_count"
             blocks = -(-st.n_core // 128)
             cbytes = blocks * (blocks + 1) // 2 * 256 * words * 8 + 4 * st.m_core

@@ -71,7 +71,7 @@ typedef struct kt_stats {
   uint32_t count_kernel;  /* pass-2 support count: 0 LDS bitmap, 1 per edge, 2 bit matrix */
   uint32_t core_words;    /* bit-matrix row words (count_kernel 2) */
   uint32_t vertex_rounds; /* the last vertex peel: 0 core numbers or one cascade launch, 1 synchronous rounds */
-  uint32_t pad;
+  uint32_t count_by_pairs; /* count_kernel 2: 1 when counted by all pairs of rows on the matrix cores, 0 by edge */
 } kt_stats;
 
 /* Library and device */

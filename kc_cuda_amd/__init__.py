@@ -65,7 +65,7 @@ class KtStats(ctypes.Structure):
                 ("m_core", ctypes.c_uint64), ("w_core", ctypes.c_uint64),
                 ("w_peeled", ctypes.c_uint64), ("truss_edges", ctypes.c_uint64),
                 ("count_kernel", ctypes.c_uint32), ("core_words", ctypes.c_uint32),
-                ("vertex_rounds", ctypes.c_uint32), ("pad", ctypes.c_uint32)]
+                ("vertex_rounds", ctypes.c_uint32), ("count_by_pairs", ctypes.c_uint32)]
 
     def as_dict(self) -> dict:
         return {name: getattr(self, name) for name, _ in self._fields_}

@@ -169,23 +169,24 @@ class Solver {
   void check_truss_count();
   // Truss decomposition of the last input graph: (u, v, t) with u < v for
   // every edge of trussness t >= 3 (the others have 2), sorted by (u, v);
-  // returns the count, copies at most cap triples. Replaces the last solve's
-  // survivors (truss_edges fails afterwards).
+  // returns the count, copies at most cap triples. The last solve's survivors
+  // are saved first (truss_edges goes on giving them; last_stats fails).
   uint64_t trussness(uint32_t* host_triples, uint64_t cap);
   // Byte-model terms of the last pass-2 core.
   void last_stats(kt_stats* out);
   // Stage access for parity tests: device CSR of the last solve.
   void csr_to_host(uint64_t* off, uint32_t* adj);
   void set_lanes(int count_lanes, int peel_lanes) { lanes_count_ = count_lanes; lanes_peel_ = peel_lanes; }
-  // Measurement of the vertex-peel push kernel: mode bit 1 stamps events at
-  // each launch's start and end, bit 2 counts the light row slots it walks
-  // and the vertices it takes (separate solves keep the counters' atomics
-  // out of the timing); push_stats sums them since set_push_probe.
+  // Measurement of the vertex peel (the sweeps for core numbers; a cascade or
+  // the push of a round where a peel runs): mode bit 1 stamps events at each
+  // launch's start and end, bit 2 counts the row slots it walks and the vertices
+  // it takes, of the sweeps over a level the first one's (separate solves keep
+  // the counters' atomics out of the timing); push_stats sums them since
+  // set_push_probe.
   void set_push_probe(int mode) { set_probe(kProbeVertexPeel, mode); }
-  // kernel: kProbeVertexPeel (the vertex-peel cascade, or the push of its
-  // rounds) or kProbeDensePeel (the bit-matrix edge-peel round); for the
-  // latter the counters are the frontier edges' d+(u) + d+(v) and their
-  // number.
+  // kernel: kProbeVertexPeel or kProbeDensePeel (the truss-level step of
+  // bit-matrix cores); for the latter the counters are the frontier edges' d+(u)
+  // + d+(v) and their number.
   static constexpr int kProbeVertexPeel = 0;
   static constexpr int kProbeDensePeel = 1;
   void set_probe(int kernel, int mode);
@@ -372,6 +373,7 @@ class Solver {
   bool peeled_by_rows_ = false;
   bool walks_ = true;  // the search over triangle lists has frontiers to walk
   uint32_t count_kind_ = 0, count_words_ = 0;  // the last timed support count
+  bool count_by_pairs_ = false;
   uint32_t walk_levels_ = 16;
   uint64_t split_build_min_ = uint64_t(1) << 22;  // fewest pairs of the build by two splits (see split_plan)
   uint32_t build_tiles_ = 4096;  // most tiles of the partitioned CSR build

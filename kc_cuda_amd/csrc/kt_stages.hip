@@ -838,9 +838,11 @@ void Solver::count_support(CoreView* cv, float* ms) {
   const int lanes = lanes_count_ ? lanes_count_ : auto_lanes(avg);
   KT_HIP(hipEventRecord(ev_[8], stream_));
   uint32_t kind = 1;
+  bool by_pairs = false;
   if (cv->dense) {
     kind = 2;
-    if (!cv->repeats && dense_by_pairs(cv->nc, cv->mc, cv->ws))
+    by_pairs = !cv->repeats && dense_by_pairs(cv->nc, cv->mc, cv->ws);
+    if (by_pairs)
       dense_count(cv->bits, cv->pref0, cv->off_u, cv->eid_u, cv->eidm, cv->nc, cv->ws, cv->sup, stream_);
     else
       dense_support(cv->off_d, cv->adj_d, cv->nc, cv->mc, cv->bits, cv->ws, nullptr, cv->sup, stream_);
@@ -855,6 +857,7 @@ void Solver::count_support(CoreView* cv, float* ms) {
     KT_HIP(hipEventElapsedTime(ms, ev_[8], ev_[9]));
     count_kind_ = kind;
     count_words_ = cv->dense ? cv->ws : 0;
+    count_by_pairs_ = by_pairs;
   }
 }
 
@@ -1430,6 +1433,7 @@ void Solver::last_stats(kt_stats* out) {
   out->n_core = cv.nc0;
   out->count_kernel = count_kind_;
   out->core_words = count_words_;
+  out->count_by_pairs = count_by_pairs_ ? 1u : 0u;
   out->vertex_rounds = vertex_rounds_ ? 1u : 0u;
   out->m_core = cv.mc0;
   out->truss_edges = last_truss_;
