@@ -423,8 +423,10 @@ bool Solver::max_core_numbers(bool allow_cut, bool fresh, uint32_t* k, uint32_t*
   depth_ = 1;
   if (fresh) fill_u32(g0.lvl, g0.n, kNone, stream_);
   *hi = 0;
-  est_whole_ = true;
-  return g0.slots <= kCoreWholeSlots && core_numbers(g0, 1, k, hi);
+  if (g0.slots > kCoreWholeSlots) return false;
+  if (core_numbers(g0, 1, k, hi)) return true;
+  est_whole_ = *hi != 0;  // (0: cut off at 16 bits)
+  return false;
 }
 
 // The largest k with a non-empty k-core (0: no edges); leaves the max-core
@@ -493,7 +495,10 @@ uint32_t Solver::max_core_gallop(bool allow_cut, bool fresh, uint32_t hi) {
   }
   uint32_t k = 1, step = 16;
   uint64_t alive = 0;
-  if (!(allow_cut && fresh && filtered_start(&g, &k, &alive))) {
+  // what the sweeps over the whole graph left (a filter's cut, which found no
+  // core before them, would reuse it)
+  const uint32_t* est = est_whole_ ? keys_.as<uint32_t>() : nullptr;
+  if (!(allow_cut && fresh && !est && filtered_start(&g, &k, &alive))) {
     const uint64_t gone = peel_vertices(*g, 1);
     if (gone >= before) return 0;
     alive = before - gone;
@@ -502,8 +507,6 @@ uint32_t Solver::max_core_gallop(bool allow_cut, bool fresh, uint32_t hi) {
     if (allow_cut && alive * 4 <= g->n && alive >= kMinCut) g = &cut_level(*g, 1, uint32_t(alive));
   }
   bool grow = true, slow = hi != 0, tried = slow;
-  // what the sweeps over the whole graph left (a filter's cut has reused it)
-  const uint32_t* est = hi && depth_ == 1 && est_whole_ ? keys_.as<uint32_t>() : nullptr;
   while (step > 0 && (!hi || k + 1 < hi)) {
     if (vertex_mode_ == 0 && mirrored_ && depth_ > 1 && !tried && g->slots <= kCoreWholeSlots) {
       uint32_t top = 0, bound = 0;

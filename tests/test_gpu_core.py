@@ -177,3 +177,19 @@ def test_pruned_and_cut_again(ctx, kept, m):
     r = ctx.solve_pairs(pairs, n)
     assert (r.max_core, r.k_hat, r.kmax, r.truss_edges) == (ref.max_core, ref.k_hat, ref.kmax, ref.truss_edges)
     np.testing.assert_array_equal(ctx.truss_edges(), canon_pairs(ref.truss))
+
+
+def test_bounds_of_the_whole_graph_after_filters_without_a_core(ctx):
+    """Stars raise the degree h-index, whose filters leave no core; the path
+    keeps the whole graph's sweeps from converging, so the peel starts from its
+    estimates."""
+    stars, leaves, path, clique = 120, 140, 150_000, 7
+    base = clique + path  # after the clique with its tail
+    centre = base + np.arange(stars) * (leaves + 1)
+    e = [_lollipop(path, clique).astype(np.int64),
+         np.column_stack([np.repeat(centre, leaves), (centre[:, None] + 1 + np.arange(leaves)).ravel()]),
+         np.column_stack([centre[:-1], centre[1:]])]
+    pairs = canon_pairs(np.concatenate(e).astype(np.uint32))
+    r = ctx.solve_pairs(pairs, int(pairs.max()) + 1)
+    assert (r.max_core, r.kmax, r.truss_edges) == (6, 7, 21)
+    np.testing.assert_array_equal(ctx.truss_edges(), _lollipop(0, clique))
