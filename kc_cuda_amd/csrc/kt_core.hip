@@ -763,6 +763,12 @@ __global__ __launch_bounds__(kBlock) void k_core_est_prune(const uint32_t* __res
   if (lane64() == 0 && c) atomicAdd(removed, c);
 }
 
+__global__ __launch_bounds__(kBlock) void k_core_clear_removed(const uint32_t* __restrict__ lvl, uint32_t n,
+                                                               uint32_t* __restrict__ deg) {
+  for (uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < n; v += uint64_t(gridDim.x) * blockDim.x)
+    if (lvl[v] != kNone) deg[v] = 0;
+}
+
 }  // namespace
 
 // --------------------------------------------------------------- wrappers ---
@@ -868,6 +874,9 @@ void core_est_max(const CoreEst& a, uint32_t* out, hipStream_t s) {
 
 void core_est_prune(const uint32_t* est, uint32_t n, uint32_t k, uint32_t* lvl, uint32_t* removed, hipStream_t s) {
   if (n) k_core_est_prune<<<std::min(grid_for(n), 1024), kBlock, 0, s>>>(est, n, k, lvl, removed);
+}
+void core_clear_removed(const uint32_t* lvl, uint32_t n, uint32_t* deg, hipStream_t s) {
+  if (n) k_core_clear_removed<<<std::min(grid_for(n), 4096), kBlock, 0, s>>>(lvl, n, deg);
 }
 void core_est_apply(const CoreEst& a, const uint32_t* top, uint32_t* lvl, hipStream_t s) {
   k_core_est_apply<<<std::min(grid_for(a.n), 4096), kBlock, 0, s>>>(a.est, a.n, a.floor, top, lvl);

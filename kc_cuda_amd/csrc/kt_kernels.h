@@ -113,8 +113,10 @@ void core_est_init(const CoreEst& a, const uint32_t* deg, const uint32_t* lvl, i
 void core_est_steps(CoreEst* a, int lanes, uint32_t count, hipStream_t s, unsigned long long* stats, hipEvent_t* ev);
 void core_est_max(const CoreEst& a, uint32_t* out, hipStream_t s);
 // alive vertices of an estimate below k are stamped removed at k; *removed (starts
-// at 0) += how many
+// at 0) += how many. clear_removed: deg = 0 for every vertex that is not alive: a
+// peel must not see one that was stamped without being peeled reach k
 void core_est_prune(const uint32_t* est, uint32_t n, uint32_t k, uint32_t* lvl, uint32_t* removed, hipStream_t s);
+void core_clear_removed(const uint32_t* lvl, uint32_t n, uint32_t* deg, hipStream_t s);
 void core_est_apply(const CoreEst& a, const uint32_t* top, uint32_t* lvl, hipStream_t s);
 // The whole of it for a small level (core_small_fits) in one launch: lvl as
 // after apply, deg of the max core's vertices = their degree in it; out[0] =

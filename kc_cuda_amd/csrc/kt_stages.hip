@@ -274,7 +274,7 @@ uint32_t Solver::degree_hindex(const LevelGraph& g0) {
 // Whole solves in ms, by a galloping peel alone, by sweeps given up after 512,
 // and so: a path of 3 k vertices 5.0, 12.4, 5.1; of 10 k 15.5, 26.7, 15.4; a
 // clique with a tail of 3 k 0.94, 5.7, 0.69; grids of 200^2 7.1, 2.9, 2.7; of
-// 600^2 79.5, 90.4, 16.7; of 1,000^2 185, 202, 65; triangulated 365, 363, 119.
+// 600^2 79.5, 90.4, 16.0; of 1,000^2 185, 202, 101; triangulated 365, 363, 148.
 bool Solver::core_numbers(LevelGraph& g, uint32_t floor, uint32_t* top, uint32_t* hi) {
   constexpr uint32_t kBatch = 16, kMaxBatch = 32, kCoreSweeps = 512, kOutWords = kMaxBatch + 5;
   const uint32_t n = g.n;
@@ -531,7 +531,10 @@ uint32_t Solver::max_core_gallop(bool allow_cut, bool fresh, uint32_t hi) {
       zero_u32(&ctl_->nalive);
       core_est_prune(est, g->n, kk, g->lvl, &ctl_->nalive, stream_);
       core_alive_degrees(g->off, g->adj, g->lvl, g->n, g->deg, heavy(), stream_);
+      core_clear_removed(g->lvl, g->n, g->deg, stream_);
       removed = read_u32(&ctl_->nalive);
+      if (trace_) std::fprintf(stderr, "[kt] estimates below k=%u: %llu of %llu\n", kk, (unsigned long long)removed,
+                               (unsigned long long)alive);
     }
     if (removed < alive) removed += peel_vertices(*g, kk, alive - removed);  // an overshoot is restored below
     if (removed < alive) {
@@ -579,6 +582,7 @@ void Solver::core_at(uint32_t k) {
   if (exact) kj = k;
   core_reopen_above(g.lvl, g.n, kj, stream_);
   core_alive_degrees(g.off, g.adj, g.lvl, g.n, g.deg, heavy(), stream_);
+  if (exact && g.loose) core_clear_removed(g.lvl, g.n, g.deg, stream_);
   if (k > kj || (exact && g.loose)) peel_vertices(g, k);
   // stamps at or below k are untouched; above k they are gone
   if (exact)

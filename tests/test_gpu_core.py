@@ -115,12 +115,27 @@ def _ladder_into_expander(columns, n):
     return np.unique(canon_pairs(e.astype(np.uint32)), axis=0), n + 2 * columns
 
 
+def _star_and_tail(leaves, path):
+    """A star on the end of a path that leads out of a ring with a chord: the
+    ring is the 2-core."""
+    ring = 104
+    i = np.arange(ring)
+    walk = ring - 1 + np.arange(path + 1)
+    hub = int(walk[-1])
+    e = np.concatenate([np.column_stack([i, (i + 1) % ring]), [[0, 2]], np.column_stack([walk[:-1], walk[1:]]),
+                        np.column_stack([np.full(leaves, hub), hub + 1 + np.arange(leaves)])])
+    return canon_pairs(e.astype(np.uint32)), hub + 1 + leaves
+
+
 LONG = {
     # one workgroup from the start, from the first sweeps on, from later ones on; peel with bounds
     "grid_20": lambda: _grid(20, False), "mesh_40": lambda: _grid(40, True), "grid_70": lambda: _grid(70, False),
     "mesh_150": lambda: _grid(150, True), "grid_256": lambda: _grid(256, False), "grid_257": lambda: _grid(257, False),
     "grid_640": lambda: _grid(640, False), "mesh_560": lambda: _grid(560, True),
     "path_4096": lambda: (_lollipop(4089, 7), 4096), "path_65536": lambda: (_lollipop(65_529, 7), 65_536),
+    # long rows beside the path: the peel goes on from the estimates
+    "star_150": lambda: _star_and_tail(150, 9000), "star_9000": lambda: _star_and_tail(9000, 12_000),
+    "star_20000": lambda: _star_and_tail(20_000, 60_000),
     # more vertices due at once than one workgroup lists
     "expander": lambda: _ladder_into_expander(300, 60_000),
 }
