@@ -270,8 +270,12 @@ __global__ __launch_bounds__(kRowsBlock) void k_group_rows(const uint2* __restri
 // -> 10.8 (two counts 1.4, splits 3.2 and 2.5, rows 3.5; 2.7 to 3.5 TB/s). It
 // is taken from 2^22 pairs on, shuffled ones too: 2^21 0.158 -> 0.186, 2^22
 // 0.288 -> 0.255, 2^23 0.525 -> 0.385, 2^25 2.67 -> 1.43.
-// Groups of as many rows as average 6,144 slots or fewer (the stage takes
-// 8,192), split by at most nine bits twice.
+// Groups of as many rows, a power of two, as average 6,144 slots or fewer (the
+// stage takes 8,192), split by at most nine bits twice, so at most 2^18 of them.
+// That holds for every vertex count up to 134 M with up to 400 M pairs; with 505
+// M pairs for 70 % of the counts from 5 to 130 M (50 M: 195 k groups; 20, 35, 40
+// and 42 M: 273 k to 328 k, which take the bucketed build and its 19 ms), with
+// 600 M for 44 %.
 bool split_plan(uint32_t n, uint64_t pairs, bool sorted, SplitPlan* p) {
   p->sorted = sorted;
   p->entries = sorted ? pairs : 2 * pairs;

@@ -17,8 +17,9 @@ double ms_between(std::chrono::steady_clock::time_point a, std::chrono::steady_c
 // buffers, the vertex-peel nest's subgraphs, and for every core edge its
 // oriented and undirected slots with edge ids, support, state, deletion
 // level, queues, triangle lists, backups and both compaction sets (160 B in all;
-// measured at most 96 B on serving and batch mixes and RMAT scale 22, pairs in
-// no order 8 B more, and 24 from 2^22 on if the core has no lists); per vertex
+// measured at most 96 B on serving and batch mixes and RMAT scale 22, 130 on a
+// lattice that is all core with lists of 36 B an edge; pairs in no order 8 B
+// more, and 24 from 2^22 on if the core has no lists); per vertex
 // offsets, degrees, levels and maps (64 B); a dense core's bit rows (at most
 // 72 B per edge, since a row is no longer than two sorted rows) and its
 // edge-id matrix (at most kServeEidmBytes); 16 MiB of fixed buffers.
